@@ -36,9 +36,7 @@ struct Engine {
     int ldz = 0;          // device z pitch: nz rounded up to a multiple of 32 cells (128 bytes)
     long long nxz = 0;    // nx * ldz, the device size of one field
     int tile_x = 16, ntx = 0, ntz = 0;
-    std::vector<int4> boxes;                        // {sx, ex, sz, ez} of every step box
-    std::vector<int> list_core, list_bz, list_bz8, list_bx;  // box indices per box class
-    DevMem d_boxes, d_list_core, d_list_bz, d_list_bz8, d_list_bx;
+    int itx0 = 0, itx1 = 0, itz0 = 0, itz1 = 0;  // rectangle of tiles with interior cells only
     int opt_tile_x = 16, opt_segment = 0, opt_lag = 1, opt_graph = 0, opt_timing = 0;
     long long opt_ckpt_budget_mb = 0;  // device memory for checkpoints and snapshot slots; 0: sqrt scheme
     // hipGraph replay of whole time loops: a loop is captured once per configuration
@@ -60,11 +58,12 @@ struct Engine {
     int opt_autotune = 0;  // pick tile_x and shots per workgroup by timing steps at the next forward run
     bool tuned = false;
     std::string tune_report;
-    int opt_spb = 8;       // shots advanced one after the other by each core-box workgroup
-    int opt_spb_edge = 1;  // the same for edge tiles (their workgroups are latency-bound)
-    int opt_spb_edge_img = 0;  // edge tiles of adjoint steps with the imaging fused in (0: opt_spb_edge)
-    int opt_band_rows = 8;     // rows of the top band (the bottom band: 8-11 more than band_rows - 8)
-    int opt_spb_img = 0;   // shots per imaging workgroup (0: 4, or opt_spb when fused)
+    // shots advanced one after the other by each workgroup of an interior tile and of a frame
+    // tile (step_groups); 0: automatic
+    int opt_spb = 0, opt_spb_edge = 0;
+    int opt_spb_edge_img = 0;  // frame tiles of adjoint steps with the imaging fused in (0: as opt_spb_edge)
+    int opt_band_rows = 8;     // accepted and kept for callers that set it; the step has no bands
+    int opt_spb_img = 0;   // shots per imaging workgroup (0: up to 4, or as the step when fused)
     // 1: imaging condition fused into the adjoint step kernels (by parts in time, sub = 1);
     // 0: the imaging kernel after each adjoint step; -1: fused on isotropic grids, where it
     // is faster (the VTI fused kernels exceed the register file)
@@ -73,9 +72,7 @@ struct Engine {
     int opt_img_buffers = 1;  // LDS window buffers of the imaging kernel (1 or 2)
     int opt_img_stream = 1;   // 1: imaging kernel on its own stream beside the next step
     int opt_img_sbp = 1;      // 1: density term by parts in time (sub = 1, separate imaging)
-    int opt_edge_stream = 1;  // edge-band launches on their own stream (1: before the core launch, 2: after)
-    hipStream_t st_edge = nullptr;       // edge-tile launches run beside the interior ones
-    hipEvent_t ev_fork = nullptr, ev_join = nullptr;
+    int opt_edge_stream = 1;  // accepted and kept for callers that set it: a step is one launch
     // imaging of adjoint step it runs on st_img beside step it+1; step it+2 (which
     // overwrites level it) and any recompute (which overwrites snapshot slots) wait for it
     hipStream_t st_img = nullptr;
@@ -86,7 +83,7 @@ struct Engine {
     int last_fwd_loop_steps = 0;
     bool vti = false;
 
-    DevMem d_model, d_deriv, d_div_tb, d_div_lr, d_tx, d_tz;
+    DevMem d_model, d_deriv, d_closure, d_div_tb, d_div_lr, d_tx, d_tz;
     std::vector<float> h_model, h_deriv;  // h_deriv: dt^2/rho[, (1+2eps) mu, (1+2eps) lambda], [nd][nx][nz]
     long long model_epoch = 0, ckpt_epoch = -1;
 
@@ -129,9 +126,6 @@ struct Engine {
         if (nxz >= (1LL << 31)) throw std::runtime_error("grid too large: nx * nz must stay below 2^31 cells");
         HIPCHECK(hipSetDevice(device));
         HIPCHECK(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
-        HIPCHECK(hipStreamCreateWithFlags(&st_edge, hipStreamNonBlocking));
-        HIPCHECK(hipEventCreateWithFlags(&ev_fork, hipEventDisableTiming));
-        HIPCHECK(hipEventCreateWithFlags(&ev_join, hipEventDisableTiming));
         HIPCHECK(hipStreamCreateWithFlags(&st_img, hipStreamNonBlocking));
         HIPCHECK(hipEventCreateWithFlags(&ev_img_in, hipEventDisableTiming));
         for (auto& e : ev_img_done) HIPCHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
@@ -145,10 +139,6 @@ struct Engine {
             (void)hipStreamSynchronize(st);
             (void)hipStreamDestroy(st);
         }
-        if (st_edge) {
-            (void)hipStreamSynchronize(st_edge);
-            (void)hipStreamDestroy(st_edge);
-        }
         if (st_img) {
             (void)hipStreamSynchronize(st_img);
             (void)hipStreamDestroy(st_img);
@@ -158,8 +148,6 @@ struct Engine {
             if (e) (void)hipEventDestroy(e);
         graph_fwd.reset();
         graph_adj.reset();
-        if (ev_fork) (void)hipEventDestroy(ev_fork);
-        if (ev_join) (void)hipEventDestroy(ev_join);
     }
 
     void set_tile(int tx)
@@ -168,77 +156,25 @@ struct Engine {
         tile_x = tx;
         ntx = tiles_x(g.nx, tile_x);
         ntz = tiles_z(ldz);
-        build_boxes();
-    }
-
-    // Step decomposition: the core [6, nx-6) x [8, core_z_end) where every stencil is
-    // interior, cut into tile_x x 64 boxes (the tile grid clipped to the core), and the
-    // edge bands around it: 120 x 8 / 64 x 16 boxes along the top and bottom (corners included),
-    // 8 x 128 boxes along the left and right sides.  Boxes partition the grid.  The
-    // band_rows option moves the core's top and bottom by band_rows - 8 rows into the
-    // grid (thicker bands in 64 x 16 boxes).
-    void build_boxes()
-    {
-        boxes.clear();
-        list_core.clear();
-        list_bz.clear();
-        list_bz8.clear();
-        list_bx.clear();
-        const int nx = g.nx, nz = g.nz;
-        const int cx0 = kCoreX0, cx1 = nx - kCoreX0;
-        const int cz0 = std::min(kCoreZ0 + (opt_band_rows - 8), nz);
-        const int cz1 = std::min(std::max(core_z_end(nz) - (opt_band_rows - 8), cz0), nz);
-        auto add = [&](std::vector<int>& list, int sx, int ex, int sz, int ez) {
-            if (ex <= sx || ez <= sz) return;
-            list.push_back((int)boxes.size());
-            boxes.push_back(make_int4(sx, ex, sz, ez));
-        };
-        for (int tix = 0; tix < ntx; tix++) {
-            int sx, ex;
-            tile_range_x(tix, ntx, tile_x, nx, sx, ex);
-            for (int tiz = 0; tiz < ntz; tiz++) {
-                int sz, ez;
-                tile_range_z(tiz, ntz, nz, ldz, sz, ez);
-                add(list_core, std::max(sx, cx0), std::min(ex, cx1), std::max(sz, cz0), std::min(ez, cz1));
-            }
+        // the tiles whose cells all lie 6 or more cells from every side: no closure rows, no
+        // SAT terms
+        itx0 = itx1 = itz0 = itz1 = 0;
+        for (int k = 0, b, e; k < ntx; k++) {
+            tile_range_x(k, ntx, tile_x, g.nx, b, e);
+            if (b < 6 || e > g.nx - 6) continue;
+            if (itx1 == 0) itx0 = k;
+            itx1 = k + 1;
         }
-        // top and bottom bands: 8-row bands in 120 x 8 boxes, taller ones (the bottom band
-        // holds 8 to 11 rows with the default band_rows) in 64 x 16 boxes; a band of more
-        // than 16 rows in rows of boxes split evenly (8 to 16 rows each).  Only a box at the
-        // grid's top or bottom takes the thin class, whose compact window serves no other.
-        auto zband = [&](int sz0, int ez) {
-            const int n = ez - sz0, nchunk = (n + 15) / 16;
-            for (int c = 0; c < nchunk; c++) {
-                const int sz = sz0 + n * c / nchunk, e = sz0 + n * (c + 1) / nchunk;
-                const bool thin = e - sz <= 8 && (sz == 0 || e == nz);
-                const int w = thin ? kBandZ8Width : 64;
-                const int nb = (nx + w - 1) / w;
-                for (int k = 0; k < nb; k++) {
-                    int sx, ex;
-                    tile_range_x(k, nb, w, nx, sx, ex);
-                    add(thin ? list_bz8 : list_bz, sx, ex, sz, e);
-                }
-            }
-        };
-        zband(0, cz0);
-        zband(cz1, nz);
-        for (int sz = cz0; sz < cz1; sz += 128) {
-            const int ez = std::min(sz + 128, cz1);
-            add(list_bx, 0, cx0, sz, ez);
-            add(list_bx, cx1, nx, sz, ez);
+        for (int k = 0, b, e; k < ntz; k++) {
+            tile_range_z(k, ntz, g.nz, ldz, b, e);
+            if (b < 6 || e > g.nz - 6) continue;
+            if (itz1 == 0) itz0 = k;
+            itz1 = k + 1;
         }
-        auto up = [&](DevMem& d, const void* h, size_t b) {
-            d.reserve(std::max<size_t>(b, 16));
-            if (b) HIPCHECK(hipMemcpyAsync(d.p, h, b, hipMemcpyHostToDevice, st));
-        };
-        up(d_boxes, boxes.data(), boxes.size() * sizeof(int4));
-        up(d_list_core, list_core.data(), list_core.size() * sizeof(int));
-        up(d_list_bz, list_bz.data(), list_bz.size() * sizeof(int));
-        up(d_list_bz8, list_bz8.data(), list_bz8.size() * sizeof(int));
-        up(d_list_bx, list_bx.data(), list_bx.size() * sizeof(int));
-        HIPCHECK(hipStreamSynchronize(st));
+        if (itx1 == 0 || itz1 == 0) itx0 = itx1 = itz0 = itz1 = 0;
     }
-    int ntiles() const { return (int)boxes.size(); }
+    int ntiles() const { return ntx * ntz; }
+    int interior_tiles() const { return (itx1 - itx0) * (itz1 - itz0); }
 
     // cos^2 taper factors per axis (taperz/taperx, spatial_operators.cpp:523-549)
     void build_tapers()
@@ -333,7 +269,7 @@ struct Engine {
             scale((long long)(nx - 1) * nz, sc2x, sc2z);
         }
         // perimeter arrays: top row and bottom row (corners included), left and right columns
-        std::vector<float> tb(4 * (size_t)nx), lr(4 * (size_t)nz);
+        std::vector<float> tb(4 * (size_t)nx), lr(4 * (size_t)ldz, 1.f);
         for (int ix = 0; ix < nx; ix++) {
             tb[ix] = (float)dvx[(long long)ix * nz];
             tb[nx + ix] = (float)dvz[(long long)ix * nz];
@@ -342,9 +278,9 @@ struct Engine {
         }
         for (int iz = 0; iz < nz; iz++) {
             lr[iz] = (float)dvx[iz];
-            lr[nz + iz] = (float)dvz[iz];
-            lr[2 * nz + iz] = (float)dvx[(long long)(nx - 1) * nz + iz];
-            lr[3 * nz + iz] = (float)dvz[(long long)(nx - 1) * nz + iz];
+            lr[ldz + iz] = (float)dvz[iz];
+            lr[2 * ldz + iz] = (float)dvx[(long long)(nx - 1) * nz + iz];
+            lr[3 * ldz + iz] = (float)dvz[(long long)(nx - 1) * nz + iz];
         }
         d_div_tb.reserve(tb.size() * sizeof(float));
         d_div_lr.reserve(lr.size() * sizeof(float));
@@ -393,7 +329,50 @@ struct Engine {
         HIPCHECK(hipMemcpy2DAsync(d_deriv.p, (size_t)ldz * sizeof(float), h_deriv.data(), (size_t)g.nz * sizeof(float),
                                   (size_t)g.nz * sizeof(float), (size_t)nd * g.nx, hipMemcpyHostToDevice, st));
         build_divisors();
+        build_closures();
         model_epoch++;
+    }
+
+    // D2 closure rows of the model (layout in StepArgs: wx[, wxx], wz): the weight of field
+    // point j in row r is the sum over the table's entries (r, j, k) of coefficient times
+    // model value at point k, formed in double, times 1 / h^2
+    void build_closures()
+    {
+        const int nx = g.nx, nz = g.nz;
+        const size_t nwx = (size_t)2 * 6 * 8 * ldz, nwz = (size_t)2 * nx * 6 * 8;
+        std::vector<float> w((vti ? 2 : 1) * nwx + nwz, 0.f);
+        const long long nc = (long long)nx * nz;
+        const double rdx2 = 1.0 / (g.dx * g.dx), rdz2 = 1.0 / (g.dz * g.dz);
+        std::vector<double> acc(nz);
+        for (int f = 0; f < (vti ? 2 : 1); f++) {
+            const float* c = f ? h_deriv.data() + nc : h_model.data() + nc;  // (1 + 2 eps) mu, mu
+            for (int side = 0; side < 2; side++)
+                for (int r = 0; r < 6; r++)
+                    for (int j = 0; j < 8; j++) {
+                        std::fill(acc.begin(), acc.end(), 0.0);
+                        for (const D2Entry& e : kD2ClosureNZ)
+                            if (e.row == r && e.point == j) {
+                                const float* p = c + (long long)(side ? nx - 1 - e.coef : e.coef) * nz;
+                                for (int iz = 0; iz < nz; iz++) acc[iz] += e.num / e.den * p[iz];
+                            }
+                        float* o = w.data() + f * nwx + ((size_t)(side * 6 + r) * 8 + j) * ldz;
+                        for (int iz = 0; iz < nz; iz++) o[iz] = (float)(acc[iz] * rdx2);
+                    }
+        }
+        const float* mu = h_model.data() + nc;
+        float* wz = w.data() + (vti ? 2 : 1) * nwx;
+        for (int side = 0; side < 2; side++)
+            for (int ix = 0; ix < nx; ix++) {
+                double v[8][6] = {};
+                const float* p = mu + (long long)ix * nz + (side ? nz - 1 : 0);
+                for (const D2Entry& e : kD2ClosureNZ)
+                    v[e.point][e.row] += e.num / e.den * p[side ? -(int)e.coef : e.coef];
+                for (int j = 0; j < 8; j++)
+                    for (int r = 0; r < 6; r++) wz[(((size_t)side * nx + ix) * 6 + r) * 8 + j] = (float)(v[j][r] * rdz2);
+            }
+        d_closure.reserve(w.size() * sizeof(float));
+        HIPCHECK(hipMemcpyAsync(d_closure.p, w.data(), w.size() * sizeof(float), hipMemcpyHostToDevice, st));
+        HIPCHECK(hipStreamSynchronize(st));
     }
 
     // ------------------------------------------------------------------
@@ -538,6 +517,29 @@ struct Engine {
     // ------------------------------------------------------------------
     long long state_stride() const { return (long long)ns * 2 * nxz; }  // one time level of all shots
 
+    // Shots per workgroup unless set: as many as keep 2048 workgroups in the launch (two
+    // rounds of 4 per CU), up to 8: a group reads its tile's model once, but a small launch
+    // wants its shots spread over the chip.
+    int spb_auto(int most) const { return (int)std::max(1LL, std::min<long long>(most, (long long)ntiles() * ns / 2048)); }
+    int spb() const { return std::max(1, std::min(opt_spb > 0 ? opt_spb : spb_auto(8), std::max(ns, 1))); }
+    int spb_edge() const
+    {
+        return std::max(1, std::min(opt_spb_edge > 0 ? opt_spb_edge : spb_auto(8), std::max(ns, 1)));
+    }
+    // shots per imaging workgroup: the separate kernel is fastest with small groups (more
+    // workgroups in flight; measured 4 < 16 < 64 at 64 shots)
+    int spb_img(bool fused) const
+    {
+        return std::max(1, std::min(opt_spb_img > 0 ? opt_spb_img : (fused ? spb() : spb_auto(4)), ns));
+    }
+    void set_groups(StepArgs& a, int n, int n_edge) const
+    {
+        a.spb = n;
+        a.ngroups = (ns + n - 1) / n;
+        a.spb_e = n_edge;
+        a.ngroups_e = (ns + n_edge - 1) / n_edge;
+    }
+
     StepArgs base_args() const
     {
         StepArgs a{};
@@ -574,8 +576,16 @@ struct Engine {
         a.irho = dv;
         a.mux = vti ? dv + nxz : nullptr;
         a.lamx = vti ? dv + 2 * nxz : nullptr;
-        a.spb = std::max(1, std::min(opt_spb, ns));
-        a.ngroups = (ns + a.spb - 1) / a.spb;
+        a.itx0 = itx0;
+        a.itx1 = itx1;
+        a.itz0 = itz0;
+        a.itz1 = itz1;
+        set_groups(a, spb(), spb_edge());
+        const float* cl = d_closure.as<float>();
+        const size_t nwx = (size_t)2 * 6 * 8 * ldz;
+        a.wx = cl;
+        a.wxx = vti ? cl + nwx : nullptr;
+        a.wz = cl + (vti ? 2 : 1) * nwx;
         a.div_tb = d_div_tb.as<float>();
         a.div_lr = d_div_lr.as<float>();
         a.taper_x = d_tx.as<float>();
@@ -655,11 +665,8 @@ struct Engine {
                 a.img_deriv = 1;
             }
             ia = a;
-            // shots per imaging workgroup: the separate kernel is fastest with small
-            // groups (more workgroups in flight; measured 4 < 16 < 64 at 64 shots)
-            const int spbi = opt_spb_img > 0 ? opt_spb_img : (fuse_img ? opt_spb : 4);
-            ia.spb = std::max(1, std::min(spbi, ns));
-            ia.ngroups = (ns + ia.spb - 1) / ia.spb;
+            const int n = spb_img(fuse_img);
+            set_groups(ia, n, fuse_img && opt_spb_edge_img > 0 ? std::min(opt_spb_edge_img, ns) : spb_edge());
             if (fuse_img) a = ia;
         }
         a.it = it;
@@ -676,29 +683,8 @@ struct Engine {
         if (rcv)
             launch_extract(L.C(), 2 * nxz, nxz, ldz, d_rcv_ext_ents.as<PointEntry>(), d_rcv_ext_ptr.as<int>(), nr, rcv,
                            it, st);
-        // edge bands on their own stream, concurrent with the core boxes (disjoint cells),
-        // or after them on the same stream
-        StepArgs e = a;
-        e.spb = std::max(1, std::min(fuse_img && opt_spb_edge_img > 0 ? opt_spb_edge_img : opt_spb_edge, ns));
-        e.ngroups = (ns + e.spb - 1) / e.spb;
         const bool img = fuse_img;
-        const int4* bx = d_boxes.as<int4>();
-        // edge_stream 1: bands enqueued before the core launch, 2: after it (they then fill
-        // the core launch's last, partial round of workgroups)
-        hipStream_t se = opt_edge_stream ? st_edge : st;
-        if (opt_edge_stream) HIPCHECK(hipEventRecord(ev_fork, st));
-        auto core = [&] {
-            launch_step(a, vti, tile_x == 32 ? BoxClass::core32 : BoxClass::core16, bx, d_list_core.as<int>(),
-                        (int)list_core.size(), img, st);
-        };
-        if (opt_edge_stream == 2) core();
-        if (opt_edge_stream) HIPCHECK(hipStreamWaitEvent(st_edge, ev_fork, 0));
-        launch_step(e, vti, BoxClass::band_z8, bx, d_list_bz8.as<int>(), (int)list_bz8.size(), img, se);
-        launch_step(e, vti, BoxClass::band_z, bx, d_list_bz.as<int>(), (int)list_bz.size(), img, se);
-        launch_step(e, vti, BoxClass::band_x, bx, d_list_bx.as<int>(), (int)list_bx.size(), img, se);
-        if (opt_edge_stream) HIPCHECK(hipEventRecord(ev_join, st_edge));
-        if (opt_edge_stream != 2) core();
-        if (opt_edge_stream) HIPCHECK(hipStreamWaitEvent(st, ev_join, 0));
+        launch_step(a, vti, tile_x, img, st);
         // point sources of this step into the new level
         const InjList& inj = adjoint ? inj_rcv : inj_src;
         InjImage im{};
@@ -845,18 +831,17 @@ struct Engine {
     {
         auto P = [](const void* p) { return (long long)(uintptr_t)p; };
         return {kind, P(p0), P(p1), flag, g.nt, ns, nr, tile_x, opt_spb, opt_spb_edge, opt_spb_edge_img, opt_lag, seg_K, nseg,
-                opt_bf16, opt_stiff, opt_edge_stream, opt_spb_img, opt_image_fused, opt_img_buffers, opt_img_stream, opt_img_sbp, P(d_ckpt16.p), P(d_ckpt_scale.p), P(d_amax.p),
+                opt_bf16, opt_stiff, opt_spb_img, opt_image_fused, opt_img_buffers, opt_img_stream, opt_img_sbp, P(d_ckpt16.p), P(d_ckpt_scale.p), P(d_amax.p),
                 P(d_fwd.p), P(d_adj.p), P(d_ckpt.p), P(d_seg.p), P(d_gshot.p), P(d_model.p), P(d_deriv.p),
-                P(d_boxes.p), P(d_list_core.p), P(d_list_bz.p), P(d_list_bz8.p), P(d_list_bx.p), P(inj_src.d_cells.p), P(inj_src.d_ptr.p),
+                P(d_closure.p), P(inj_src.d_cells.p), P(inj_src.d_ptr.p),
                 P(inj_src.d_ctx.p), P(inj_src.d_ctz.p), P(inj_src.d_cw.p), P(inj_rcv.d_cells.p), P(inj_rcv.d_ptr.p),
                 P(inj_rcv.d_ctx.p), P(inj_rcv.d_ctz.p), P(d_rcv_ext_ptr.p), src_nc,
                 P(inj_rcv.d_cw.p), (long long)inj_src.cells.size(), (long long)inj_rcv.cells.size(), P(d_src_ents.p),
                 P(d_rcv_ents.p), P(d_rcv_ext_ents.p), P(d_src_shot_ptr.p), P(d_rcv_shot_ptr.p), P(d_tx.p), P(d_tz.p),
-                P(d_div_tb.p), P(d_div_lr.p), (long long)list_core.size(), (long long)list_bz.size(), (long long)list_bz8.size(),
-                (long long)list_bx.size(), (long long)boxes.size()};
+                P(d_div_tb.p), P(d_div_lr.p)};
     }
 
-    // Runs body (which only enqueues device work on st / st_edge) directly, or, with the
+    // Runs body (which only enqueues device work on st) directly, or, with the
     // graph option, replays its capture when the key matches and captures it otherwise.
     template <class F>
     void run_loop(LoopGraph& G, const std::vector<long long>& key, F body)
@@ -916,64 +901,43 @@ struct Engine {
         int btx = opt_tile_x, bspb = opt_spb, bspe = opt_spb_edge;
         tune_report.clear();
         const long long steps0 = stat_steps;
-        int bes = opt_edge_stream;
-        double t_es2[2][5][3];  // the edge_stream = 2 time of each (tile, spb, spb_edge)
-        for (auto& a : t_es2)
-            for (auto& b : a)
-                for (double& c : b) c = 1e300;
         for (int tx : {16, 32})
             for (int spb : {1, 2, 4, 8, 16}) {
                 if (spb > 1 && spb > ns) continue;
-                for (int spe : {1, 2, 4})
-                    for (int es : {1, 2, 0}) {
-                        if (spe > 1 && spe > ns) continue;
-                        set_tile(tx);
-                        opt_spb = spb;
-                        opt_spb_edge = spe;
-                        opt_edge_stream = es;
-                        Levels L = levels_in(d_fwd);
-                        init_levels(L, false, dsrc);
-                        for (int it = 0; it < nsteps; it++) {
-                            if (it == nsteps - timed) HIPCHECK(hipEventRecord(e0, st));
-                            step(L, it, false, dsrc, nullptr);
-                        }
-                        HIPCHECK(hipEventRecord(e1, st));
-                        HIPCHECK(hipEventSynchronize(e1));
-                        float ms = 0.f;
-                        HIPCHECK(hipEventElapsedTime(&ms, e0, e1));
-                        const double us = 1e3 * ms / std::min(timed, nsteps);
-                        char buf[112];
-                        snprintf(buf, sizeof(buf), "%stile_x=%d spb=%d spb_edge=%d edge_stream=%d: %.1f us",
-                                 tune_report.empty() ? "" : "; ", tx, spb, spe, es, us);
-                        tune_report += buf;
-                        if (es == 2) {
-                            const int ispb = spb == 1 ? 0 : spb == 2 ? 1 : spb == 4 ? 2 : spb == 8 ? 3 : 4;
-                            t_es2[tx == 32][ispb][spe == 1 ? 0 : spe == 2 ? 1 : 2] = us;
-                        }
-                        if (us < best) {
-                            best = us;
-                            btx = tx;
-                            bspb = spb;
-                            bspe = spe;
-                            bes = es;
-                        }
+                for (int spe : {1, 2, 4, 8}) {
+                    if (spe > 1 && spe > ns) continue;
+                    set_tile(tx);
+                    opt_spb = spb;
+                    opt_spb_edge = spe;
+                    Levels L = levels_in(d_fwd);
+                    init_levels(L, false, dsrc);
+                    for (int it = 0; it < nsteps; it++) {
+                        if (it == nsteps - timed) HIPCHECK(hipEventRecord(e0, st));
+                        step(L, it, false, dsrc, nullptr);
                     }
+                    HIPCHECK(hipEventRecord(e1, st));
+                    HIPCHECK(hipEventSynchronize(e1));
+                    float ms = 0.f;
+                    HIPCHECK(hipEventElapsedTime(&ms, e0, e1));
+                    const double us = 1e3 * ms / std::min(timed, nsteps);
+                    char buf[96];
+                    snprintf(buf, sizeof(buf), "%stile_x=%d spb=%d spb_edge=%d: %.1f us", tune_report.empty() ? "" : "; ",
+                             tx, spb, spe, us);
+                    tune_report += buf;
+                    if (us < best) {
+                        best = us;
+                        btx = tx;
+                        bspb = spb;
+                        bspe = spe;
+                    }
+                }
             }
         (void)hipEventDestroy(e0);
         (void)hipEventDestroy(e1);
-        // the forward step cannot tell the edge-stream orders apart (within 1%), but the
-        // graph-replayed gradient can: the core launch issued before the edge bands
-        // (edge_stream 2) took 6.45 s per gradient of 64 shots on 500 x 1700 (nt 4000)
-        // against 6.66 s with the bands first, so that order wins forward-step ties
-        {
-            const int ispb = bspb == 1 ? 0 : bspb == 2 ? 1 : bspb == 4 ? 2 : bspb == 8 ? 3 : 4;
-            if (bes != 2 && t_es2[btx == 32][ispb][bspe == 1 ? 0 : bspe == 2 ? 1 : 2] <= 1.015 * best) bes = 2;
-        }
         set_tile(btx);
         opt_tile_x = btx;
         opt_spb = bspb;
         opt_spb_edge = bspe;
-        opt_edge_stream = bes;
         stat_steps = steps0;
         tuned = true;
     }
@@ -1296,8 +1260,7 @@ struct Engine {
                 load_segment(0, dsrc);
                 StepArgs ia = base_args();
                 sbp_image_args(ia, 0);
-                ia.spb = std::max(1, std::min(opt_spb_img > 0 ? opt_spb_img : 4, ns));
-                ia.ngroups = (ns + ia.spb - 1) / ia.spb;
+                set_groups(ia, spb_img(false), spb_edge());
                 ia.aprev = Ac.P();
                 ia.curr = Ac.C();
                 ia.next = Ac.C();  // weight 0
@@ -1559,7 +1522,6 @@ int fwi2d_engine_set_option(fwi2d_engine* e, const char* key, long long value)
         } else if (k == "band_rows") {
             if (value != 8 && value != 12 && value != 16) throw std::runtime_error("band_rows must be 8, 12 or 16");
             x->opt_band_rows = (int)value;
-            x->build_boxes();
         } else if (k == "shots_per_block_edge_img") {
             if (value < 0 || value > 64) throw std::runtime_error("shots_per_block_edge_img must be in [0, 64]");
             x->opt_spb_edge_img = (int)value;
@@ -1590,8 +1552,8 @@ long long fwi2d_engine_get_stat(fwi2d_engine* e, const char* key)
     if (k == "segment") return x->seg_K;
     if (k == "nseg") return x->nseg;
     if (k == "tile_x") return x->tile_x;
-    if (k == "shots_per_block") return x->opt_spb;
-    if (k == "shots_per_block_edge") return x->opt_spb_edge;
+    if (k == "shots_per_block") return x->spb();
+    if (k == "shots_per_block_edge") return x->spb_edge();
     if (k == "shots_per_block_edge_img") return x->opt_spb_edge_img;
     if (k == "band_rows") return x->opt_band_rows;
     if (k == "shots_per_block_img") return x->opt_spb_img;
@@ -1601,7 +1563,7 @@ long long fwi2d_engine_get_stat(fwi2d_engine* e, const char* key)
     if (k == "image_stream") return x->opt_img_stream;
     if (k == "image_sbp") return x->opt_img_sbp;
     if (k == "ntiles") return x->ntiles();
-    if (k == "interior_tiles") return (long long)x->list_core.size();
+    if (k == "interior_tiles") return x->interior_tiles();
     if (k == "graph_captures") return x->graph_captures;
     if (k == "graph_replays") return x->graph_replays;
     if (k == "nrec") return x->nr;

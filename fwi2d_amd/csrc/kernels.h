@@ -37,14 +37,20 @@ struct InjCell {
 struct StepArgs {
     int nx, nz, ldz, ntx, ntz, nshots, nt, it, taper_prev;
     int spb, ngroups;      // shots per workgroup, shot groups (ceil(nshots / spb))
+    int spb_e, ngroups_e;  // the same for frame tiles
+    int itx0, itx1, itz0, itz1;  // the tiles [itx0, itx1) x [itz0, itz1) hold interior cells only
     float rdx, rdz, rdx2, rdz2, dt, dt2, sat_x, sat_z;
     float c1x, c2x, c1z, c2z;  // interior first-derivative coefficients divided by dx, dz
     int bc_top, bc_bottom, bc_left, bc_right;
     const float *lam, *mu, *rho, *c13, *eps;
     const float* irho;     // dt^2 / rho
     const float *mux, *lamx;  // VTI: (1 + 2 eps) mu, (1 + 2 eps) lambda
+    // D2 closure rows of the model, times 1 / h^2: x columns 0-5 from the left and right
+    // [2 sides][6 columns][8 points][ldz] for mu (wx) and, VTI, (1 + 2 eps) mu (wxx); z rows
+    // 0-5 from the top and bottom [2 sides][nx][6 rows][8 points] for mu
+    const float *wx, *wxx, *wz;
     const float *div_tb;   // [2 sides][2 comps][nx] absorbing divisors, top then bottom
-    const float *div_lr;   // [2 sides][2 comps][nz]
+    const float *div_lr;   // [2 sides][2 comps][ldz]
     const float *taper_x;  // [nx]
     const float *taper_z;  // [ldz]
     const float* prev;     // shot 0 base of [2][nx][ldz]; shot stride below
@@ -94,19 +100,8 @@ int tiles_z(int ldz);
 void tile_range_x(int k, int ntile, int T, int n, int& s, int& e);
 void tile_range_z(int k, int ntile, int nz, int ldz, int& s, int& e);
 
-// Box shapes of the step decomposition: core boxes (TX x 64, every stencil interior) and
-// edge-band boxes (120 x 8 for 8-row bands and 64 x 16 for taller ones along the top and
-// bottom, 8 x 128 along the sides).  The 8-row boxes are 120 wide so that their state
-// window is 128 columns: two window quads and two product quads per thread.
-enum class BoxClass { core16, core32, band_z, band_x, band_z8 };
-constexpr int kBandZ8Width = 120;
-constexpr int kCoreX0 = 6;   // core: x in [6, nx - 6), z in [8, core_z_end(nz))
-constexpr int kCoreZ0 = 8;
-inline int core_z_end(int nz) { return ((nz - 8) / 4) * 4; }
-
-// n boxes listed in list (indices into boxes: {sx, ex, sz, ez}) of one class
-void launch_step(const StepArgs& a, bool vti, BoxClass c, const int4* boxes, const int* list, int n, bool image,
-                 hipStream_t s);
+// one time step of every shot over the tile grid
+void launch_step(const StepArgs& a, bool vti, int tile_x, bool image, hipStream_t s);
 void launch_init_prev(float* prev, long long shot_stride, long long nxz, int ldz, int nshots, const int* shot_ptr,
                       const PointEntry* ents, const float* trace, hipStream_t s);
 void launch_scale_prev(float* prev, const float* rho, float half_dt2, long long nxz, int nshots, hipStream_t s);

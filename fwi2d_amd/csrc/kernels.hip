@@ -2,10 +2,9 @@
 //
 // Layout: every field is [x][ldz] with z contiguous (index ix*ldz + iz), the reference's
 // [x][z] order with z padded to a multiple of 32 cells (128-byte columns).  Workgroups
-// of 256 threads own a box of cells and a group of shots; a thread moves 4 consecutive
-// z cells (a quad) with 128-bit accesses.  The time step runs over a box decomposition
-// (interior core boxes and edge bands, built by the engine); the imaging kernel runs
-// over the tile grid below.
+// of 256 threads own a tile of cells and a group of shots; a thread moves 4 consecutive
+// z cells (a quad) with 128-bit accesses.  The time step and the imaging kernel run over
+// the tile grid below.
 //
 // Tile grid: tiles start at multiples of the tile size except the last one in each
 // direction, which is anchored to end at the grid edge (start = n - T).  Each tile
@@ -190,8 +189,8 @@ __device__ __forceinline__ float d2_apply(const W5& w, const float* pu, int s)
     return w.c * pu[0] + w.m1 * pu[-s] + w.p1 * pu[s] + w.m2 * pu[-2 * s] + w.p2 * pu[2 * s];
 }
 
-// Closure rows of D2(c): row R of the 6 x 8 x 8 table applied to one or two fields
-// sharing the coefficient, from the edge point along stride st.  The table's non-zeros
+// Closure rows of D2(c): row R of the 6 x 8 x 8 table applied to a field, from the edge
+// point along stride st.  The table's non-zeros
 // are compile-time immediates; the weights of the 8 field points are formed first.
 constexpr int kD2NZ = sizeof(kD2ClosureNZ) / sizeof(kD2ClosureNZ[0]);
 constexpr int d2_row_begin(int r)
@@ -201,9 +200,8 @@ constexpr int d2_row_begin(int r)
     return i;
 }
 
-template <int R, bool TWO>
-__device__ __forceinline__ void d2_closure_row(const float* qu, const float* qv, const float* qc, int st, float& ou,
-                                               float& ov)
+template <int R>
+__device__ __forceinline__ float d2_closure_row(const float* qu, const float* qc, int st)
 {
     float val[8];
 #pragma unroll
@@ -213,47 +211,28 @@ __device__ __forceinline__ void d2_closure_row(const float* qu, const float* qv,
     for (int i = b; i < e; i++)
         val[kD2ClosureNZ[i].point] +=
             (float)(kD2ClosureNZ[i].num / kD2ClosureNZ[i].den) * qc[kD2ClosureNZ[i].coef * st];
-    float cu = 0.f, cv = 0.f;
+    float cu = 0.f;
 #pragma unroll
-    for (int j = 0; j < 8; j++) {
-        cu += val[j] * qu[j * st];
-        if (TWO) cv += val[j] * qv[j * st];
-    }
-    ou = cu;
-    ov = cv;
+    for (int j = 0; j < 8; j++) cu += val[j] * qu[j * st];
+    return cu;
 }
 
-// closure rows of D2(c) for one field (TWO = false) or two fields sharing the coefficient
-template <bool TWO>
-__device__ __forceinline__ void d2_closure_any(const float* pu, const float* pv, const float* pc, int s, int g, int n,
-                                               float& ou, float& ov)
+// closure rows of D2(c) at point g of n
+__device__ __forceinline__ float d2_closure(const float* pu, const float* pc, int s, int g, int n)
 {
     const bool top = g < 6;
     const int r = top ? g : n - 1 - g;
     const int st = top ? s : -s;
     const int o = top ? -g * s : r * s;
-    const float *qu = pu + o, *qv = pv + o, *qc = pc + o;
+    const float *qu = pu + o, *qc = pc + o;
     switch (r) {
-    case 0: d2_closure_row<0, TWO>(qu, qv, qc, st, ou, ov); break;
-    case 1: d2_closure_row<1, TWO>(qu, qv, qc, st, ou, ov); break;
-    case 2: d2_closure_row<2, TWO>(qu, qv, qc, st, ou, ov); break;
-    case 3: d2_closure_row<3, TWO>(qu, qv, qc, st, ou, ov); break;
-    case 4: d2_closure_row<4, TWO>(qu, qv, qc, st, ou, ov); break;
-    default: d2_closure_row<5, TWO>(qu, qv, qc, st, ou, ov); break;
+    case 0: return d2_closure_row<0>(qu, qc, st);
+    case 1: return d2_closure_row<1>(qu, qc, st);
+    case 2: return d2_closure_row<2>(qu, qc, st);
+    case 3: return d2_closure_row<3>(qu, qc, st);
+    case 4: return d2_closure_row<4>(qu, qc, st);
+    default: return d2_closure_row<5>(qu, qc, st);
     }
-}
-
-__device__ __forceinline__ float d2_closure(const float* pu, const float* pc, int s, int g, int n)
-{
-    float ou, ov;
-    d2_closure_any<false>(pu, pu, pc, s, g, n, ou, ov);
-    return ou;
-}
-
-__device__ __forceinline__ void d2_closure2(const float* pu, const float* pv, const float* pc, int s, int g, int n,
-                                            float& ou, float& ov)
-{
-    d2_closure_any<true>(pu, pv, pc, s, g, n, ou, ov);
 }
 
 // one-sided outward boundary derivative sum_k SC[k] u[k*s] (times h)
@@ -268,83 +247,70 @@ __device__ __forceinline__ float d1_row0(const float* p, int s) { return d1_clos
 // ---------------------------------------------------------------------------
 // Fused time step
 //
-// A workgroup owns a 64 (z) x TX (x) tile and advances a group of shots through it one
-// after the other, so that the coefficient window and the per-cell factors are read
-// once per tile, not once per shot.  Per shot: the state window (halo 4 in x, 8 in z)
-// is staged in LDS, the products of first derivatives are formed on the tile +/- 2 (x)
-// and +/- 4 (z), then each thread computes the new level of its quads (4 consecutive z
-// cells).  The x and z parts of every stencil choose between the vectorised interior
-// path and the closure path independently, so only quads that really touch a closure
-// row take it.  The next shot's window is loaded into registers before the current
-// shot's arithmetic, which hides its latency.
+// A workgroup owns a 64 (z) x TX (x) tile of the tile grid and advances a group of shots
+// through it one after the other, so that the coefficient window and the per-cell factors
+// are read once per tile, not once per shot.  Per shot: the state window (halo 4 in x, 8 in
+// z) goes straight from global memory into LDS, the products of first derivatives are
+// formed on the tile +/- 2 (x) and +/- 4 (z), then each thread computes the new level of its
+// quads (4 consecutive z cells; column-major, so that a wavefront covers 4 whole columns).
+//
+// Tiles whose cells are all interior run without closure code.  The frame of tiles around
+// them runs the same phases plus the SBP closures and SAT terms, arranged so that the code
+// stays small: closure rows are table-driven loops, not one instance per row.
+//   * Along x the closure columns are whole quads: the D2(mu) weights of a closure column's
+//     8 points come from a model array (formed once per model), D1 coefficients from an LDS
+//     table.
+//   * Along z a closure row is part of a quad.  Every quad forms the interior rows, and the
+//     closure rows are dealt one cell per thread in passes of their own: the products of
+//     rows 0-3 from either side, then the z terms (with the top and bottom SAT terms) of
+//     rows 0-5, and the left and right SAT terms, which go to the quads' owners through the
+//     out-of-grid cells of the state windows.
+// The instance-per-row form this replaced (34-60 KB of code per kernel, edge bands beside a
+// core launch) was bound by instruction fetch: one band workgroup took 30 us alone, and a
+// step of one shot on 201 x 601 cells 117 us (the core launch 6.4 us of it); it takes 14 us
+// in this form (one launch), a 64-shot step on 500 x 1700 392 us instead of 401.  A frame
+// tile costs about 1.7 times an interior one, in VALU work (1209 against 527 vector
+// instructions per wavefront and shot at first, most of the surplus addresses), so it loads
+// per shot what its passes need and keeps no D2 weights: spills cost it more than both.
 // ---------------------------------------------------------------------------
-// Thin z bands (TZ <= 16) map lanes row-major: a wavefront holds one quad row of 64
-// consecutive columns, so the z closure row of every lane of a wave is the same and the
-// closure coefficients are read with scalar loads.  Their LDS columns then hold an odd
-// number of quads, which keeps the column-strided 16-byte reads free of bank conflicts.
-// 8-row bands (TZ = 8) hold compact windows: 16 state rows and 12 product rows, starting
-// at row 0 for the top band; elsewhere the state rows start 8 and the product rows 4
-// above the box (the interior product quads read 4 state rows above themselves, the
-// bottom closure rows the 8 rows above the last one).
-template <int TX, int TZ_>
+template <int TX_>
 struct StepShape {
-    static constexpr int TZ = TZ_;
-    static constexpr bool ROWMAJ = TZ <= 16;
-    static constexpr int BX = ROWMAJ ? (TX + 63) / 64 * 64 : TX;  // lanes per quad row (row-major)
-    static constexpr bool COMPACT = TZ == 8;
+    static constexpr int TX = TX_, TZ = kTileZ;
     static constexpr int HX = 4, HZ = 8;
-    static constexpr int WX = TX + 2 * HX;                     // state window columns
-    static constexpr int WQ = COMPACT ? 4 : (TZ + 2 * HZ) / 4; // state window quads per column
-    static constexpr int WZ = 4 * (ROWMAJ ? (WQ | 1) : WQ);    // LDS column stride of the window
-    static constexpr int IX = TX + 4;                          // product columns
-    static constexpr int PQ = COMPACT ? 3 : (TZ + 8) / 4;      // product quads: rows [sz-4, sz+TZ+4)
-    static constexpr int PZ = 4 * (ROWMAJ ? (PQ | 1) : PQ);    // LDS column stride of the products
-    static constexpr int IXP = ROWMAJ ? (IX + 63) / 64 * 64 : IX;  // product slots per quad row
-    static constexpr int QC = TZ / 4;                          // new-level quads per column
+    static constexpr int WX = TX + 2 * HX;       // state window columns
+    static constexpr int WQ = (TZ + 2 * HZ) / 4; // state window quads per column
+    static constexpr int WZ = 4 * WQ;            // LDS column stride of the window
+    static constexpr int IX = TX + 4;            // product columns
+    static constexpr int PQ = (TZ + 8) / 4;      // product quads: rows [sz-4, sz+TZ+4)
+    static constexpr int PZ = 4 * PQ;            // LDS column stride of the products
+    static constexpr int QC = TZ / 4;            // new-level quads per column
     static constexpr int NQ1 = (WX * WQ + kThreads - 1) / kThreads;  // window quads per thread
-    static constexpr int NQ2 = (IXP * PQ + kThreads - 1) / kThreads; // product quads per thread
-    static constexpr int NQ3 = (BX * QC + kThreads - 1) / kThreads;  // new-level quads per thread
-    static_assert(ROWMAJ || (TX * QC) % kThreads == 0, "box shape must give every thread whole quads");
+    static constexpr int NQ2 = (IX * PQ + kThreads - 1) / kThreads;  // product quads per thread
+    static constexpr int NQ3 = TX * QC / kThreads;                   // new-level quads per thread
+    static_assert((TX * QC) % kThreads == 0, "tile must give every thread whole quads");
 };
 
 struct TileInfo {
-    int tile, sx, ex, sz, ez, wsx, wsz, plx, phx, plz, phz, pz0;
+    int sx, ex, sz, ez, wsx, wsz, plx, phx, plz, phz, pz0;
 };
 
-// new-level quad i of a box: column-major, so that a wavefront covers whole columns
-// (contiguous 16-byte quads along z); row-major in thin z bands, where the quad row is
-// uniform over a wavefront and is made a scalar
+// new-level quad i of a tile
 template <class S>
 __device__ __forceinline__ void out_quad(const TileInfo& t, int i, int& gx, int& z0)
 {
-    if constexpr (S::ROWMAJ) {
-        const int row = __builtin_amdgcn_readfirstlane(i / S::BX);
-        gx = t.sx + (i - row * S::BX);
-        z0 = t.sz + 4 * row;
-    } else {
-        gx = t.sx + i / S::QC;
-        z0 = t.sz + 4 * (i % S::QC);
-    }
+    gx = t.sx + i / S::QC;
+    z0 = t.sz + 4 * (i % S::QC);
 }
 
-// product quad of slot i: column lc of the IX product columns, quad row lq of PQ;
-// false for a slot that holds none
-template <class S>
-__device__ __forceinline__ bool prod_slot(int i, int& lc, int& lq)
-{
-    if constexpr (S::ROWMAJ) {
-        lq = __builtin_amdgcn_readfirstlane(i / S::IXP);
-        lc = i - lq * S::IXP;
-        return lc < S::IX && lq < S::PQ;
-    } else {
-        lc = i / S::PQ;
-        lq = i - lc * S::PQ;
-        return i < S::IX * S::PQ;
-    }
-}
+// D1 rows 0-5 on points 0-7 in LDS (rows 4 and 5 are interior rows), row stride rs
+struct EdgeTable {
+    const float* c;
+    int rs;
+};
 
 struct StepSmem {
     float *ux, *uz, *mu, *mux, *px, *pz, *qx, *qz;
+    EdgeTable tb;
 };
 
 // D1 of a 12-cell column (cells z0-4 .. z0+7) at the 4 quad cells
@@ -385,35 +351,144 @@ __device__ __forceinline__ void load_col12(const float* base, int i, float* c)
     }
 }
 
-// D2(c) u at global index g of n along stride s: interior weights or closure rows
-__device__ __forceinline__ void d2_any2(const float* pu, const float* pv, const float* pc, int s, int g, int n,
-                                        float& ou, float& ov)
+// D1 rows 0-5 from a side on the 8 points next to it: four closure rows and the first two
+// interior ones
+struct EdgeD1 {
+    float c[48];
+};
+constexpr EdgeD1 edge_d1_table()
 {
-    if (g >= 6 && g < n - 6) {
-        const W5 w = d2_weights(pc, s);
-        ou = d2_apply(w, pu, s);
-        ov = d2_apply(w, pv, s);
-    } else {
-        d2_closure2(pu, pv, pc, s, g, n, ou, ov);
+    EdgeD1 t{};
+    for (int r = 0; r < 4; r++)
+        for (int j = 0; j < 6; j++) t.c[8 * r + j] = (float)kD1Closure[r][j];
+    for (int r = 4; r < 6; r++) {
+        t.c[8 * r + r - 2] = (float)-kD1Interior[1];
+        t.c[8 * r + r - 1] = (float)-kD1Interior[0];
+        t.c[8 * r + r + 1] = (float)kD1Interior[0];
+        t.c[8 * r + r + 2] = (float)kD1Interior[1];
+    }
+    return t;
+}
+__constant__ EdgeD1 cEdgeD1 = edge_d1_table();
+
+// One launch for all tiles: the frame's workgroups first (their extra passes make them the
+// slowest), then the interior rectangle's, each class spread over all XCDs (the frame's
+// block count rounded up to a multiple of 8, the extra blocks idle) and remapped within its
+// class so that an XCD runs neighbouring tiles.
+// ---- table-driven closure rows -------------------------------------------------------
+// A closure row of point g of n: the edge point's offset o from g and the inward step st
+// along a line of stride s, the row r from the edge, and the sign of D1 there.
+struct EdgeRow {
+    int o, st, r;
+    float sg;
+};
+__device__ __forceinline__ EdgeRow edge_row(int g, int n, int s)
+{
+    const bool far = 2 * g >= n;
+    const int r = far ? n - 1 - g : g;
+    return {(far ? r : -r) * s, far ? -s : s, r, far ? -1.f : 1.f};
+}
+
+// D1 (times h) of two fields at point g of n along stride s: interior or closure row
+__device__ __forceinline__ void d1_pair(const float* u, const float* v, int s, int g, int n, EdgeTable tb,
+                                        float& du, float& dv)
+{
+    if (g >= 4 && g < n - 4) {
+        du = d1_int(u, s);
+        dv = d1_int(v, s);
+        return;
+    }
+    const EdgeRow e = edge_row(g, n, s);
+    float a = 0.f, b = 0.f;
+#pragma unroll
+    for (int j = 0; j < 6; j++) {
+        const float c = tb.c[tb.rs * e.r + j];
+        a += c * u[e.o + j * e.st];
+        b += c * v[e.o + j * e.st];
+    }
+    du = e.sg * a;
+    dv = e.sg * b;
+}
+
+// The N cells of a column next to its top or bottom cell p, from the side inwards.  They are
+// read in memory order (immediate offsets from one address, all in flight at once; a loop
+// with the side's step as its stride waits for each) and reversed in registers.
+template <int N>
+__device__ __forceinline__ void edge_cells(const float* p, bool far, float* e)
+{
+    const float* b = far ? p - (N - 1) : p;
+    float v[N];
+#pragma unroll
+    for (int i = 0; i < N; i++) v[i] = b[i];
+#pragma unroll
+    for (int j = 0; j < N; j++) e[j] = far ? v[N - 1 - j] : v[j];
+}
+__device__ __forceinline__ void edge_coefficients(EdgeTable tb, int r, float* c)
+{
+    unpack(ld4(tb.c + tb.rs * r), c);
+    unpack(ld4(tb.c + tb.rs * r + 4), c + 4);
+}
+// D1 along z (times h) of closure row r from the top or bottom, whose boundary cell is p;
+// c: the row's coefficients
+__device__ __forceinline__ float d1z_closure(const float* p, bool far, const float* c)
+{
+    float e[6], v = 0.f;
+    edge_cells<6>(p, far, e);
+#pragma unroll
+    for (int j = 0; j < 6; j++) v += c[j] * e[j];
+    return far ? -v : v;
+}
+
+// D1 along x (times h) of two fields at the 4 cells of a quad of a closure column (rows 0-3
+// from a side), column stride CS
+template <int CS>
+__device__ __forceinline__ void d1_quad_closure(const float* u, const float* v, int gx, int nx, EdgeTable tb,
+                                                float* du, float* dv)
+{
+    const EdgeRow e = edge_row(gx, nx, CS);
+#pragma unroll
+    for (int k = 0; k < 4; k++) du[k] = dv[k] = 0.f;
+#pragma unroll 2
+    for (int j = 0; j < 6; j++) {
+        const float c = e.sg * tb.c[tb.rs * e.r + j];
+        float U[4], V[4];
+        unpack(ld4(u + e.o + j * e.st), U);
+        unpack(ld4(v + e.o + j * e.st), V);
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            du[k] += c * U[k];
+            dv[k] += c * V[k];
+        }
     }
 }
 
-__device__ __forceinline__ float d2_any(const float* pu, const float* pc, int s, int g, int n)
+// ---- products of first derivatives on one quad --------------------------------------
+template <bool VTI>
+__device__ __forceinline__ void products(const float* lam, const float* lamx, const float* c13, const float* mu,
+                                         const float* dxux, const float* dxuz, const float* dzux, const float* dzuz,
+                                         int k, float* p, float* pz, float* qx, float* qz)
 {
-    if (g >= 6 && g < n - 6) return d2_apply(d2_weights(pc, s), pu, s);
-    return d2_closure(pu, pc, s, g, n);
+    if (!VTI) {
+        p[k] = lam[k] * (dxux[k] + dzuz[k]);
+        pz[k] = 0.f;
+    } else {
+        p[k] = lamx[k] * dxux[k] + c13[k] * dzuz[k];
+        pz[k] = lam[k] * dzuz[k] + c13[k] * dxux[k];
+    }
+    qx[k] = mu[k] * dxuz[k];
+    qz[k] = mu[k] * dzux[k];
 }
 
-// ---- products of first derivatives on one quad --------------------------------------
+// z rows by the interior stencil whatever the row: in frame tiles product_pass replaces the
+// closure rows
 template <bool VTI, class S, bool EDGE>
 __device__ __forceinline__ void product_quad(const StepArgs& a, const StepSmem& sm, const TileInfo& t, int gx, int z0,
                                              float4 lam4, float4 lamx4, float4 c134, float* p, float* pz, float* qx,
                                              float* qz)
 {
-    const int nx = a.nx, nz = a.nz;
     const int w = (gx - t.wsx) * S::WZ + (z0 - t.wsz);
     float dxux[4], dxuz[4], dzux[4], dzuz[4];
-    if (!EDGE || (gx >= 4 && gx < nx - 4)) {
+    if (!EDGE || (gx >= 4 && gx < a.nx - 4)) {
         float X[4][4], Z[4][4];
         const int off[4] = {-2, -1, 1, 2};
 #pragma unroll
@@ -427,26 +502,19 @@ __device__ __forceinline__ void product_quad(const StepArgs& a, const StepSmem& 
             dxuz[k] = a.c1x * (Z[2][k] - Z[1][k]) + a.c2x * (Z[3][k] - Z[0][k]);
         }
     } else if constexpr (EDGE) {
-#pragma unroll 1
+        d1_quad_closure<S::WZ>(&sm.ux[w], &sm.uz[w], gx, a.nx, sm.tb, dxux, dxuz);
+#pragma unroll
         for (int k = 0; k < 4; k++) {
-            dxux[k] = d1_closure(&sm.ux[w + k], S::WZ, gx, nx) * a.rdx;
-            dxuz[k] = d1_closure(&sm.uz[w + k], S::WZ, gx, nx) * a.rdx;
+            dxux[k] *= a.rdx;
+            dxuz[k] *= a.rdx;
         }
     }
-    if (!EDGE || (z0 >= 4 && z0 + 3 < nz - 4)) {
+    {
         float Uc[12], Zc[12];
         load_col12(sm.ux, w, Uc);
         load_col12(sm.uz, w, Zc);
         d1_quad_z(Uc, dzux, a.c1z, a.c2z);
         d1_quad_z(Zc, dzuz, a.c1z, a.c2z);
-    } else if constexpr (EDGE) {
-#pragma unroll 1
-        for (int k = 0; k < 4; k++) {
-            const int gz = z0 + k;
-            const bool in = gz >= 0 && gz < nz;
-            dzux[k] = in ? d1<false>(&sm.ux[w + k], 1, gz, nz) * a.rdz : 0.f;
-            dzuz[k] = in ? d1<false>(&sm.uz[w + k], 1, gz, nz) * a.rdz : 0.f;
-        }
     }
     float mu[4], lam[4], lamx[4], c13[4];
     unpack(ld4(&sm.mu[w]), mu);
@@ -454,64 +522,201 @@ __device__ __forceinline__ void product_quad(const StepArgs& a, const StepSmem& 
     unpack(lamx4, lamx);
     unpack(c134, c13);
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
-        if (!VTI) {
-            p[k] = lam[k] * (dxux[k] + dzuz[k]);
-            pz[k] = 0.f;
-        } else {
-            p[k] = lamx[k] * dxux[k] + c13[k] * dzuz[k];
-            pz[k] = lam[k] * dzuz[k] + c13[k] * dxux[k];
-        }
-        qx[k] = mu[k] * dxuz[k];
-        qz[k] = mu[k] * dzux[k];
+    for (int k = 0; k < 4; k++)
+        products<VTI>(lam, lamx, c13, mu, dxux, dxuz, dzux, dzuz, k, p, pz, qx, qz);
+}
+
+// Frame tiles at the top or bottom: the products of the closure rows (0-3 from the side)
+// over the tile's product columns, one cell per thread: cell c of the pass, whose model
+// values are loaded ahead of the shot's window.
+struct PCell {
+    int gx, gz;
+    float lam, lamx, c13;
+};
+template <bool VTI, class S>
+__device__ __forceinline__ bool p_cell(const StepArgs& a, const TileInfo& t, int c, bool top, bool bot, PCell& e)
+{
+    constexpr int per = 4 * S::IX;
+    if (c >= (top + bot) * per) return false;
+    const bool far = !top || c >= per;
+    const int i = c - (top && far ? per : 0);
+    e.gx = t.plx + (i >> 2);
+    e.gz = far ? a.nz - 1 - (i & 3) : i & 3;
+    if (e.gx >= t.phx) return false;
+    const int g = e.gx * a.ldz + e.gz;
+    e.lam = a.lam[g];
+    if (VTI) {
+        e.lamx = a.lamx[g];
+        e.c13 = a.c13[g];
+    }
+    return true;
+}
+template <bool VTI, class S>
+__device__ __forceinline__ void p_cell_run(const StepArgs& a, const StepSmem& sm, const TileInfo& t, const PCell& e)
+{
+    const int w = (e.gx - t.wsx) * S::WZ + (e.gz - t.wsz);
+    float dxux, dxuz, dzux, dzuz;
+    d1_pair(&sm.ux[w], &sm.uz[w], S::WZ, e.gx, a.nx, sm.tb, dxux, dxuz);
+    const bool far = e.gz >= 4;
+    const int r = far ? a.nz - 1 - e.gz : e.gz, wb = w + (far ? r : -r);
+    float c[8];
+    edge_coefficients(sm.tb, r, c);
+    dzux = d1z_closure(&sm.ux[wb], far, c);
+    dzuz = d1z_closure(&sm.uz[wb], far, c);
+    dxux *= a.rdx;
+    dxuz *= a.rdx;
+    dzux *= a.rdz;
+    dzuz *= a.rdz;
+    const float mu = sm.mu[w];
+    float p, pz, qx, qz;
+    products<VTI>(&e.lam, &e.lamx, &e.c13, &mu, &dxux, &dxuz, &dzux, &dzuz, 0, &p, &pz, &qx, &qz);
+    const int o = (e.gx - t.plx) * S::PZ + (e.gz - t.pz0);
+    sm.px[o] = p;
+    if (VTI) sm.pz[o] = pz;
+    sm.qx[o] = qx;
+    sm.qz[o] = qz;
+}
+
+// The passes hand their terms to the quads' owners through cells of the state window outside
+// the grid, which no result that is used reads: the term of a top row 8 window rows above
+// its cell, of a bottom row 8 below, of a left or right boundary cell one column outside; x
+// component in the ux window, z component in the uz window.
+constexpr int kTermRows = 8;
+
+// previous level at one cell, tapered as the step takes it
+__device__ __forceinline__ void prev_at(const StepArgs& a, const float* prev, long long nxz, int gx, int gz, float& px,
+                                        float& pz)
+{
+    const int g = gx * a.ldz + gz;
+    px = prev[g];
+    pz = prev[nxz + g];
+    if (a.taper_prev) {
+        px = (px * a.taper_z[gz]) * a.taper_x[gx];
+        pz = (pz * a.taper_z[gz]) * a.taper_x[gx];
     }
 }
 
-// ---- SAT terms of one perimeter cell (we_op.cpp:726-822, 1705-1800) -------------------
+// The z part of the right-hand side (D2z[mu] ux, 2 D2z[mu] uz, Dz of the products) of the
+// closure rows 0-5 from the top or bottom, one cell per thread, and on the boundary row the
+// SAT terms of that side (we_op.cpp:726-774, 1705-1752).  Cell c of the pass, whose D2
+// weights and boundary values are loaded ahead of the shot's window.
+struct ZCell {
+    int gx, r;
+    bool bot;
+    float w[8], lam, rho, f1, prx, prz;
+};
 template <bool VTI, class S>
-__device__ __forceinline__ void sat_cell(const StepArgs& a, const float* sux, const float* suz, float mu0, int gx,
-                                         int gz, float prx, float prz, float& rx, float& rz)
+__device__ __forceinline__ bool z_cell(const StepArgs& a, const TileInfo& t, int c, bool top, bool bot,
+                                       const float* prev, long long nxz, ZCell& e)
 {
-    const int nx = a.nx, nz = a.nz;
-    const int g = gx * a.ldz + gz;
-    const float lam0 = a.lam[g];
-    const float rho0 = a.rho[g];
-    const float f1tb = VTI ? a.c13[g] : lam0;
-    const float epsf = VTI ? 1.f + 2.f * a.eps[g] : 1.f;
-    for (int side = 0; side < 2; side++) {
-        const int bc = side ? a.bc_bottom : a.bc_top;
-        if (bc == 0 || gz != (side ? nz - 1 : 0)) continue;
-        const float sgn = side ? 1.f : -1.f;
-        const int sn = side ? -1 : 1;  // inward step along z
-        float tt = sgn * mu0 * d1<false>(suz, S::WZ, gx, nx) * a.rdx + mu0 * bnd_deriv(sux, sn) * a.rdz;
-        if (bc == 2) tt -= (0.5f * sqrtf(mu0 * rho0)) * prx / a.dt;
-        rx -= a.sat_z * tt;
-        tt = sgn * f1tb * d1<false>(sux, S::WZ, gx, nx) * a.rdx + (2.f * mu0) * bnd_deriv(suz, sn) * a.rdz;
-        if (bc == 2) tt -= (0.5f * sqrtf((lam0 + 2.f * mu0) * rho0)) * prz / a.dt;
-        rz -= a.sat_z * tt;
-        rz += (a.sat_z * a.rdz) * lam0 * d1_row0(suz, sn);
+    constexpr int per = 6 * S::TX;
+    if (c >= (top + bot) * per) return false;
+    e.bot = !top || c >= per;
+    const int i = c - (top && e.bot ? per : 0);
+    e.r = i / S::TX;
+    e.gx = t.sx + i % S::TX;
+    if (e.gx >= t.ex) return false;
+    // weights [side][nx][6 rows][8 points], divided by dz^2
+    const float* W = a.wz + (((e.bot ? a.nx : 0) + e.gx) * 6 + e.r) * 8;
+    unpack(ld4(W), e.w);
+    unpack(ld4(W + 4), e.w + 4);
+    if (e.r == 0) {
+        const int gz = e.bot ? a.nz - 1 : 0, g = e.gx * a.ldz + gz;
+        e.lam = a.lam[g];
+        e.rho = a.rho[g];
+        e.f1 = VTI ? a.c13[g] : e.lam;
+        prev_at(a, prev, nxz, e.gx, gz, e.prx, e.prz);
     }
-    for (int side = 0; side < 2; side++) {
-        const int bc = side ? a.bc_right : a.bc_left;
-        if (bc == 0 || gx != (side ? nx - 1 : 0)) continue;
-        const float sgn = side ? 1.f : -1.f;
-        const int sn = side ? -S::WZ : S::WZ;  // inward step along x
-        const float f2 = epsf * (2.f * mu0);
-        float tt = sgn * f1tb * d1<false>(suz, 1, gz, nz) * a.rdz + f2 * bnd_deriv(sux, sn) * a.rdx;
-        if (bc == 2) tt -= (0.5f * sqrtf(epsf * (lam0 + 2.f * mu0) * rho0)) * prx / a.dt;
-        rx -= a.sat_x * tt;
-        rx += (a.sat_x * a.rdx) * (epsf * lam0) * d1_row0(sux, sn);
-        tt = sgn * mu0 * d1<false>(sux, 1, gz, nz) * a.rdz + mu0 * bnd_deriv(suz, sn) * a.rdx;
-        if (bc == 2) tt -= (0.5f * sqrtf(mu0 * rho0)) * prz / a.dt;
-        rz -= a.sat_x * tt;
+    return true;
+}
+template <bool VTI, class S>
+__device__ __forceinline__ void z_cell_run(const StepArgs& a, const StepSmem& sm, const TileInfo& t, const ZCell& e)
+{
+    const int st = e.bot ? -1 : 1, edge = e.bot ? a.nz - 1 : 0;
+    const int w = (e.gx - t.wsx) * S::WZ + (edge - t.wsz);  // the boundary cell
+    const int q = (e.gx - t.plx) * S::PZ + (edge - t.pz0);
+    float c[8], ux[8], uz[8], v[8];
+    edge_coefficients(sm.tb, e.r, c);
+    edge_cells<8>(&sm.ux[w], e.bot, ux);
+    edge_cells<8>(&sm.uz[w], e.bot, uz);
+    float d2x = 0.f, d2z = 0.f, dp = 0.f, dq = 0.f;
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+        d2x += e.w[j] * ux[j];
+        d2z += e.w[j] * uz[j];
+    }
+    edge_cells<8>((VTI ? sm.pz : sm.px) + q, e.bot, v);
+#pragma unroll
+    for (int j = 0; j < 8; j++) dp += c[j] * v[j];
+    edge_cells<8>(sm.qx + q, e.bot, v);
+#pragma unroll
+    for (int j = 0; j < 8; j++) dq += c[j] * v[j];
+    const float sg = e.bot ? -a.rdz : a.rdz;
+    float rx = d2x + sg * dq, rz = 2.f * d2z + sg * dp;
+    const int bc = e.bot ? a.bc_bottom : a.bc_top;
+    if (e.r == 0 && bc != 0) {
+        const float mu0 = sm.mu[w];
+        const float out = e.bot ? a.rdx : -a.rdx;
+        float dxx, dxz;
+        d1_pair(&sm.ux[w], &sm.uz[w], S::WZ, e.gx, a.nx, sm.tb, dxx, dxz);
+        float tx = mu0 * (out * dxz) + mu0 * bnd_deriv(ux, 1) * a.rdz;
+        float tz = e.f1 * (out * dxx) + (2.f * mu0) * bnd_deriv(uz, 1) * a.rdz;
+        if (bc == 2) {
+            tx -= (0.5f * sqrtf(mu0 * e.rho)) * e.prx / a.dt;
+            tz -= (0.5f * sqrtf((e.lam + 2.f * mu0) * e.rho)) * e.prz / a.dt;
+        }
+        rx -= a.sat_z * tx;
+        rz -= a.sat_z * tz;
+        rz += (a.sat_z * a.rdz) * e.lam * d1_row0(uz, 1);
+    }
+    const int o = w + st * (e.r - kTermRows);
+    sm.ux[o] = rx;
+    sm.uz[o] = rz;
+}
+
+// The SAT terms of the left and right boundary columns of a tile (we_op.cpp:776-822,
+// 1754-1800), one cell per thread.
+template <bool VTI, class S>
+__device__ __forceinline__ void x_sat_pass(const StepArgs& a, const StepSmem& sm, const TileInfo& t, int tid,
+                                           bool left, bool right, const float* prev, long long nxz)
+{
+    for (int c = tid; c < 2 * S::TZ; c += kThreads) {
+        const bool rt = c >= S::TZ;
+        const int gz = t.sz + (rt ? c - S::TZ : c);
+        if (!(rt ? right : left) || gz >= t.ez) continue;
+        const int gx = rt ? a.nx - 1 : 0, sn = rt ? -S::WZ : S::WZ;
+        const int w = (gx - t.wsx) * S::WZ + (gz - t.wsz), g = gx * a.ldz + gz;
+        const float *ux = &sm.ux[w], *uz = &sm.uz[w];
+        const float mu0 = sm.mu[w], lam0 = a.lam[g], rho0 = a.rho[g], f1 = VTI ? a.c13[g] : lam0;
+        const float epsf = VTI ? 1.f + 2.f * a.eps[g] : 1.f;
+        const int bc = rt ? a.bc_right : a.bc_left;
+        float rx = 0.f, rz = 0.f;
+        if (bc != 0) {
+            const float out = rt ? a.rdz : -a.rdz;
+            float dzx, dzz;
+            d1_pair(ux, uz, 1, gz, a.nz, sm.tb, dzx, dzz);
+            float tx = f1 * (out * dzz) + (epsf * (2.f * mu0)) * bnd_deriv(ux, sn) * a.rdx;
+            float tz = mu0 * (out * dzx) + mu0 * bnd_deriv(uz, sn) * a.rdx;
+            if (bc == 2) {
+                float prx, prz;
+                prev_at(a, prev, nxz, gx, gz, prx, prz);
+                tx -= (0.5f * sqrtf(epsf * (lam0 + 2.f * mu0) * rho0)) * prx / a.dt;
+                tz -= (0.5f * sqrtf(mu0 * rho0)) * prz / a.dt;
+            }
+            rx = (a.sat_x * a.rdx) * (epsf * lam0) * d1_row0(ux, sn) - a.sat_x * tx;
+            rz = -a.sat_x * tz;
+        }
+        sm.ux[w - sn] = rx;
+        sm.uz[w - sn] = rz;
     }
 }
 
 // ---- right-hand side of one quad before sources: volume terms (we_op.cpp:690-720,
-// 1665-1700) and SAT terms ----------------------------------------------------------
+// 1665-1700).  Frame tiles (EDGE): the x part in rx, rz and the z part by the interior rows
+// in zx, zz, for frame_terms to complete ------------------------------------------------
 template <bool VTI, class S, bool EDGE, bool CW>
 __device__ __forceinline__ void rhs_quad(const StepArgs& a, const StepSmem& sm, const TileInfo& t, int gx, int z0,
-                                         const float* prx, const float* prz, float* rx, float* rz, const QuadW& qw)
+                                         float* rx, float* rz, float* zx, float* zz, const QuadW& qw)
 {
     const int nx = a.nx, nz = a.nz;
     const int w = (gx - t.wsx) * S::WZ + (z0 - t.wsz);
@@ -563,23 +768,52 @@ __device__ __forceinline__ void rhs_quad(const StepArgs& a, const StepSmem& sm, 
             rz[k] += a.c1x * (Q[2][k] - Q[1][k]) + a.c2x * (Q[3][k] - Q[0][k]);
         }
     } else if constexpr (EDGE) {
-#pragma unroll 1
-        for (int k = 0; k < 4; k++) {
-            if (VTI) {
-                rx[k] = 2.f * d2_closure(&sm.ux[w + k], &sm.mux[w + k], S::WZ, gx, nx) * a.rdx2;
-                rz[k] = d2_closure(&sm.uz[w + k], &sm.mu[w + k], S::WZ, gx, nx) * a.rdx2;
-            } else {
-                float dxx, dxz;
-                d2_closure2(&sm.ux[w + k], &sm.uz[w + k], &sm.mu[w + k], S::WZ, gx, nx, dxx, dxz);
-                rx[k] = 2.f * dxx * a.rdx2;
-                rz[k] = dxz * a.rdx2;
+        // closure column r from a side: weights [side][column][point][ldz], divided by dx^2
+        const EdgeRow e = edge_row(gx, nx, 1);
+        const size_t wo = (size_t)((gx >= 6 ? 6 : 0) + e.r) * 8 * a.ldz + z0;
+        const float *W = a.wx + wo, *WX = VTI ? a.wxx + wo : W;
+        float d2u[4], d2z[4], dp[4], dq[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) d2u[k] = d2z[k] = dp[k] = dq[k] = 0.f;
+#pragma unroll 2
+        for (int j = 0; j < 8; j++) {
+            const int o = e.o + j * e.st;
+            const float c = sm.tb.c[sm.tb.rs * e.r + j];
+            float wj[4], xj[4], U[4], Z[4];
+            unpack(ld4(W + (size_t)j * a.ldz), wj);
+            if (VTI) unpack(ld4(WX + (size_t)j * a.ldz), xj);
+            unpack(ld4(&sm.ux[w + o * S::WZ]), U);
+            unpack(ld4(&sm.uz[w + o * S::WZ]), Z);
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                d2u[k] += (VTI ? xj[k] : wj[k]) * U[k];
+                d2z[k] += wj[k] * Z[k];
             }
-            rx[k] += d1<false>(&sm.px[q + k], S::PZ, gx, nx) * a.rdx;
-            rz[k] += d1<false>(&sm.qz[q + k], S::PZ, gx, nx) * a.rdx;
+            if (c != 0.f) {  // the other points may lie before the product columns
+                float P[4], Q[4];
+                unpack(ld4(&sm.px[q + o * S::PZ]), P);
+                unpack(ld4(&sm.qz[q + o * S::PZ]), Q);
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    dp[k] += c * P[k];
+                    dq[k] += c * Q[k];
+                }
+            }
+        }
+        const float sg = e.sg * a.rdx;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            rx[k] = 2.f * d2u[k] + sg * dp[k];
+            rz[k] = d2z[k] + sg * dq[k];
         }
     }
     // z part: D2z[2mu] uz, D2z[mu] ux, Dz of the products
-    if (!EDGE || (z0 >= 6 && z0 + 3 < nz - 6)) {
+    if (EDGE) {
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int k = 0; k < 4; k++) zx[k] = zz[k] = 0.f;
+    }
+    {
         float Uc[12], Zc[12], d2zx[4], d2zz[4];
         load_col12(sm.ux, w, Uc);
         load_col12(sm.uz, w, Zc);
@@ -602,48 +836,70 @@ __device__ __forceinline__ void rhs_quad(const StepArgs& a, const StepSmem& sm, 
 #pragma unroll
         for (int k = 0; k < 4; k++) {
             if constexpr (CW) {  // cached weights already carry 1/dz^2
-                rz[k] += 2.f * d2zz[k];
-                rx[k] += d2zx[k];
+                zz[k] += 2.f * d2zz[k];
+                zx[k] += d2zx[k];
             } else {
-                rz[k] += 2.f * d2zz[k] * a.rdz2;
-                rx[k] += d2zx[k] * a.rdz2;
+                zz[k] += 2.f * d2zz[k] * a.rdz2;
+                zx[k] += d2zx[k] * a.rdz2;
             }
-            rz[k] += dpz[k];
-            rx[k] += dqz[k];
-        }
-    } else if constexpr (EDGE) {
-#pragma unroll 1
-        for (int k = 0; k < 4; k++) {
-            const int gz = z0 + k;
-            if (gz >= nz) continue;
-            float dzz, dzx;
-            d2_any2(&sm.uz[w + k], &sm.ux[w + k], &sm.mu[w + k], 1, gz, nz, dzz, dzx);
-            rz[k] += 2.f * dzz * a.rdz2;
-            rx[k] += dzx * a.rdz2;
-            rz[k] += d1<false>(VTI ? &sm.pz[q + k] : &sm.px[q + k], 1, gz, nz) * a.rdz;
-            rx[k] += d1<false>(&sm.qx[q + k], 1, gz, nz) * a.rdz;
+            zz[k] += dpz[k];
+            zx[k] += dqz[k];
         }
     }
-    // SAT lines
-    if (EDGE && (gx == 0 || gx == nx - 1 || z0 == 0 || z0 + 3 >= nz - 1)) {
-#pragma unroll 1
+}
+
+// Frame tiles: the z part of one quad with its closure rows, and the left and right SAT terms
+template <class S>
+__device__ __forceinline__ void frame_terms(const StepArgs& a, const StepSmem& sm, const TileInfo& t, int gx, int z0,
+                                            float* rx, float* rz, float* zx, float* zz)
+{
+    const int nx = a.nx, nz = a.nz;
+    const int w = (gx - t.wsx) * S::WZ + (z0 - t.wsz);
+    float tx[4], tz[4];
+    if (z0 < 6) {  // quads 0 and 4: rows 0-5
+        unpack(ld4(&sm.ux[w - kTermRows]), tx);
+        unpack(ld4(&sm.uz[w - kTermRows]), tz);
+#pragma unroll
         for (int k = 0; k < 4; k++) {
-            const int gz = z0 + k;
-            if (gz >= nz) continue;
-            if (gz == 0 || gz == nz - 1 || gx == 0 || gx == nx - 1)
-                sat_cell<VTI, S>(a, &sm.ux[w + k], &sm.uz[w + k], sm.mu[w + k], gx, gz, prx[k], prz[k], rx[k], rz[k]);
+            zx[k] = k < 2 || z0 == 0 ? tx[k] : zx[k];
+            zz[k] = k < 2 || z0 == 0 ? tz[k] : zz[k];
+        }
+    }
+    if (z0 + 3 >= nz - 6) {  // (nz 12 and 13: a quad holds rows of both sides)
+        unpack(ld4(&sm.ux[w + kTermRows]), tx);
+        unpack(ld4(&sm.uz[w + kTermRows]), tz);
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            zx[k] = z0 + k >= nz - 6 ? tx[k] : zx[k];
+            zz[k] = z0 + k >= nz - 6 ? tz[k] : zz[k];
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        rx[k] += zx[k];
+        rz[k] += zz[k];
+    }
+    if (gx == 0 || gx == nx - 1) {
+        const int o = gx == 0 ? w - S::WZ : w + S::WZ;
+        unpack(ld4(&sm.ux[o]), tx);
+        unpack(ld4(&sm.uz[o]), tz);
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            rx[k] += tx[k];
+            rz[k] += tz[k];
         }
     }
 }
 
 // First derivatives of a pair of fields (u, v) at the 4 cells of a quad from an LDS
-// array with column stride CS: (dx u, dz u, dx v, dz v), scaled by 1/h.
+// array with column stride CS: (dx u, dz u, dx v, dz v), scaled by 1/h.  In frame tiles
+// (EDGE) the z derivatives of the closure rows come from d1z_pass: u and v are arrays whose
+// rows start H above the tile, row0 their index of the quad's column at the tile's row 0.
 template <bool EDGE, int CS>
-__device__ __forceinline__ void quad_derivs(const StepArgs& a, const float* u, const float* v, int w, int gx, int z0,
-                                            float* xu, float* zu, float* xv, float* zv)
+__device__ __forceinline__ void quad_derivs(const StepArgs& a, const float* u, const float* v, int w, int row0, int gx,
+                                            int z0, EdgeTable tb, float* xu, float* zu, float* xv, float* zv)
 {
     const int nx = a.nx, nz = a.nz;
-    const float rdx = a.rdx, rdz = a.rdz;
     if (!EDGE || (gx >= 4 && gx < nx - 4)) {
         float U[4][4], V[4][4];
         const int off[4] = {-2, -1, 1, 2};
@@ -658,26 +914,55 @@ __device__ __forceinline__ void quad_derivs(const StepArgs& a, const float* u, c
             xv[k] = a.c1x * (V[2][k] - V[1][k]) + a.c2x * (V[3][k] - V[0][k]);
         }
     } else if constexpr (EDGE) {
-#pragma unroll 1
+        d1_quad_closure<CS>(u + w, v + w, gx, nx, tb, xu, xv);
+#pragma unroll
         for (int k = 0; k < 4; k++) {
-            xu[k] = d1_closure(&u[w + k], CS, gx, nx) * rdx;
-            xv[k] = d1_closure(&v[w + k], CS, gx, nx) * rdx;
+            xu[k] *= a.rdx;
+            xv[k] *= a.rdx;
         }
     }
-    if (!EDGE || (z0 >= 4 && z0 + 3 < nz - 4)) {
+    {
         float Uc[12], Vc[12];
         load_col12(u, w, Uc);
         load_col12(v, w, Vc);
         d1_quad_z(Uc, zu, a.c1z, a.c2z);
         d1_quad_z(Vc, zv, a.c1z, a.c2z);
-    } else if constexpr (EDGE) {
-#pragma unroll 1
-        for (int k = 0; k < 4; k++) {
-            const int gz = z0 + k;
-            const bool in = gz < nz;
-            zu[k] = in ? d1<false>(&u[w + k], 1, gz, nz) * rdz : 0.f;
-            zv[k] = in ? d1<false>(&v[w + k], 1, gz, nz) * rdz : 0.f;
+    }
+    if constexpr (EDGE) {
+        if (z0 < 4 || z0 + 3 >= nz - 4) {
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const int gz = z0 + k;
+                const bool bot = gz >= 4;
+                if ((bot && gz < nz - 4) || gz >= nz) continue;
+                const int i = row0 + (bot ? kTileZ + nz - 1 - gz : gz - 4);
+                zu[k] = u[i];
+                zv[k] = v[i];
+            }
         }
+    }
+}
+
+// Frame tiles at the top or bottom: the z derivatives (times 1/h) of two fields on the
+// closure rows 0-3 from the side, one cell per thread, into the arrays' rows outside the
+// grid: row r of the top at r - 4, of the bottom at r below the tile.  u and v have column
+// stride CS and first column wx; row0 is their index of the first tile column's row 0.
+template <int TX, int CS>
+__device__ __forceinline__ void d1z_pass(const StepArgs& a, float* u, float* v, int row0, int sx, int ex, int sz,
+                                         int tid, bool near, bool far, EdgeTable tb)
+{
+    constexpr int per = 4 * TX;
+    for (int c = tid; c < (near + far) * per; c += kThreads) {
+        const bool bot = !near || c >= per;
+        const int i = c - (near && bot ? per : 0);
+        const int col = i >> 2, r = i & 3;
+        if (sx + col >= ex) continue;
+        const int w = row0 + col * CS, wb = w + (bot ? a.nz - 1 : 0) - sz;
+        float cf[8];
+        edge_coefficients(tb, r, cf);
+        const float du = d1z_closure(&u[wb], bot, cf), dv = d1z_closure(&v[wb], bot, cf);
+        u[w + (bot ? kTileZ + r : r - 4)] = du * a.rdz;
+        v[w + (bot ? kTileZ + r : r - 4)] = dv * a.rdz;
     }
 }
 
@@ -782,7 +1067,6 @@ __device__ __forceinline__ void opaque(int& v) { __asm__ volatile("" : "+s"(v));
 __device__ __forceinline__ void opaque_v(int& v) { __asm__ volatile("" : "+v"(v)); }
 __device__ __forceinline__ void opaque(TileInfo& t)
 {
-    opaque(t.tile);
     opaque(t.sx);
     opaque(t.ex);
     opaque(t.sz);
@@ -807,10 +1091,7 @@ __device__ __forceinline__ void quad_to_lds(const float* src, float* lds_wave)
     __builtin_amdgcn_global_load_lds(src, (__attribute__((address_space(3))) void*)lds_wave, 16, 0, 0);
 }
 
-// A workgroup advances the shots of one group through one box of the grid.  Boxes of the
-// core (EDGE = false) hold only cells whose stencils are all interior, so no closure or
-// SAT code is compiled in; boxes of the edge bands (EDGE = true) take the closure and
-// SAT paths where a quad needs them.
+// One tile and shot group of a time step (see above).  EDGE: a frame tile.
 // IMG (the image_fused option; by default the imaging runs in k_img): adjoint step it with
 // the imaging by parts in time fused in (see k_img with SBP): the density term of
 // snapshot j = f0 against wn next + wc curr + wp prev at the cells (prev as stored, before
@@ -820,49 +1101,26 @@ __device__ __forceinline__ void quad_to_lds(const float* src, float* lds_wave)
 // products once the new level is done.  The gradient contributions of the workgroup's
 // shots are summed in registers and added once per launch to the gradient slab of the
 // group's first shot.
-template <bool VTI, int TX, int TZ, bool EDGE, bool IMG>
-__global__ void __launch_bounds__(kThreads)
-k_step(const StepArgs a, const int4* boxes, const int* list)
+template <bool VTI, class S, bool EDGE, bool IMG>
+__device__ __forceinline__ void step_tile(const StepArgs& a, const StepSmem& sm, int tix, int tiz, int s0, int s1)
 {
-    using S = StepShape<TX, TZ>;
-    __shared__ __attribute__((aligned(16))) float sUx[S::WX * S::WZ];
-    __shared__ __attribute__((aligned(16))) float sUz[S::WX * S::WZ];
-    __shared__ __attribute__((aligned(16))) float sMu[S::WX * S::WZ];
-    __shared__ __attribute__((aligned(16))) float sMuX[VTI ? S::WX * S::WZ : 4];  // (1+2eps) mu
-    __shared__ __attribute__((aligned(16))) float sPx[S::IX * S::PZ];
-    __shared__ __attribute__((aligned(16))) float sPz[VTI ? S::IX * S::PZ : 4];
-    __shared__ __attribute__((aligned(16))) float sQx[S::IX * S::PZ];
-    __shared__ __attribute__((aligned(16))) float sQz[S::IX * S::PZ];
-    StepSmem sm{sUx, sUz, sMu, sMuX, sPx, sPz, sQx, sQz};
     // IMG: snapshot fm's window in the product layout, over the products (dead by then)
-    float* const sFx = sPx;
-    float* const sFz = sQx;
-
-    const int lin = xcd_remap(blockIdx.x, gridDim.x);
+    float* const sFx = sm.px;
+    float* const sFz = sm.qx;
     TileInfo t;
-    const int slot = lin / a.ngroups;
-    const int group = lin - slot * a.ngroups;
-    t.tile = list[slot];
-    const int4 box = boxes[t.tile];
     const int nx = a.nx, nz = a.nz, ldz = a.ldz;
-    t.sx = box.x;
-    t.ex = box.y;
-    t.sz = box.z;
-    t.ez = box.w;
+    tile_range_x_hd(tix, a.ntx, S::TX, nx, t.sx, t.ex);
+    tile_range_z_hd(tiz, a.ntz, nz, ldz, t.sz, t.ez);
     t.wsx = window_start(t.sx, S::HX);
-    if constexpr (S::COMPACT) {
-        t.wsz = t.sz == 0 ? 0 : t.sz - 8;
-        t.pz0 = t.sz == 0 ? 0 : t.sz - 4;
-    } else {
-        t.wsz = t.sz - S::HZ;
-        t.pz0 = t.sz - 4;
-    }
+    t.wsz = t.sz - S::HZ;
+    t.pz0 = t.sz - 4;
     product_range(t.sx, t.ex, nx, t.plx, t.phx);
     product_range(t.sz, t.ez, nz, t.plz, t.phz);
+    // closure rows in the tile
+    const bool top = EDGE && t.sz == 0, bot = EDGE && tiz == a.ntz - 1;
+    const bool left = EDGE && t.sx == 0, right = EDGE && tix == a.ntx - 1;
     const long long nxz = (long long)nx * ldz;
     const int tid = threadIdx.x;
-    const int s0 = group * a.spb;
-    const int s1 = min(a.nshots, s0 + a.spb);
 
     // ---- per tile: coefficient window, product coefficients, new-level factors ----
 #pragma unroll
@@ -875,42 +1133,51 @@ k_step(const StepArgs a, const int4* boxes, const int* list)
             const int g = ok ? gx * ldz + gz : 0;
             const float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
             const int o = lx * S::WZ + 4 * lq;
-            st4(&sMu[o], ok ? ld4(a.mu + g) : z4);
-            if (VTI) st4(&sMuX[o], ok ? ld4(a.mux + g) : z4);
+            st4(&sm.mu[o], ok ? ld4(a.mu + g) : z4);
+            if (VTI) st4(&sm.mux[o], ok ? ld4(a.mux + g) : z4);
         }
     }
+    // interior tiles hold the product coefficients and the new level's factors across the
+    // shots; frame tiles, whose passes need the registers, load them per shot
     float4 plam[S::NQ2], plamx[VTI ? S::NQ2 : 1], pc13[VTI ? S::NQ2 : 1];
+    auto load_coefficients = [&](const TileInfo& t, int tid) {
 #pragma unroll
-    for (int m = 0; m < S::NQ2; m++) {
-        const int i = tid + m * kThreads;
-        int lc, lq;
-        const bool slot = prod_slot<S>(i, lc, lq);
-        const int gx = t.plx + lc, z0 = t.pz0 + 4 * lq;
-        const bool ok = slot && gx < t.phx && z0 + 3 >= t.plz && z0 < t.phz;
-        const int g = ok ? gx * ldz + z0 : 0;
-        const float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
-        plam[m] = ok ? ld4(a.lam + g) : z4;
-        if (VTI) {
-            plamx[m] = ok ? ld4(a.lamx + g) : z4;
-            pc13[m] = ok ? ld4(a.c13 + g) : z4;
+        for (int m = 0; m < S::NQ2; m++) {
+            const int i = tid + m * kThreads;
+            const int lc = i / S::PQ, lq = i - lc * S::PQ;
+            const int gx = t.plx + lc, z0 = t.pz0 + 4 * lq;
+            const bool ok = i < S::IX * S::PQ && gx < t.phx && z0 + 3 >= t.plz && z0 < t.phz;
+            const int g = ok ? gx * ldz + z0 : 0;
+            const float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
+            plam[m] = ok ? ld4(a.lam + g) : z4;
+            if (VTI) {
+                plamx[m] = ok ? ld4(a.lamx + g) : z4;
+                pc13[m] = ok ? ld4(a.c13 + g) : z4;
+            }
         }
-    }
+    };
     float4 qir[S::NQ3], qtz[S::NQ3];
     float qtx[S::NQ3];
+    auto load_factors = [&](const TileInfo& t, int tid) {
 #pragma unroll
-    for (int m = 0; m < S::NQ3; m++) {
-        const int i = tid + m * kThreads;
-        int gx, gz;
-        out_quad<S>(t, i, gx, gz);
-        const bool ok = gx < t.ex && gz < t.ez;
-        const int g = ok ? gx * ldz + gz : 0;
-        const float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
-        qir[m] = ok ? ld4(a.irho + g) : z4;
-        qtz[m] = ok ? ld4(a.taper_z + gz) : z4;
-        qtx[m] = ok ? a.taper_x[gx] : 0.f;
+        for (int m = 0; m < S::NQ3; m++) {
+            const int i = tid + m * kThreads;
+            int gx, gz;
+            out_quad<S>(t, i, gx, gz);
+            const bool ok = gx < t.ex && gz < t.ez;
+            const int g = ok ? gx * ldz + gz : 0;
+            const float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
+            qir[m] = ok ? ld4(a.irho + g) : z4;
+            qtz[m] = ok ? ld4(a.taper_z + gz) : z4;
+            qtx[m] = ok ? a.taper_x[gx] : 0.f;
+        }
+    };
+    if (!EDGE) {
+        load_coefficients(t, tid);
+        load_factors(t, tid);
     }
 
-    // ---- D2 weights of the new-level quads (core boxes, isotropic): once per workgroup ----
+    // ---- D2 weights of the new-level quads (interior tiles, isotropic): once per workgroup ----
     // (not with IMG: the imaging's accumulators and second phase need the registers)
     constexpr bool CW = !EDGE && !VTI && S::NQ3 == 1 && !IMG;
     QuadW qw[CW ? S::NQ3 : 1];
@@ -925,8 +1192,8 @@ k_step(const StepArgs a, const int4* boxes, const int* list)
             const int w = (gx - t.wsx) * S::WZ + (z0 - t.wsz);
             float M[5][4], Mc[12];
 #pragma unroll
-            for (int c = 0; c < 5; c++) unpack(ld4(&sMu[w + (c - 2) * S::WZ]), M[c]);
-            load_col12(sMu, w, Mc);
+            for (int c = 0; c < 5; c++) unpack(ld4(&sm.mu[w + (c - 2) * S::WZ]), M[c]);
+            load_col12(sm.mu, w, Mc);
 #pragma unroll
             for (int k = 0; k < 4; k++) {
                 const float mk[5] = {M[0][k], M[1][k], M[2][k], M[3][k], M[4][k]};
@@ -936,28 +1203,7 @@ k_step(const StepArgs a, const int4* boxes, const int* list)
         }
     }
 
-    // ---- state window of one shot into registers ----
-    float4 wux[S::NQ1], wuz[S::NQ1];
-    auto load_window = [&](int shot, int tid, const TileInfo& t) {
-        const float* cux = a.curr + shot * a.shot_stride;
-#pragma unroll
-        for (int m = 0; m < S::NQ1; m++) {
-            const int i = tid + m * kThreads;
-            const int lx = i / S::WQ, lq = i - lx * S::WQ;
-            const int gx = t.wsx + lx, gz = t.wsz + 4 * lq;
-            const bool ok = i < S::WX * S::WQ && gx >= 0 && gx < nx && gz >= 0 && gz < ldz;
-            const int g = ok ? gx * ldz + gz : 0;
-            const float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
-            wux[m] = ok ? ld4(cux + g) : z4;
-            wuz[m] = ok ? ld4(cux + nxz + g) : z4;
-        }
-    };
-    // core boxes: the state window goes straight from global memory into LDS at the start
-    // of each shot (no register staging); other boxes prefetch the next shot's window
-    // into registers during this shot
-    constexpr bool DMA = !EDGE && S::WZ == 4 * S::WQ;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    if (!DMA && s0 < s1) load_window(s0, tid, t);
 
     float gl[IMG ? S::NQ3 : 1][4], gm[IMG ? S::NQ3 : 1][4], gr[IMG ? S::NQ3 : 1][4];
     float g3[IMG && VTI ? S::NQ3 : 1][4], g4[IMG && VTI ? S::NQ3 : 1][4];  // VTI stiffness mode
@@ -981,124 +1227,192 @@ k_step(const StepArgs a, const int4* boxes, const int* list)
         // previous level of this shot's new-level quads
         float4 qprx[S::NQ3], qprz[S::NQ3];
         const float* pux = a.prev + shot * a.shot_stride;
+        auto load_prev = [&] {
 #pragma unroll
         for (int m = 0; m < S::NQ3; m++) {
             const int i = tid + m * kThreads;
             int gx, gz;
-        out_quad<S>(t, i, gx, gz);
+            out_quad<S>(t, i, gx, gz);
             const bool ok = gx < t.ex && gz < t.ez;
             const int g = ok ? gx * ldz + gz : 0;
             const float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
             qprx[m] = ok ? ld4(pux + g) : z4;
             qprz[m] = ok ? ld4(pux + nxz + g) : z4;
         }
+        };
+        if (!EDGE) load_prev();
+        if (EDGE) load_coefficients(t, tid);
+        // frame tiles: this thread's cells of the closure passes, with what they read of the
+        // model and the previous level
+        // (the z pass takes two of the four wavefronts, alternating with the shot and the
+        // workgroup, so that it does not fall on the same SIMDs in every workgroup of a CU)
+        PCell pc;
+        ZCell zc;
+        const int ztid = tid ^ (((shot ^ tix) & 1) << 7);
+        bool has_p = false, has_z = false;
+        if (EDGE && (top || bot)) {
+            has_p = p_cell<VTI, S>(a, t, kThreads - 1 - tid, top, bot, pc);
+            has_z = z_cell<VTI, S>(a, t, ztid, top, bot, pux, nxz, zc);
+        }
         __syncthreads();  // the previous shot is done with the LDS state and products
-        if constexpr (DMA) {
-            const float* cux = a.curr + shot * a.shot_stride;
+        if (EDGE && VTI && shot == s0 && tid < 48)
+            const_cast<float*>(sm.tb.c)[sm.tb.rs * (tid >> 3) + (tid & 7)] = cEdgeD1.c[tid];
+        const float* cux = a.curr + shot * a.shot_stride;
 #pragma unroll
-            for (int m = 0; m < S::NQ1; m++) {
-                const int i = tid + m * kThreads;
-                if (i < S::WX * S::WQ) {
-                    const int lx = i / S::WQ, lq = i - lx * S::WQ;
-                    const int gx = t.wsx + lx, gz = t.wsz + 4 * lq;
-                    const bool ok = gx >= 0 && gx < nx && gz >= 0 && gz < ldz;
-                    const int g = gx * ldz + gz;
-                    const int o = 4 * (m * kThreads + wave * 64);  // window quad i at 4 i
-                    quad_to_lds(ok ? cux + g : kZeroQuad, &sUx[o]);
-                    quad_to_lds(ok ? cux + nxz + g : kZeroQuad, &sUz[o]);
-                }
-            }
-            __builtin_amdgcn_s_waitcnt(0);
-        } else {
-#pragma unroll
-            for (int m = 0; m < S::NQ1; m++) {
-                const int i = tid + m * kThreads;
-                if (i < S::WX * S::WQ) {
-                    const int lx = i / S::WQ, lq = i - lx * S::WQ;
-                    const int o = lx * S::WZ + 4 * lq;
-                    st4(&sUx[o], wux[m]);
-                    st4(&sUz[o], wuz[m]);
-                }
+        for (int m = 0; m < S::NQ1; m++) {
+            const int i = tid + m * kThreads;
+            if (i < S::WX * S::WQ) {
+                const int lx = i / S::WQ, lq = i - lx * S::WQ;
+                const int gx = t.wsx + lx, gz = t.wsz + 4 * lq;
+                const bool ok = gx >= 0 && gx < nx && gz >= 0 && gz < ldz;
+                const int g = gx * ldz + gz;
+                const int o = 4 * (m * kThreads + wave * 64);  // window quad i at 4 i
+                quad_to_lds(ok ? cux + g : kZeroQuad, &sm.ux[o]);
+                quad_to_lds(ok ? cux + nxz + g : kZeroQuad, &sm.uz[o]);
             }
         }
+        __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
-        if (!DMA && shot + 1 < s1) load_window(shot + 1, tid, t);
 
         // products of first derivatives
 #pragma unroll
         for (int m = 0; m < S::NQ2; m++) {
             const int i = tid + m * kThreads;
-            int lc, lq;
-            if (!prod_slot<S>(i, lc, lq)) continue;
+            if (i >= S::IX * S::PQ) continue;
+            const int lc = i / S::PQ, lq = i - lc * S::PQ;
             const int gx = t.plx + lc, z0 = t.pz0 + 4 * lq;
             float p[4] = {0.f, 0.f, 0.f, 0.f}, pz[4] = {0.f, 0.f, 0.f, 0.f}, qx[4] = {0.f, 0.f, 0.f, 0.f},
                   qz[4] = {0.f, 0.f, 0.f, 0.f};
             if (gx < t.phx && z0 + 3 >= t.plz && z0 < t.phz)
                 product_quad<VTI, S, EDGE>(a, sm, t, gx, z0, plam[m], VTI ? plamx[m] : plam[m], VTI ? pc13[m] : plam[m],
-                                      p, pz, qx, qz);
+                                           p, pz, qx, qz);
             const int o = lc * S::PZ + 4 * lq;
-            st4(&sPx[o], make_float4(p[0], p[1], p[2], p[3]));
-            if (VTI) st4(&sPz[o], make_float4(pz[0], pz[1], pz[2], pz[3]));
-            st4(&sQx[o], make_float4(qx[0], qx[1], qx[2], qx[3]));
-            st4(&sQz[o], make_float4(qz[0], qz[1], qz[2], qz[3]));
+            if (EDGE && ((top && z0 >= 0 && z0 < 4) || z0 + 3 >= nz - 4)) {
+                // the closure rows are the pass's
+#pragma unroll
+                for (int k = 0; k < 4; k++)
+                    if (z0 >= 4 && z0 + k < nz - 4) {
+                        sm.px[o + k] = p[k];
+                        if (VTI) sm.pz[o + k] = pz[k];
+                        sm.qx[o + k] = qx[k];
+                        sm.qz[o + k] = qz[k];
+                    }
+                continue;
+            }
+            st4(&sm.px[o], make_float4(p[0], p[1], p[2], p[3]));
+            if (VTI) st4(&sm.pz[o], make_float4(pz[0], pz[1], pz[2], pz[3]));
+            st4(&sm.qx[o], make_float4(qx[0], qx[1], qx[2], qx[3]));
+            st4(&sm.qz[o], make_float4(qz[0], qz[1], qz[2], qz[3]));
+        }
+        if (EDGE && (top || bot)) {
+            if (has_p) p_cell_run<VTI, S>(a, sm, t, pc);
+            if (8 * S::IX > kThreads && p_cell<VTI, S>(a, t, 2 * kThreads - 1 - tid, top, bot, pc))
+                p_cell_run<VTI, S>(a, sm, t, pc);
         }
         __syncthreads();
 
-        // new level
+        // new level; frame tiles: the closure and SAT terms and the quads' own parts, then
+        // (after a barrier) the rest of the step
         float* nux = a.next + shot * a.shot_stride;
         float* nuz = nux + nxz;
+        float erx[EDGE ? S::NQ3 : 1][4], erz[EDGE ? S::NQ3 : 1][4], ezx[EDGE ? S::NQ3 : 1][4], ezz[EDGE ? S::NQ3 : 1][4];
+        if constexpr (EDGE) {
+            if (top || bot) {
+                if (has_z) z_cell_run<VTI, S>(a, sm, t, zc);
+                if (12 * S::TX > kThreads && z_cell<VTI, S>(a, t, kThreads + ztid, top, bot, pux, nxz, zc))
+                    z_cell_run<VTI, S>(a, sm, t, zc);
+            }
+            if (left || right) x_sat_pass<VTI, S>(a, sm, t, tid, left, right, pux, nxz);
+#pragma unroll
+            for (int m = 0; m < S::NQ3; m++) {
+                const int i = tid + m * kThreads;
+                int gx, z0;
+                out_quad<S>(t, i, gx, z0);
+                if (gx >= t.ex || z0 >= t.ez) continue;
+                rhs_quad<VTI, S, EDGE, CW>(a, sm, t, gx, z0, erx[m], erz[m], ezx[m], ezz[m], qw[0]);
+#pragma unroll
+                for (int k = 0; k < 4; k++)  // formed here, not sunk past the barrier with their inputs kept
+                    __asm__ volatile("" : "+v"(erx[m][k]), "+v"(erz[m][k]), "+v"(ezx[m][k]), "+v"(ezz[m][k]));
+            }
+            load_factors(t, tid);
+            load_prev();
+            __syncthreads();
+        }
 #pragma unroll
         for (int m = 0; m < S::NQ3; m++) {
             const int i = tid + m * kThreads;
             int gx, z0;
             out_quad<S>(t, i, gx, z0);
             if (gx >= t.ex || z0 >= t.ez) continue;
+            float rx[4], rz[4];
+            if constexpr (EDGE) {
+                frame_terms<S>(a, sm, t, gx, z0, erx[m], erz[m], ezx[m], ezz[m]);
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    rx[k] = erx[m][k];
+                    rz[k] = erz[m][k];
+                }
+            } else {
+                rhs_quad<VTI, S, EDGE, CW>(a, sm, t, gx, z0, rx, rz, rx, rz, qw[CW ? m : 0]);
+            }
             float prx[4], prz[4], ir[4], tz[4];
             unpack(qprx[m], prx);
             unpack(qprz[m], prz);
             unpack(qir[m], ir);
             unpack(qtz[m], tz);
             const float txf = qtx[m];
-            if (a.taper_prev) {
+            // factors of 1 instead of a branch, which would keep the right-hand side's inputs
+            // live across it
+            const float txp = a.taper_prev ? txf : 1.f;
 #pragma unroll
-                for (int k = 0; k < 4; k++) {
-                    prx[k] = (prx[k] * tz[k]) * txf;
-                    prz[k] = (prz[k] * tz[k]) * txf;
-                }
+            for (int k = 0; k < 4; k++) {
+                const float tzp = a.taper_prev ? tz[k] : 1.f;
+                prx[k] = (prx[k] * tzp) * txp;
+                prz[k] = (prz[k] * tzp) * txp;
             }
-            float rx[4], rz[4];
-            rhs_quad<VTI, S, EDGE, CW>(a, sm, t, gx, z0, prx, prz, rx, rz, qw[CW ? m : 0]);
             const int wq = (gx - t.wsx) * S::WZ + (z0 - t.wsz);
             float cx[4], cz[4], vx[4], vz[4];
-            unpack(ld4(&sUx[wq]), cx);
-            unpack(ld4(&sUz[wq]), cz);
+            unpack(ld4(&sm.ux[wq]), cx);
+            unpack(ld4(&sm.uz[wq]), cz);
 #pragma unroll
             for (int k = 0; k < 4; k++) {
                 // leapfrog (we_op.cpp:824-830) with ir = dt^2 / rho
                 vx[k] = ir[k] * rx[k] + (2.f * cx[k] - prx[k]);
                 vz[k] = ir[k] * rz[k] + (2.f * cz[k] - prz[k]);
             }
-            if (EDGE && (gx == 0 || gx == nx - 1 || z0 == 0 || z0 + 3 >= nz - 1)) {
+            if constexpr (EDGE) {
                 // implicit part of the absorbing SAT on the perimeter (spatial_operators.cpp:307-521)
-                for (int k = 0; k < 4; k++) {
-                    const int gz = z0 + k;
-                    if (gz >= nz) continue;
-                    const bool edge = (gz == 0) | (gz == nz - 1) | (gx == 0) | (gx == nx - 1);
-                    if (!edge) continue;
-                    float dvx, dvz;
-                    if (gz == 0) { dvx = a.div_tb[gx]; dvz = a.div_tb[nx + gx]; }
-                    else if (gz == nz - 1) { dvx = a.div_tb[2 * nx + gx]; dvz = a.div_tb[3 * nx + gx]; }
-                    else if (gx == 0) { dvx = a.div_lr[gz]; dvz = a.div_lr[nz + gz]; }
-                    else { dvx = a.div_lr[2 * nz + gz]; dvz = a.div_lr[3 * nz + gz]; }
-                    vx[k] = vx[k] / dvx;
-                    vz[k] = vz[k] / dvz;
+                if (gx == 0 || gx == nx - 1) {  // the corners' divisors are in both arrays
+                    const float* d = a.div_lr + (gx ? 2 * ldz : 0) + z0;
+                    float dx[4], dz[4];
+                    unpack(ld4(d), dx);
+                    unpack(ld4(d + ldz), dz);
+#pragma unroll
+                    for (int k = 0; k < 4; k++) {
+                        vx[k] = vx[k] / dx[k];
+                        vz[k] = vz[k] / dz[k];
+                    }
+                } else {
+                    if (z0 == 0) {
+                        vx[0] = vx[0] / a.div_tb[gx];
+                        vz[0] = vz[0] / a.div_tb[nx + gx];
+                    }
+                    if (z0 == ((nz - 1) & ~3)) {
+                        const float dx = a.div_tb[2 * nx + gx], dz = a.div_tb[3 * nx + gx];
+#pragma unroll
+                        for (int k = 0; k < 4; k++)
+                            if (k == ((nz - 1) & 3)) {  // the same for all lanes
+                                vx[k] = vx[k] / dx;
+                                vz[k] = vz[k] / dz;
+                            }
+                    }
                 }
             }
             // cos^2 taper of the new level (we_op.cpp:846-861); cells past nz stay zero
             float ox[4], oz[4];
 #pragma unroll
             for (int k = 0; k < 4; k++) {
-                const bool in = z0 + k < nz;
+                const bool in = !EDGE || z0 + k < nz;
                 ox[k] = in ? (vx[k] * tz[k]) * txf : 0.f;
                 oz[k] = in ? (vz[k] * tz[k]) * txf : 0.f;
             }
@@ -1119,7 +1433,7 @@ k_step(const StepArgs a, const int4* boxes, const int* list)
                 for (int k = 0; k < 4; k++) {
                     const float ax = a.wn * ox[k] + a.wc * cx[k] + a.wp * pvx[k];
                     const float az = a.wn * oz[k] + a.wc * cz[k] + a.wp * pvz[k];
-                    const float r = z0 + k < nz ? f0x[k] * ax + f0z[k] * az : 0.f;
+                    const float r = !EDGE || z0 + k < nz ? f0x[k] * ax + f0z[k] * az : 0.f;
                     if (VTI) {
                         gr[m][k] += st ? 0.f : r;
                         g4[VTI ? m : 0][k] += st ? r : 0.f;
@@ -1136,41 +1450,37 @@ k_step(const StepArgs a, const int4* boxes, const int* list)
 #pragma unroll
             for (int m = 0; m < S::NQ2; m++) {
                 const int i = tid + m * kThreads;
-                int lc, lq;
-                const bool slot = prod_slot<S>(i, lc, lq);
-                const int gx = t.plx + lc, z0 = t.pz0 + 4 * lq;
-                const bool ok = slot && gx < nx && z0 >= 0 && z0 < ldz;
-                const int g = ok ? gx * ldz + z0 : 0;
-                if constexpr (DMA && !S::ROWMAJ) {
-                    // quad i at float 4 i (column-major product slots), as the window DMA
-                    if (slot) {
-                        const int o = 4 * (m * kThreads + wave * 64);
-                        quad_to_lds(ok ? Fm + g : kZeroQuad, &sFx[o]);
-                        quad_to_lds(ok ? Fm + nxz + g : kZeroQuad, &sFz[o]);
-                    }
-                } else {
-                    if (!slot) continue;
-                    const float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
-                    const int o = lc * S::PZ + 4 * lq;
-                    st4(&sFx[o], ok ? ld4(Fm + g) : z4);
-                    st4(&sFz[o], ok ? ld4(Fm + nxz + g) : z4);
+                if (i < S::IX * S::PQ) {
+                    const int lc = i / S::PQ, lq = i - lc * S::PQ;
+                    const int gx = t.plx + lc, z0 = t.pz0 + 4 * lq;
+                    const bool ok = gx < nx && z0 >= 0 && z0 < ldz;
+                    const int g = ok ? gx * ldz + z0 : 0;
+                    const int o = 4 * (m * kThreads + wave * 64);  // quad i at float 4 i, as the state window
+                    quad_to_lds(ok ? Fm + g : kZeroQuad, &sFx[o]);
+                    quad_to_lds(ok ? Fm + nxz + g : kZeroQuad, &sFz[o]);
                 }
             }
-            if constexpr (DMA && !S::ROWMAJ) __builtin_amdgcn_s_waitcnt(0);
+            __builtin_amdgcn_s_waitcnt(0);
             __syncthreads();
+            const int wrow = (t.sx - t.wsx) * S::WZ + S::HZ, frow = (t.sx - t.plx) * S::PZ + 4;
+            if (EDGE && (top || bot)) {
+                d1z_pass<S::TX, S::WZ>(a, sm.ux, sm.uz, wrow, t.sx, t.ex, t.sz, tid, top, bot, sm.tb);
+                d1z_pass<S::TX, S::PZ>(a, sFx, sFz, frow, t.sx, t.ex, t.sz, tid, top, bot, sm.tb);
+                __syncthreads();
+            }
 #pragma unroll
             for (int m = 0; m < S::NQ3; m++) {
                 const int i = tid + m * kThreads;
                 int gx, z0;
                 out_quad<S>(t, i, gx, z0);
                 if (gx >= t.ex || z0 >= t.ez) continue;
-                const int wq = (gx - t.wsx) * S::WZ + (z0 - t.wsz);
-                const int q = (gx - t.plx) * S::PZ + (z0 - t.pz0);
+                const int col = gx - t.sx;
+                const int wq = wrow + col * S::WZ + (z0 - t.sz), q = frow + col * S::PZ + (z0 - t.sz);
                 // adjoint derivatives of the step's current level, forward derivatives of
                 // snapshot j-1 (we_op.cpp:519-541)
                 float axx[4], azx[4], axz[4], azz[4], t0x[4], t1z[4], t2x[4], t3z[4];
-                quad_derivs<EDGE, S::WZ>(a, sUx, sUz, wq, gx, z0, axx, azx, axz, azz);
-                quad_derivs<EDGE, S::PZ>(a, sFx, sFz, q, gx, z0, t0x, t3z, t2x, t1z);
+                quad_derivs<EDGE, S::WZ>(a, sm.ux, sm.uz, wq, wrow + col * S::WZ, gx, z0, sm.tb, axx, azx, axz, azz);
+                quad_derivs<EDGE, S::PZ>(a, sFx, sFz, q, frow + col * S::PZ, gx, z0, sm.tb, t0x, t3z, t2x, t1z);
                 image_stiff<VTI>(a, (long long)gx * ldz + z0, z0, axx, azx, axz, azz, t0x, t1z, t2x, t3z, gl[m],
                                  gm[m], gr[m], g3[VTI ? m : 0]);
             }
@@ -1201,6 +1511,66 @@ k_step(const StepArgs a, const int4* boxes, const int* list)
     }
 }
 
+// wavefronts per SIMD the registers must leave room for: the LDS's share
+constexpr int step_waves(bool vti, int tx, bool img) { return tx == 32 ? 2 : (vti || img ? (vti && img ? 2 : 3) : 4); }
+
+template <bool VTI, int TX, bool IMG>
+__global__ void __launch_bounds__(kThreads, step_waves(VTI, TX, IMG)) k_step(const StepArgs a)
+{
+    using S = StepShape<TX>;
+    __shared__ __attribute__((aligned(16))) float sUx[S::WX * S::WZ];
+    __shared__ __attribute__((aligned(16))) float sUz[S::WX * S::WZ];
+    __shared__ __attribute__((aligned(16))) float sMu[S::WX * S::WZ];
+    __shared__ __attribute__((aligned(16))) float sMuX[VTI ? S::WX * S::WZ : 4];  // (1+2eps) mu
+    __shared__ __attribute__((aligned(16))) float sPx[S::IX * S::PZ];
+    __shared__ __attribute__((aligned(16))) float sPz[VTI ? S::IX * S::PZ : 4];
+    __shared__ __attribute__((aligned(16))) float sQx[S::IX * S::PZ];
+    __shared__ __attribute__((aligned(16))) float sQz[S::IX * S::PZ];
+    // frame tiles' D1 table; VTI: in the (1 + 2 eps) mu window, for the 42 LDS granules that
+    // leave 3 workgroups per CU
+    __shared__ __attribute__((aligned(16))) float sT[VTI ? 4 : 48];
+    StepSmem sm{sUx, sUz, sMu, sMuX, sPx, sPz, sQx, sQz, {sT, 8}};
+
+    const int nin_x = a.itx1 - a.itx0, nin_z = a.itz1 - a.itz0;
+    const int nin = nin_x * nin_z, nedge = a.ntx * a.ntz - nin;
+    const int ne = nedge * a.ngroups_e, ne8 = (ne + 7) & ~7;
+    const int b = blockIdx.x;
+    if (b < ne8) {
+        if (b >= ne) return;  // padding: the whole workgroup leaves before any barrier
+        if (!VTI && threadIdx.x < 48) sT[threadIdx.x] = cEdgeD1.c[threadIdx.x];  // read after the first barrier
+        // frame: the rows of tiles above and below the rectangle, then its side columns
+        const int lin = xcd_remap(b, ne);
+        const int tile = lin / a.ngroups_e, grp = lin - tile * a.ngroups_e;
+        const int top = a.itz0 * a.ntx, bot = (a.ntz - a.itz1) * a.ntx;
+        int tix, tiz;
+        if (tile < top + bot) {
+            const int r = tile < top ? tile : tile - top;
+            tix = r % a.ntx;
+            tiz = (tile < top ? 0 : a.itz1) + r / a.ntx;
+        } else {
+            const int r = tile - top - bot, w = a.ntx - nin_x;
+            const int c = r % w;
+            tiz = a.itz0 + r / w;
+            tix = c < a.itx0 ? c : a.itx1 + (c - a.itx0);
+        }
+        if (VTI) {
+            // out-of-grid cells of the (1 + 2 eps) mu window: 8 rows above or below the grid, or
+            // the first or last window column
+            const bool t = tiz == 0, b = tiz == a.ntz - 1;
+            sm.tb = {sMuX + (t ? 0 : b ? S::TZ + S::HZ : tix == 0 ? S::HZ : (S::WX - 1) * S::WZ + S::HZ),
+                     t || b ? S::WZ : 8};
+        }
+        const int s0 = grp * a.spb_e;
+        step_tile<VTI, S, true, IMG>(a, sm, tix, tiz, s0, min(a.nshots, s0 + a.spb_e));
+    } else {
+        const int lin = xcd_remap(b - ne8, gridDim.x - ne8);
+        const int tile = lin / a.ngroups, grp = lin - tile * a.ngroups;
+        const int s0 = grp * a.spb;
+        step_tile<VTI, S, false, IMG>(a, sm, a.itx0 + tile / nin_z, a.itz0 + tile % nin_z, s0,
+                                      min(a.nshots, s0 + a.spb));
+    }
+}
+
 // ---------------------------------------------------------------------------
 // Imaging condition after an adjoint step (compute_gradients, we_op.cpp:505-562).
 // a.curr is the lagged adjoint level (its first derivatives are imaged), a.next the
@@ -1210,7 +1580,8 @@ k_step(const StepArgs a, const int4* boxes, const int* list)
 // go through LDS, the next shot's windows are loaded into registers meanwhile, and the
 // contributions are summed in registers and added once to the gradient slab of the
 // group's first shot.  Tiles with every cell at least 4 from the edges take the interior
-// stencils only; the others choose per quad.
+// stencils only; the others the closure columns per quad and the closure rows from a pass
+// with one cell per thread (d1z_pass).
 // ---------------------------------------------------------------------------
 // SBP = true: the density term by parts in time (a.aprev is the derivative level, the
 // cell values are the adjoint levels it and it+1, see StepArgs).
@@ -1226,6 +1597,9 @@ __global__ void __launch_bounds__(kThreads) k_img(const StepArgs a)
     // [buffer][Ax, Az, Fx, Fz][window]: window quad i of an array at float offset 4 i, so
     // that the quads a wavefront loads are consecutive in LDS
     __shared__ __attribute__((aligned(16))) float sW[NBUF * 4 * WS];
+    __shared__ __attribute__((aligned(16))) float sT[48];
+    if (threadIdx.x < 48) sT[threadIdx.x] = cEdgeD1.c[threadIdx.x];  // read after the first barrier
+    const EdgeTable tb{sT, 8};
 
     // group-major order: the tiles of one shot group follow each other (z first), so that
     // the window halos a tile shares with its neighbours are still in the XCD's L2
@@ -1240,6 +1614,7 @@ __global__ void __launch_bounds__(kThreads) k_img(const StepArgs a)
     tile_range_z_hd(tiz, a.ntz, nz, ldz, sz, ez);
     const int wsx = window_start(sx, HX), wsz = sz - HZ;
     const bool inner = sx >= 4 && ex <= nx - 4 && sz >= 4 && ez <= nz - 4;
+    const bool top = sz == 0, bot = tiz == a.ntz - 1;
     const long long nxz = (long long)nx * ldz;
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1313,10 +1688,17 @@ __global__ void __launch_bounds__(kThreads) k_img(const StepArgs a)
         __syncthreads();
         // the next shot's windows go into the other buffer while this one is imaged
         if (NBUF == 2 && shot + 1 < s1) issue_windows(shot + 1, b ^ 1);
-        const float* sAx = sW + b * 4 * WS;
-        const float* sAz = sAx + WS;
-        const float* sFx = sAx + 2 * WS;
-        const float* sFz = sAx + 3 * WS;
+        float* const sAx = sW + b * 4 * WS;
+        float* const sAz = sAx + WS;
+        float* const sFx = sAx + 2 * WS;
+        float* const sFz = sAx + 3 * WS;
+        const int wrow = (sx - wsx) * WZ + HZ;
+        if ((top || bot) && !(SBP && !a.img_deriv)) {
+            // z derivatives of the closure rows, into the windows' rows outside the grid
+            d1z_pass<TX, WZ>(a, sAx, sAz, wrow, sx, ex, sz, tid, top, bot, tb);
+            d1z_pass<TX, WZ>(a, sFx, sFz, wrow, sx, ex, sz, tid, top, bot, tb);
+            __syncthreads();
+        }
 #pragma unroll
         for (int m = 0; m < NQ3; m++) {
             const int i = tid + m * kThreads;
@@ -1365,12 +1747,13 @@ __global__ void __launch_bounds__(kThreads) k_img(const StepArgs a)
             if (SBP && !a.img_deriv) continue;
             __builtin_amdgcn_sched_barrier(0);
             float axx[4], azx[4], axz[4], azz[4], t0x[4], t1z[4], t2x[4], t3z[4];
+            const int row0 = w - (z0 - sz);
             if (inner) {
-                quad_derivs<false, WZ>(a, sAx, sAz, w, gx, z0, axx, azx, axz, azz);
-                quad_derivs<false, WZ>(a, sFx, sFz, w, gx, z0, t0x, t3z, t2x, t1z);
+                quad_derivs<false, WZ>(a, sAx, sAz, w, row0, gx, z0, tb, axx, azx, axz, azz);
+                quad_derivs<false, WZ>(a, sFx, sFz, w, row0, gx, z0, tb, t0x, t3z, t2x, t1z);
             } else {
-                quad_derivs<true, WZ>(a, sAx, sAz, w, gx, z0, axx, azx, axz, azz);
-                quad_derivs<true, WZ>(a, sFx, sFz, w, gx, z0, t0x, t3z, t2x, t1z);
+                quad_derivs<true, WZ>(a, sAx, sAz, w, row0, gx, z0, tb, axx, azx, axz, azz);
+                quad_derivs<true, WZ>(a, sFx, sFz, w, row0, gx, z0, tb, t0x, t3z, t2x, t1z);
             }
             const long long g = (long long)gx * ldz + z0;
             image_stiff<VTI>(a, g, z0, axx, azx, axz, azz, t0x, t1z, t2x, t3z, gl[m], gm[m], gr[m],
@@ -1479,8 +1862,8 @@ __global__ void k_inject_cells(const InjCell* cells, int ncell, const int* ptr, 
     float dx = 1.f, dz = 1.f;
     if (gz == 0) { dx = div_tb[gx]; dz = div_tb[nx + gx]; }
     else if (gz == nz - 1) { dx = div_tb[2 * nx + gx]; dz = div_tb[3 * nx + gx]; }
-    else if (gx == 0) { dx = div_lr[gz]; dz = div_lr[nz + gz]; }
-    else if (gx == nx - 1) { dx = div_lr[2 * nz + gz]; dz = div_lr[3 * nz + gz]; }
+    else if (gx == 0) { dx = div_lr[gz]; dz = div_lr[ldz + gz]; }
+    else if (gx == nx - 1) { dx = div_lr[2 * ldz + gz]; dz = div_lr[3 * ldz + gz]; }
     const float f = irho[g] * taper_z[gz] * taper_x[gx];
     float* u = next + cell.shot * shot_stride + g;
     const float ix = f * fx / dx, iz = f * fz / dz;
@@ -1738,33 +2121,21 @@ static inline int grid_for(long long n, int cap = 4096)
     return (int)(b < 1 ? 1 : (b > cap ? cap : b));
 }
 
-template <bool VTI, int TX, int TZ, bool EDGE>
-static void step_launch(const StepArgs& a, const int4* boxes, const int* list, int n, bool image, hipStream_t s)
+template <bool VTI, int TX>
+static void step_launch(const StepArgs& a, bool image, hipStream_t s)
 {
-    const int nb = n * a.ngroups;
-    if (nb <= 0) return;
-    if (image) hipLaunchKernelGGL((k_step<VTI, TX, TZ, EDGE, true>), dim3(nb), dim3(kThreads), 0, s, a, boxes, list);
-    else hipLaunchKernelGGL((k_step<VTI, TX, TZ, EDGE, false>), dim3(nb), dim3(kThreads), 0, s, a, boxes, list);
+    const int nin = (a.itx1 - a.itx0) * (a.itz1 - a.itz0), ne = (a.ntx * a.ntz - nin) * a.ngroups_e;
+    const dim3 grid(((ne + 7) & ~7) + nin * a.ngroups);
+    if (image) hipLaunchKernelGGL((k_step<VTI, TX, true>), grid, dim3(kThreads), 0, s, a);
+    else hipLaunchKernelGGL((k_step<VTI, TX, false>), grid, dim3(kThreads), 0, s, a);
 }
 
-template <bool VTI>
-static void step_class(const StepArgs& a, BoxClass c, const int4* boxes, const int* list, int n, bool image,
-                       hipStream_t s)
+void launch_step(const StepArgs& a, bool vti, int tile_x, bool image, hipStream_t s)
 {
-    switch (c) {
-    case BoxClass::core16: step_launch<VTI, 16, 64, false>(a, boxes, list, n, image, s); break;
-    case BoxClass::core32: step_launch<VTI, 32, 64, false>(a, boxes, list, n, image, s); break;
-    case BoxClass::band_z: step_launch<VTI, 64, 16, true>(a, boxes, list, n, image, s); break;
-    case BoxClass::band_z8: step_launch<VTI, kBandZ8Width, 8, true>(a, boxes, list, n, image, s); break;
-    case BoxClass::band_x: step_launch<VTI, 8, 128, true>(a, boxes, list, n, image, s); break;
-    }
-}
-
-void launch_step(const StepArgs& a, bool vti, BoxClass c, const int4* boxes, const int* list, int n, bool image,
-                 hipStream_t s)
-{
-    if (vti) step_class<true>(a, c, boxes, list, n, image, s);
-    else step_class<false>(a, c, boxes, list, n, image, s);
+    if (vti && tile_x == 32) step_launch<true, 32>(a, image, s);
+    else if (vti) step_launch<true, 16>(a, image, s);
+    else if (tile_x == 32) step_launch<false, 32>(a, image, s);
+    else step_launch<false, 16>(a, image, s);
 }
 
 template <bool VTI, int NBUF, bool SBP>

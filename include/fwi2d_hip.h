@@ -118,13 +118,14 @@ int fwi2d_dot_f64_noalloc(int device, const float* a, const float* b, const floa
 
 /* Tuning and test options (no reference counterpart): "tile_x" (16 | 32 cells per tile
    along x), "shots_per_block" (1..64 shots advanced in turn by one step workgroup of an
-   interior tile), "shots_per_block_edge" (the same for tiles at the grid edge),
-   "shots_per_block_edge_img" (the same for edge tiles of adjoint steps with the imaging
-   fused in; 0, the default: "shots_per_block_edge"),
-   "edge_stream" (1: edge-band launches run on a second stream beside the core launch,
-   enqueued before it; 2: the same, enqueued after it; 0: after it on the same stream),
-   "shots_per_block_img" (shots per imaging workgroup; 0: 4, or "shots_per_block" when
-   fused),
+   interior tile; by default up to 8, fewer where the launch would otherwise have less than
+   2048 workgroups; the stat reads the number in effect), "shots_per_block_edge" (the same
+   for tiles at the grid edge), "shots_per_block_edge_img" (the same for edge tiles of
+   adjoint steps with the imaging fused in; 0, the default: "shots_per_block_edge"),
+   "edge_stream" (0, 1 or 2) and "band_rows" (8, 12 or 16) (accepted without effect: a step
+   is one launch over all tiles),
+   "shots_per_block_img" (shots per imaging workgroup; 0: up to 4, or "shots_per_block"
+   when fused),
    "image_fused" (1: the imaging condition runs inside the adjoint step kernels, by parts
    in time (with sub = 1 and the imaging lag; otherwise as 0); 0: in its own kernel after
    each adjoint step and its point sources; -1, the default: 1 on isotropic grids, 0 on
@@ -138,8 +139,7 @@ int fwi2d_dot_f64_noalloc(int device, const float* a, const float* b, const floa
    levels; 0: the reference's direct form with three snapshots per launch; the two agree
    to rounding),
    "autotune" (1: at the next forward run, time a few steps of every tile_x,
-   shots-per-workgroup and edge_stream choice and keep the fastest, edge_stream 2 winning
-   ties within 1.5% (it replays the gradient faster); forward results are unchanged),
+   shots-per-workgroup choice and keep the fastest; forward results are unchanged),
    "checkpoint_format" (0 FP32; 1 BF16, 2 FP16: checkpoint levels stored in 16 bits with
    a max-abs scale per level and shot, which halves their memory; the gradient then
    carries the error of the recomputation from rounded levels),
