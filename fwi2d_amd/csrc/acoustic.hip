@@ -167,8 +167,11 @@ struct Acoustic {
         }
         ns = nshots;
         nr = r;
-        inj_src.build(se, st);
-        inj_rcv.build(re, st);
+        std::vector<int> xt(g.nx), zt(g.nz);
+        for (int i = 0; i < g.nx; i++) xt[i] = i / kAcTX;
+        for (int i = 0; i < g.nz; i++) zt[i] = i / kAcTZ;
+        inj_src.build(se, xt, zt, ntx, ntz, ns, st);
+        inj_rcv.build(re, xt, zt, ntx, ntz, ns, st);
         ext.swap(xe);
         up(d_ext, ext.data(), ext.size() * sizeof(PointEntry));
         HIPCHECK(hipStreamSynchronize(st));

@@ -93,8 +93,7 @@ struct Engine {
     double gauge = 0.0;    // > 0: DAS receivers of this gauge length
     DevMem d_das_cs;       // DAS: cos, sin of each channel's dip (the operator level's strain)
     std::vector<PointEntry> src_ents, rcv_ents;  // flat, ordered by shot
-    std::vector<int> src_shot_ptr, rcv_shot_ptr;
-    DevMem d_src_ents, d_rcv_ents, d_src_shot_ptr, d_rcv_shot_ptr;
+    DevMem d_points;  // PointTables of the forward and adjoint runs
     InjList inj_src, inj_rcv;  // sources (forward) and receivers (adjoint) as injectors
 
     // state and checkpoints
@@ -172,6 +171,32 @@ struct Engine {
             itz1 = k + 1;
         }
         if (itx1 == 0 || itz1 == 0) itx0 = itx1 = itz0 = itz1 = 0;
+        if (ns > 0) build_points();
+    }
+
+    // the injectors' cells by tile and shot, and the point tables on the device
+    void build_points()
+    {
+        std::vector<int> xt(g.nx), zt(g.nz);
+        for (int k = 0, b, e; k < ntx; k++) {
+            tile_range_x(k, ntx, tile_x, g.nx, b, e);
+            std::fill(xt.begin() + b, xt.begin() + e, k);
+        }
+        for (int k = 0, b, e; k < ntz; k++) {
+            tile_range_z(k, ntz, g.nz, ldz, b, e);
+            std::fill(zt.begin() + b, zt.begin() + e, k);
+        }
+        PointTable t[2];
+        for (int d = 0; d < 2; d++) {
+            InjList& inj = d ? inj_rcv : inj_src;
+            inj.build(d ? rcv_ents : src_ents, xt, zt, ntx, ntz, ns, st);
+            t[d] = {inj.d_cells.as<InjCell>(), inj.d_tile_ptr.as<int>(), inj.d_ptr.as<int>(), inj.d_ctx.as<long long>(),
+                    inj.d_ctz.as<long long>(), inj.d_cw.as<float>(), d_rcv_ext_ents.as<PointEntry>(),
+                    d_rcv_ext_ptr.as<int>(), nr};
+        }
+        d_points.reserve(sizeof(t));
+        HIPCHECK(hipMemcpyAsync(d_points.p, t, sizeof(t), hipMemcpyHostToDevice, st));
+        HIPCHECK(hipStreamSynchronize(st));
     }
     int ntiles() const { return ntx * ntz; }
     int interior_tiles() const { return (itx1 - itx0) * (itz1 - itz0); }
@@ -410,7 +435,7 @@ struct Engine {
         }
         const int nt = g.nt;
         std::vector<PointEntry> se, re, xe;
-        std::vector<int> sp(nshots + 1, 0), rp(nshots + 1, 0), xp(1, 0);
+        std::vector<int> xp(1, 0);
         int r = 0;
         for (int s = 0; s < nshots; s++) {
             const Pivot q = pivot(sxz[2 * s], sxz[2 * s + 1], ox, oz);
@@ -436,7 +461,6 @@ struct Engine {
                 se.push_back(a);
                 se.push_back(b);
             }
-            sp[s + 1] = (int)se.size();
             for (int k = 0; k < nrec[s]; k++, r++) {
                 const double x = rxz[2 * r], z = rxz[2 * r + 1];
                 const long long tx = (long long)r * nt, tz = (long long)(nrt + r) * nt;
@@ -473,7 +497,6 @@ struct Engine {
                 }
                 xp.push_back((int)xe.size());
             }
-            rp[s + 1] = (int)re.size();
         }
         ns = nshots;
         nr = nrt;
@@ -493,20 +516,13 @@ struct Engine {
         rcv_ents.swap(re);
         rcv_ext_ents.swap(xe);
         rcv_ext_ptr.swap(xp);
-        src_shot_ptr.swap(sp);
-        rcv_shot_ptr.swap(rp);
         auto up = [&](DevMem& d, const void* h, size_t b) {
             d.reserve(std::max<size_t>(b, 16));
             if (b) HIPCHECK(hipMemcpyAsync(d.p, h, b, hipMemcpyHostToDevice, st));
         };
-        up(d_src_ents, src_ents.data(), src_ents.size() * sizeof(PointEntry));
-        up(d_rcv_ents, rcv_ents.data(), rcv_ents.size() * sizeof(PointEntry));
         up(d_rcv_ext_ents, rcv_ext_ents.data(), rcv_ext_ents.size() * sizeof(PointEntry));
         up(d_rcv_ext_ptr, rcv_ext_ptr.data(), rcv_ext_ptr.size() * sizeof(int));
-        up(d_src_shot_ptr, src_shot_ptr.data(), src_shot_ptr.size() * sizeof(int));
-        up(d_rcv_shot_ptr, rcv_shot_ptr.data(), rcv_shot_ptr.size() * sizeof(int));
-        inj_src.build(src_ents, st);
-        inj_rcv.build(rcv_ents, st);
+        build_points();
         ckpt_epoch = -1;
         tuned = false;
         HIPCHECK(hipStreamSynchronize(st));
@@ -631,13 +647,10 @@ struct Engine {
         L.prev = 0;
         L.curr = 1;
         L.next = 2;
-        if (adjoint)
-            launch_init_prev(L.P(), 2 * nxz, nxz, ldz, ns, d_rcv_shot_ptr.as<int>(), d_rcv_ents.as<PointEntry>(), traces,
-                             st);
-        else
-            launch_init_prev(L.P(), 2 * nxz, nxz, ldz, ns, d_src_shot_ptr.as<int>(), d_src_ents.as<PointEntry>(), traces,
-                             st);
-        launch_scale_prev(L.P(), d_model.as<float>() + 2 * nxz, (float)(0.5 * g.dt * g.dt), nxz, ns, st);
+        const InjList& inj = adjoint ? inj_rcv : inj_src;
+        launch_init_cells(inj.d_cells.as<InjCell>(), (int)inj.cells.size(), inj.d_ptr.as<int>(),
+                          inj.d_ctx.as<long long>(), inj.d_ctz.as<long long>(), inj.d_cw.as<float>(), traces, L.P(),
+                          2 * nxz, nxz, ldz, d_model.as<float>() + 2 * nxz, (float)(0.5 * g.dt * g.dt), st);
     }
 
     // img_idx >= 0: image forward snapshot img_idx in this adjoint step (its segment must
@@ -679,29 +692,12 @@ struct Engine {
             HIPCHECK(hipStreamWaitEvent(st, ev_img_done[it & 1], 0));
             img_out[it & 1] = false;
         }
-        // extraction of the current level (forward)
-        if (rcv)
-            launch_extract(L.C(), 2 * nxz, nxz, ldz, d_rcv_ext_ents.as<PointEntry>(), d_rcv_ext_ptr.as<int>(), nr, rcv,
-                           it, st);
-        const bool img = fuse_img;
-        launch_step(a, vti, tile_x, img, st);
-        // point sources of this step into the new level
-        const InjList& inj = adjoint ? inj_rcv : inj_src;
-        InjImage im{};
-        if (img) {
-            im.on = 1;
-            im.wn = a.wn;
-            im.f0 = a.f0;
-            im.fshot_stride = a.fshot_stride;
-            im.grad = a.grad;
-            im.gslab_stride = a.gslab_stride;
-            im.rho_off = (long long)(a.stiff ? 4 : 2) * nxz;
-        }
-        launch_inject_cells(inj.d_cells.as<InjCell>(), (int)inj.cells.size(), inj.d_ptr.as<int>(),
-                            inj.d_ctx.as<long long>(), inj.d_ctz.as<long long>(), inj.d_cw.as<float>(), traces, it,
-                            L.N(), 2 * nxz, nxz, g.nx, g.nz, ldz,
-                            d_deriv.as<float>(), d_tx.as<float>(), d_tz.as<float>(), d_div_tb.as<float>(),
-                            d_div_lr.as<float>(), im, st);
+        // point sources of this step into the new level; extraction of the current level (forward)
+        a.points = d_points.as<PointTable>() + (adjoint ? 1 : 0);
+        a.inj_trace = traces;
+        a.rec_trace = rcv;
+        a.nrec = nr;
+        launch_step(a, vti, tile_x, fuse_img, (int)(adjoint ? inj_rcv : inj_src).cells.size(), st);
         if (img_idx >= 0 && !fuse_img) {
             ia.aprev = L.P();
             ia.curr = L.C();
@@ -835,9 +831,10 @@ struct Engine {
                 P(d_fwd.p), P(d_adj.p), P(d_ckpt.p), P(d_seg.p), P(d_gshot.p), P(d_model.p), P(d_deriv.p),
                 P(d_closure.p), P(inj_src.d_cells.p), P(inj_src.d_ptr.p),
                 P(inj_src.d_ctx.p), P(inj_src.d_ctz.p), P(inj_src.d_cw.p), P(inj_rcv.d_cells.p), P(inj_rcv.d_ptr.p),
-                P(inj_rcv.d_ctx.p), P(inj_rcv.d_ctz.p), P(d_rcv_ext_ptr.p), src_nc,
-                P(inj_rcv.d_cw.p), (long long)inj_src.cells.size(), (long long)inj_rcv.cells.size(), P(d_src_ents.p),
-                P(d_rcv_ents.p), P(d_rcv_ext_ents.p), P(d_src_shot_ptr.p), P(d_rcv_shot_ptr.p), P(d_tx.p), P(d_tz.p),
+                P(inj_rcv.d_ctx.p), P(inj_rcv.d_ctz.p), P(d_rcv_ext_ptr.p), src_nc, P(d_points.p),
+                P(inj_src.d_tile_ptr.p), P(inj_rcv.d_tile_ptr.p),
+                P(inj_rcv.d_cw.p), (long long)inj_src.cells.size(), (long long)inj_rcv.cells.size(),
+                P(d_rcv_ext_ents.p), P(d_tx.p), P(d_tz.p),
                 P(d_div_tb.p), P(d_div_lr.p)};
     }
 

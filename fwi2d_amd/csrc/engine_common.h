@@ -41,18 +41,21 @@ struct DevMem {
     ~DevMem() { release(); }
 };
 
-// Cells touched by the point injectors of all shots, with their contributions (trace
-// offset of the x component, weight) in injector order -- host build, device copy
+// Cells touched by the point injectors of all shots, ordered by (tile, shot), with their
+// contributions (trace offsets, weight) in injector order -- host build, device copy
 struct InjList {
     std::vector<InjCell> cells;
-    std::vector<int> ptr;
+    std::vector<int> ptr, tile_ptr;
     std::vector<long long> ctx, ctz;  // trace offsets read by the x and z field components
     std::vector<float> cw;
-    DevMem d_cells, d_ptr, d_ctx, d_ctz, d_cw;
-    void build(const std::vector<PointEntry>& ents, hipStream_t s)
+    DevMem d_cells, d_ptr, d_tile_ptr, d_ctx, d_ctz, d_cw;
+    // xt, zt: the tile column and row of every grid column and row (ntz tile rows), for cells
+    // ordered by (tile, shot)
+    void build(const std::vector<PointEntry>& ents, const std::vector<int>& xt, const std::vector<int>& zt, int ntx,
+               int ntz, int nshots, hipStream_t s)
     {
         struct C {
-            int shot, gx, gz, k;
+            int tile, shot, gx, gz, k;
             long long tx, tz;
             float w;
         };
@@ -62,9 +65,11 @@ struct InjList {
             const PointEntry& e = ents[k];
             for (int ix = 0; ix < 3; ix++)
                 for (int iz = 0; iz < 3; iz++)
-                    all.push_back({e.shot, e.xi0 + ix, e.zi0 + iz, k, e.trace, e.tz, e.wx[ix] * e.wz[iz]});
+                    all.push_back({xt[e.xi0 + ix] * ntz + zt[e.zi0 + iz], e.shot, e.xi0 + ix, e.zi0 + iz, k, e.trace,
+                                   e.tz, e.wx[ix] * e.wz[iz]});
         }
         std::stable_sort(all.begin(), all.end(), [](const C& a, const C& b) {
+            if (a.tile != b.tile) return a.tile < b.tile;
             if (a.shot != b.shot) return a.shot < b.shot;
             if (a.gx != b.gx) return a.gx < b.gx;
             if (a.gz != b.gz) return a.gz < b.gz;
@@ -85,12 +90,16 @@ struct InjList {
             cw.push_back(all[i].w);
         }
         if (!all.empty()) ptr.push_back((int)ctx.size());
+        tile_ptr.assign((size_t)ntx * ntz * nshots + 1, 0);
+        for (const InjCell& c : cells) tile_ptr[((size_t)xt[c.gx] * ntz + zt[c.gz]) * nshots + c.shot + 1]++;
+        for (size_t i = 1; i < tile_ptr.size(); i++) tile_ptr[i] += tile_ptr[i - 1];
         auto up = [&](DevMem& d, const void* h, size_t b) {
             d.reserve(std::max<size_t>(b, 16));
             if (b) HIPCHECK(hipMemcpyAsync(d.p, h, b, hipMemcpyHostToDevice, s));
         };
         up(d_cells, cells.data(), cells.size() * sizeof(InjCell));
         up(d_ptr, ptr.data(), ptr.size() * sizeof(int));
+        up(d_tile_ptr, tile_ptr.data(), tile_ptr.size() * sizeof(int));
         up(d_ctx, ctx.data(), ctx.size() * sizeof(long long));
         up(d_ctz, ctz.data(), ctz.size() * sizeof(long long));
         up(d_cw, cw.data(), cw.size() * sizeof(float));

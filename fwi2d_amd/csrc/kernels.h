@@ -34,6 +34,20 @@ struct InjCell {
     int shot, gx, gz, pad;
 };
 
+// Point sources and receivers of a propagation, in device memory: the touched cells ordered
+// by (tile, shot), so that a step's workgroup adds the sources of its own tile, and the
+// receivers' footprints.
+struct PointTable {
+    const InjCell* cells;
+    const int* tile_ptr;  // [tiles x shots + 1]: cells of a tile's shot
+    const int* ptr;       // [cells + 1]: contributions of a cell
+    const long long *ctx, *ctz;
+    const float* w;
+    const PointEntry* rec;  // receiver r: footprints rec_ptr[r] .. rec_ptr[r + 1]
+    const int* rec_ptr;
+    int nrec;
+};
+
 struct StepArgs {
     int nx, nz, ldz, ntx, ntz, nshots, nt, it, taper_prev;
     int spb, ngroups;      // shots per workgroup, shot groups (ceil(nshots / spb))
@@ -74,6 +88,11 @@ struct StepArgs {
     const float* aprev;
     float wn, wc, wp;
     int img_deriv;             // 0: snapshot j has no stiffness terms (only density terms)
+    // point sources added to the new level, receivers read from the current one
+    const PointTable* points;
+    const float* inj_trace;
+    float* rec_trace;          // null: no receivers
+    int nrec;
 };
 
 struct ImageArgs {
@@ -100,27 +119,13 @@ int tiles_z(int ldz);
 void tile_range_x(int k, int ntile, int T, int n, int& s, int& e);
 void tile_range_z(int k, int ntile, int nz, int ldz, int& s, int& e);
 
-// one time step of every shot over the tile grid
-void launch_step(const StepArgs& a, bool vti, int tile_x, bool image, hipStream_t s);
-void launch_init_prev(float* prev, long long shot_stride, long long nxz, int ldz, int nshots, const int* shot_ptr,
-                      const PointEntry* ents, const float* trace, hipStream_t s);
-void launch_scale_prev(float* prev, const float* rho, float half_dt2, long long nxz, int nshots, hipStream_t s);
-// Density-term share of the point sources of a fused imaging step (by parts in time,
-// on = 0: no imaging): wn f0 . (injected x, z) into the shot's gradient slab at rho_off,
-// the offset of the density component in a slab.
-struct InjImage {
-    int on;
-    float wn;
-    const float* f0;
-    long long fshot_stride;
-    float* grad;
-    long long gslab_stride, rho_off;
-};
-void launch_inject_cells(const InjCell* cells, int ncell, const int* ptr, const long long* ctx, const long long* ctz,
-                         const float* cw, const float* trace, int it, float* next, long long shot_stride,
-                         long long nxz, int nx, int nz, int ldz, const float* irho, const float* taper_x,
-                         const float* taper_z, const float* div_tb, const float* div_lr, const InjImage& im,
-                         hipStream_t s);
+// one time step of every shot over the tile grid, with its ncell point source cells and
+// receivers (a.points)
+void launch_step(const StepArgs& a, bool vti, int tile_x, bool image, int ncell, hipStream_t s);
+// initial condition: prev = 1/2 dt^2 / rho * sum of the cell's contributions at sample 0
+void launch_init_cells(const InjCell* cells, int ncell, const int* ptr, const long long* ctx, const long long* ctz,
+                       const float* cw, const float* trace, float* prev, long long shot_stride, long long nxz, int ldz,
+                       const float* rho, float half_dt2, hipStream_t s);
 // receiver r sums the footprints ents[rptr[r]] .. ents[rptr[r+1]-1] into its traces
 void launch_extract(const float* state, long long shot_stride, long long nxz, int ldz, const PointEntry* ents,
                     const int* rptr, int nrec, float* trace, int it, hipStream_t s);

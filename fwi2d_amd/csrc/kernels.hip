@@ -1091,19 +1091,91 @@ __device__ __forceinline__ void quad_to_lds(const float* src, float* lds_wave)
     __builtin_amdgcn_global_load_lds(src, (__attribute__((address_space(3))) void*)lds_wave, 16, 0, 0);
 }
 
+// receiver component k of 2 nrec (receiver k / 2): its footprints of one level into its trace
+__device__ __forceinline__ void extract_component(int k, const float* state, long long shot_stride, long long nxz,
+                                                  int ldz, const PointEntry* ents, const int* rptr, float* trace,
+                                                  int it)
+{
+    const int r = k >> 1, comp = k & 1;
+    float v = 0.f;
+    long long out = 0;
+    for (int f = rptr[r]; f < rptr[r + 1]; f++) {
+        const PointEntry en = ents[f];
+        const float* u = state + en.shot * shot_stride + comp * nxz;
+        for (int ix = 0; ix < 3; ix++)
+            for (int iz = 0; iz < 3; iz++) v += en.wx[ix] * en.wz[iz] * u[(long long)(en.xi0 + ix) * ldz + en.zi0 + iz];
+        out = comp ? en.tz : en.trace;
+    }
+    if (rptr[r + 1] > rptr[r]) trace[out + it] = v;
+}
+
+// Point sources (we_op.cpp:722-724), added to the new level once it is stored: cells c0, c0 +
+// 256, ... before c1, one thread per touched cell summing its contributions in injector order.  The step
+// forms next = (dt^2/rho (r + s) + 2 curr - prev) / d * taper, which is linear in the
+// source term s, so the sources add dt^2/rho * s / d * taper (d: the absorbing divisor on
+// the perimeter, 1 elsewhere).  img: the imaging fused into the step took the new level before this increment;
+// its share of the density term by parts, wn f0 . (increment), goes to the shot's own slab.
+__device__ __forceinline__ void inject_cells(const StepArgs& a, int c0, int c1, bool img, long long nxz)
+{
+    const PointTable& pt = *a.points;
+    const int nx = a.nx, nz = a.nz, ldz = a.ldz;
+    for (int c = c0; c < c1; c += kThreads) {
+        const InjCell cell = pt.cells[c];
+        float fx = 0.f, fz = 0.f;
+        for (int k = pt.ptr[c]; k < pt.ptr[c + 1]; k++) {
+            fx += pt.w[k] * a.inj_trace[pt.ctx[k] + a.it];
+            fz += pt.w[k] * a.inj_trace[pt.ctz[k] + a.it];
+        }
+        const int gx = cell.gx, gz = cell.gz;
+        const long long g = (long long)gx * ldz + gz;
+        float dx = 1.f, dz = 1.f;
+        if (gz == 0) { dx = a.div_tb[gx]; dz = a.div_tb[nx + gx]; }
+        else if (gz == nz - 1) { dx = a.div_tb[2 * nx + gx]; dz = a.div_tb[3 * nx + gx]; }
+        else if (gx == 0) { dx = a.div_lr[gz]; dz = a.div_lr[ldz + gz]; }
+        else if (gx == nx - 1) { dx = a.div_lr[2 * ldz + gz]; dz = a.div_lr[3 * ldz + gz]; }
+        const float f = a.irho[g] * a.taper_z[gz] * a.taper_x[gx];
+        const float ix = f * fx / dx, iz = f * fz / dz;
+        float* u = a.next + cell.shot * a.shot_stride + g;
+        u[0] += ix;
+        u[nxz] += iz;
+        if (img) {
+            const long long fo = cell.shot * a.fshot_stride + g;
+            a.grad[cell.shot * a.gslab_stride + (a.stiff ? 4 : 2) * nxz + g] +=
+                a.wn * (ix * a.f0[fo] + iz * a.f0[fo + nxz]);
+        }
+    }
+}
+
+// The point sources and receivers of a step in a launch of their own (the sources go into
+// the new level, the receivers read the current one): blocks [0, nsrc) the sources' cells,
+// the others the receivers' components.
+__global__ void __launch_bounds__(kThreads) k_points(const StepArgs a, int ncell, int nsrc, int img)
+{
+    const long long nxz = (long long)a.nx * a.ldz;
+    if ((int)blockIdx.x < nsrc) {
+        const int c = blockIdx.x * kThreads + threadIdx.x;
+        inject_cells(a, c, min(c + 1, ncell), img != 0, nxz);
+    } else {
+        const int k = (blockIdx.x - nsrc) * kThreads + threadIdx.x;
+        if (k < 2 * a.nrec)
+            extract_component(k, a.curr, a.shot_stride, nxz, a.ldz, a.points->rec, a.points->rec_ptr, a.rec_trace, a.it);
+    }
+}
+
 // One tile and shot group of a time step (see above).  EDGE: a frame tile.
 // IMG (the image_fused option; by default the imaging runs in k_img): adjoint step it with
 // the imaging by parts in time fused in (see k_img with SBP): the density term of
 // snapshot j = f0 against wn next + wc curr + wp prev at the cells (prev as stored, before
-// the step's taper; next before the step's point sources, whose share k_inject_cells
+// the step's taper; next before the step's point sources, whose share inject_cells
 // adds), and the stiffness terms of snapshot j-1 = fm, whose derivatives meet those of the
 // step's current level (the reference's lag).  fm's window goes through the LDS of the
 // products once the new level is done.  The gradient contributions of the workgroup's
 // shots are summed in registers and added once per launch to the gradient slab of the
 // group's first shot.
-template <bool VTI, class S, bool EDGE, bool IMG>
+template <bool VTI, class S, bool EDGE, bool IMG, bool PTS>
 __device__ __forceinline__ void step_tile(const StepArgs& a, const StepSmem& sm, int tix, int tiz, int s0, int s1)
 {
+    const int* const tile_ptr = PTS ? a.points->tile_ptr + (tix * a.ntz + tiz) * a.nshots : nullptr;
     // IMG: snapshot fm's window in the product layout, over the products (dead by then)
     float* const sFx = sm.px;
     float* const sFz = sm.qx;
@@ -1227,6 +1299,7 @@ __device__ __forceinline__ void step_tile(const StepArgs& a, const StepSmem& sm,
         // previous level of this shot's new-level quads
         float4 qprx[S::NQ3], qprz[S::NQ3];
         const float* pux = a.prev + shot * a.shot_stride;
+        const int inj0 = PTS ? tile_ptr[shot] : 0, inj1 = PTS ? tile_ptr[shot + 1] : 0;  // the sources' cells
         auto load_prev = [&] {
 #pragma unroll
         for (int m = 0; m < S::NQ3; m++) {
@@ -1485,8 +1558,13 @@ __device__ __forceinline__ void step_tile(const StepArgs& a, const StepSmem& sm,
                                  gm[m], gr[m], g3[VTI ? m : 0]);
             }
         }
+        if (PTS && inj1 > inj0) {
+            __syncthreads();  // the tile's new level is stored
+            inject_cells(a, inj0 + tid, inj1, IMG, nxz);
+        }
     }
     if constexpr (IMG) {
+        if (PTS) __syncthreads();  // the point sources' shares of the first shot are in its slab
         float* G = a.grad + s0 * a.gslab_stride;
 #pragma unroll
         for (int m = 0; m < S::NQ3; m++) {
@@ -1514,7 +1592,8 @@ __device__ __forceinline__ void step_tile(const StepArgs& a, const StepSmem& sm,
 // wavefronts per SIMD the registers must leave room for: the LDS's share
 constexpr int step_waves(bool vti, int tx, bool img) { return tx == 32 ? 2 : (vti || img ? (vti && img ? 2 : 3) : 4); }
 
-template <bool VTI, int TX, bool IMG>
+// PTS: the launch also takes the point sources and receivers (see step_launch).
+template <bool VTI, int TX, bool IMG, bool PTS>
 __global__ void __launch_bounds__(kThreads, step_waves(VTI, TX, IMG)) k_step(const StepArgs a)
 {
     using S = StepShape<TX>;
@@ -1561,12 +1640,19 @@ __global__ void __launch_bounds__(kThreads, step_waves(VTI, TX, IMG)) k_step(con
                      t || b ? S::WZ : 8};
         }
         const int s0 = grp * a.spb_e;
-        step_tile<VTI, S, true, IMG>(a, sm, tix, tiz, s0, min(a.nshots, s0 + a.spb_e));
+        step_tile<VTI, S, true, IMG, PTS>(a, sm, tix, tiz, s0, min(a.nshots, s0 + a.spb_e));
+    } else if (PTS && b >= ne8 + nin * a.ngroups) {
+        // receivers of the current level
+        const PointTable& pt = *a.points;
+        const int k = (b - ne8 - nin * a.ngroups) * kThreads + threadIdx.x;
+        if (k < 2 * pt.nrec)
+            extract_component(k, a.curr, a.shot_stride, (long long)a.nx * a.ldz, a.ldz, pt.rec, pt.rec_ptr, a.rec_trace,
+                              a.it);
     } else {
-        const int lin = xcd_remap(b - ne8, gridDim.x - ne8);
+        const int lin = xcd_remap(b - ne8, nin * a.ngroups);
         const int tile = lin / a.ngroups, grp = lin - tile * a.ngroups;
         const int s0 = grp * a.spb;
-        step_tile<VTI, S, false, IMG>(a, sm, a.itx0 + tile / nin_z, a.itz0 + tile % nin_z, s0,
+        step_tile<VTI, S, false, IMG, PTS>(a, sm, a.itx0 + tile / nin_z, a.itz0 + tile % nin_z, s0,
                                       min(a.nshots, s0 + a.spb));
     }
 }
@@ -1785,96 +1871,34 @@ __global__ void __launch_bounds__(kThreads) k_img(const StepArgs a)
 }
 
 // ---------------------------------------------------------------------------
-// Initial condition: prev = 1/2 dt^2/rho * inject(trace[0])  (we_op.cpp:655-663)
+// Initial condition: prev = 1/2 dt^2/rho * inject(trace[0])  (we_op.cpp:655-663) on a zero
+// level, one thread per touched cell summing its contributions in injector order
 // ---------------------------------------------------------------------------
-__global__ void k_init_prev(float* prev, long long shot_stride, long long nxz, int ldz, const int* shot_ptr,
-                            const PointEntry* ents, const float* trace)
-{
-    // one single-thread block per shot: deterministic accumulation order over its injectors
-    const int s = blockIdx.x;
-    const int b = shot_ptr[s], e = shot_ptr[s + 1];
-    float* px = prev + s * shot_stride;
-    float* pz = px + nxz;
-    for (int k = b; k < e; k++) {
-        const PointEntry en = ents[k];
-        const float vx = trace[en.trace], vz = trace[en.tz];
-        for (int ix = 0; ix < 3; ix++)
-            for (int iz = 0; iz < 3; iz++) {
-                const long long g = (long long)(en.xi0 + ix) * ldz + (en.zi0 + iz);
-                const float w = en.wx[ix] * en.wz[iz];
-                px[g] += w * vx;
-                pz[g] += w * vz;
-            }
-    }
-}
-
-__global__ void k_scale_prev(float* prev, const float* rho, float half_dt2, long long nxz, int nshots)
-{
-    const long long n = 2 * nxz * nshots;
-    for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) {
-        const long long g = i % nxz;
-        prev[i] *= half_dt2 / rho[g];
-    }
-}
-
-// extraction of one level from global memory (used for the last level)
-__global__ void k_extract(const float* state, long long shot_stride, long long nxz, int ldz, const PointEntry* ents,
-                          const int* rptr, int nrec, float* trace, int it)
-{
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= 2 * nrec) return;
-    const int r = k >> 1, comp = k & 1;
-    float v = 0.f;
-    long long out = 0;
-    for (int f = rptr[r]; f < rptr[r + 1]; f++) {
-        const PointEntry en = ents[f];
-        const float* u = state + en.shot * shot_stride + comp * nxz;
-        for (int ix = 0; ix < 3; ix++)
-            for (int iz = 0; iz < 3; iz++) v += en.wx[ix] * en.wz[iz] * u[(long long)(en.xi0 + ix) * ldz + en.zi0 + iz];
-        out = comp ? en.tz : en.trace;
-    }
-    if (rptr[r + 1] > rptr[r]) trace[out + it] = v;
-}
-
-// ---------------------------------------------------------------------------
-// Point sources of a step (we_op.cpp:722-724): added to the new level after the step,
-// one thread per touched cell summing its contributions in a fixed order.  The step
-// forms next = (dt^2/rho (r + s) + 2 curr - prev) / d * taper, which is linear in the
-// source term s, so the sources add dt^2/rho * s / d * taper (d: the absorbing divisor on
-// the perimeter, 1 elsewhere).
-// ---------------------------------------------------------------------------
-__global__ void k_inject_cells(const InjCell* cells, int ncell, const int* ptr, const long long* ctx,
-                               const long long* ctz, const float* cw, const float* trace, int it, float* next,
-                               long long shot_stride, long long nxz, int nx, int nz, int ldz, const float* irho,
-                               const float* taper_x, const float* taper_z, const float* div_tb, const float* div_lr,
-                               const InjImage im)
+__global__ void k_init_cells(const InjCell* cells, int ncell, const int* ptr, const long long* ctx,
+                             const long long* ctz, const float* cw, const float* trace, float* prev,
+                             long long shot_stride, long long nxz, int ldz, const float* rho, float half_dt2)
 {
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= ncell) return;
     const InjCell cell = cells[c];
     float fx = 0.f, fz = 0.f;
     for (int k = ptr[c]; k < ptr[c + 1]; k++) {
-        fx += cw[k] * trace[ctx[k] + it];
-        fz += cw[k] * trace[ctz[k] + it];
+        fx += cw[k] * trace[ctx[k]];
+        fz += cw[k] * trace[ctz[k]];
     }
-    const int gx = cell.gx, gz = cell.gz;
-    const long long g = (long long)gx * ldz + gz;
-    float dx = 1.f, dz = 1.f;
-    if (gz == 0) { dx = div_tb[gx]; dz = div_tb[nx + gx]; }
-    else if (gz == nz - 1) { dx = div_tb[2 * nx + gx]; dz = div_tb[3 * nx + gx]; }
-    else if (gx == 0) { dx = div_lr[gz]; dz = div_lr[ldz + gz]; }
-    else if (gx == nx - 1) { dx = div_lr[2 * ldz + gz]; dz = div_lr[3 * ldz + gz]; }
-    const float f = irho[g] * taper_z[gz] * taper_x[gx];
-    float* u = next + cell.shot * shot_stride + g;
-    const float ix = f * fx / dx, iz = f * fz / dz;
-    u[0] += ix;
-    u[nxz] += iz;
-    if (im.on) {
-        // the fused imaging step took the new level before this increment: add its share
-        // of the density term by parts, wn f0 . (ix, iz), to the shot's own gradient slab
-        const long long fo = cell.shot * im.fshot_stride + g;
-        im.grad[cell.shot * im.gslab_stride + im.rho_off + g] += im.wn * (ix * im.f0[fo] + iz * im.f0[fo + nxz]);
-    }
+    const long long g = (long long)cell.gx * ldz + cell.gz;
+    const float f = half_dt2 / rho[g];
+    float* u = prev + cell.shot * shot_stride + g;
+    u[0] = fx * f;
+    u[nxz] = fz * f;
+}
+
+// extraction of one level (the last one; the others are read by the step that follows them)
+__global__ void k_extract(const float* state, long long shot_stride, long long nxz, int ldz, const PointEntry* ents,
+                          const int* rptr, int nrec, float* trace, int it)
+{
+    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k < 2 * nrec) extract_component(k, state, shot_stride, nxz, ldz, ents, rptr, trace, it);
 }
 
 // ---------------------------------------------------------------------------
@@ -2122,20 +2146,37 @@ static inline int grid_for(long long n, int cap = 4096)
 }
 
 template <bool VTI, int TX>
-static void step_launch(const StepArgs& a, bool image, hipStream_t s)
+static void step_launch(const StepArgs& a, bool image, int ncell, hipStream_t s)
 {
     const int nin = (a.itx1 - a.itx0) * (a.itz1 - a.itz0), ne = (a.ntx * a.ntz - nin) * a.ngroups_e;
-    const dim3 grid(((ne + 7) & ~7) + nin * a.ngroups);
-    if (image) hipLaunchKernelGGL((k_step<VTI, TX, true>), grid, dim3(kThreads), 0, s, a);
-    else hipLaunchKernelGGL((k_step<VTI, TX, false>), grid, dim3(kThreads), 0, s, a);
+    const int nstep = ((ne + 7) & ~7) + nin * a.ngroups;
+    const int nrec = a.rec_trace ? (2 * a.nrec + kThreads - 1) / kThreads : 0;
+    // Point sources and receivers: in the step's launch while its workgroups fit the chip about
+    // once (4 per CU): one shot on 201 x 601 takes 12.4 us a step instead of 14.6 and 8.5 in
+    // launches of their own.  In larger launches the step kernel without their code keeps its
+    // registers: 64 shots of 500 x 1700 took 455 us a step with them in the launch, 392 us and
+    // 8 us for k_points without.
+    if constexpr (TX == 16) {
+        if (nstep <= 1024) {
+            const dim3 grid(nstep + nrec);
+            if (image) hipLaunchKernelGGL((k_step<VTI, TX, true, true>), grid, dim3(kThreads), 0, s, a);
+            else hipLaunchKernelGGL((k_step<VTI, TX, false, true>), grid, dim3(kThreads), 0, s, a);
+            return;
+        }
+    }
+    if (image) hipLaunchKernelGGL((k_step<VTI, TX, true, false>), dim3(nstep), dim3(kThreads), 0, s, a);
+    else hipLaunchKernelGGL((k_step<VTI, TX, false, false>), dim3(nstep), dim3(kThreads), 0, s, a);
+    const int nsrc = (ncell + kThreads - 1) / kThreads;
+    if (nsrc + nrec > 0)
+        hipLaunchKernelGGL(k_points, dim3(nsrc + nrec), dim3(kThreads), 0, s, a, ncell, nsrc, image ? 1 : 0);
 }
 
-void launch_step(const StepArgs& a, bool vti, int tile_x, bool image, hipStream_t s)
+void launch_step(const StepArgs& a, bool vti, int tile_x, bool image, int ncell, hipStream_t s)
 {
-    if (vti && tile_x == 32) step_launch<true, 32>(a, image, s);
-    else if (vti) step_launch<true, 16>(a, image, s);
-    else if (tile_x == 32) step_launch<false, 32>(a, image, s);
-    else step_launch<false, 16>(a, image, s);
+    if (vti && tile_x == 32) step_launch<true, 32>(a, image, ncell, s);
+    else if (vti) step_launch<true, 16>(a, image, ncell, s);
+    else if (tile_x == 32) step_launch<false, 32>(a, image, ncell, s);
+    else step_launch<false, 16>(a, image, ncell, s);
 }
 
 template <bool VTI, int NBUF, bool SBP>
@@ -2179,28 +2220,13 @@ void launch_image(const ImageArgs& a, bool vti, int tile_x, hipStream_t s)
     else image_dispatch<false>(a, tile_x, s);
 }
 
-void launch_init_prev(float* prev, long long shot_stride, long long nxz, int ldz, int nshots, const int* shot_ptr,
-                      const PointEntry* ents, const float* trace, hipStream_t s)
-{
-    hipLaunchKernelGGL(k_init_prev, dim3(nshots), dim3(1), 0, s, prev, shot_stride, nxz, ldz, shot_ptr, ents, trace);
-}
-
-void launch_scale_prev(float* prev, const float* rho, float half_dt2, long long nxz, int nshots, hipStream_t s)
-{
-    hipLaunchKernelGGL(k_scale_prev, dim3(grid_for(2 * nxz * nshots)), dim3(kThreads), 0, s, prev, rho, half_dt2, nxz,
-                       nshots);
-}
-
-void launch_inject_cells(const InjCell* cells, int ncell, const int* ptr, const long long* ctx, const long long* ctz,
-                         const float* cw, const float* trace, int it, float* next, long long shot_stride,
-                         long long nxz, int nx, int nz, int ldz, const float* irho, const float* taper_x,
-                         const float* taper_z, const float* div_tb, const float* div_lr, const InjImage& im,
-                         hipStream_t s)
+void launch_init_cells(const InjCell* cells, int ncell, const int* ptr, const long long* ctx, const long long* ctz,
+                       const float* cw, const float* trace, float* prev, long long shot_stride, long long nxz, int ldz,
+                       const float* rho, float half_dt2, hipStream_t s)
 {
     if (ncell <= 0) return;
-    hipLaunchKernelGGL(k_inject_cells, dim3((ncell + kThreads - 1) / kThreads), dim3(kThreads), 0, s, cells, ncell,
-                       ptr, ctx, ctz, cw, trace, it, next, shot_stride, nxz, nx, nz, ldz, irho, taper_x,
-                       taper_z, div_tb, div_lr, im);
+    hipLaunchKernelGGL(k_init_cells, dim3((ncell + kThreads - 1) / kThreads), dim3(kThreads), 0, s, cells, ncell, ptr,
+                       ctx, ctz, cw, trace, prev, shot_stride, nxz, ldz, rho, half_dt2);
 }
 
 void launch_extract(const float* state, long long shot_stride, long long nxz, int ldz, const PointEntry* ents,
