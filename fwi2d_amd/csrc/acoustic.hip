@@ -41,7 +41,7 @@ struct Acoustic {
     int ns = 0, nr = 0;
     bool model_ready = false;
     long long model_epoch = 0, snap_epoch = -1;
-    DevMem d_K, d_ri, d_kdt2, d_div, d_tx, d_tz;
+    DevMem d_stage, d_K, d_ri, d_kdt2, d_div, d_tx, d_tz;
     DevMem d_lev, d_full, d_gslab, d_gout, d_src, d_rcv, d_adj;
     // snapshot segments: checkpoints, the segment buffer, recompute levels, the forward
     // run's source traces
@@ -102,29 +102,16 @@ struct Acoustic {
     // cell takes v dt / (2 h H0) from each absorbing side it lies on)
     void set_model(const float* m)
     {
-        const int nx = g.nx, nz = g.nz;
-        std::vector<float> K(nxz, 0.f), ri(nxz, 0.f), kd(nxz, 0.f), dv(nxz, 1.f);
-        const bool ab[4] = {g.bc_top == 2, g.bc_bottom == 2, g.bc_left == 2, g.bc_right == 2};
-        for (int ix = 0; ix < nx; ix++)
-            for (int iz = 0; iz < nz; iz++) {
-                const long long i = (long long)ix * ldz + iz;
-                const float k = m[(long long)ix * nz + iz], r = m[(long long)nx * nz + (long long)ix * nz + iz];
-                if (!(k > 0) || !(r > 0)) throw std::runtime_error("K and 1/rho must be positive");
-                K[i] = k;
-                ri[i] = r;
-                kd[i] = (float)(g.dt * g.dt * (double)k);
-                const double v = std::sqrt((double)k * r) * g.dt, h0 = kHWeights[0];
-                double s = 0;
-                if (ab[0] && iz == 0) s += v / (2 * g.dz * h0);
-                if (ab[1] && iz == nz - 1) s += v / (2 * g.dz * h0);
-                if (ab[2] && ix == 0) s += v / (2 * g.dx * h0);
-                if (ab[3] && ix == nx - 1) s += v / (2 * g.dx * h0);
-                dv[i] = (float)(1 + s);
-            }
-        up(d_K, K.data(), K.size() * sizeof(float));
-        up(d_ri, ri.data(), ri.size() * sizeof(float));
-        up(d_kdt2, kd.data(), kd.size() * sizeof(float));
-        up(d_div, dv.data(), dv.size() * sizeof(float));
+        const size_t n = (size_t)2 * g.nx * g.nz;
+        bool positive = true;
+        for (size_t i = 0; i < n; i++) positive &= m[i] > 0;
+        if (!positive) throw std::runtime_error("K and 1/rho must be positive");
+        up(d_stage, m, n * sizeof(float));
+        for (DevMem* d : {&d_K, &d_ri, &d_kdt2, &d_div}) d->reserve((size_t)nxz * sizeof(float));
+        const int4 ab = make_int4(g.bc_top == 2, g.bc_bottom == 2, g.bc_left == 2, g.bc_right == 2);
+        launch_amodel(d_stage.as<float>(), g.nx, g.nz, ldz, g.dt, 1.0 / (2 * g.dx * kHWeights[0]),
+                      1.0 / (2 * g.dz * kHWeights[0]), ab, d_K.as<float>(), d_ri.as<float>(), d_kdt2.as<float>(),
+                      d_div.as<float>(), st);
         HIPCHECK(hipStreamSynchronize(st));
         model_ready = true;
         model_epoch++;
@@ -503,12 +490,12 @@ struct Acoustic {
         d_gslab.reserve((size_t)groups * 2 * nxz * sizeof(float));
         launch_fill(d_gslab.as<float>(), (long long)groups * 2 * nxz, 0.f, st);
         propagate(true, inj_rcv, dadj, nullptr, false);
-        d_gout.reserve((size_t)2 * nxz * sizeof(float));
-        launch_sum_shots(d_gslab.as<float>(), 2 * nxz, groups, 2 * nxz, d_gout.as<float>(), 0, st);
-        // [2][nx][ldz] -> [2][nx][nz]
-        HIPCHECK(hipMemcpy2DAsync(grad, (size_t)g.nz * sizeof(float), d_gout.p, (size_t)ldz * sizeof(float),
-                                  (size_t)g.nz * sizeof(float), (size_t)2 * g.nx,
-                                  grad_dev ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost, st));
+        const size_t ngrad = (size_t)2 * g.nx * g.nz;
+        if (!grad_dev) d_gout.reserve(ngrad * sizeof(float));
+        float* out = grad_dev ? grad : d_gout.as<float>();
+        launch_sum_slabs(d_gslab.as<float>(), 2 * nxz, groups, 2LL * g.nx, g.nz, ldz, out, st);
+        if (!grad_dev)
+            HIPCHECK(hipMemcpyAsync(grad, out, ngrad * sizeof(float), hipMemcpyDeviceToHost, st));
         HIPCHECK(hipStreamSynchronize(st));
         HIPCHECK(hipGetLastError());
     }

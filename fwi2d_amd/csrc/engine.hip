@@ -84,7 +84,7 @@ struct Engine {
     bool vti = false;
 
     DevMem d_model, d_deriv, d_closure, d_div_tb, d_div_lr, d_tx, d_tz;
-    std::vector<float> h_model, h_deriv;  // h_deriv: dt^2/rho[, (1+2eps) mu, (1+2eps) lambda], [nd][nx][nz]
+    DevMem d_stage;  // the model as it was given, [np][nx][nz]
     long long model_epoch = 0, ckpt_epoch = -1;
 
     // acquisition
@@ -217,18 +217,23 @@ struct Engine {
     // Divisors 1 + c dt/(2 h h0) of the absorbing boundaries, with the corner
     // accumulation of esat_scale_boundaries / vtisat_scale_boundaries
     // (spatial_operators.cpp:307-521) for the full grid.
-    void build_divisors()
+    void build_divisors(const float* m)
     {
         const int nx = g.nx, nz = g.nz;
         const long long nc = (long long)nx * nz;  // host model is [np][nx][nz]
-        const float* la = h_model.data();
+        const float* la = m;
         const float* mu = la + nc;
         const float* rho = la + 2 * nc;
         const float* eps = vti ? la + 4 * nc : nullptr;
-        std::vector<double> dvx(nc, 1.0), dvz(nc, 1.0);
+        // of the perimeter cells only: top row, bottom row, left and right columns between them
+        std::vector<double> dvx(2 * ((size_t)nx + nz), 1.0), dvz(2 * ((size_t)nx + nz), 1.0);
+        auto at = [&](long long i) -> size_t {
+            const int ix = (int)(i / nz), iz = (int)(i % nz);
+            return iz == 0 ? ix : iz == nz - 1 ? nx + ix : ix == 0 ? 2 * nx + iz : 2 * nx + nz + iz;
+        };
         const double h0 = kH0, dt = g.dt, dx = g.dx, dz = g.dz;
         auto vpx2 = [&](long long i) { return (vti ? (1 + 2 * (double)eps[i]) : 1.0) * ((double)la[i] + 2 * (double)mu[i]); };
-        auto scale = [&](long long i, double sx, double sz) { dvx[i] = 1 + sx; dvz[i] = 1 + sz; };
+        auto scale = [&](long long i, double sx, double sz) { dvx[at(i)] = 1 + sx; dvz[at(i)] = 1 + sz; };
         const bool top = g.bc_top == 2, bottom = g.bc_bottom == 2, left = g.bc_left == 2, right = g.bc_right == 2;
         double sc1x = 0, sc1z = 0, sc2x = 0, sc2z = 0;
         if (top) {
@@ -296,16 +301,18 @@ struct Engine {
         // perimeter arrays: top row and bottom row (corners included), left and right columns
         std::vector<float> tb(4 * (size_t)nx), lr(4 * (size_t)ldz, 1.f);
         for (int ix = 0; ix < nx; ix++) {
-            tb[ix] = (float)dvx[(long long)ix * nz];
-            tb[nx + ix] = (float)dvz[(long long)ix * nz];
-            tb[2 * nx + ix] = (float)dvx[(long long)ix * nz + nz - 1];
-            tb[3 * nx + ix] = (float)dvz[(long long)ix * nz + nz - 1];
+            const long long t = (long long)ix * nz;
+            tb[ix] = (float)dvx[at(t)];
+            tb[nx + ix] = (float)dvz[at(t)];
+            tb[2 * nx + ix] = (float)dvx[at(t + nz - 1)];
+            tb[3 * nx + ix] = (float)dvz[at(t + nz - 1)];
         }
         for (int iz = 0; iz < nz; iz++) {
-            lr[iz] = (float)dvx[iz];
-            lr[ldz + iz] = (float)dvz[iz];
-            lr[2 * ldz + iz] = (float)dvx[(long long)(nx - 1) * nz + iz];
-            lr[3 * ldz + iz] = (float)dvz[(long long)(nx - 1) * nz + iz];
+            const long long r = (long long)(nx - 1) * nz + iz;
+            lr[iz] = (float)dvx[at(iz)];
+            lr[ldz + iz] = (float)dvz[at(iz)];
+            lr[2 * ldz + iz] = (float)dvx[at(r)];
+            lr[3 * ldz + iz] = (float)dvz[at(r)];
         }
         d_div_tb.reserve(tb.size() * sizeof(float));
         d_div_lr.reserve(lr.size() * sizeof(float));
@@ -316,52 +323,30 @@ struct Engine {
 
     void set_model(const float* m)
     {
+        // one contiguous copy, and the padded fields and the step's factors on the device (a
+        // 2-D copy from pageable memory goes column by column: 20 ms of a 601 x 201 model's set)
         const size_t n = (size_t)np * g.nx * g.nz;  // host model is [np][nx][nz]
-        for (size_t i = 0; i < n; i++)
-            if (!std::isfinite(m[i])) throw std::runtime_error("model contains a non-finite value");
-        h_model.assign(m, m + n);
+        bool finite = true, positive = true;
+        for (size_t i = 0; i < n; i++) finite &= std::fabs(m[i]) <= 3.4028235e38f;
+        if (!finite) throw std::runtime_error("model contains a non-finite value");
         const long long nc = (long long)g.nx * g.nz;
-        const float* rho = m + 2 * nc;
-        const float* mu = m + nc;
-        for (long long i = 0; i < nc; i++)
-            if (!(rho[i] > 0) || !(mu[i] > 0)) throw std::runtime_error("model must have rho > 0 and mu > 0");
-        // device copy with z pitch ldz; padding cells hold lambda = mu = c13 = eps = 0, rho = 1
+        for (long long i = 0; i < nc; i++) positive &= (m[nc + i] > 0) & (m[2 * nc + i] > 0);
+        if (!positive) throw std::runtime_error("model must have rho > 0 and mu > 0");
+        d_stage.reserve(n * sizeof(float));
+        HIPCHECK(hipMemcpyAsync(d_stage.p, m, n * sizeof(float), hipMemcpyHostToDevice, st));
         d_model.reserve((size_t)np * nxz * sizeof(float));
-        for (int c = 0; c < np; c++) launch_fill(d_model.as<float>() + c * nxz, nxz, c == 2 ? 1.f : 0.f, st);
-        HIPCHECK(hipMemcpy2DAsync(d_model.p, (size_t)ldz * sizeof(float), m, (size_t)g.nz * sizeof(float),
-                                  (size_t)g.nz * sizeof(float), (size_t)np * g.nx, hipMemcpyHostToDevice, st));
-        // per-cell factors of the step, formed in double and rounded once
-        // VTI imaging factors (we_op.cpp:1510-1519): delta recovered from c13, then
-        // d c13 / d lambda and d c13 / d mu
-        const int nd = vti ? 6 : 1;
-        h_deriv.resize((size_t)nd * nc);
-        for (long long i = 0; i < nc; i++) {
-            h_deriv[i] = (float)(g.dt * g.dt / (double)rho[i]);
-            if (vti) {
-                const double l = m[i], u = mu[i], c = m[3 * nc + i];
-                const double e = 1.0 + 2.0 * (double)m[4 * nc + i];
-                h_deriv[nc + i] = (float)(e * u);
-                h_deriv[2 * nc + i] = (float)(e * l);
-                const double del = ((c + u) * (c + u) - (l + u) * (l + u)) / (2.0 * (l + u) * (l + 2.0 * u));
-                const double v1 = std::sqrt(2.0 * (l + 2.0 * u) * (l + u) * del + (l + u) * (l + u));
-                h_deriv[3 * nc + i] = (float)e;
-                h_deriv[4 * nc + i] = (float)(((1.0 + 2.0 * del) * l + (1.0 + 3.0 * del) * u) / v1);
-                h_deriv[5 * nc + i] = (float)(((1.0 + 3.0 * del) * l + (1.0 + 4.0 * del) * u) / v1 - 1.0);
-            }
-        }
-        d_deriv.reserve((size_t)nd * nxz * sizeof(float));
-        launch_fill(d_deriv.as<float>(), nd * nxz, 0.f, st);
-        HIPCHECK(hipMemcpy2DAsync(d_deriv.p, (size_t)ldz * sizeof(float), h_deriv.data(), (size_t)g.nz * sizeof(float),
-                                  (size_t)g.nz * sizeof(float), (size_t)nd * g.nx, hipMemcpyHostToDevice, st));
-        build_divisors();
-        build_closures();
+        d_deriv.reserve((size_t)(vti ? 6 : 1) * nxz * sizeof(float));
+        launch_model(d_stage.as<float>(), np, g.nx, g.nz, ldz, g.dt * g.dt, d_model.as<float>(), d_deriv.as<float>(),
+                     st);
+        build_divisors(m);
+        build_closures(m);
         model_epoch++;
     }
 
     // D2 closure rows of the model (layout in StepArgs: wx[, wxx], wz): the weight of field
     // point j in row r is the sum over the table's entries (r, j, k) of coefficient times
     // model value at point k, formed in double, times 1 / h^2
-    void build_closures()
+    void build_closures(const float* m)
     {
         const int nx = g.nx, nz = g.nz;
         const size_t nwx = (size_t)2 * 6 * 8 * ldz, nwz = (size_t)2 * nx * 6 * 8;
@@ -370,21 +355,24 @@ struct Engine {
         const double rdx2 = 1.0 / (g.dx * g.dx), rdz2 = 1.0 / (g.dz * g.dz);
         std::vector<double> acc(nz);
         for (int f = 0; f < (vti ? 2 : 1); f++) {
-            const float* c = f ? h_deriv.data() + nc : h_model.data() + nc;  // (1 + 2 eps) mu, mu
+            const float *mu = m + nc, *eps = f ? m + 4 * nc : nullptr;  // (1 + 2 eps) mu, mu
             for (int side = 0; side < 2; side++)
                 for (int r = 0; r < 6; r++)
                     for (int j = 0; j < 8; j++) {
                         std::fill(acc.begin(), acc.end(), 0.0);
                         for (const D2Entry& e : kD2ClosureNZ)
                             if (e.row == r && e.point == j) {
-                                const float* p = c + (long long)(side ? nx - 1 - e.coef : e.coef) * nz;
-                                for (int iz = 0; iz < nz; iz++) acc[iz] += e.num / e.den * p[iz];
+                                const long long p = (long long)(side ? nx - 1 - e.coef : e.coef) * nz;
+                                for (int iz = 0; iz < nz; iz++) {
+                                    const double u = mu[p + iz];
+                                    acc[iz] += e.num / e.den * (f ? (float)((1.0 + 2.0 * (double)eps[p + iz]) * u) : u);
+                                }
                             }
                         float* o = w.data() + f * nwx + ((size_t)(side * 6 + r) * 8 + j) * ldz;
                         for (int iz = 0; iz < nz; iz++) o[iz] = (float)(acc[iz] * rdx2);
                     }
         }
-        const float* mu = h_model.data() + nc;
+        const float* mu = m + nc;
         float* wz = w.data() + (vti ? 2 : 1) * nwx;
         for (int side = 0; side < 2; side++)
             for (int ix = 0; ix < nx; ix++) {
@@ -1293,9 +1281,10 @@ struct Engine {
             }
             image(A, 0, dsrc);
         }
-        d_gout.reserve((size_t)np * nxz * sizeof(float));
-        float* out = d_gout.as<float>();
-        launch_sum_shots(d_gshot.as<float>(), (long long)np * nxz, nslab, (long long)np * nxz, out, 0, st);
+        const size_t ngrad = (size_t)np * g.nx * g.nz;
+        if (!grad_dev) d_gout.reserve(ngrad * sizeof(float));
+        float* out = grad_dev ? grad : d_gout.as<float>();
+        launch_sum_slabs(d_gshot.as<float>(), (long long)np * nxz, nslab, (long long)np * g.nx, g.nz, ldz, out, st);
         if (opt_timing) {
             HIPCHECK(hipEventRecord(ev1, st));
             HIPCHECK(hipEventSynchronize(ev1));
@@ -1305,10 +1294,8 @@ struct Engine {
             (void)hipEventDestroy(ev0);
             (void)hipEventDestroy(ev1);
         }
-        // [np][nx][ldz] -> [np][nx][nz]
-        HIPCHECK(hipMemcpy2DAsync(grad, (size_t)g.nz * sizeof(float), out, (size_t)ldz * sizeof(float),
-                                  (size_t)g.nz * sizeof(float), (size_t)np * g.nx,
-                                  grad_dev ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost, st));
+        if (!grad_dev)
+            HIPCHECK(hipMemcpyAsync(grad, out, ngrad * sizeof(float), hipMemcpyDeviceToHost, st));
         HIPCHECK(hipStreamSynchronize(st));
         HIPCHECK(hipGetLastError());
     }

@@ -36,52 +36,114 @@ void check(int rc)
     if (rc) throw std::runtime_error(fwi2d_last_error());
 }
 
-// analyzeModel (we_op.cpp:267-474) for 3 or 5 parameters: bounds, the Vs <= Vp/sqrt(2)
-// and Thomsen-delta admissibility clips, and the propagation time axis.
+// analyzeModel (we_op.cpp:267-474): bounds, the Vs <= Vp/sqrt(2) and Thomsen-delta
+// admissibility clips, and the propagation time axis.
 struct TimeAxis {
     int nt;
     double dt;
     int sub;
 };
 
-TimeAxis analyze_model(const fwi2d_op_desc& d, std::vector<double>& m)
+// f(begin, end) over [0, n) on up to 16 host threads, in equal parts of at least 16384; an
+// exception is rethrown here once every started thread has joined.
+template <class F>
+void parallel_ranges(size_t n, F&& f)
 {
-    const long long n = (long long)d.nx * d.nz;
-    double* vp = m.data();
-    double* vs = vp + n;
-    double* rho = vp + 2 * n;
-    auto clip = [&](double* a, double lo, double hi) {
-        for (long long i = 0; i < n; i++) a[i] = std::max(lo, std::min(hi, a[i]));
+    const size_t hw = std::min(16u, std::max(1u, std::thread::hardware_concurrency()));
+    const size_t parts = std::max<size_t>(1, std::min(hw, n / 16384));
+    if (parts == 1) {
+        f((size_t)0, n);
+        return;
+    }
+    std::mutex mu;
+    std::exception_ptr err;
+    auto work = [&](size_t p) {
+        try {
+            f(n * p / parts, n * (p + 1) / parts);
+        } catch (...) {
+            std::lock_guard<std::mutex> lk(mu);
+            if (!err) err = std::current_exception();
+        }
     };
-    if (d.nparam == 2) {  // acoustic (vp, rho): always clipped (we_op.cpp:399-421)
-        rho = vp + n;
-        clip(vp, d.vpmin, d.vpmax);
-        clip(rho, d.rhomin, d.rhomax);
+    std::vector<std::thread> pool;
+    try {
+        pool.reserve(parts);
+        for (size_t p = 1; p < parts; p++) pool.emplace_back(work, p);
+    } catch (...) {
+        for (auto& t : pool) t.join();
+        throw;
     }
-    if (d.nparam == 5) {
-        double* del = vp + 3 * n;
-        for (long long i = 0; i < n; i++) {
-            const double v1 = -0.5 * (1 - vs[i] * vs[i] / (vp[i] * vp[i]));
-            const double v2 = 2.0 / (vp[i] * vp[i] / (vs[i] * vs[i]) - 1);
-            if (del[i] < v1) del[i] = 0.9999 * v1;
-            else if (del[i] > v2) del[i] = 0.9999 * v2;
-        }
-    }
-    if (d.nparam != 2 && !d.soft_clip) {
-        clip(vp, d.vpmin, d.vpmax);
-        clip(vs, d.vsmin, d.vsmax);
-        clip(rho, d.rhomin, d.rhomax);
-        if (d.nparam == 5) {
-            clip(vp + 3 * n, d.deltamin, d.deltamax);
-            clip(vp + 4 * n, d.epsilonmin, d.epsilonmax);
-        }
-        for (long long i = 0; i < n; i++)
-            if (vp[i] < std::sqrt(2.0) * vs[i]) vs[i] = vp[i] / std::sqrt(2.0001);
-    }
+    work(0);
+    for (auto& t : pool) t.join();
+    if (err) std::rethrow_exception(err);
+}
+
+// analyzeModel's bounds and admissibility clips and convert_model (we_op.cpp:476-494,
+// 1441-1462; acoustic 1863-1881) cell by cell, in double, into out: (vp, vs, rho[, delta, eps])
+// -> (lambda, mu, rho[, c13, eps]), (vp, rho) -> (K = rho vp^2, 1/rho).  Returns the largest
+// velocity of the clipped model; throws for a non-finite input value.
+double analyze_convert(const fwi2d_op_desc& d, const float* in, float* out)
+{
+    const size_t n = (size_t)d.nx * d.nz;
+    auto clip = [](double v, double lo, double hi) { return std::max(lo, std::min(hi, v)); };
     double vmax = -1e300;
-    for (long long i = 0; i < n; i++) vmax = std::max(vmax, vp[i]);
-    if (d.nparam == 5)
-        for (long long i = 0; i < n; i++) vmax = std::max(vmax, vp[i] * std::sqrt(1 + 2 * vp[4 * n + i]));
+    bool finite = true;
+    std::mutex merge;
+    parallel_ranges(n, [&](size_t b, size_t e) {
+        double vm = -1e300;
+        bool ok = true;
+        for (size_t i = b; i < e; i++) {
+            for (int c = 0; c < d.nparam; c++) ok &= std::isfinite(in[c * n + i]);
+            double vp = in[i];
+            if (d.nparam == 2) {  // acoustic (vp, rho): always clipped (we_op.cpp:399-421)
+                vp = clip(vp, d.vpmin, d.vpmax);
+                const double rho = clip(in[n + i], d.rhomin, d.rhomax);
+                vm = std::max(vm, vp);
+                out[i] = (float)(rho * vp * vp);
+                out[n + i] = (float)(1.0 / rho);
+                continue;
+            }
+            double vs = in[n + i], rho = in[2 * n + i], del = 0, eps = 0;
+            if (d.nparam == 5) {
+                del = in[3 * n + i];
+                eps = in[4 * n + i];
+                const double v1 = -0.5 * (1 - vs * vs / (vp * vp));
+                const double v2 = 2.0 / (vp * vp / (vs * vs) - 1);
+                if (del < v1) del = 0.9999 * v1;
+                else if (del > v2) del = 0.9999 * v2;
+            }
+            if (!d.soft_clip) {
+                vp = clip(vp, d.vpmin, d.vpmax);
+                vs = clip(vs, d.vsmin, d.vsmax);
+                rho = clip(rho, d.rhomin, d.rhomax);
+                if (d.nparam == 5) {
+                    del = clip(del, d.deltamin, d.deltamax);
+                    eps = clip(eps, d.epsilonmin, d.epsilonmax);
+                }
+                if (vp < std::sqrt(2.0) * vs) vs = vp / std::sqrt(2.0001);
+            }
+            vm = std::max(vm, vp);
+            if (d.nparam == 5) vm = std::max(vm, vp * std::sqrt(1 + 2 * eps));
+            const double la = rho * (vp * vp - 2 * vs * vs), mu = rho * vs * vs;
+            out[i] = (float)la;
+            out[n + i] = (float)mu;
+            out[2 * n + i] = (float)rho;
+            if (d.nparam == 5) {
+                out[3 * n + i] = (float)(std::sqrt(2 * (la + 2 * mu) * (la + mu) * del + (la + mu) * (la + mu)) - mu);
+                out[4 * n + i] = (float)eps;
+            }
+        }
+        std::lock_guard<std::mutex> lk(merge);
+        vmax = std::max(vmax, vm);
+        finite = finite && ok;
+    });
+    if (!finite) throw std::runtime_error("model contains a non-finite value");
+    return vmax;
+}
+
+// the propagation time axis of analyzeModel (we_op.cpp:430-474) for the largest velocity
+TimeAxis time_axis(const fwi2d_op_desc& d, double vmax)
+{
     const double hmin = std::min(d.dx, d.dz);
     const double tmax = (d.nt_data - 1) * d.dt_data;
     double dt = d.dt;
@@ -96,26 +158,6 @@ TimeAxis analyze_model(const fwi2d_op_desc& d, std::vector<double>& m)
     t.nt = (int)std::lround(tmax / dt) + 1;
     t.sub = d.sub < 0 ? (int)std::lround(d.dt_data / dt) : d.sub;
     return t;
-}
-
-// convert_model (we_op.cpp:476-494, 1441-1462): (vp, vs, rho[, delta, eps]) -> (lambda, mu, rho[, c13, eps]);
-// the acoustic nl_we_op_a::convert_model (we_op.cpp:1863-1881): (vp, rho) -> (K = rho vp^2, 1/rho)
-void convert_model(std::vector<double>& m, int np, long long n)
-{
-    if (np == 2) {
-        for (long long i = 0; i < n; i++) {
-            m[i] = m[n + i] * m[i] * m[i];
-            m[n + i] = 1.0 / m[n + i];
-        }
-        return;
-    }
-    for (long long i = 0; i < n; i++) {
-        const double vp = m[i], vs = m[n + i], rho = m[2 * n + i];
-        const double la = rho * (vp * vp - 2 * vs * vs), mu = rho * vs * vs;
-        m[i] = la;
-        m[n + i] = mu;
-        if (np == 5) m[3 * n + i] = std::sqrt(2 * (la + 2 * mu) * (la + mu) * m[3 * n + i] + (la + mu) * (la + mu)) - mu;
-    }
 }
 
 // sinc_resampler (operator.cpp:808-856, alpha = 0.5) and linear_resampler (760-806):
@@ -514,7 +556,7 @@ struct fwi2d_op {
     std::vector<float> src_prop;    // source traces at the propagation step
     fwi2d::TraceMatrix tm_fwd;      // receiver traces -> data [nt_data][nt]
     fwi2d::TraceMatrix tm_adj;      // data -> adjoint sources [nt][nt_data]
-    bool shots_set = false;
+    std::vector<float> graw;        // raw gradient of the last apply_jacobianT
 
     int np() const { return d.nparam; }
     bool acoustic() const { return d.nparam == 2; }
@@ -522,17 +564,13 @@ struct fwi2d_op {
     int ncd() const { return acoustic() ? 1 : 2; }               // data components
     long long nxz() const { return (long long)d.nx * d.nz; }
 
-    // model (physical) -> analysed + converted float model; sets the time axis
-    std::vector<float> prepare(const float* pmod)
+    // model (physical) -> analysed + converted float model, in `conv`; sets the time axis
+    std::vector<float> conv;
+    const std::vector<float>& prepare(const float* pmod)
     {
-        const long long n = nxz();
-        std::vector<double> m(pmod, pmod + (size_t)np() * n);
-        for (double v : m)
-            if (!std::isfinite(v)) throw std::runtime_error("model contains a non-finite value");
-        TimeAxis t = analyze_model(d, m);
-        convert_model(m, np(), n);
-        ensure_engine(t);
-        return std::vector<float>(m.begin(), m.end());
+        conv.resize((size_t)np() * nxz());
+        ensure_engine(time_axis(d, analyze_convert(d, pmod, conv.data())));
+        return conv;
     }
 
     void ensure_engine(const TimeAxis& t)
@@ -626,7 +664,7 @@ struct fwi2d_op {
 
     void apply_forward(bool add, const float* pmod, float* pdat)
     {
-        std::vector<float> m = prepare(pmod);
+        const std::vector<float>& m = prepare(pmod);
         if (nr == 0) {  // no traces: the run only leaves checkpoints
             std::vector<float> rcv;
             run_forward(m, rcv);
@@ -635,21 +673,23 @@ struct fwi2d_op {
         set_model(m);
         ckpt_model.clear();
         const size_t n = (size_t)ncd() * nr * d.nt_data;
-        std::vector<float> out(n);
+        std::vector<float> sum(add ? n : 0);
+        float* out = add ? sum.data() : pdat;
         const bool keep = axis.sub > 0;
-        if (acoustic()) fwi2d::acoustic_forward_traces(aeng, src_prop.data(), keep, tm_fwd, out.data());
-        else fwi2d::engine_forward_traces(eng, src_prop.data(), keep, tm_fwd, out.data());
+        if (acoustic()) fwi2d::acoustic_forward_traces(aeng, src_prop.data(), keep, tm_fwd, out);
+        else fwi2d::engine_forward_traces(eng, src_prop.data(), keep, tm_fwd, out);
         if (keep) ckpt_model = m;
-        for (size_t i = 0; i < n; i++) pdat[i] = add ? pdat[i] + out[i] : out[i];
+        if (add)
+            for (size_t i = 0; i < n; i++) pdat[i] += out[i];
     }
 
     void apply_jacobianT(bool add, float* pmod, const float* pmod0, const float* pdat)
     {
-        std::vector<float> m = prepare(pmod0);
+        const std::vector<float>& m = prepare(pmod0);
         if (axis.sub <= 0) throw std::runtime_error("apply_jacobianT needs sub != 0");
-        const long long n = nxz();
-        const int ng = acoustic() ? 2 : 3;  // raw gradient fields
-        std::vector<float> graw((size_t)(acoustic() ? 2 : np()) * n, 0.f);
+        const size_t n = (size_t)nxz();
+        const bool ac = acoustic();
+        graw.resize((size_t)(ac ? 2 : np()) * n);
         if (nr > 0) {  // no traces: no adjoint sources, a zero gradient
             if (ckpt_model != m) {  // no checkpoints of this model: run the forward first
                 std::vector<float> rcv;
@@ -657,34 +697,32 @@ struct fwi2d_op {
             }
             // (DAS channels: the device maps strain to gauge-end differences first,
             // dipole_to_strain's adjoint; it commutes with the per-trace time map)
-            if (acoustic()) fwi2d::acoustic_adjoint_traces(aeng, pdat, tm_adj, graw.data());
+            if (ac) fwi2d::acoustic_adjoint_traces(aeng, pdat, tm_adj, graw.data());
             else fwi2d::engine_adjoint_traces(eng, pdat, tm_adj, graw.data());
-        }
-        // H quadrature (we_op.cpp:1192-1199) and chain rule (we_op.cpp:1208-1230)
-        std::vector<double> gd(graw.begin(), graw.end());
-        for (int c = 0; c < ng; c++)
-            for (int ix = 0; ix < d.nx; ix++)
-                for (int iz = 0; iz < d.nz; iz++)
-                    gd[c * n + (long long)ix * d.nz + iz] *= h_weight(d.nz, iz) * d.dz * h_weight(d.nx, ix) * d.dx;
-        if (acoustic()) {
-            // (K, 1/rho) -> (vp, rho): g_rho = (1/rho) K g_K - (1/rho)^2 g_1/rho, g_vp = 2 sqrt(K rho) g_K
-            for (long long i = 0; i < n; i++) {
-                const double K = m[i], ri = m[n + i];
-                const double gk = gd[i], gri = gd[n + i];
-                gd[n + i] = ri * K * gk - ri * ri * gri;
-                gd[i] = 2 * std::sqrt(K / ri) * gk;
-            }
         } else {
-            for (long long i = 0; i < n; i++) {
-                const double la = m[i], mu = m[n + i], rho = m[2 * n + i];
-                const double gl = gd[i], gm = gd[n + i], gr = gd[2 * n + i];
-                gd[2 * n + i] = (la / rho) * gl + (mu / rho) * gm + gr;
-                gd[n + i] = 2 * std::sqrt(mu * rho) * (gm - 2 * gl);
-                gd[i] = 2 * std::sqrt(rho * (la + 2 * mu)) * gl;
-            }
-            for (long long i = 3 * n; i < np() * n; i++) gd[i] = 0.0;
+            std::fill(graw.begin(), graw.end(), 0.f);
         }
-        for (long long i = 0; i < np() * n; i++) pmod[i] = (float)((add ? (double)pmod[i] : 0.0) + gd[i]);
+        // H quadrature (we_op.cpp:1192-1199) and chain rule (we_op.cpp:1208-1230), cell by cell
+        parallel_ranges(n, [&](size_t b, size_t e) {
+            auto put = [&](size_t i, double v) { pmod[i] = (float)((add ? (double)pmod[i] : 0.0) + v); };
+            for (size_t i = b; i < e; i++) {
+                const int ix = (int)(i / d.nz), iz = (int)(i - (size_t)ix * d.nz);
+                const double h = h_weight(d.nz, iz) * d.dz * h_weight(d.nx, ix) * d.dx;
+                if (ac) {
+                    // (K, 1/rho) -> (vp, rho): g_rho = (1/rho) K g_K - (1/rho)^2 g_1/rho, g_vp = 2 sqrt(K rho) g_K
+                    const double K = m[i], ri = m[n + i], gk = graw[i] * h, gri = graw[n + i] * h;
+                    put(n + i, ri * K * gk - ri * ri * gri);
+                    put(i, 2 * std::sqrt(K / ri) * gk);
+                } else {
+                    const double la = m[i], mu = m[n + i], rho = m[2 * n + i];
+                    const double gl = graw[i] * h, gm = graw[n + i] * h, gr = graw[2 * n + i] * h;
+                    put(2 * n + i, (la / rho) * gl + (mu / rho) * gm + gr);
+                    put(n + i, 2 * std::sqrt(mu * rho) * (gm - 2 * gl));
+                    put(i, 2 * std::sqrt(rho * (la + 2 * mu)) * gl);
+                    for (int c = 3; c < np(); c++) put(c * n + i, 0.0);
+                }
+            }
+        });
     }
 
     ~fwi2d_op()
@@ -711,6 +749,7 @@ struct fwi2d_nlls {
     std::vector<float> gmask;  // gradient mask, empty: none
     TraceFilter filt;          // prepared filter, empty: none
     std::vector<float> r;      // residual of the last evaluation
+    std::vector<float> u, af, gr;  // workspaces of evaluate: modelled data, adjoint source, gradient
     double dnorm = 1.0;        // nlls_fwi_eco's data norm (optimization.hpp:569-574), else 1
     size_t ndata = 0, nmodel = 0;
 
@@ -777,11 +816,11 @@ struct fwi2d_nlls {
         const int n = nt();
         const double dt = op->d.dt_data;
         const size_t T = ntr();
-        std::vector<float> u(ndata);
+        u.resize(ndata);
         op->apply_forward(false, m, u.data());
         r.resize(ndata);
         std::vector<double> fpart(T);
-        std::vector<float> af(g ? ndata : 0);
+        if (g) af.resize(ndata);
         // trace by trace (each independent, so the result does not depend on the threads):
         // res (optimization.hpp:346-374, 660-776): r = P(F(m)) - P(d), P the processing;
         // the trace's share of getFunc (optimization.hpp:375-385, 929-942):
@@ -849,10 +888,11 @@ struct fwi2d_nlls {
             *func = 0.5 * dt * f / dnorm;
         }
         if (!g) return;
-        std::vector<float> gr(nmodel);
+        gr.resize(nmodel);
         op->apply_jacobianT(false, gr.data(), m, af.data());
-        for (size_t i = 0; i < nmodel; i++)
-            g[i] = (float)((gmask.empty() ? 1.0 : (double)gmask[i]) * (gr[i] / dnorm));
+        parallel_ranges(nmodel, [&](size_t b, size_t e) {
+            for (size_t i = b; i < e; i++) g[i] = (float)((gmask.empty() ? 1.0 : (double)gmask[i]) * (gr[i] / dnorm));
+        });
     }
 };
 

@@ -135,8 +135,16 @@ void launch_image(const ImageArgs& a, bool vti, int tile_x, hipStream_t s);
 // one (sbp: the density term by parts, a.aprev the lagged level, see StepArgs); nbuf 2:
 // the next shot's windows load into a second LDS buffer during this shot
 void launch_img(const StepArgs& a, bool vti, int tile_x, int nbuf, bool sbp, hipStream_t s);
-void launch_sum_shots(const float* per_shot, long long shot_stride, int nshots, long long n, float* out,
-                      int accumulate, hipStream_t s);
+// sum of nslab gradient slabs of ncol columns into out, columns unpadded from ldz to nz
+void launch_sum_slabs(const float* slabs, long long stride, int nslab, long long ncol, int nz, int ldz, float* out,
+                      hipStream_t s);
+// device fields of a model on the device: elastic [np][nx][nz] into the padded fields and the
+// step's factors; acoustic (K, 1/rho) into K, 1/rho, dt^2 K and the boundary divisors (fx, fz:
+// 1 / (2 h H0))
+void launch_model(const float* m, int np, int nx, int nz, int ldz, double dt2, float* model, float* deriv,
+                  hipStream_t s);
+void launch_amodel(const float* m, int nx, int nz, int ldz, double dt, double fx, double fz, int4 ab, float* K,
+                   float* ri, float* kd, float* dv, hipStream_t s);
 void launch_fill(float* p, long long n, float v, hipStream_t s);
 // out [ntr][nrow] = per-trace row-compressed matrix (ptr [nrow + 1], col, w) times in [ntr][ncol]
 void launch_trace_matvec(const int* ptr, const int* col, const double* w, int nrow, int ncol, const float* in,

@@ -1993,12 +1993,75 @@ __global__ void __launch_bounds__(kThreads) k_image(const ImageArgs a)
 // ---------------------------------------------------------------------------
 // Utilities
 // ---------------------------------------------------------------------------
-__global__ void k_sum_shots(const float* per_shot, long long shot_stride, int nshots, long long n, float* out, int acc)
+// sum of the gradient slabs in slab order; columns of ldz cells in, of nz out
+__global__ void k_sum_slabs(const float* slabs, long long stride, int nslab, long long ncol, int nz, int ldz,
+                            float* out)
 {
+    const long long n = ncol * nz;
     for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) {
-        float v = acc ? out[i] : 0.f;
-        for (int s = 0; s < nshots; s++) v += per_shot[s * shot_stride + i];
+        const long long c = i / nz, p = c * ldz + (i - c * nz);
+        float v = 0.f;
+        for (int s = 0; s < nslab; s++) v += slabs[s * stride + p];
         out[i] = v;
+    }
+}
+
+// The elastic model's device fields from the model [np][nx][nz]: the padded fields (padding
+// cells hold lambda = mu = c13 = eps = 0, rho = 1), and the per-cell factors of the step,
+// formed in double and rounded once: dt^2 / rho and, VTI, (1 + 2 eps) mu, (1 + 2 eps) lambda
+// and the imaging factors 1 + 2 eps, d c13 / d lambda, d c13 / d mu (we_op.cpp:1510-1519, delta
+// recovered from c13); zero in the padding.
+__global__ void k_model(const float* m, int np, int nx, int nz, int ldz, double dt2, float* model, float* deriv)
+{
+    const long long nc = (long long)nx * nz, nxz = (long long)nx * ldz;
+    for (long long p = blockIdx.x * (long long)blockDim.x + threadIdx.x; p < nxz;
+         p += (long long)gridDim.x * blockDim.x) {
+        const long long ix = p / ldz;
+        const int iz = (int)(p - ix * ldz);
+        const bool in = iz < nz;
+        const long long i = ix * nz + iz;
+        for (int c = 0; c < np; c++) model[c * nxz + p] = in ? m[c * nc + i] : (c == 2 ? 1.f : 0.f);
+        deriv[p] = in ? (float)(dt2 / (double)m[2 * nc + i]) : 0.f;
+        if (np == 5) {
+            float d[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
+            if (in) {
+                const double l = m[i], u = m[nc + i], c = m[3 * nc + i], e = 1.0 + 2.0 * (double)m[4 * nc + i];
+                const double del = ((c + u) * (c + u) - (l + u) * (l + u)) / (2.0 * (l + u) * (l + 2.0 * u));
+                const double v1 = sqrt(2.0 * (l + 2.0 * u) * (l + u) * del + (l + u) * (l + u));
+                d[0] = (float)(e * u);
+                d[1] = (float)(e * l);
+                d[2] = (float)e;
+                d[3] = (float)(((1.0 + 2.0 * del) * l + (1.0 + 3.0 * del) * u) / v1);
+                d[4] = (float)(((1.0 + 3.0 * del) * l + (1.0 + 4.0 * del) * u) / v1 - 1.0);
+            }
+            for (int k = 0; k < 5; k++) deriv[(k + 1) * nxz + p] = d[k];
+        }
+    }
+}
+
+// The acoustic model's device fields from (K, 1/rho) [2][nx][nz]: both padded with zeros, the
+// leapfrog factor dt^2 K, and the divisors of the absorbing sides (asat_scale_boundaries,
+// spatial_operators.cpp:779-860: a boundary cell takes v dt / (2 h H0) from each absorbing side
+// it lies on; ab: top, bottom, left, right), formed in double.
+__global__ void k_amodel(const float* m, int nx, int nz, int ldz, double dt, double fx, double fz, int4 ab, float* K,
+                         float* ri, float* kd, float* dv)
+{
+    const long long nc = (long long)nx * nz, nxz = (long long)nx * ldz;
+    for (long long p = blockIdx.x * (long long)blockDim.x + threadIdx.x; p < nxz;
+         p += (long long)gridDim.x * blockDim.x) {
+        const int ix = (int)(p / ldz), iz = (int)(p - (long long)ix * ldz);
+        const bool in = iz < nz;
+        const long long i = (long long)ix * nz + iz;
+        const double k = in ? (double)m[i] : 0.0, r = in ? (double)m[nc + i] : 0.0, v = sqrt(k * r) * dt;
+        double s = 0;
+        if (ab.x && iz == 0) s += v * fz;
+        if (ab.y && iz == nz - 1) s += v * fz;
+        if (ab.z && ix == 0) s += v * fx;
+        if (ab.w && ix == nx - 1) s += v * fx;
+        K[p] = (float)k;
+        ri[p] = (float)r;
+        kd[p] = (float)(dt * dt * k);
+        dv[p] = (float)(1 + s);
     }
 }
 
@@ -2237,10 +2300,25 @@ void launch_extract(const float* state, long long shot_stride, long long nxz, in
                        shot_stride, nxz, ldz, ents, rptr, nrec, trace, it);
 }
 
-void launch_sum_shots(const float* per_shot, long long shot_stride, int nshots, long long n, float* out, int acc,
+void launch_sum_slabs(const float* slabs, long long stride, int nslab, long long ncol, int nz, int ldz, float* out,
                       hipStream_t s)
 {
-    hipLaunchKernelGGL(k_sum_shots, dim3(grid_for(n)), dim3(kThreads), 0, s, per_shot, shot_stride, nshots, n, out, acc);
+    hipLaunchKernelGGL(k_sum_slabs, dim3(grid_for(ncol * nz)), dim3(kThreads), 0, s, slabs, stride, nslab, ncol, nz,
+                       ldz, out);
+}
+
+void launch_model(const float* m, int np, int nx, int nz, int ldz, double dt2, float* model, float* deriv,
+                  hipStream_t s)
+{
+    hipLaunchKernelGGL(k_model, dim3(grid_for((long long)nx * ldz)), dim3(kThreads), 0, s, m, np, nx, nz, ldz, dt2,
+                       model, deriv);
+}
+
+void launch_amodel(const float* m, int nx, int nz, int ldz, double dt, double fx, double fz, int4 ab, float* K,
+                   float* ri, float* kd, float* dv, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_amodel, dim3(grid_for((long long)nx * ldz)), dim3(kThreads), 0, s, m, nx, nz, ldz, dt, fx, fz,
+                       ab, K, ri, kd, dv);
 }
 
 void launch_fill(float* p, long long n, float v, hipStream_t s)
