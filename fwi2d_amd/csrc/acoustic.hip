@@ -3,13 +3,15 @@
 //
 // One pressure-like field per shot, [shot][nx][ldz] with ldz = nz rounded up to a quad;
 // model (K, 1/rho) = (rho vp^2, 1/rho) as convert_model (we_op.cpp:1863-1881) produces
-// it.  A time step is one launch over 32 x 32 tiles of every shot (k_astep), then the
-// point sources (k_ainject).  The forward run keeps every sub-th level on the device (the
+// it.  A time step is one launch over 32 x 32 tiles of every shot (k_astep), point sources and
+// receivers included.  The forward run keeps every sub-th level on the device (the
 // reference's full wavefield) when that history fits the snapshot budget, and otherwise
 // checkpoints of segments of about sqrt(2 nsnap) snapshots from which the adjoint run
-// recomputes them, one segment at a time; the adjoint run images them (k_agrad) the way
-// the reference's compute_gradients does, into one gradient slab per shot that are
-// summed at the end.  The reference never ran this operator on a GPU.
+// recomputes them, one segment at a time; a step writes a level that is kept straight into its
+// slot, and the next steps read it there.  The adjoint run images the snapshots the way the
+// reference's compute_gradients does, into one gradient slab per shot group that are summed at
+// the end: with every level kept (sub 1) by parts in time inside the step, otherwise one
+// launch per snapshot (k_agrad).  The reference never ran this operator on a GPU.
 #include <algorithm>
 #include <cmath>
 #include <stdexcept>
@@ -41,22 +43,19 @@ struct Acoustic {
     int ns = 0, nr = 0;
     bool model_ready = false;
     long long model_epoch = 0, snap_epoch = -1;
-    DevMem d_stage, d_K, d_ri, d_kdt2, d_div, d_tx, d_tz;
+    DevMem d_stage, d_K, d_ri, d_kdt2, d_div, d_closure, d_tx, d_tz;
     DevMem d_lev, d_full, d_gslab, d_gout, d_src, d_rcv, d_adj;
     // snapshot segments: checkpoints, the segment buffer, recompute levels, the forward
     // run's source traces
     DevMem d_ckpt, d_seg, d_rlev, d_fsrc;
     long long snapshot_budget_mib = 131072;  // whole snapshot history up to this size (128 GiB)
-    // 1: the adjoint step kernel images the snapshots; 0 (default): k_agrad before the step,
-    // faster: fused, the step kernel holds 151 VGPRs and 42 KB of LDS, 3 wavefronts per SIMD,
-    // and a 64-shot 500 x 1700 adjoint step with imaging takes 566 us against 211 + 300 us
-    int image_fused = 0;
+    int image_fused = 0;  // accepted without effect: the step images the snapshots when sub is 1
     bool whole = true;
     int seg_K = 0, nseg = 0, seg_loaded = -1;
     long long stat_recompute_steps = 0;
     InjList inj_src, inj_rcv;
     std::vector<PointEntry> ext;
-    DevMem d_ext;
+    DevMem d_ext, d_points;
 
     Acoustic(const fwi2d_grid& grid, double stiffness, int dev) : g(grid), device(dev)
     {
@@ -112,6 +111,9 @@ struct Acoustic {
         launch_amodel(d_stage.as<float>(), g.nx, g.nz, ldz, g.dt, 1.0 / (2 * g.dx * kHWeights[0]),
                       1.0 / (2 * g.dz * kHWeights[0]), ab, d_K.as<float>(), d_ri.as<float>(), d_kdt2.as<float>(),
                       d_div.as<float>(), st);
+        d_closure.reserve((2 * 48 * (size_t)ldz + 2 * 48 * (size_t)g.nx) * sizeof(float));
+        launch_closures(d_ri.as<float>(), g.nx, g.nz, ldz, d_closure.as<float>(),
+                        d_closure.as<float>() + 2 * 48 * (size_t)ldz, st);
         HIPCHECK(hipStreamSynchronize(st));
         model_ready = true;
         model_epoch++;
@@ -161,6 +163,18 @@ struct Acoustic {
         inj_rcv.build(re, xt, zt, ntx, ntz, ns, st);
         ext.swap(xe);
         up(d_ext, ext.data(), ext.size() * sizeof(PointEntry));
+        PointTable t[2] = {};  // the forward run's points, the adjoint run's
+        for (int d = 0; d < 2; d++) {
+            InjList& inj = d ? inj_rcv : inj_src;
+            t[d].cells = inj.d_cells.as<InjCell>();
+            t[d].tile_ptr = inj.d_tile_ptr.as<int>();
+            t[d].ptr = inj.d_ptr.as<int>();
+            t[d].ctx = inj.d_ctx.as<long long>();
+            t[d].w = inj.d_cw.as<float>();
+            t[d].rec = d_ext.as<PointEntry>();
+            t[d].nrec = nr;
+        }
+        up(d_points, t, sizeof(t));
         HIPCHECK(hipStreamSynchronize(st));
         snap_epoch = -1;
     }
@@ -183,6 +197,7 @@ struct Acoustic {
         // shots per step workgroup: up to 8 while the launch keeps 2048 or more workgroups
         // (64 shots of 500 x 1700: 8 shots 209 us a step, 16 shots 214 us)
         a.spb = (int)std::max(1LL, std::min(8LL, (long long)ntx * ntz * ns / 2048));
+        a.stream = 3 * state() * (long long)sizeof(float) > kStreamBytes;
         // the rectangle of tiles whose cells are all interior along both axes (no closure
         // rows, no SAT terms): columns 6..nx-7, rows 6..nz-7
         auto interior = [](int n, int t, int ntiles, int& i0, int& i1) {
@@ -213,6 +228,8 @@ struct Acoustic {
         a.ri = d_ri.as<float>();
         a.kdt2 = d_kdt2.as<float>();
         a.div = d_div.as<float>();
+        a.wx = d_closure.as<float>();
+        a.wz = a.wx + 2 * 48 * (size_t)ldz;
         a.taper_x = d_tx.as<float>();
         a.taper_z = d_tz.as<float>();
         a.shot_stride = nxz;
@@ -224,14 +241,15 @@ struct Acoustic {
     // snapshot slots 1 + nt/sub, as the reference allocates its full wavefield
     // (we_op.cpp:923); a slot past the last stored level stays zero
     int nsnap() const { return g.sub > 0 ? 1 + g.nt / g.sub : 0; }
-    float* level(int k) { return d_lev.as<float>() + (long long)k * ns * nxz; }
-    float* snap(int idx) { return d_full.as<float>() + (long long)idx * ns * nxz; }
+    long long state() const { return (long long)ns * nxz; }  // one time level of all shots
+    float* snap(int idx) { return d_full.as<float>() + idx * state(); }
 
     // Segments of K snapshots (K about sqrt(2 nsnap)); segment j owns snapshots jK ..
-    // (j+1)K - 1 and its buffer holds jK - 1 .. (j+1)K (K + 2 slots), every snapshot its
-    // imaging reads.  Segment j >= 1 restarts from the levels (curr, prev) at step
-    // (jK - 1) sub, stored by the forward run, which also keeps the last segment's
-    // snapshots; the adjoint run images the segments last to first, recomputing each.
+    // (j+1)K - 1.  Segment j >= 1 restarts from the levels (curr, prev) at step (jK - 1) sub,
+    // stored by the forward run, which also keeps the last segment's snapshots; the adjoint
+    // run images the segments last to first, recomputing each.  The imaging of sub > 1 reads
+    // both neighbours of a snapshot: jK - 1 is the segment's own checkpoint, and the buffer
+    // holds (j+1)K too (K + 1 slots).
     void plan_segments()
     {
         const int n = nsnap();
@@ -240,128 +258,155 @@ struct Acoustic {
         seg_K = std::max(1, std::min(n, (int)std::ceil(std::sqrt(2.0 * n))));
         nseg = (n + seg_K - 1) / seg_K;
     }
-    int seg_base(int j) const { return std::max(j * seg_K - 1, 0); }
-    int seg_last(int j) const { return std::min((j + 1) * seg_K, nsnap() - 1); }
-    float* slot(int j, int idx) { return d_seg.as<float>() + (long long)(idx - seg_base(j)) * ns * nxz; }
-    float* ckpt(int k) { return d_ckpt.as<float>() + (long long)k * ns * nxz; }
-    // snapshot idx as the imaging of a snapshot of segment j reads it (segment j loaded:
-    // its buffer holds the neighbours jK - 1 and (j+1)K too)
-    float* snapshot(int j, int idx) { return whole ? snap(idx) : slot(j, idx); }
+    bool by_parts() const { return g.sub == 1; }
+    int seg_last(int j) const { return std::min((j + 1) * seg_K - (by_parts() ? 1 : 0), nsnap() - 1); }
+    float* slot(int j, int idx) { return d_seg.as<float>() + (idx - j * seg_K) * state(); }
+    float* ckpt(int k) { return d_ckpt.as<float>() + k * state(); }
+    // snapshot idx as the imaging of a snapshot of segment j (loaded) reads it
+    float* snapshot(int j, int idx)
+    {
+        if (whole) return snap(idx);
+        return idx < j * seg_K ? ckpt(2 * (j - 1)) : slot(j, idx);
+    }
+    int last_written() const { return (g.nt - 1) / g.sub; }  // snapshot slots past it stay zero
 
-    // one step it on levels (p, c, n): the step kernel, then the point sources; with
-    // img_idx >= 0 (adjoint run, the image_fused option) the step kernel also images
-    // snapshot img_idx against c
-    void step(float* p, float* c, float* n, int it, const InjList& inj, const float* tr, int img_idx = -1)
+    // The places that keep level it of the forward run (at most one snapshot slot, a restart
+    // level and a restart's previous level)
+    int kept(int it, float** out)
+    {
+        const int sub = g.sub, idx = it / sub;
+        int n = 0;
+        if (whole) {
+            if (it % sub == 0) out[n++] = snap(idx);
+            return n;
+        }
+        if (it % sub == 0 && idx >= (nseg - 1) * seg_K) out[n++] = slot(nseg - 1, idx);
+        for (int d = 0; d < 2; d++) {  // (jK - 1) sub - d
+            const int l = it + d, j = (l / sub + 1) / seg_K;
+            if (l % sub == 0 && (l / sub + 1) % seg_K == 0 && j >= 1 && j < nseg && l < g.nt - 1)
+                out[n++] = ckpt(2 * (j - 1) + d);
+        }
+        return n;
+    }
+
+    // a level of the scratch buffer lev (three levels) that is neither p nor c
+    float* scratch(float* lev, const float* p, const float* c) const
+    {
+        for (int k = 0; k < 2; k++, lev += state())
+            if (lev != p && lev != c) return lev;
+        return lev;
+    }
+
+    // one step it on levels (p, c, n), with the point sources of the forward or the adjoint run
+    // and its receivers (rcv, may be null); with img_idx >= 0 also images snapshot img_idx by parts
+    void step(float* p, float* c, float* n, int it, bool adjoint, const float* tr, float* rcv = nullptr,
+              int img_idx = -1)
     {
         AcousticArgs a = img_idx >= 0 ? image_args(img_idx) : base_args();
-        a.img = img_idx >= 0;
+        if (img_idx >= 0) {
+            a.img = 1;
+            // weights of the neighbours' adjoint levels; the first step's level is zero and its
+            // previous one the initial condition, so only the next one counts there
+            a.img_deriv = it > 0;
+            const double dtg = g.dt, w = it > 0 ? gdamp_weight(img_idx) : 0.0;
+            a.wk = (float)(w / dtg);
+            a.dwn = (float)((gdamp_weight(img_idx - 1) - w) / dtg);
+            a.dwp = it > 0 ? (float)((gdamp_weight(img_idx + 1) - w) / dtg) : 0.f;
+        }
         a.taper_prev = it > 0;
         a.prev = p;
         a.curr = c;
         a.next = n;
+        a.it = it;
+        a.points = d_points.as<PointTable>() + (adjoint ? 1 : 0);
+        a.inj_trace = tr;
+        a.rec_trace = rcv;
+        a.nrec = nr;
         launch_astep(a, st);
-        launch_ainject(inj.d_cells.as<InjCell>(), (int)inj.cells.size(), inj.d_ptr.as<int>(),
-                       inj.d_ctx.as<long long>(), inj.d_cw.as<float>(), tr, it, n, nxz, ldz, a.kdt2, a.div, a.taper_x,
-                       a.taper_z, false, st);
     }
 
-    // the initial condition prev = 1/2 K dt^2 inject(trace sample 0) (we_op.cpp:1977-1979)
-    // on zeroed levels
-    void init_levels(float* lev, const InjList& inj, const float* tr)
+    // the initial condition (we_op.cpp:1977-1979): p = 1/2 K dt^2 inject(trace sample 0), c = 0
+    void init_levels(float* p, float* c, const InjList& inj, const float* tr)
     {
-        const long long ss = (long long)ns * nxz;
-        launch_fill(lev, 3 * ss, 0.f, st);
-        AcousticArgs a = base_args();
-        launch_ainject(inj.d_cells.as<InjCell>(), (int)inj.cells.size(), inj.d_ptr.as<int>(),
-                       inj.d_ctx.as<long long>(), inj.d_cw.as<float>(), tr, 0, lev, nxz, ldz, a.kdt2, a.div, a.taper_x,
-                       a.taper_z, true, st);
+        launch_fill(p, state(), 0.f, st);
+        launch_fill(c, state(), 0.f, st);
+        launch_ainit(inj.d_cells.as<InjCell>(), (int)inj.cells.size(), inj.d_ptr.as<int>(), inj.d_ctx.as<long long>(),
+                     inj.d_cw.as<float>(), tr, p, nxz, ldz, d_kdt2.as<float>(), st);
+    }
+    void copy_level(float* dst, const float* src)
+    {
+        HIPCHECK(hipMemcpyAsync(dst, src, state() * sizeof(float), hipMemcpyDeviceToDevice, st));
     }
 
     // recompute segment j's snapshots from its checkpoint into the segment buffer
     void load_segment(int j)
     {
         if (seg_loaded == j) return;
-        const long long ss = (long long)ns * nxz;
-        const int sub = g.sub, lastw = (g.nt - 1) / sub;  // last written snapshot
-        const int b = seg_base(j), e = seg_last(j);
-        launch_fill(slot(j, b), (long long)(e - b + 1) * ss, 0.f, st);  // slots past lastw stay zero
-        d_rlev.reserve((size_t)3 * ss * sizeof(float));
+        const int sub = g.sub, b = j * seg_K, e = seg_last(j);
+        if (e > last_written()) launch_fill(slot(j, e), state(), 0.f, st);
+        d_rlev.reserve((size_t)3 * state() * sizeof(float));
         float* R = d_rlev.as<float>();
-        int ip = 0, ic = 1, in = 2, it = 0;
+        float *p = R, *c = R + state();
+        int it = 0;
         if (j == 0) {
-            init_levels(R, inj_src, d_fsrc.as<float>());
+            c = slot(0, 0);
+            init_levels(p, c, inj_src, d_fsrc.as<float>());
         } else {
-            HIPCHECK(hipMemcpyAsync(R + ic * ss, ckpt(2 * (j - 1)), ss * sizeof(float), hipMemcpyDeviceToDevice, st));
-            HIPCHECK(hipMemcpyAsync(R + ip * ss, ckpt(2 * (j - 1) + 1), ss * sizeof(float), hipMemcpyDeviceToDevice, st));
-            it = b * sub;
+            c = ckpt(2 * (j - 1));
+            p = ckpt(2 * (j - 1) + 1);
+            it = (b - 1) * sub;
         }
-        const int end = std::min(e, lastw) * sub;
-        for (;; it++) {
-            if (it % sub == 0 && it / sub >= b)
-                HIPCHECK(hipMemcpyAsync(slot(j, it / sub), R + ic * ss, ss * sizeof(float), hipMemcpyDeviceToDevice, st));
-            if (it >= end) break;
-            step(R + ip * ss, R + ic * ss, R + in * ss, it, inj_src, d_fsrc.as<float>());
+        for (const int end = std::min(e, last_written()) * sub; it < end; it++) {
+            float* n = (it + 1) % sub == 0 && (it + 1) / sub >= b ? slot(j, (it + 1) / sub) : scratch(R, p, c);
+            step(p, c, n, it, false, d_fsrc.as<float>());
             stat_recompute_steps++;
-            const int t = ip;
-            ip = ic;
-            ic = in;
-            in = t;
+            p = c;
+            c = n;
         }
         seg_loaded = j;
     }
 
-    // one propagation (we_op.cpp:1937-2135): sources inj with traces tr; the forward run
-    // extracts into rcv and keeps snapshots (or checkpoints), the adjoint run images them
-    // into the slabs
-    void propagate(bool adjoint, const InjList& inj, const float* tr, float* rcv, bool keep)
+    // the forward run (we_op.cpp:1937-2135): sources with traces tr, receivers into rcv (may be
+    // null), snapshots or checkpoints if keep.  A level that is kept is written where it stays;
+    // further places get copies.
+    void propagate_forward(const float* tr, float* rcv, bool keep)
+    {
+        const int nt = g.nt;
+        d_lev.reserve((size_t)3 * state() * sizeof(float));
+        float *L = d_lev.as<float>(), *p = L, *c = L + state(), *to[3];
+        int nk = keep ? kept(0, to) : 0;
+        if (nk > 0) c = to[0];
+        init_levels(p, c, inj_src, tr);
+        for (int k = 1; k < nk; k++) copy_level(to[k], c);
+        for (int it = 0; it < nt - 1; it++) {
+            nk = keep ? kept(it + 1, to) : 0;
+            float* n = nk > 0 ? to[0] : scratch(L, p, c);
+            step(p, c, n, it, false, tr, rcv);
+            for (int k = 1; k < nk; k++) copy_level(to[k], n);
+            p = c;
+            c = n;
+        }
+        if (rcv) launch_aextract(c, nxz, ldz, d_ext.as<PointEntry>(), nr, rcv, nt - 1, st);
+    }
+
+    // the adjoint run: the same propagation from the receivers with traces tr, imaging the
+    // snapshots into the slabs
+    void propagate_adjoint(const float* tr)
     {
         const int nt = g.nt, sub = g.sub;
-        const long long ss = (long long)ns * nxz;
-        d_lev.reserve((size_t)3 * ss * sizeof(float));
-        init_levels(level(0), inj, tr);
-        int ip = 0, ic = 1, in = 2;
-        const int jlast = nseg - 1;
-        auto capture = [&](int it) {  // forward run: snapshots and checkpoints of level it
-            if (!keep) return;
-            if (whole) {
-                if (it % sub == 0)
-                    HIPCHECK(hipMemcpyAsync(snap(it / sub), level(ic), ss * sizeof(float), hipMemcpyDeviceToDevice, st));
-                return;
-            }
-            if (it % sub == 0 && it / sub >= seg_base(jlast))
-                HIPCHECK(hipMemcpyAsync(slot(jlast, it / sub), level(ic), ss * sizeof(float), hipMemcpyDeviceToDevice,
-                                        st));
-            if (it % sub == 0 && (it / sub + 1) % seg_K == 0 && it / sub + 1 < nseg * seg_K && it < nt - 1) {
-                const int j = (it / sub + 1) / seg_K;  // level (jK - 1) sub starts segment j
-                if (j >= 1 && j < nseg) {
-                    HIPCHECK(hipMemcpyAsync(ckpt(2 * (j - 1)), level(ic), ss * sizeof(float), hipMemcpyDeviceToDevice,
-                                            st));
-                    HIPCHECK(hipMemcpyAsync(ckpt(2 * (j - 1) + 1), level(ip), ss * sizeof(float),
-                                            hipMemcpyDeviceToDevice, st));
-                }
-            }
-        };
+        d_lev.reserve((size_t)3 * state() * sizeof(float));
+        float *L = d_lev.as<float>(), *p = L, *c = L + state();
+        init_levels(p, c, inj_rcv, tr);
         for (int it = 0; it < nt - 1; it++) {
-            int img_idx = -1;
-            if (!adjoint) {
-                capture(it);
-                if (rcv) launch_aextract(level(ic), nxz, ldz, d_ext.as<PointEntry>(), nr, rcv, it, st);
-            } else if ((nt - 1 - it) % sub == 0 && it != 0) {
-                if (image_fused) img_idx = (nt - 1 - it) / sub;
-                else image(level(ic), (nt - 1 - it) / sub);
-            }
-            step(level(ip), level(ic), level(in), it, inj, tr, img_idx);
-            const int t = ip;
-            ip = ic;
-            ic = in;
-            in = t;
+            const int idx = (nt - 1 - it) / sub;
+            if (!by_parts() && (nt - 1 - it) % sub == 0 && it != 0) image(c, idx);
+            float* n = scratch(L, p, c);
+            step(p, c, n, it, true, tr, nullptr, by_parts() ? idx : -1);
+            p = c;
+            c = n;
         }
-        if (!adjoint) {
-            capture(nt - 1);
-            if (rcv) launch_aextract(level(ic), nxz, ldz, d_ext.as<PointEntry>(), nr, rcv, nt - 1, st);
-        } else {
-            image(level(ic), 0);
-        }
+        // snapshot 0 is the zero initial level: by parts, nothing is left for it
+        if (!by_parts()) image(c, 0);
     }
 
     // compute_gradients (we_op.cpp:1883-1935) of snapshot idx with the adjoint level adj
@@ -372,24 +417,32 @@ struct Acoustic {
         launch_agrad(a, st);
     }
 
+    // weight of snapshot idx (the reference's gradient damping in time)
+    double gdamp_weight(int idx) const
+    {
+        const double t = idx * (g.sub * g.dt);
+        double w = 1.0;
+        if (g.gdamp_tmax - t > 0 && t - g.gdamp_tmin >= 0)
+            w = std::cos(g.gdamp_power * M_PI * (t - g.gdamp_tmin) / (g.gdamp_tmax - g.gdamp_tmin));
+        return w * w;
+    }
+
     // the imaging arguments of snapshot idx (its segment loaded first)
     AcousticArgs image_args(int idx)
     {
         AcousticArgs a = base_args();
         const int last = g.nt / g.sub;
-        const double dtg = g.sub * g.dt, t = idx * dtg;
-        double w = 1.0;
-        if (g.gdamp_tmax - t > 0 && t - g.gdamp_tmin >= 0)
-            w = std::cos(g.gdamp_power * M_PI * (t - g.gdamp_tmin) / (g.gdamp_tmax - g.gdamp_tmin));
-        w *= w;
+        const double dtg = g.sub * g.dt, w = gdamp_weight(idx);
         a.mode = (idx > 0 && idx < last) ? 0 : (idx == 0 ? 1 : 2);
         a.wk = (float)(w / dtg);
         a.wr = (float)(idx == 0 ? w * 0.5 * dtg : w * dtg);
         const int j = whole ? 0 : idx / seg_K;
         if (!whole) load_segment(j);
         a.f0 = snapshot(j, idx);
-        a.fm = a.mode != 1 ? snapshot(j, idx - 1) : nullptr;
-        a.fp = a.mode != 2 ? snapshot(j, idx + 1) : nullptr;
+        if (!by_parts()) {
+            a.fm = a.mode != 1 ? snapshot(j, idx - 1) : nullptr;
+            a.fp = a.mode != 2 ? snapshot(j, idx + 1) : nullptr;
+        }
         a.fshot_stride = nxz;
         a.grad = d_gslab.as<float>();
         a.gslab_stride = 2 * nxz;
@@ -450,22 +503,23 @@ struct Acoustic {
         }
         if (keep) {
             plan_segments();
-            const long long ss = (long long)ns * nxz;
+            const long long ss = state();
             if (whole) {
                 d_full.reserve((size_t)nsnap() * ss * sizeof(float));
-                for (int idx = (nt - 1) / g.sub + 1; idx < nsnap(); idx++) launch_fill(snap(idx), ss, 0.f, st);
+                for (int idx = last_written() + 1; idx < nsnap(); idx++) launch_fill(snap(idx), ss, 0.f, st);
             } else {
                 d_ckpt.reserve((size_t)std::max(2 * (nseg - 1), 1) * ss * sizeof(float));
-                d_seg.reserve((size_t)(seg_K + 2) * ss * sizeof(float));
+                d_seg.reserve((size_t)(seg_K + 1) * ss * sizeof(float));
                 const int jl = nseg - 1;
-                launch_fill(slot(jl, seg_base(jl)), (long long)(seg_last(jl) - seg_base(jl) + 1) * ss, 0.f, st);
+                for (int idx = std::max(last_written() + 1, jl * seg_K); idx < nsnap(); idx++)
+                    launch_fill(slot(jl, idx), ss, 0.f, st);
                 // the recomputation re-runs the sources: keep their traces
                 d_fsrc.reserve((size_t)ns * nt * sizeof(float));
                 HIPCHECK(hipMemcpyAsync(d_fsrc.p, dsrc, (size_t)ns * nt * sizeof(float), hipMemcpyDeviceToDevice, st));
                 seg_loaded = jl;
             }
         }
-        propagate(false, inj_src, dsrc, nr > 0 ? drcv : nullptr, keep);
+        propagate_forward(dsrc, nr > 0 ? drcv : nullptr, keep);
         if (!on_device && nr > 0)
             HIPCHECK(hipMemcpyAsync(rcv, drcv, (size_t)nr * nt * sizeof(float), hipMemcpyDeviceToHost, st));
         HIPCHECK(hipStreamSynchronize(st));
@@ -489,7 +543,7 @@ struct Acoustic {
         const int groups = (ns + base_args().spb - 1) / base_args().spb;  // one slab per shot group
         d_gslab.reserve((size_t)groups * 2 * nxz * sizeof(float));
         launch_fill(d_gslab.as<float>(), (long long)groups * 2 * nxz, 0.f, st);
-        propagate(true, inj_rcv, dadj, nullptr, false);
+        propagate_adjoint(dadj);
         const size_t ngrad = (size_t)2 * g.nx * g.nz;
         if (!grad_dev) d_gout.reserve(ngrad * sizeof(float));
         float* out = grad_dev ? grad : d_gout.as<float>();

@@ -145,6 +145,9 @@ void launch_model(const float* m, int np, int nx, int nz, int ldz, double dt2, f
                   hipStream_t s);
 void launch_amodel(const float* m, int nx, int nz, int ldz, double dt, double fx, double fz, int4 ab, float* K,
                    float* ri, float* kd, float* dv, hipStream_t s);
+// D2(c) closure rows (times h^2) of a coefficient c [nx][ldz]: wx [2 sides][6 rows][8 points][ldz],
+// wz [2 sides][nx][6 rows][8 points]
+void launch_closures(const float* c, int nx, int nz, int ldz, float* wx, float* wz, hipStream_t s);
 void launch_fill(float* p, long long n, float v, hipStream_t s);
 // out [ntr][nrow] = per-trace row-compressed matrix (ptr [nrow + 1], col, w) times in [ntr][ncol]
 void launch_trace_matvec(const int* ptr, const int* col, const double* w, int nrow, int ncol, const float* in,
@@ -169,40 +172,45 @@ void launch_reduce_f64(const double* partial, int n, double* out, hipStream_t s)
 constexpr int kAcTX = 32, kAcTZ = 32;  // step and imaging tiles (x, z)
 
 struct AcousticArgs {
-    int nx, nz, ldz, nshots, ntx, ntz, taper_prev;
-    int spb;                     // k_astep: shots per workgroup (consecutive shots of one tile)
+    int nx, nz, ldz, nshots, ntx, ntz, taper_prev, it;
+    int spb;                     // shots per workgroup (consecutive shots of one tile)
+    int stream;                  // k_astep: prev and next are read and written past the caches
     int itx0, itx1, itz0, itz1;  // k_astep: the tiles [itx0, itx1) x [itz0, itz1) hold interior cells only
     int bc[4];                   // top, bottom, left, right: 1 Dirichlet, 2 absorbing, 3 Neumann
-    float rdx2, rdz2;            // 1 / dx^2, 1 / dz^2
+    float rdx, rdz, rdx2, rdz2;  // 1 / dx, 1 / dz and their squares
     float dir_x[4], dir_z[4];    // Dirichlet SAT S^T terms SC[k] / (H[k] h^2)
     float pen_x, pen_z;          // Dirichlet penalty 1 / (a H0 h^2)
     float neu_x, neu_z;          // Neumann / absorbing 1 / (H0 h^2)
     float abs_x, abs_z;          // absorbing 1 / (2 dt H0 h)
     const float *K, *ri, *kdt2, *div, *taper_x, *taper_z;  // [nx][ldz] (tapers per axis)
+    const float *wx, *wz;        // D2[1/rho] closure rows (launch_closures)
     const float* prev;
     const float* curr;
     float* next;
     long long shot_stride;       // nx * ldz
-    // imaging (k_agrad): adjoint level curr against snapshots f0 (idx), fm, fp
+    // point sources added to the new level, receivers read from the current one (null: none)
+    const PointTable* points;
+    const float* inj_trace;
+    float* rec_trace;
+    int nrec;
+    // imaging: adjoint level curr against snapshot f0 (k_agrad: and its neighbours fm, fp)
     const float *f0, *fm, *fp;
     long long fshot_stride;
     float* grad;                 // per shot-group slabs [groups][2][nx][ldz] (groups of spb shots)
     long long gslab_stride;
-    int mode;                    // 0 interior snapshot, 1 the first, 2 the last
-    int img;                     // k_astep: image snapshot f0 with the adjoint level curr as well
-    float wk;                    // K term weight w / dtg
+    int mode;                    // k_agrad: 0 interior snapshot, 1 the first, 2 the last
+    int img;                     // k_astep: image snapshot f0 by parts in time as well
+    int img_deriv;               // k_astep: 0: snapshot f0 has no 1/rho term
+    float wk, dwn, dwp;          // K term weight w / dtg; k_astep: those of the neighbours less it
     float wr;                    // 1/rho term weight w dtg (halved for the first snapshot)
-    float rdx, rdz;              // 1 / dx, 1 / dz
 };
-// one time step of every shot: next from prev and curr (no point sources)
+// one time step of every shot: next from prev and curr, with the point sources
 void launch_astep(const AcousticArgs& a, hipStream_t s);
-// imaging condition of one snapshot for every shot, into the per-shot slabs
+// imaging condition of one snapshot for every shot, into the shot groups' slabs
 void launch_agrad(const AcousticArgs& a, hipStream_t s);
-// point sources: next[cell] += scale[cell] * sum_k w[k] trace[off[k] + it] / div * taper
-// (scale = dt^2 K; with init: prev = 1/2 dt^2 K sum_k ..., no divisor or taper)
-void launch_ainject(const InjCell* cells, int ncell, const int* ptr, const long long* off, const float* w,
-                    const float* trace, int it, float* u, long long shot_stride, int ldz, const float* kdt2,
-                    const float* div, const float* taper_x, const float* taper_z, bool init, hipStream_t s);
+// initial condition: u[cell] = 1/2 scale[cell] * sum_k w[k] trace[off[k]] (scale = dt^2 K)
+void launch_ainit(const InjCell* cells, int ncell, const int* ptr, const long long* off, const float* w,
+                  const float* trace, float* u, long long shot_stride, int ldz, const float* kdt2, hipStream_t s);
 // receivers: trace[r][it] = sum over the 9 footprint cells of w * u (shot of the receiver)
 void launch_aextract(const float* u, long long shot_stride, int ldz, const PointEntry* ents, int nrec, float* trace,
                      int it, hipStream_t s);

@@ -95,6 +95,21 @@ __device__ __forceinline__ float4 ld4(const float* p)
     return *reinterpret_cast<const float4*>(__builtin_assume_aligned(p, 16));
 }
 __device__ __forceinline__ void st4(float* p, float4 v) { *reinterpret_cast<float4*>(__builtin_assume_aligned(p, 16)) = v; }
+typedef float v4f __attribute__((ext_vector_type(4)));
+// the same with a uniform choice of the streaming form (data that no cache will hold until it is
+// used again leaves the room to data that is)
+__device__ __forceinline__ float4 ld4(const float* p, bool stream)
+{
+    if (!stream) return ld4(p);
+    const v4f v = __builtin_nontemporal_load(reinterpret_cast<const v4f*>(__builtin_assume_aligned(p, 16)));
+    return make_float4(v[0], v[1], v[2], v[3]);
+}
+__device__ __forceinline__ void st4(float* p, float4 v, bool stream)
+{
+    const v4f x = {v.x, v.y, v.z, v.w};
+    if (stream) __builtin_nontemporal_store(x, reinterpret_cast<v4f*>(__builtin_assume_aligned(p, 16)));
+    else st4(p, v);
+}
 __device__ __forceinline__ void unpack(float4 v, float* d)
 {
     d[0] = v.x;
@@ -187,52 +202,6 @@ __device__ __forceinline__ W5 d2_scaled(W5 w, float f)
 __device__ __forceinline__ float d2_apply(const W5& w, const float* pu, int s)
 {
     return w.c * pu[0] + w.m1 * pu[-s] + w.p1 * pu[s] + w.m2 * pu[-2 * s] + w.p2 * pu[2 * s];
-}
-
-// Closure rows of D2(c): row R of the 6 x 8 x 8 table applied to a field, from the edge
-// point along stride st.  The table's non-zeros
-// are compile-time immediates; the weights of the 8 field points are formed first.
-constexpr int kD2NZ = sizeof(kD2ClosureNZ) / sizeof(kD2ClosureNZ[0]);
-constexpr int d2_row_begin(int r)
-{
-    int i = 0;
-    while (i < kD2NZ && kD2ClosureNZ[i].row < r) i++;
-    return i;
-}
-
-template <int R>
-__device__ __forceinline__ float d2_closure_row(const float* qu, const float* qc, int st)
-{
-    float val[8];
-#pragma unroll
-    for (int j = 0; j < 8; j++) val[j] = 0.f;
-    constexpr int b = d2_row_begin(R), e = d2_row_begin(R + 1);
-#pragma unroll
-    for (int i = b; i < e; i++)
-        val[kD2ClosureNZ[i].point] +=
-            (float)(kD2ClosureNZ[i].num / kD2ClosureNZ[i].den) * qc[kD2ClosureNZ[i].coef * st];
-    float cu = 0.f;
-#pragma unroll
-    for (int j = 0; j < 8; j++) cu += val[j] * qu[j * st];
-    return cu;
-}
-
-// closure rows of D2(c) at point g of n
-__device__ __forceinline__ float d2_closure(const float* pu, const float* pc, int s, int g, int n)
-{
-    const bool top = g < 6;
-    const int r = top ? g : n - 1 - g;
-    const int st = top ? s : -s;
-    const int o = top ? -g * s : r * s;
-    const float *qu = pu + o, *qc = pc + o;
-    switch (r) {
-    case 0: return d2_closure_row<0>(qu, qc, st);
-    case 1: return d2_closure_row<1>(qu, qc, st);
-    case 2: return d2_closure_row<2>(qu, qc, st);
-    case 3: return d2_closure_row<3>(qu, qc, st);
-    case 4: return d2_closure_row<4>(qu, qc, st);
-    default: return d2_closure_row<5>(qu, qc, st);
-    }
 }
 
 // one-sided outward boundary derivative sum_k SC[k] u[k*s] (times h)
@@ -334,7 +303,6 @@ __device__ __forceinline__ void d2_quad_z(const float* m, const float* u1, const
 // i is a multiple of 4: the reads are indexed in quads, so that the compiler knows their
 // 16-byte alignment and emits 128-bit LDS reads (not pairs of 64-bit ones, which conflict
 // on banks for lanes 16 bytes apart)
-typedef float v4f __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ void load_col12(const float* base, int i, float* c)
 {
@@ -2065,6 +2033,40 @@ __global__ void k_amodel(const float* m, int nx, int nz, int ldz, double dt, dou
     }
 }
 
+// D2 closure rows as a dense table [row][field point][coefficient point]
+struct ClosureD2 {
+    float c[6 * 8 * 8];
+};
+constexpr ClosureD2 closure_d2_table()
+{
+    ClosureD2 t{};
+    for (const D2Entry& e : kD2ClosureNZ) t.c[(e.row * 8 + e.point) * 8 + e.coef] = (float)(e.num / e.den);
+    return t;
+}
+__constant__ ClosureD2 cClosureD2 = closure_d2_table();
+
+// D2(c) closure rows of a model (see launch_closures): the weight of field point j in row r is
+// sum_k table(r, j, k) c_k over the coefficients k cells in from the side.  One thread per x
+// weight (consecutive threads down z) or z weight; runs once per model.
+__global__ void k_closures(const float* c, int nx, int nz, int ldz, float* wx, float* wz)
+{
+    const long long nwx = 2LL * 6 * 8 * ldz, nwz = 2LL * nx * 6 * 8;
+    for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < nwx + nwz;
+         i += (long long)gridDim.x * blockDim.x) {
+        const bool x = i < nwx;
+        const long long line = x ? i / ldz : (i - nwx) / 48;  // (side 6 + row) 8 + point, or side nx + column
+        const int z = (int)(x ? i - line * ldz : 0);
+        const int rj = (int)(x ? line % 48 : (i - nwx) - line * 48);
+        const bool far = line >= (x ? 48 : nx);
+        long long p = x ? (far ? (long long)(nx - 1) * ldz : 0) + z : (line - (far ? nx : 0)) * ldz + (far ? nz - 1 : 0);
+        const long long st = (x ? ldz : 1) * (far ? -1 : 1);
+        float v = 0.f;
+        for (int k = 0; k < 8; k++, p += st) v += cClosureD2.c[rj * 8 + k] * c[p];
+        if (x) wx[i] = v;
+        else wz[i - nwx] = v;
+    }
+}
+
 __global__ void k_fill(float* p, long long n, float v)
 {
     for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) p[i] = v;
@@ -2321,6 +2323,11 @@ void launch_amodel(const float* m, int nx, int nz, int ldz, double dt, double fx
                        ab, K, ri, kd, dv);
 }
 
+void launch_closures(const float* c, int nx, int nz, int ldz, float* wx, float* wz, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_closures, dim3(grid_for(2LL * 48 * (ldz + nx))), dim3(kThreads), 0, s, c, nx, nz, ldz, wx, wz);
+}
+
 void launch_fill(float* p, long long n, float v, hipStream_t s)
 {
     hipLaunchKernelGGL(k_fill, dim3(grid_for(n)), dim3(kThreads), 0, s, p, n, v);
@@ -2378,278 +2385,539 @@ void launch_reduce_f64(const double* partial, int n, double* out, hipStream_t s)
 // ---------------------------------------------------------------------------
 // Acoustic operator (nl_we_op_a::propagate, we_op.cpp:1937-2135; the SAT terms and their
 // scaling, spatial_operators.cpp:551-860).  A workgroup owns a 32 (x) x 32 (z) tile of
-// a group of shots; the level and 1/rho windows go through LDS (8 rows above and below
-// the tile, which holds every closure row a tile can need; the columns as below), and
-// each thread forms the new level of one quad (column-major, so a wavefront covers 8
-// whole columns): D2x + D2z of the 1/rho-weighted Laplacian (interior weights or closure
-// rows per axis), the SAT terms of the boundary cells, the leapfrog with dt^2 K, the
-// absorbing boundary divisor and the cos^2 taper.  The reference tapers the current
-// level in place after each step; here the previous level is tapered on load instead
-// (taper_prev), which gives the same values.
+// a group of shots; the level windows go straight from global memory into LDS, one shot ahead
+// (two buffers), and each thread forms the new level of one quad (column-major, so a
+// wavefront covers 8 whole columns) from 128-bit LDS reads: D2x + D2z of the 1/rho-weighted
+// Laplacian, the SAT terms of the boundary cells, the leapfrog with dt^2 K, the absorbing
+// boundary divisor and the cos^2 taper.  The reference tapers the current level in place after
+// each step; here the previous level is tapered on load instead (taper_prev), which gives the
+// same values.  Frame tiles take their closures as the elastic step's do: columns along x from
+// model weight arrays, rows along z one cell per thread, handed to the quads' owners through
+// window cells outside the grid.
 // ---------------------------------------------------------------------------
-constexpr int kAcH = 8;
-constexpr int kAcWZ = kAcTZ + 2 * kAcH, kAcWQ = kAcWZ / 4;
 static_assert(kAcTX * (kAcTZ / 4) == kThreads, "one quad per thread");
 
-// SAT terms of one side at a cell k cells in from it (0 <= k < 4), added to rhs: pu / pc
-// point at the side's boundary cell of the cell's line in the level / 1/rho windows, st
-// the window stride pointing inwards, p the cell's previous level (absorbing), K the
-// boundary cell's bulk modulus (absorbing).
-__device__ __forceinline__ float ac_sat(int kind, int k, const float* pu, const float* pc, int st, float p, float K,
-                                        const float* dir, float pen, float neu, float absc)
+// bnd_deriv of 4 values with the order of its roundings written out
+__device__ __forceinline__ float ac_bnd(float u0, float u1, float u2, float u3)
 {
-    if (kind == 1) {
-        // Dirichlet (free surface): + H^-1 S^T (ri u)_0 on the first 4 cells, - penalty at 0
-        float v = dir[k] * pc[0] * pu[0];
-        if (k == 0) v -= pc[0] * pu[0] * pen;
-        return v;
-    }
-    if (k != 0) return 0.f;
-    // Neumann: - H^-1 (ri S u)_0; absorbing: + the impedance term of the previous level
-    float v = -neu * pc[0] * bnd_deriv(pu, st);
-    if (kind == 2) v += absc * p / sqrtf(K / pc[0]);
-    return v;
+    return __builtin_fmaf(cSC[3], u3, __builtin_fmaf(cSC[2], u2, __builtin_fmaf(cSC[0], u0, cSC[1] * u1)));
+}
+// d2_apply and d2_weights with the order of their roundings written out, so
+// that the results do not depend on how the compiler contracts the expressions around them (the
+// 1/rho gradient on a free surface is a sum of large cancelling terms: a change of the rounding
+// alone moves single values by up to 1e-3 of the gradient's rms).  CF: the centre's product is
+// rounded, not the lower neighbour's; MN, PN: on the lower and the upper side the nearer
+// coefficient's product is; sf: the nearest pair's product is, not the centre's.
+template <bool CF>
+__device__ __forceinline__ float ac_d2(const W5& w, float m2, float m1, float u0, float p1, float p2)
+{
+    auto fma = [](float a, float b, float c) { return __builtin_fmaf(a, b, c); };
+    const float v = CF ? fma(w.m1, m1, w.c * u0) : fma(w.c, u0, w.m1 * m1);
+    return fma(w.p2, p2, fma(w.m2, m2, fma(w.p1, p1, v)));
+}
+template <bool MN, bool PN>
+__device__ __forceinline__ W5 ac_weights(float m2, float m1, float f0, float p1, float p2, bool sf = false)
+{
+    auto fma = [](float a, float b, float c) { return __builtin_fmaf(a, b, c); };
+    auto two = [&](bool near, float cf, float f, float cn, float n) {
+        return near ? fma(cf, f, cn * n) : fma(cn, n, cf * f);
+    };
+    W5 w;
+    const float s = m1 + p1;
+    w.c = fma(cD2I[2], m2 + p2, sf ? fma(cD2I[0], f0, cD2I[1] * s) : fma(cD2I[1], s, cD2I[0] * f0));
+    w.m1 = fma(cD2I[6], p1, fma(cD2I[5], f0, two(MN, cD2I[3], m2, cD2I[4], m1)));
+    w.p1 = fma(cD2I[6], m1, fma(cD2I[5], f0, two(PN, cD2I[3], p2, cD2I[4], p1)));
+    w.m2 = fma(cD2I[9], f0, two(MN, cD2I[7], m2, cD2I[8], m1));
+    w.p2 = fma(cD2I[9], f0, two(PN, cD2I[7], p2, cD2I[8], p1));
+    return w;
 }
 
-// The step's level window is narrower in x than the imaging windows: 2 columns before the
-// tile and 6 after it, the window moved left to start at column nx - 8 at the far side.
-// That holds every point a tile's cells read: interior D2 rows +-2, the closure rows of
-// columns 0-5 read columns 0-7 (first tile) and those of columns nx-6..nx-1 columns
-// nx-8..nx-1 (a tile holding such a column ends at most 5 columns before its window does),
-// and the SAT terms the boundary column and its 3 neighbours.
-constexpr int kAcSHL = 2, kAcSWX = kAcTX + kAcSHL + 6;
+// The level windows.  An interior tile reads 2 columns and (whole quads) 4 rows around it.  A
+// frame tile's window holds 2 columns before the tile and 6 after it, moved left to start at
+// column nx - 8 at the far side, and 8 rows each side.  That holds every point its cells read:
+// interior D2 rows +-2, the closure rows of columns 0-5 read columns 0-7 (first tile) and those of
+// columns nx-6..nx-1 columns nx-8..nx-1 (a tile holding such a column ends at most 5 columns
+// before its window does), and the SAT terms the boundary column and its 3 neighbours.
+template <bool EDGE>
+struct AcShape {
+    static constexpr int HL = 2, HZ = EDGE ? 8 : 4;
+    static constexpr int WX = kAcTX + HL + (EDGE ? 6 : 2);
+    static constexpr int WZ = kAcTZ + 2 * HZ, WQ = WZ / 4;  // LDS column stride, quads of a column
+    static constexpr int NQ = (WX * WQ + kThreads - 1) / kThreads;
+};
+constexpr int kAcWin = AcShape<true>::WX * AcShape<true>::WZ;  // floats of the largest window
+
+struct AcTile {
+    int sx, ex, sz, ez, wsx, wsz;
+};
+template <bool EDGE>
+__device__ __forceinline__ AcTile ac_tile(const AcousticArgs& a, int tix, int tiz)
+{
+    AcTile t;
+    t.sx = tix * kAcTX;
+    t.sz = tiz * kAcTZ;
+    t.ex = min(t.sx + kAcTX, a.nx);
+    t.ez = min(t.sz + kAcTZ, a.ldz);
+    t.wsx = t.sx - AcShape<EDGE>::HL;
+    if (EDGE) t.wsx = min(t.wsx, a.nx - 8);
+    t.wsz = t.sz - AcShape<EDGE>::HZ;
+    return t;
+}
 
 __device__ __forceinline__ float sel4(const float (&v)[4], int k)
 {
     return k == 0 ? v[0] : (k == 1 ? v[1] : (k == 2 ? v[2] : v[3]));
 }
 
-__device__ __forceinline__ void ac_window_x(const float* u, float* sU, int wsx, int wsz, int nx, int ldz)
+// 4 floats at a uniform address plus a 32-bit offset in floats (an address in scalar registers
+// and one vector register)
+__device__ __forceinline__ const float* at(const float* base, unsigned i)
 {
-    for (int i = threadIdx.x; i < kAcSWX * kAcWQ; i += kThreads) {
-        const int lx = i / kAcWQ, lq = i - lx * kAcWQ;
-        const int gx = wsx + lx, gz = wsz + 4 * lq;
-        const bool ok = gx >= 0 && gx < nx && gz >= 0 && gz < ldz;
-        st4(&sU[lx * kAcWZ + 4 * lq], ok ? ld4(u + (long long)gx * ldz + gz) : make_float4(0.f, 0.f, 0.f, 0.f));
-    }
+    return reinterpret_cast<const float*>(reinterpret_cast<const char*>(base) + 4 * i);
+}
+__device__ __forceinline__ float* at(float* base, unsigned i)
+{
+    return reinterpret_cast<float*>(reinterpret_cast<char*>(base) + 4 * i);
 }
 
-// The new level of one frame cell with closure rows or SAT terms (the reference's
-// Dxx_var/Dzz_var closures and asat_* terms, then the leapfrog, the boundary divisor and
-// the taper), from the level window U and the 1/rho window R (w: the cell's window index)
-__device__ __forceinline__ float ac_frame_cell(const AcousticArgs& a, const float* U, const float* R, int w, int wsx,
-                                               int wsz, int gx, int gz, long long so)
-{
-    const int nx = a.nx, nz = a.nz, ldz = a.ldz;
-    const long long gi = (long long)gx * ldz + gz;
-    const float* pu = &U[w];
-    const float* pc = &R[w];
-    const float tzk = a.taper_z[gz], tx = a.taper_x[gx];
-    float p = a.prev[so + gi];
-    if (a.taper_prev) p = (p * tzk) * tx;
-    const float lx = (gx >= 6 && gx < nx - 6) ? d2_apply(d2_weights(pc, kAcWZ), pu, kAcWZ)
-                                              : d2_closure(pu, pc, kAcWZ, gx, nx);
-    const float lz = (gz >= 6 && gz < nz - 6) ? d2_apply(d2_weights(pc, 1), pu, 1) : d2_closure(pu, pc, 1, gz, nz);
-    float rhs = lx * a.rdx2 + lz * a.rdz2;
-    const int col = (gx - wsx) * kAcWZ;
-    if (gz < 4) {  // top side, boundary cell (gx, 0)
-        const int bb = col - wsz;
-        rhs += ac_sat(a.bc[0], gz, &U[bb], &R[bb], 1, p, gz == 0 ? a.K[gi - gz] : 0.f, a.dir_z, a.pen_z, a.neu_z,
-                      a.abs_z);
-    }
-    if (gz >= nz - 4) {  // bottom side, boundary cell (gx, nz - 1)
-        const int bb = col + (nz - 1 - wsz);
-        rhs += ac_sat(a.bc[1], nz - 1 - gz, &U[bb], &R[bb], -1, p, gz == nz - 1 ? a.K[gi] : 0.f, a.dir_z, a.pen_z,
-                      a.neu_z, a.abs_z);
-    }
-    if (gx < 4) {  // left side, boundary cell (0, gz)
-        const int bb = (0 - wsx) * kAcWZ + (gz - wsz);
-        rhs += ac_sat(a.bc[2], gx, &U[bb], &R[bb], kAcWZ, p, gx == 0 ? a.K[gi] : 0.f, a.dir_x, a.pen_x, a.neu_x,
-                      a.abs_x);
-    }
-    if (gx >= nx - 4) {  // right side, boundary cell (nx - 1, gz)
-        const int bb = (nx - 1 - wsx) * kAcWZ + (gz - wsz);
-        rhs += ac_sat(a.bc[3], nx - 1 - gx, &U[bb], &R[bb], -kAcWZ, p, gx == nx - 1 ? a.K[gi] : 0.f, a.dir_x,
-                      a.pen_x, a.neu_x, a.abs_x);
-    }
-    // leapfrog (we_op.cpp:2093-2098), boundary divisor (asat_scale_boundaries), taper
-    const float v = (a.kdt2[gi] * rhs + (2.f * pu[0] - p)) / a.div[gi];
-    return (v * tzk) * tx;
-}
-
-// A workgroup steps one 32 x 32 tile of a.spb consecutive shots: the 1/rho window, dt^2 K,
-// the boundary divisor and the tapers are loaded once (and, for tiles of interior cells
-// only, the D2 weights of the cells formed once); the shots' level windows alternate
-// between two LDS buffers, the next shot's loaded while the current one is computed (one
-// barrier per shot).  EDGE = false: a tile of the rectangle of interior tiles; EDGE = true:
-// a tile of the frame around it, whose interior cells take the interior rows (weights
-// formed per shot) and whose other cells the closure rows and SAT terms, dealt one cell
-// per thread.
-// IMG: the adjoint step also images snapshot a.f0 of every shot against the level it
-// reads (the curr window is the adjoint level compute_gradients takes), as k_agrad does,
-// with the snapshot's window double buffered beside the level's.
-template <bool EDGE, bool IMG>
-__device__ __forceinline__ void astep_tile(const AcousticArgs& a, int tix, int tiz, int grp, float* sR,
-                                           float (*sU)[kAcSWX * kAcWZ], float* sO, float (*sF)[kAcSWX * kAcWZ])
-{
-    const int sx = tix * kAcTX, sz = tiz * kAcTZ;
-    const int nx = a.nx, nz = a.nz, ldz = a.ldz;
-    const int ex = min(sx + kAcTX, nx), ez = min(sz + kAcTZ, ldz);
-    const int wsx = min(sx - kAcSHL, nx - 8), wsz = sz - kAcH;
-    const int s0 = grp * a.spb, s1 = min(s0 + a.spb, a.nshots);
-    for (int i = threadIdx.x; i < kAcSWX * kAcWQ; i += kThreads) {
-        const int lx = i / kAcWQ, lq = i - lx * kAcWQ;
-        const int gx = wsx + lx, gz = wsz + 4 * lq;
-        const bool ok = gx >= 0 && gx < nx && gz >= 0 && gz < ldz;
-        st4(&sR[lx * kAcWZ + 4 * lq], ok ? ld4(a.ri + (long long)gx * ldz + gz) : make_float4(0.f, 0.f, 0.f, 0.f));
-    }
-    ac_window_x(a.curr + (long long)s0 * a.shot_stride, sU[0], wsx, wsz, nx, ldz);
-    if (IMG) ac_window_x(a.f0 + (long long)s0 * a.fshot_stride, sF[0], wsx, wsz, nx, ldz);
-    const int q = threadIdx.x;  // quads column-major: a wavefront covers 8 whole columns
-    const int col_q = q / (kAcTZ / 4), row_q = q % (kAcTZ / 4);
-    const int gx = sx + col_q, z0 = sz + 4 * row_q;
-    const bool active = gx < ex && z0 < ez;
-    const long long g = active ? (long long)gx * ldz + z0 : 0;
-    float kd[4], dv[4], tz[4];
-    unpack(ld4(a.kdt2 + g), kd);
-    unpack(ld4(a.div + g), dv);
-    unpack(ld4(a.taper_z + (active ? z0 : 0)), tz);
-    const float tx = a.taper_x[active ? gx : 0];
-    const int col = (active ? gx - wsx : 2) * kAcWZ;  // an in-window column either way
-    const int zw = (active ? z0 : sz) - wsz;
-    __syncthreads();
-    // interior D2 weights of the quad's cells, once for all shots (interior tiles; a frame
-    // tile forms them per shot: held across the shot loop they cost a wavefront per SIMD)
-    W5 wx[4], wz[4];
-    if (!EDGE) {
+// The thread's quads of a window: window quad i goes to float 4 i of the LDS window and comes
+// from float off of the level (kOutside: outside the grid, zeros).  Interior tiles' windows lie
+// inside the grid: such a tile starts at a multiple of 32 rows, ends before row nz - 6, and
+// before column nx - 6.
+constexpr int kOutside = -1;
+template <bool EDGE>
+struct AcQuads {
+    using S = AcShape<EDGE>;
+    int off[S::NQ];
+    __device__ __forceinline__ AcQuads(const AcousticArgs& a, const AcTile& t)
+    {
 #pragma unroll
-        for (int k = 0; k < 4; k++) {
-            wx[k] = d2_weights(&sR[col + zw + k], kAcWZ);
-            wz[k] = d2_weights(&sR[col + zw + k], 1);
+        for (int m = 0; m < S::NQ; m++) {
+            const int i = threadIdx.x + m * kThreads, lx = i / S::WQ;
+            const int gx = t.wsx + lx, gz = t.wsz + 4 * (i - lx * S::WQ);
+            off[m] = !EDGE || (gx >= 0 && gx < a.nx && gz >= 0 && gz < a.ldz) ? gx * a.ldz + gz : kOutside;
         }
     }
-    const bool inx = gx >= 6 && gx < nx - 6;
-    // frame tiles: the cells with closure rows or SAT terms (the tile's columns within 6 of
-    // a side, then its rows within 6 of a side in the other columns), dealt to all the
-    // workgroup's threads one cell each, consecutive threads along a row or down a column
-    const int zr = min(ez, nz), nrr = zr - sz, ncx = ex - sx;
-    const int cl = sx < 6 ? min(6, ex) - sx : 0, crs = max(nx - 6, sx + cl), cr = max(0, ex - crs);
-    const int rt = sz < 6 ? max(0, min(6, zr) - sz) : 0, rbs = max(nz - 6, sz + rt), rb = max(0, zr - rbs);
-    const int nsc = cl + cr, nsr = rt + rb, nnc = ncx - nsc;
-    const int nslow = EDGE ? nsc * nrr + nnc * nsr : 0;
-    // imaging: the group's gradient slab and the K term's weights w / (dtg K^2)
-    float gk[4] = {0.f, 0.f, 0.f, 0.f}, gr[4] = {0.f, 0.f, 0.f, 0.f}, kw[4] = {0.f, 0.f, 0.f, 0.f};
-    float* G = a.grad + (long long)grp * a.gslab_stride + g;
-    if (IMG && active) {
+    __device__ __forceinline__ void load(const float* u, float* w) const
+    {
+        const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+#pragma unroll
+        for (int m = 0; m < S::NQ; m++)
+            if (threadIdx.x + m * kThreads < S::WX * S::WQ)
+                quad_to_lds(!EDGE || off[m] != kOutside ? at(u, off[m]) : kZeroQuad, w + 4 * (m * kThreads + wave * 64));
+    }
+};
+
+// A closure row of a frame tile's cell along z: column gx, row r from the top or bottom, its D2
+// weights, and on the boundary row the bulk modulus and the tapered previous level
+struct AcCell {
+    int gx, r;
+    bool bot;
+    float w[8], K, p;
+};
+// cell c of the tile's pass: rows 0-5 of the top (where the tile holds it), then of the bottom
+__device__ __forceinline__ bool ac_cell(const AcousticArgs& a, const AcTile& t, int c, int ntop, int nbot,
+                                        const float* prev, AcCell& e)
+{
+    const int row = c / kAcTX;
+    e.gx = t.sx + (c - row * kAcTX);
+    if (row >= ntop + nbot || e.gx >= t.ex) return false;
+    e.bot = row >= ntop;
+    const int gz = e.bot ? max(a.nz - 6, t.sz) + (row - ntop) : row;
+    e.r = e.bot ? a.nz - 1 - gz : gz;
+    const float* W = a.wz + (((e.bot ? a.nx : 0) + e.gx) * 6 + e.r) * 8;
+    unpack(ld4(W), e.w);
+    unpack(ld4(W + 4), e.w + 4);
+    if (e.r == 0) {
+        const int g = e.gx * a.ldz + gz;
+        e.K = a.K[g];
+        e.p = prev[g];
+        if (a.taper_prev) e.p = (e.p * a.taper_z[gz]) * a.taper_x[e.gx];
+    }
+    return true;
+}
+// D2z[1/rho] (times h^2) of the cell into the level window's cell 8 rows outside, on rows 0-3 its
+// side's SAT terms into the 1/rho window's; IMG: the z derivatives of the level and of the snapshot F on rows 0-3, into F's cells 4 and 8
+// rows outside
+template <bool IMG>
+__device__ __forceinline__ void ac_cell_run(const AcousticArgs& a, const AcTile& t, const AcCell& e, float* U,
+                                            float* R, float* F, EdgeTable tb)
+{
+    const int st = e.bot ? -1 : 1;
+    const int w = (e.gx - t.wsx) * AcShape<true>::WZ + (e.bot ? a.nz - 1 : 0) - t.wsz;  // the boundary cell
+    float u[8], v = 0.f, sat = 0.f;
+    edge_cells<8>(&U[w], e.bot, u);
+#pragma unroll
+    for (int j = 0; j < 8; j++) v += e.w[j] * u[j];
+    const int bc = e.bot ? a.bc[1] : a.bc[0];
+    const float ri = R[w];
+    if (bc == 1) {
+        // Dirichlet (free surface): + H^-1 S^T (ri u)_0 on the first 4 cells, - penalty at 0
+        if (e.r < 4) sat = sel4(a.dir_z, e.r) * ri * u[0];
+        if (e.r == 0) sat -= ri * u[0] * a.pen_z;
+    } else if (e.r == 0) {
+        // Neumann: - H^-1 (ri S u)_0; absorbing: + the impedance term of the previous level
+        sat = -a.neu_z * ri * ac_bnd(u[0], u[1], u[2], u[3]);
+        if (bc == 2) sat += a.abs_z * e.p / sqrtf(e.K / ri);
+    }
+    const int o = w + st * e.r;
+    U[o - st * 8] = v;
+    if (e.r < 4) R[o - st * 8] = sat;
+    if (IMG && e.r < 4) {
+        float c[8];
+        edge_coefficients(tb, e.r, c);
+        float du = 0.f;
+#pragma unroll
+        for (int j = 0; j < 6; j++) du += c[j] * u[j];
+        F[o - st * 4] = (e.bot ? -du : du) * a.rdz;
+        F[o - st * 8] = d1z_closure(&F[w], e.bot, c) * a.rdz;
+    }
+}
+
+// x part of the Laplacian (times h^2) of a closure column's quad (columns 0-5 from a side), and
+// its SAT terms into sat;
+// w: the quad's window index, g its model index, p the tapered previous level
+__device__ __forceinline__ void ac_closure_column(const AcousticArgs& a, const float* U, const float* R, int w, int gx,
+                                                  int z0, int g, const float* p, float* rhs, float* sat)
+{
+    const EdgeRow e = edge_row(gx, a.nx, 1);
+    const float* W = a.wx + ((size_t)((e.sg < 0 ? 6 : 0) + e.r) * 8) * a.ldz + z0;
+    const int w0 = w + e.o * AcShape<true>::WZ, st = e.st * AcShape<true>::WZ;
+    float ub[4][4], ri[4];  // the 4 cells next to the side
+#pragma unroll
+    for (int k = 0; k < 4; k++) rhs[k] = 0.f;
+    unpack(ld4(&R[w0]), ri);
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+        float wj[4], u[4];
+        unpack(ld4(W + (size_t)j * a.ldz), wj);
+        unpack(ld4(&U[w0 + j * st]), u);
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            rhs[k] += wj[k] * u[k];
+            if (j < 4) ub[j][k] = u[k];
+        }
+    }
+    const int bc = e.sg < 0 ? a.bc[3] : a.bc[2];
+    if (bc == 1) {
+        if (e.r < 4) {
+            const float d = sel4(a.dir_x, e.r);
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                sat[k] = d * ri[k] * ub[0][k];
+                if (e.r == 0) sat[k] -= ri[k] * ub[0][k] * a.pen_x;
+            }
+        }
+    } else if (e.r == 0) {
         float K[4];
         unpack(ld4(a.K + g), K);
 #pragma unroll
-        for (int k = 0; k < 4; k++) kw[k] = a.wk / (K[k] * K[k]);
-        unpack(ld4(G), gk);
-        unpack(ld4(G + a.shot_stride), gr);
+        for (int k = 0; k < 4; k++) {
+            sat[k] = -a.neu_x * ri[k] * ac_bnd(ub[0][k], ub[1][k], ub[2][k], ub[3][k]);
+            if (bc == 2) sat[k] += a.abs_x * p[k] / sqrtf(K[k] / ri[k]);
+        }
     }
+}
+
+// D1 along x of a quad of two windows: interior or closure column
+template <bool EDGE>
+__device__ __forceinline__ void ac_d1x(const AcousticArgs& a, const float* u, const float* v, int w, int gx,
+                                       EdgeTable tb, float* du, float* dv)
+{
+    if (!EDGE || (gx >= 4 && gx < a.nx - 4)) {
+        auto d1x = [&](const float* f, float* d) {
+            float X[4][4];
+#pragma unroll
+            for (int c = 0; c < 4; c++) unpack(ld4(&f[w + (c < 2 ? c - 2 : c - 1) * AcShape<EDGE>::WZ]), X[c]);
+#pragma unroll
+            for (int k = 0; k < 4; k++) d[k] = cD1I[0] * (X[2][k] - X[1][k]) + cD1I[1] * (X[3][k] - X[0][k]);
+        };
+        d1x(u, du);
+        d1x(v, dv);
+    } else if constexpr (EDGE) {
+        d1_quad_closure<AcShape<true>::WZ>(u + w, v + w, gx, a.nx, tb, du, dv);
+    }
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        du[k] *= a.rdx;
+        dv[k] *= a.rdx;
+    }
+}
+
+// Point sources of a tile's shot (we_op.cpp injects them into the right-hand side): the new
+// level's cells c0, c0 + 256, ... before c1 get dt^2 K f over the divisor, tapered; sums in
+// injector order.  IMG: the increment's share of the K gradient by parts, which the imaging did
+// not see, goes to the group's slab.
+template <bool IMG>
+__device__ __forceinline__ void ac_inject(const AcousticArgs& a, int c0, int c1, float* G)
+{
+    const PointTable& pt = *a.points;
+    for (int c = c0; c < c1; c += kThreads) {
+        const InjCell cell = pt.cells[c];
+        float f = 0.f;
+        for (int k = pt.ptr[c]; k < pt.ptr[c + 1]; k++) f += pt.w[k] * a.inj_trace[pt.ctx[k] + a.it];
+        const int g = cell.gx * a.ldz + cell.gz;
+        const float inc = ((a.kdt2[g] * f / a.div[g]) * a.taper_z[cell.gz]) * a.taper_x[cell.gx];
+        a.next[cell.shot * a.shot_stride + g] += inc;
+        if (IMG) G[g] -= (a.wk + a.dwn) * inc * a.f0[cell.shot * a.fshot_stride + g] / (a.K[g] * a.K[g]);
+    }
+}
+
+// One tile of a.spb consecutive shots.  EDGE = false: a tile of the rectangle of interior tiles,
+// whose D2 weights, dt^2 K and tapers stay in registers across the shots; EDGE =
+// true: a frame tile, which forms the weights of its interior cells per shot.
+// IMG (an adjoint step): the imaging of snapshot j = f0 by parts in time, as in the elastic step.
+// The K gradient -sum_j (w_j / dtg) / K^2 a_j (F_j+1 - 2 F_j + F_j-1) collected per snapshot is
+// -F_j / K^2 times the second difference of w a / dtg, formed as wk (next - 2 curr + prev) +
+// dwn next + dwp prev (prev as stored; the point sources' share of next is ac_inject's), so a
+// step reads one snapshot, and its 1/rho term meets the step's own level (img_deriv): 16 B per
+// shot-cell instead of the 12 B of a step and 16 B of a separate k_agrad.
+template <bool EDGE, bool IMG>
+__device__ __forceinline__ void astep_tile(const AcousticArgs& a, int tix, int tiz, int grp, float* sR, float* sU,
+                                           float* sF, EdgeTable tb)
+{
+    constexpr int WZ = AcShape<EDGE>::WZ;
+    const AcTile t = ac_tile<EDGE>(a, tix, tiz);
+    const int nx = a.nx, nz = a.nz, ldz = a.ldz, tid = threadIdx.x;
+    const int s0 = grp * a.spb, s1 = min(s0 + a.spb, a.nshots);
+    const int* const tile_ptr = a.points->tile_ptr + (tix * a.ntz + tiz) * a.nshots;
+    AcQuads<EDGE> q(a, t);
+    q.load(a.ri, sR);
+    q.load(a.curr + s0 * a.shot_stride, sU);
+    if (IMG) q.load(a.f0 + s0 * a.fshot_stride, sF);
+    // threads past the last column compute the tile's first one and store nothing
+    const bool active = t.sx + tid / (kAcTZ / 4) < t.ex;
+    int gx = active ? t.sx + tid / (kAcTZ / 4) : t.sx, z0 = t.sz + 4 * (tid % (kAcTZ / 4));
+    int g = gx * ldz + z0, w = (gx - t.wsx) * WZ + (z0 - t.wsz);
+    float kd[4], tz[4], pn[4];  // pn: the previous level of the next shot, in flight with its windows
+    unpack(ld4(at(a.prev + s0 * a.shot_stride, g), a.stream), pn);
+    unpack(ld4(a.kdt2 + g), kd);
+    unpack(ld4(a.taper_z + z0), tz);
+    const float tx = a.taper_x[gx];
+    // closure rows of the tile: rows 0 .. ntop - 1 and the nbot last rows of the grid it holds
+    const int zr = min(t.ez, nz);
+    const int ntop = EDGE && t.sz == 0 ? min(6, zr) : 0;
+    const int nbot = EDGE ? max(0, zr - max(nz - 6, t.sz)) : 0;
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    W5 wx[EDGE ? 1 : 4], wz[EDGE ? 1 : 4];
+    if constexpr (!EDGE) {
+        float M[5][4], Mc[12];
+#pragma unroll
+        for (int c = 0; c < 5; c++) unpack(ld4(&sR[w + (c - 2) * WZ]), M[c]);
+        load_col12(sR, w, Mc);
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const float* z = &Mc[4 + k];
+            wx[k] = ac_weights<true, false>(M[0][k], M[1][k], M[2][k], M[3][k], M[4][k]);
+            wz[k] = k == 0   ? ac_weights<true, true>(z[-2], z[-1], z[0], z[1], z[2])
+                    : k == 1 ? ac_weights<false, true>(z[-2], z[-1], z[0], z[1], z[2])
+                             : ac_weights<true, false>(z[-2], z[-1], z[0], z[1], z[2]);
+        }
+    }
+    float gk[4] = {0.f, 0.f, 0.f, 0.f}, gr[4] = {0.f, 0.f, 0.f, 0.f};
+    float* const G = IMG ? a.grad + grp * a.gslab_stride : nullptr;
+    if (IMG) unpack(ld4(G + a.shot_stride + g), gr);
     for (int sh = s0; sh < s1; sh++) {
         const int b = (sh - s0) & 1;
-        const long long so = (long long)sh * a.shot_stride;
-        if (sh + 1 < s1) {
-            ac_window_x(a.curr + so + a.shot_stride, sU[b ^ 1], wsx, wsz, nx, ldz);
-            if (IMG) ac_window_x(a.f0 + (long long)(sh + 1) * a.fshot_stride, sF[b ^ 1], wsx, wsz, nx, ldz);
+        float* const U = sU + b * kAcWin;
+        float* const F = IMG ? sF + b * kAcWin : nullptr;
+        const float* prev = a.prev + sh * a.shot_stride;
+        const int inj0 = tile_ptr[sh], inj1 = tile_ptr[sh + 1];  // the sources' cells
+        int cell = tid;
+        // addresses are formed per shot: held (or advanced) across the shots, they spill
+        opaque_v(g);
+        opaque_v(w);
+#pragma unroll
+        for (int m = 0; m < AcShape<EDGE>::NQ; m++) opaque_v(q.off[m]);
+        if constexpr (EDGE) {
+            opaque_v(gx);
+            opaque_v(z0);
+            opaque_v(cell);
         }
-        if (active) {
-            float pv[4], out[4];
-            unpack(ld4(a.prev + so + g), pv);
-            const float* U = sU[b];
-            if (!EDGE) {
+        float pv[4], p[4];
 #pragma unroll
-                for (int k = 0; k < 4; k++) {
-                    const float* pu = &U[col + zw + k];
-                    float p = pv[k];
-                    if (a.taper_prev) p = (p * tz[k]) * tx;
-                    const float rhs = d2_apply(wx[k], pu, kAcWZ) * a.rdx2 + d2_apply(wz[k], pu, 1) * a.rdz2;
-                    // leapfrog (we_op.cpp:2093-2098), boundary divisor, taper
-                    const float v = (kd[k] * rhs + (2.f * pu[0] - p)) / dv[k];
-                    out[k] = (v * tz[k]) * tx;
+        for (int k = 0; k < 4; k++) pv[k] = pn[k];
+        AcCell e;
+        if (sh + 1 < s1) {  // the next shot's windows, while this one is computed
+            unpack(ld4(at(prev + a.shot_stride, g), a.stream), pn);
+            q.load(a.curr + (sh + 1) * a.shot_stride, sU + (b ^ 1) * kAcWin);
+            if (IMG) q.load(a.f0 + (sh + 1) * a.fshot_stride, sF + (b ^ 1) * kAcWin);
+        }
+        const float txp = a.taper_prev ? tx : 1.f;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            p[k] = (pv[k] * (a.taper_prev ? tz[k] : 1.f)) * txp;
+            __asm__("" : "+v"(p[k]));  // rounded as the stored level would be, not fused into 2 u - p
+        }
+        float rhs[4], zt[4], Uc[12], sat[EDGE ? 4 : 1] = {};  // D2 along x and z times h^2, SAT terms
+        if constexpr (EDGE) {
+            // x, then z, the reads of one not held beside the other's
+            const bool closure_x = gx < 6 || gx >= nx - 6;
+            if (!closure_x) {
+                float X[5][4], M[5][4];
+#pragma unroll
+                for (int c = 0; c < 5; c++) {
+                    unpack(ld4(&U[w + (c - 2) * WZ]), X[c]);
+                    unpack(ld4(&sR[w + (c - 2) * WZ]), M[c]);
                 }
-            } else {
-                // the interior cells of the quad (weights formed per shot) and the rows
-                // past nz (zero) into the output tile; the other cells follow below
 #pragma unroll
-                for (int k = 0; k < 4; k++) {
-                    const int gz = z0 + k;
-                    const float* pu = &U[col + zw + k];
-                    const float* pc = &sR[col + zw + k];
-                    if (gz >= nz) {
-                        sO[(gx - sx) * kAcTZ + (gz - sz)] = 0.f;  // rows past nz stay zero
-                    } else if (inx && gz >= 6 && gz < nz - 6) {
-                        float p = pv[k];
-                        if (a.taper_prev) p = (p * tz[k]) * tx;
-                        const float rhs = d2_apply(d2_weights(pc, kAcWZ), pu, kAcWZ) * a.rdx2 +
-                                          d2_apply(d2_weights(pc, 1), pu, 1) * a.rdz2;
-                        const float v = (kd[k] * rhs + (2.f * pu[0] - p)) / dv[k];
-                        sO[(gx - sx) * kAcTZ + (gz - sz)] = (v * tz[k]) * tx;
+                for (int k = 0; k < 4; k++)
+                    rhs[k] = ac_d2<true>(ac_weights<true, false>(M[0][k], M[1][k], M[2][k], M[3][k], M[4][k],
+                                                                 z0 + k < 6 || z0 + k >= nz - 6),
+                                         X[0][k], X[1][k], X[2][k], X[3][k], X[4][k]);
+            } else {
+                ac_closure_column(a, U, sR, w, gx, z0, g, p, rhs, sat);
+            }
+#pragma unroll
+            for (int k = 0; k < 4; k++) __asm__ volatile("" : "+v"(rhs[k]), "+v"(sat[k]));
+            __builtin_amdgcn_sched_barrier(0);
+            float Mc[12];
+            load_col12(sR, w, Mc);
+            load_col12(U, w, Uc);
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const float *c = &Mc[4 + k], *u = &Uc[4 + k];
+                zt[k] = ac_d2<true>(ac_weights<true, false>(c[-2], c[-1], c[0], c[1], c[2], closure_x), u[-2], u[-1], u[0],
+                                    u[1], u[2]);
+            }
+        } else {
+            float X[5][4];
+#pragma unroll
+            for (int c = 0; c < 5; c++) unpack(ld4(&U[w + (c - 2) * WZ]), X[c]);
+            load_col12(U, w, Uc);
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const float* u = &Uc[4 + k];
+                rhs[k] = ac_d2<false>(wx[k], X[0][k], X[1][k], X[2][k], X[3][k], X[4][k]);
+                zt[k] = k == 0 ? ac_d2<false>(wz[k], u[-2], u[-1], u[0], u[1], u[2])
+                               : ac_d2<true>(wz[k], u[-2], u[-1], u[0], u[1], u[2]);
+            }
+        }
+        if (EDGE && ntop + nbot > 0) {
+#pragma unroll
+            for (int k = 0; k < 4; k++) __asm__ volatile("" : "+v"(zt[k]));
+            bool has = ac_cell(a, t, cell, ntop, nbot, prev, e);
+#pragma unroll 1
+            while (has) {
+                ac_cell_run<IMG>(a, t, e, U, sR, F, tb);
+                cell += kThreads;
+                has = ac_cell(a, t, cell, ntop, nbot, prev, e);
+            }
+            __syncthreads();  // the closure rows' terms are in the windows
+            float c[4];
+            if (z0 < 6) {
+                unpack(ld4(&U[w - 8]), c);
+#pragma unroll
+                for (int k = 0; k < 4; k++) zt[k] = z0 + k < 6 ? c[k] : zt[k];
+            }
+            if (z0 + 3 >= nz - 6) {
+                unpack(ld4(&U[w + 8]), c);
+#pragma unroll
+                for (int k = 0; k < 4; k++) zt[k] = z0 + k >= nz - 6 ? c[k] : zt[k];
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < 4; k++) rhs[k] = __builtin_fmaf(rhs[k], a.rdx2, zt[k] * a.rdz2);
+        if constexpr (EDGE) {  // SAT terms: top, bottom, then the column's
+            float c[4];
+            if (z0 < 4) {
+                unpack(ld4(&sR[w - 8]), c);
+#pragma unroll
+                for (int k = 0; k < 4; k++) rhs[k] += c[k];
+            }
+            if (z0 + 3 >= nz - 4) {
+                unpack(ld4(&sR[w + 8]), c);
+#pragma unroll
+                for (int k = 0; k < 4; k++) rhs[k] += z0 + k >= nz - 4 ? c[k] : 0.f;
+            }
+#pragma unroll
+            for (int k = 0; k < 4; k++) rhs[k] += sat[k];
+        }
+        float out[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) out[k] = kd[k] * rhs[k] + (2.f * Uc[4 + k] - p[k]);  // leapfrog (we_op.cpp:2093-2098)
+        if (EDGE && (gx == 0 || gx == nx - 1 || z0 == 0 || z0 + 3 >= nz - 1)) {
+            float dv[4];  // boundary divisor (asat_scale_boundaries)
+            unpack(ld4(a.div + g), dv);
+#pragma unroll
+            for (int k = 0; k < 4; k++) out[k] = out[k] / dv[k];
+        }
+#pragma unroll
+        for (int k = 0; k < 4; k++) out[k] = !EDGE || z0 + k < nz ? (out[k] * tz[k]) * tx : 0.f;
+        if (active) st4(at(a.next + sh * a.shot_stride, g), make_float4(out[0], out[1], out[2], out[3]), a.stream);
+        if constexpr (IMG) {
+            __builtin_amdgcn_sched_barrier(0);  // no reads for the imaging while the step's are held
+            float Fc[12], ax[4], az[4], fx[4], fz[4];
+            load_col12(F, w, Fc);
+            // K term by parts (1 / K^2 at the end)
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+                gk[k] += Fc[4 + k] * (a.wk * ((out[k] - Uc[4 + k]) + (pv[k] - Uc[4 + k])) + (a.dwn * out[k] + a.dwp * pv[k]));
+            ac_d1x<EDGE>(a, U, F, w, gx, tb, ax, fx);
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                az[k] = (cD1I[0] * (Uc[5 + k] - Uc[3 + k]) + cD1I[1] * (Uc[6 + k] - Uc[2 + k])) * a.rdz;
+                fz[k] = (cD1I[0] * (Fc[5 + k] - Fc[3 + k]) + cD1I[1] * (Fc[6 + k] - Fc[2 + k])) * a.rdz;
+            }
+            if (EDGE && ntop + nbot > 0) {
+                float c[4], d[4];
+                if (z0 < 4) {
+                    unpack(ld4(&F[w - 4]), az);
+                    unpack(ld4(&F[w - 8]), fz);
+                }
+                if (z0 + 3 >= nz - 4) {
+                    unpack(ld4(&F[w + 4]), c);
+                    unpack(ld4(&F[w + 8]), d);
+#pragma unroll
+                    for (int k = 0; k < 4; k++) {
+                        az[k] = z0 + k >= nz - 4 ? c[k] : az[k];
+                        fz[k] = z0 + k >= nz - 4 ? d[k] : fz[k];
                     }
                 }
             }
-            if (!EDGE) st4(a.next + so + g, make_float4(out[0], out[1], out[2], out[3]));
-            if (IMG) {
-                // compute_gradients of this shot (we_op.cpp:1883-1935), as k_agrad
-                const long long fo = (long long)sh * a.fshot_stride;
-                float fm[4] = {0.f, 0.f, 0.f, 0.f}, fp[4] = {0.f, 0.f, 0.f, 0.f};
-                if (a.mode != 1) unpack(ld4(a.fm + fo + g), fm);
-                if (a.mode != 2) unpack(ld4(a.fp + fo + g), fp);
 #pragma unroll
-                for (int k = 0; k < 4; k++) {
-                    const int gz = z0 + k;
-                    if (gz >= nz) continue;
-                    const float* pa = &U[col + zw + k];
-                    const float* pf = &sF[b][col + zw + k];
-                    const float ax = d1<false>(pa, kAcWZ, gx, nx) * a.rdx, az = d1<false>(pa, 1, gz, nz) * a.rdz;
-                    const float fx = d1<false>(pf, kAcWZ, gx, nx) * a.rdx, fz = d1<false>(pf, 1, gz, nz) * a.rdz;
-                    const float d2 =
-                        a.mode == 0 ? fp[k] - 2.f * pf[0] + fm[k] : (a.mode == 1 ? fp[k] - pf[0] : -pf[0] + fm[k]);
-                    gk[k] -= kw[k] * pa[0] * d2;
-                    gr[k] += a.wr * (ax * fx + az * fz);
-                }
-            }
+            for (int k = 0; k < 4; k++)
+                if (!EDGE || z0 + k < nz) gr[k] += a.wr * (ax[k] * fx[k] + az[k] * fz[k]);
         }
-        if (EDGE) {
-#pragma unroll 1
-            for (int c = threadIdx.x; c < nslow; c += kThreads) {
-                int cx, cz;
-                if (c < nsc * nrr) {
-                    const int j = c / nrr;
-                    cz = sz + (c - j * nrr);
-                    cx = j < cl ? sx + j : crs + (j - cl);
-                } else {
-                    const int c2 = c - nsc * nrr, r = c2 / nnc;
-                    cx = sx + cl + (c2 - r * nnc);
-                    cz = r < rt ? sz + r : rbs + (r - rt);
-                }
-                sO[(cx - sx) * kAcTZ + (cz - sz)] =
-                    ac_frame_cell(a, sU[b], sR, (cx - wsx) * kAcWZ + (cz - wsz), wsx, wsz, cx, cz, so);
-            }
-            __syncthreads();  // the output tile is complete
-            if (active) st4(a.next + so + g, ld4(&sO[(gx - sx) * kAcTZ + (z0 - sz)]));
-        }
-        __syncthreads();  // the next shot's window is in; this shot's window is read
+        __builtin_amdgcn_s_waitcnt(0);
+        __syncthreads();  // the next shot's windows are in, this one's are read, the new level is stored
+        if (inj1 > inj0) ac_inject<IMG>(a, inj0 + tid, inj1, G);
     }
+    if (IMG) __syncthreads();  // the point sources' shares are in the slab
     if (IMG && active) {
-        st4(G, make_float4(gk[0], gk[1], gk[2], gk[3]));
-        st4(G + a.shot_stride, make_float4(gr[0], gr[1], gr[2], gr[3]));
+        float K[4], v[4];
+        unpack(ld4(a.K + g), K);
+        unpack(ld4(G + g), v);
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+            if (z0 + k < nz) v[k] -= gk[k] / (K[k] * K[k]);
+        st4(G + g, make_float4(v[0], v[1], v[2], v[3]));
+        if (a.img_deriv) st4(G + a.shot_stride + g, make_float4(gr[0], gr[1], gr[2], gr[3]));
     }
 }
 
 // One launch for all tiles: the frame tiles' workgroups first (their closure rows make
 // them the slowest), then the interior rectangle's, each class spread over all XCDs (the
 // frame's block count rounded up to a multiple of 8, the extra blocks idle) and remapped
-// within its class so that an XCD runs neighbouring tiles.
+// within its class so that an XCD runs neighbouring tiles; then the receivers of the current
+// level.
+// Bound by memory latency: 12 B per shot-cell (16 imaged) at 4.1 (3.3) TB/s for 64 shots of
+// 500 x 1700, 159 us a step and 266 us an imaged one.  The form before (loads through
+// registers, the frame's cells dealt one per thread with one code instance per closure row, a
+// launch of its own for the imaging, the points and each kept level) took 208 us a step, 299 us
+// an imaging launch and 78 us a copy.  Waves per SIMD: scratch reloads in the shot loop wait for
+// the windows in flight, so the bounds are the tightest ones that do not spill there (5 and 4
+// instead: 246 and 650 us); what the frame spills costs 1%.  Streamed levels (stream): 151
+// instead of 168 us above the memory-side cache's size, 2 to 12% slower below it.
 template <bool IMG>
-__global__ void __launch_bounds__(kThreads) k_astep(const AcousticArgs a)
+__global__ void __launch_bounds__(kThreads, IMG ? 3 : 4) k_astep(const AcousticArgs a)
 {
-    __shared__ __attribute__((aligned(16))) float sR[kAcSWX * kAcWZ];
-    __shared__ __attribute__((aligned(16))) float sU[2][kAcSWX * kAcWZ];
-    __shared__ __attribute__((aligned(16))) float sO[kAcTX * kAcTZ];  // a frame tile's new level
-    __shared__ __attribute__((aligned(16))) float sF[IMG ? 2 : 1][IMG ? kAcSWX * kAcWZ : 4];  // snapshot windows
+    __shared__ __attribute__((aligned(16))) float sR[kAcWin];
+    __shared__ __attribute__((aligned(16))) float sU[2 * kAcWin];
+    __shared__ __attribute__((aligned(16))) float sF[IMG ? 2 * kAcWin : 4];  // snapshot windows
+    __shared__ __attribute__((aligned(16))) float sT[IMG ? 48 : 4];
+    const EdgeTable tb{sT, 8};
     const int nin_x = a.itx1 - a.itx0, nin_z = a.itz1 - a.itz0;
     const int nin = nin_x * nin_z, nedge = a.ntx * a.ntz - nin;
     const int groups = (a.nshots + a.spb - 1) / a.spb;
@@ -2657,6 +2925,7 @@ __global__ void __launch_bounds__(kThreads) k_astep(const AcousticArgs a)
     const int b = blockIdx.x;
     if (b < ne8) {
         if (b >= ne) return;  // padding: the whole workgroup leaves before any barrier
+        if (IMG && threadIdx.x < 48) sT[threadIdx.x] = cEdgeD1.c[threadIdx.x];  // read after the first barrier
         // frame: the rows of tiles above and below the rectangle, then its side columns
         const int lin = xcd_remap(b, ne);
         const int grp = lin / nedge, tile = lin - grp * nedge;
@@ -2672,78 +2941,123 @@ __global__ void __launch_bounds__(kThreads) k_astep(const AcousticArgs a)
             tiz = a.itz0 + r / w;
             tix = c < a.itx0 ? c : a.itx1 + (c - a.itx0);
         }
-        astep_tile<true, IMG>(a, tix, tiz, grp, sR, sU, sO, reinterpret_cast<float (*)[kAcSWX * kAcWZ]>(&sF[0][0]));
-    } else {
-        const int lin = xcd_remap(b - ne8, gridDim.x - ne8);
+        astep_tile<true, IMG>(a, tix, tiz, grp, sR, sU, sF, tb);
+    } else if (b < ne8 + nin * groups) {
+        const int lin = xcd_remap(b - ne8, nin * groups);
         const int grp = lin / nin, tile = lin - grp * nin;
-        astep_tile<false, IMG>(a, a.itx0 + tile / nin_z, a.itz0 + tile % nin_z, grp, sR, sU, sO,
-                               reinterpret_cast<float (*)[kAcSWX * kAcWZ]>(&sF[0][0]));
+        astep_tile<false, IMG>(a, a.itx0 + tile / nin_z, a.itz0 + tile % nin_z, grp, sR, sU, sF, tb);
+    } else {
+        const int r = (b - ne8 - nin * groups) * kThreads + threadIdx.x;
+        if (r < a.nrec) {
+            const PointEntry e = a.points->rec[r];
+            const float* p = a.curr + e.shot * a.shot_stride;
+            float v = 0.f;
+            for (int ix = 0; ix < 3; ix++)
+                for (int iz = 0; iz < 3; iz++)
+                    v += e.wx[ix] * e.wz[iz] * p[(long long)(e.xi0 + ix) * a.ldz + e.zi0 + iz];
+            a.rec_trace[e.trace + a.it] = v;
+        }
     }
 }
 
 // nl_we_op_a::compute_gradients (we_op.cpp:1883-1935) for every shot: the K term from the
 // second time difference of the snapshots against the adjoint level, the 1/rho term
 // from first derivatives of both.  A workgroup images one tile of a.spb consecutive
-// shots (the step kernel's groups and windows, adjoint level and snapshot windows double
-// buffered), sums their terms in shot order in registers and adds the sum to the group's
+// shots (the step kernel's groups and windows, adjoint level and snapshot windows one shot
+// ahead), sums their terms in shot order in registers and adds the sum to the group's
 // gradient slab once.
-__global__ void __launch_bounds__(kThreads) k_agrad(const AcousticArgs a)
+__global__ void __launch_bounds__(kThreads, 5) k_agrad(const AcousticArgs a)
 {
-    __shared__ __attribute__((aligned(16))) float sA[2][kAcSWX * kAcWZ];
-    __shared__ __attribute__((aligned(16))) float sF[2][kAcSWX * kAcWZ];
-    const int ntile = a.ntx * a.ntz;
+    __shared__ __attribute__((aligned(16))) float sA[2 * kAcWin];
+    __shared__ __attribute__((aligned(16))) float sF[2 * kAcWin];
+    __shared__ __attribute__((aligned(16))) float sT[48];
+    const EdgeTable tb{sT, 8};
+    const int ntile = a.ntx * a.ntz, tid = threadIdx.x;
+    if (tid < 48) sT[tid] = cEdgeD1.c[tid];  // read after the first barrier
     const int lin = xcd_remap(blockIdx.x, gridDim.x);
     const int grp = lin / ntile, tile = lin - grp * ntile;
     const int tix = tile / a.ntz, tiz = tile - tix * a.ntz;
-    const int sx = tix * kAcTX, sz = tiz * kAcTZ;
-    const int nx = a.nx, nz = a.nz, ldz = a.ldz;
-    const int ex = min(sx + kAcTX, nx), ez = min(sz + kAcTZ, ldz);
-    // the step's window: D1 rows read +-2 points inside, the closure rows the 6 points
-    // next to a side
-    const int wsx = min(sx - kAcSHL, nx - 8), wsz = sz - kAcH;
+    constexpr int WZ = AcShape<true>::WZ;
+    const AcTile t = ac_tile<true>(a, tix, tiz);
+    const int nz = a.nz, ldz = a.ldz;
     const int s0 = grp * a.spb, s1 = min(s0 + a.spb, a.nshots);
-    ac_window_x(a.curr + (long long)s0 * a.shot_stride, sA[0], wsx, wsz, nx, ldz);
-    ac_window_x(a.f0 + (long long)s0 * a.fshot_stride, sF[0], wsx, wsz, nx, ldz);
-    const int q = threadIdx.x;
-    const int gx = sx + q / (kAcTZ / 4), z0 = sz + 4 * (q % (kAcTZ / 4));
-    const bool active = gx < ex && z0 < ez;
-    const long long g = active ? (long long)gx * ldz + z0 : 0;
-    float K[4], gk[4], gr[4];
+    const AcQuads<true> q(a, t);
+    q.load(a.curr + s0 * a.shot_stride, sA);
+    q.load(a.f0 + s0 * a.fshot_stride, sF);
+    // threads past the last column compute the tile's first one and store nothing
+    const bool active = t.sx + tid / (kAcTZ / 4) < t.ex;
+    const int gx = active ? t.sx + tid / (kAcTZ / 4) : t.sx, z0 = t.sz + 4 * (tid % (kAcTZ / 4));
+    const int g = gx * ldz + z0, w = (gx - t.wsx) * WZ + (z0 - t.wsz);
+    const int zr = min(t.ez, nz);
+    const int ntop = t.sz == 0 ? min(4, zr) : 0, nbot = max(0, zr - max(nz - 4, t.sz));
+    float K[4], kw[4], gk[4], gr[4];  // kw: the K term's weight w / (dtg K^2)
+    float* const G = a.grad + grp * a.gslab_stride + g;
     unpack(ld4(a.K + g), K);
-    float* G = a.grad + (long long)grp * a.gslab_stride + g;
     unpack(ld4(G), gk);
     unpack(ld4(G + a.shot_stride), gr);
-    float kw[4];  // the K term's weight w / (dtg K^2)
 #pragma unroll
-    for (int k = 0; k < 4; k++) kw[k] = active ? a.wk / (K[k] * K[k]) : 0.f;
-    const int col = (active ? gx - wsx : 2) * kAcWZ;
-    const int zw = (active ? z0 : sz) - wsz;
+    for (int k = 0; k < 4; k++) kw[k] = z0 + k < nz ? a.wk / (K[k] * K[k]) : 0.f;
+    __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
     for (int sh = s0; sh < s1; sh++) {
         const int b = (sh - s0) & 1;
-        const long long fo = (long long)sh * a.fshot_stride;
+        float *const A = sA + b * kAcWin, *const F = sF + b * kAcWin;
+        const long long fo = sh * a.fshot_stride + g;
+        float fm[4] = {0.f, 0.f, 0.f, 0.f}, fp[4] = {0.f, 0.f, 0.f, 0.f};
+        if (a.mode != 1) unpack(ld4(a.fm + fo), fm);
+        if (a.mode != 2) unpack(ld4(a.fp + fo), fp);
         if (sh + 1 < s1) {
-            ac_window_x(a.curr + (long long)(sh + 1) * a.shot_stride, sA[b ^ 1], wsx, wsz, nx, ldz);
-            ac_window_x(a.f0 + fo + a.fshot_stride, sF[b ^ 1], wsx, wsz, nx, ldz);
+            q.load(a.curr + (sh + 1) * a.shot_stride, sA + (b ^ 1) * kAcWin);
+            q.load(a.f0 + (sh + 1) * a.fshot_stride, sF + (b ^ 1) * kAcWin);
         }
-        if (active) {
-            float fm[4] = {0.f, 0.f, 0.f, 0.f}, fp[4] = {0.f, 0.f, 0.f, 0.f};
-            if (a.mode != 1) unpack(ld4(a.fm + fo + g), fm);
-            if (a.mode != 2) unpack(ld4(a.fp + fo + g), fp);
+        if (ntop + nbot > 0) {
+            // z derivatives of rows 0-3 from the top and bottom, one cell per thread, into the
+            // windows' cells 8 rows outside
+            for (int c = tid; c < (ntop + nbot) * kAcTX; c += kThreads) {
+                const int row = c / kAcTX, col = c - row * kAcTX;
+                const bool bot = row >= ntop;
+                const int gz = bot ? max(nz - 4, t.sz) + (row - ntop) : row, r = bot ? nz - 1 - gz : gz;
+                if (t.sx + col >= t.ex) continue;
+                const int wb = (t.sx + col - t.wsx) * WZ + (bot ? nz - 1 : 0) - t.wsz, o = wb + (bot ? 8 - r : r - 8);
+                float cf[8];
+                edge_coefficients(tb, r, cf);
+                A[o] = d1z_closure(&A[wb], bot, cf) * a.rdz;
+                F[o] = d1z_closure(&F[wb], bot, cf) * a.rdz;
+            }
+            __syncthreads();
+        }
+        float Ac[12], Fc[12], ax[4], az[4], fx[4], fz[4];
+        load_col12(A, w, Ac);
+        load_col12(F, w, Fc);
 #pragma unroll
-            for (int k = 0; k < 4; k++) {
-                const int gz = z0 + k;
-                if (gz >= nz) continue;
-                const float* pa = &sA[b][col + zw + k];
-                const float* pf = &sF[b][col + zw + k];
-                const float ax = d1<false>(pa, kAcWZ, gx, nx) * a.rdx, az = d1<false>(pa, 1, gz, nz) * a.rdz;
-                const float fx = d1<false>(pf, kAcWZ, gx, nx) * a.rdx, fz = d1<false>(pf, 1, gz, nz) * a.rdz;
-                const float d2 =
-                    a.mode == 0 ? fp[k] - 2.f * pf[0] + fm[k] : (a.mode == 1 ? fp[k] - pf[0] : -pf[0] + fm[k]);
-                gk[k] -= kw[k] * pa[0] * d2;
-                gr[k] += a.wr * (ax * fx + az * fz);
+        for (int k = 0; k < 4; k++) {
+            const float f = Fc[4 + k];
+            const float d2 = a.mode == 0 ? fp[k] - 2.f * f + fm[k] : (a.mode == 1 ? fp[k] - f : -f + fm[k]);
+            gk[k] -= kw[k] * Ac[4 + k] * d2;
+            az[k] = (cD1I[0] * (Ac[5 + k] - Ac[3 + k]) + cD1I[1] * (Ac[6 + k] - Ac[2 + k])) * a.rdz;
+            fz[k] = (cD1I[0] * (Fc[5 + k] - Fc[3 + k]) + cD1I[1] * (Fc[6 + k] - Fc[2 + k])) * a.rdz;
+        }
+        ac_d1x<true>(a, A, F, w, gx, tb, ax, fx);
+        if (ntop + nbot > 0) {
+            float c[4], d[4];
+            if (z0 < 4) {
+                unpack(ld4(&A[w - 8]), az);
+                unpack(ld4(&F[w - 8]), fz);
+            }
+            if (z0 + 3 >= nz - 4) {
+                unpack(ld4(&A[w + 8]), c);
+                unpack(ld4(&F[w + 8]), d);
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    az[k] = z0 + k >= nz - 4 ? c[k] : az[k];
+                    fz[k] = z0 + k >= nz - 4 ? d[k] : fz[k];
+                }
             }
         }
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+            if (z0 + k < nz) gr[k] += a.wr * (ax[k] * fx[k] + az[k] * fz[k]);
+        __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();  // the next shot's windows are in; this shot's are read
     }
     if (active) {
@@ -2752,23 +3066,18 @@ __global__ void __launch_bounds__(kThreads) k_agrad(const AcousticArgs a)
     }
 }
 
-// point sources of the acoustic operator: per touched cell, the sum of its contributions
-// in injector order, times dt^2 K (the leapfrog's factor), over the boundary divisor and
-// times the taper, as the reference's injection into the right-hand side becomes after
-// the step; init: the initial condition prev = 1/2 dt^2 K inject(trace sample 0)
-__global__ void k_ainject(const InjCell* cells, int ncell, const int* ptr, const long long* off, const float* w,
-                          const float* trace, int it, float* u, long long shot_stride, int ldz, const float* kdt2,
-                          const float* div, const float* taper_x, const float* taper_z, int init)
+// Initial condition prev = 1/2 dt^2 K inject(trace sample 0) on a zero level, one thread per
+// touched cell summing its contributions in injector order
+__global__ void k_ainit(const InjCell* cells, int ncell, const int* ptr, const long long* off, const float* w,
+                        const float* trace, float* u, long long shot_stride, int ldz, const float* kdt2)
 {
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= ncell) return;
     const InjCell cell = cells[c];
     float f = 0.f;
-    for (int k = ptr[c]; k < ptr[c + 1]; k++) f += w[k] * trace[off[k] + it];
+    for (int k = ptr[c]; k < ptr[c + 1]; k++) f += w[k] * trace[off[k]];
     const long long g = (long long)cell.gx * ldz + cell.gz;
-    float* p = u + cell.shot * shot_stride + g;
-    if (init) *p += 0.5f * kdt2[g] * f;
-    else *p += ((kdt2[g] * f / div[g]) * taper_z[cell.gz]) * taper_x[cell.gx];
+    u[cell.shot * shot_stride + g] = 0.5f * kdt2[g] * f;
 }
 
 __global__ void k_aextract(const float* u, long long shot_stride, int ldz, const PointEntry* ents, int nrec,
@@ -2788,7 +3097,8 @@ void launch_astep(const AcousticArgs& a, hipStream_t s)
 {
     const int groups = (a.nshots + a.spb - 1) / a.spb;
     const int nin = (a.itx1 - a.itx0) * (a.itz1 - a.itz0), ne = (a.ntx * a.ntz - nin) * groups;
-    const dim3 grid(((ne + 7) & ~7) + nin * groups);
+    const int nrec = a.rec_trace ? (a.nrec + kThreads - 1) / kThreads : 0;
+    const dim3 grid(((ne + 7) & ~7) + nin * groups + nrec);
     if (a.img) hipLaunchKernelGGL(k_astep<true>, grid, dim3(kThreads), 0, s, a);
     else hipLaunchKernelGGL(k_astep<false>, grid, dim3(kThreads), 0, s, a);
 }
@@ -2799,13 +3109,12 @@ void launch_agrad(const AcousticArgs& a, hipStream_t s)
     hipLaunchKernelGGL(k_agrad, dim3(a.ntx * a.ntz * groups), dim3(kThreads), 0, s, a);
 }
 
-void launch_ainject(const InjCell* cells, int ncell, const int* ptr, const long long* off, const float* w,
-                    const float* trace, int it, float* u, long long shot_stride, int ldz, const float* kdt2,
-                    const float* div, const float* taper_x, const float* taper_z, bool init, hipStream_t s)
+void launch_ainit(const InjCell* cells, int ncell, const int* ptr, const long long* off, const float* w,
+                  const float* trace, float* u, long long shot_stride, int ldz, const float* kdt2, hipStream_t s)
 {
     if (ncell <= 0) return;
-    hipLaunchKernelGGL(k_ainject, dim3((ncell + 127) / 128), dim3(128), 0, s, cells, ncell, ptr, off, w, trace, it, u,
-                       shot_stride, ldz, kdt2, div, taper_x, taper_z, init ? 1 : 0);
+    hipLaunchKernelGGL(k_ainit, dim3((ncell + 127) / 128), dim3(128), 0, s, cells, ncell, ptr, off, w, trace, u,
+                       shot_stride, ldz, kdt2);
 }
 
 void launch_aextract(const float* u, long long shot_stride, int ldz, const PointEntry* ents, int nrec, float* trace,

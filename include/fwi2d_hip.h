@@ -208,9 +208,8 @@ int fwi2d_acoustic_adjoint(fwi2d_acoustic* e, const float* adj, float* grad, int
 
 /* Options (no counterpart in the reference, which keeps every snapshot on the host):
    "snapshot_budget" (MiB, default 131072): the largest snapshot history kept whole; 0
-   always checkpoints; "image_fused" (1: the adjoint step kernel images the snapshots as
-   it steps; 0, the default and faster: a separate imaging kernel before each imaged step;
-   the gradients are identical).
+   always checkpoints; "image_fused" (0 or 1, accepted without effect: the adjoint step
+   images the snapshots by parts in time when sub is 1, a separate kernel does otherwise).
    Statistics: "image_fused", "recompute_steps" (total), "whole_snapshots" (1 or 0,
    the last forward run's choice), "segment", "nseg", "snapshot_budget",
    "shots_per_block" (of the step kernel); -1 for an unknown key. */
