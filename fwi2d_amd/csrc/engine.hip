@@ -345,7 +345,10 @@ struct Engine {
 
     // D2 closure rows of the model (layout in StepArgs: wx[, wxx], wz): the weight of field
     // point j in row r is the sum over the table's entries (r, j, k) of coefficient times
-    // model value at point k, formed in double, times 1 / h^2
+    // model value at point k, formed in double, times 1 / h^2.  Row 0 of a side with a boundary
+    // condition takes the SAT's boundary derivative, -1 / (H0 h) c S u, with it: the two cancel to
+    // a tenth of either, and rounded apart they left the free surface with an error of its own at
+    // every step.
     void build_closures(const float* m)
     {
         const int nx = g.nx, nz = g.nz;
@@ -354,20 +357,25 @@ struct Engine {
         const long long nc = (long long)nx * nz;
         const double rdx2 = 1.0 / (g.dx * g.dx), rdz2 = 1.0 / (g.dz * g.dz);
         std::vector<double> acc(nz);
+        const int bcx[2] = {g.bc_left, g.bc_right}, bcz[2] = {g.bc_top, g.bc_bottom};
+        double sat[8] = {};
+        for (int j = 0; j < 4; j++) sat[j] = -kBoundaryDeriv[j] / kH0;
         for (int f = 0; f < (vti ? 2 : 1); f++) {
             const float *mu = m + nc, *eps = f ? m + 4 * nc : nullptr;  // (1 + 2 eps) mu, mu
+            auto add = [&](double w, long long p) {
+                for (int iz = 0; iz < nz; iz++) {
+                    const double u = mu[p + iz];
+                    acc[iz] += w * (f ? (float)((1.0 + 2.0 * (double)eps[p + iz]) * u) : u);
+                }
+            };
             for (int side = 0; side < 2; side++)
                 for (int r = 0; r < 6; r++)
                     for (int j = 0; j < 8; j++) {
                         std::fill(acc.begin(), acc.end(), 0.0);
                         for (const D2Entry& e : kD2ClosureNZ)
-                            if (e.row == r && e.point == j) {
-                                const long long p = (long long)(side ? nx - 1 - e.coef : e.coef) * nz;
-                                for (int iz = 0; iz < nz; iz++) {
-                                    const double u = mu[p + iz];
-                                    acc[iz] += e.num / e.den * (f ? (float)((1.0 + 2.0 * (double)eps[p + iz]) * u) : u);
-                                }
-                            }
+                            if (e.row == r && e.point == j)
+                                add(e.num / e.den, (long long)(side ? nx - 1 - e.coef : e.coef) * nz);
+                        if (r == 0 && bcx[side] != 0) add(sat[j], (long long)(side ? nx - 1 : 0) * nz);
                         float* o = w.data() + f * nwx + ((size_t)(side * 6 + r) * 8 + j) * ldz;
                         for (int iz = 0; iz < nz; iz++) o[iz] = (float)(acc[iz] * rdx2);
                     }
@@ -380,6 +388,8 @@ struct Engine {
                 const float* p = mu + (long long)ix * nz + (side ? nz - 1 : 0);
                 for (const D2Entry& e : kD2ClosureNZ)
                     v[e.point][e.row] += e.num / e.den * p[side ? -(int)e.coef : e.coef];
+                if (bcz[side] != 0)
+                    for (int j = 0; j < 8; j++) v[j][0] += sat[j] * p[0];
                 for (int j = 0; j < 8; j++)
                     for (int r = 0; r < 6; r++) wz[(((size_t)side * nx + ix) * 6 + r) * 8 + j] = (float)(v[j][r] * rdz2);
             }
@@ -556,12 +566,12 @@ struct Engine {
         a.nt = g.nt;
         a.rdx = (float)(1.0 / g.dx);
         a.rdz = (float)(1.0 / g.dz);
-        a.rdx2 = (float)(1.0 / (g.dx * g.dx));
-        a.rdz2 = (float)(1.0 / (g.dz * g.dz));
+        a.rdx2 = (float)(1.0 / (24 * g.dx * g.dx));
+        a.rdz2 = (float)(1.0 / (24 * g.dz * g.dz));
         a.c1x = (float)(kD1Interior[0] / g.dx);
-        a.c2x = (float)(kD1Interior[1] / g.dx);
+        a.c2x = d1_interior_far(a.c1x, g.dx);
         a.c1z = (float)(kD1Interior[0] / g.dz);
-        a.c2z = (float)(kD1Interior[1] / g.dz);
+        a.c2z = d1_interior_far(a.c1z, g.dz);
         a.dt = (float)g.dt;
         a.dt2 = (float)g.dt * (float)g.dt;
         a.sat_x = (float)(1.0 / (g.dx * kH0));

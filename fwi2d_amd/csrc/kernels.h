@@ -53,7 +53,7 @@ struct StepArgs {
     int spb, ngroups;      // shots per workgroup, shot groups (ceil(nshots / spb))
     int spb_e, ngroups_e;  // the same for frame tiles
     int itx0, itx1, itz0, itz1;  // the tiles [itx0, itx1) x [itz0, itz1) hold interior cells only
-    float rdx, rdz, rdx2, rdz2, dt, dt2, sat_x, sat_z;
+    float rdx, rdz, rdx2, rdz2, dt, dt2, sat_x, sat_z;  // rdx2, rdz2: 1 / (24 dx^2), 1 / (24 dz^2)
     float c1x, c2x, c1z, c2z;  // interior first-derivative coefficients divided by dx, dz
     int bc_top, bc_bottom, bc_left, bc_right;
     const float *lam, *mu, *rho, *c13, *eps;
@@ -61,7 +61,8 @@ struct StepArgs {
     const float *mux, *lamx;  // VTI: (1 + 2 eps) mu, (1 + 2 eps) lambda
     // D2 closure rows of the model, times 1 / h^2: x columns 0-5 from the left and right
     // [2 sides][6 columns][8 points][ldz] for mu (wx) and, VTI, (1 + 2 eps) mu (wxx); z rows
-    // 0-5 from the top and bottom [2 sides][nx][6 rows][8 points] for mu
+    // 0-5 from the top and bottom [2 sides][nx][6 rows][8 points] for mu.  Row 0 of a side with a
+    // boundary condition includes its SAT's boundary derivative
     const float *wx, *wxx, *wz;
     const float *div_tb;   // [2 sides][2 comps][nx] absorbing divisors, top then bottom
     const float *div_lr;   // [2 sides][2 comps][ldz]

@@ -17,20 +17,23 @@
 
 namespace fwi2d {
 
-__constant__ float cD1I[2];
-__constant__ float cSC[4];
+__constant__ float cD1I[2];   // elastic interior rows (see kD2Interior24)
 __constant__ float cD2I[10];
+__constant__ float cD1A[2];   // acoustic: the rows rounded one by one
+__constant__ float cD2A[10];
+__constant__ float cSC[4];
 
 void upload_constants(hipStream_t s)
 {
-    float d1i[2], sc[4], d2i[10];
-    d1i[0] = (float)kD1Interior[0];
-    d1i[1] = (float)kD1Interior[1];
+    float d1a[2], sc[4], d2a[10];
+    for (int i = 0; i < 2; i++) d1a[i] = (float)kD1Interior[i];
     for (int i = 0; i < 4; i++) sc[i] = (float)kBoundaryDeriv[i];
-    for (int i = 0; i < 10; i++) d2i[i] = (float)kD2Interior[i];
-    (void)hipMemcpyToSymbolAsync(HIP_SYMBOL(cD1I), d1i, sizeof(d1i), 0, hipMemcpyHostToDevice, s);
+    for (int i = 0; i < 10; i++) d2a[i] = (float)kD2Interior[i];
+    (void)hipMemcpyToSymbolAsync(HIP_SYMBOL(cD1I), kD1InteriorF, sizeof(kD1InteriorF), 0, hipMemcpyHostToDevice, s);
+    (void)hipMemcpyToSymbolAsync(HIP_SYMBOL(cD2I), kD2Interior24, sizeof(kD2Interior24), 0, hipMemcpyHostToDevice, s);
+    (void)hipMemcpyToSymbolAsync(HIP_SYMBOL(cD1A), d1a, sizeof(d1a), 0, hipMemcpyHostToDevice, s);
+    (void)hipMemcpyToSymbolAsync(HIP_SYMBOL(cD2A), d2a, sizeof(d2a), 0, hipMemcpyHostToDevice, s);
     (void)hipMemcpyToSymbolAsync(HIP_SYMBOL(cSC), sc, sizeof(sc), 0, hipMemcpyHostToDevice, s);
-    (void)hipMemcpyToSymbolAsync(HIP_SYMBOL(cD2I), d2i, sizeof(d2i), 0, hipMemcpyHostToDevice, s);
     (void)hipStreamSynchronize(s);
 }
 
@@ -166,7 +169,7 @@ __device__ __forceinline__ float d1(const float* p, int s, int g, int n)
     return d1_closure(p, s, g, n);
 }
 
-// interior weights of D2(c) at one point: u[-2..2] coefficients (Dzz_var/Dxx_var interior)
+// interior weights of D2(c) at one point, times 24 h^2: u[-2..2] coefficients (Dzz_var/Dxx_var interior)
 struct W5 {
     float m2, m1, c, p1, p2;
 };
@@ -203,15 +206,6 @@ __device__ __forceinline__ float d2_apply(const W5& w, const float* pu, int s)
 {
     return w.c * pu[0] + w.m1 * pu[-s] + w.p1 * pu[s] + w.m2 * pu[-2 * s] + w.p2 * pu[2 * s];
 }
-
-// one-sided outward boundary derivative sum_k SC[k] u[k*s] (times h)
-__device__ __forceinline__ float bnd_deriv(const float* p, int s)
-{
-    return cSC[0] * p[0] + cSC[1] * p[s] + cSC[2] * p[2 * s] + cSC[3] * p[3 * s];
-}
-
-// sum_j B[0][j] u[j*s]: first closure row (times h), used by the normal complement terms
-__device__ __forceinline__ float d1_row0(const float* p, int s) { return d1_closure_row<0>(p, s); }
 
 // ---------------------------------------------------------------------------
 // Fused time step
@@ -330,10 +324,10 @@ constexpr EdgeD1 edge_d1_table()
     for (int r = 0; r < 4; r++)
         for (int j = 0; j < 6; j++) t.c[8 * r + j] = (float)kD1Closure[r][j];
     for (int r = 4; r < 6; r++) {
-        t.c[8 * r + r - 2] = (float)-kD1Interior[1];
-        t.c[8 * r + r - 1] = (float)-kD1Interior[0];
-        t.c[8 * r + r + 1] = (float)kD1Interior[0];
-        t.c[8 * r + r + 2] = (float)kD1Interior[1];
+        t.c[8 * r + r - 2] = -kD1InteriorF[1];
+        t.c[8 * r + r - 1] = -kD1InteriorF[0];
+        t.c[8 * r + r + 1] = kD1InteriorF[0];
+        t.c[8 * r + r + 2] = kD1InteriorF[1];
     }
     return t;
 }
@@ -565,15 +559,19 @@ __device__ __forceinline__ void prev_at(const StepArgs& a, const float* prev, lo
 }
 
 // The z part of the right-hand side (D2z[mu] ux, 2 D2z[mu] uz, Dz of the products) of the
-// closure rows 0-5 from the top or bottom, one cell per thread, and on the boundary row the
-// SAT terms of that side (we_op.cpp:726-774, 1705-1752).  Cell c of the pass, whose D2
-// weights and boundary values are loaded ahead of the shot's window.
+// closure rows 0-5 from the top or bottom, one cell per thread, with the SAT terms of that side
+// on the boundary row (we_op.cpp:726-774, 1705-1752).  Those are minus the boundary derivative,
+// which the row's D2 weights hold, and, for the traction's derivatives along the side and the
+// scheme's complement term together, plus the products there over H0 h: that turns the row's
+// first D1 coefficient -24/17 into 24/17.  Absorbing sides add the impedance term of the
+// previous level.  Cell c of the pass, whose D2 weights and boundary values are loaded ahead
+// of the shot's window.
 struct ZCell {
     int gx, r;
     bool bot;
-    float w[8], lam, rho, f1, prx, prz;
+    float w[8], lam, rho, prx, prz;
 };
-template <bool VTI, class S>
+template <class S>
 __device__ __forceinline__ bool z_cell(const StepArgs& a, const TileInfo& t, int c, bool top, bool bot,
                                        const float* prev, long long nxz, ZCell& e)
 {
@@ -588,11 +586,10 @@ __device__ __forceinline__ bool z_cell(const StepArgs& a, const TileInfo& t, int
     const float* W = a.wz + (((e.bot ? a.nx : 0) + e.gx) * 6 + e.r) * 8;
     unpack(ld4(W), e.w);
     unpack(ld4(W + 4), e.w + 4);
-    if (e.r == 0) {
+    if (e.r == 0 && (e.bot ? a.bc_bottom : a.bc_top) == 2) {
         const int gz = e.bot ? a.nz - 1 : 0, g = e.gx * a.ldz + gz;
         e.lam = a.lam[g];
         e.rho = a.rho[g];
-        e.f1 = VTI ? a.c13[g] : e.lam;
         prev_at(a, prev, nxz, e.gx, gz, e.prx, e.prz);
     }
     return true;
@@ -605,6 +602,8 @@ __device__ __forceinline__ void z_cell_run(const StepArgs& a, const StepSmem& sm
     const int q = (e.gx - t.plx) * S::PZ + (edge - t.pz0);
     float c[8], ux[8], uz[8], v[8];
     edge_coefficients(sm.tb, e.r, c);
+    const int bc = e.bot ? a.bc_bottom : a.bc_top;
+    if (e.r == 0 && bc != 0) c[0] = -c[0];
     edge_cells<8>(&sm.ux[w], e.bot, ux);
     edge_cells<8>(&sm.uz[w], e.bot, uz);
     float d2x = 0.f, d2z = 0.f, dp = 0.f, dq = 0.f;
@@ -621,29 +620,19 @@ __device__ __forceinline__ void z_cell_run(const StepArgs& a, const StepSmem& sm
     for (int j = 0; j < 8; j++) dq += c[j] * v[j];
     const float sg = e.bot ? -a.rdz : a.rdz;
     float rx = d2x + sg * dq, rz = 2.f * d2z + sg * dp;
-    const int bc = e.bot ? a.bc_bottom : a.bc_top;
-    if (e.r == 0 && bc != 0) {
+    if (e.r == 0 && bc == 2) {
         const float mu0 = sm.mu[w];
-        const float out = e.bot ? a.rdx : -a.rdx;
-        float dxx, dxz;
-        d1_pair(&sm.ux[w], &sm.uz[w], S::WZ, e.gx, a.nx, sm.tb, dxx, dxz);
-        float tx = mu0 * (out * dxz) + mu0 * bnd_deriv(ux, 1) * a.rdz;
-        float tz = e.f1 * (out * dxx) + (2.f * mu0) * bnd_deriv(uz, 1) * a.rdz;
-        if (bc == 2) {
-            tx -= (0.5f * sqrtf(mu0 * e.rho)) * e.prx / a.dt;
-            tz -= (0.5f * sqrtf((e.lam + 2.f * mu0) * e.rho)) * e.prz / a.dt;
-        }
-        rx -= a.sat_z * tx;
-        rz -= a.sat_z * tz;
-        rz += (a.sat_z * a.rdz) * e.lam * d1_row0(uz, 1);
+        rx += a.sat_z * ((0.5f * sqrtf(mu0 * e.rho)) * e.prx / a.dt);
+        rz += a.sat_z * ((0.5f * sqrtf((e.lam + 2.f * mu0) * e.rho)) * e.prz / a.dt);
     }
     const int o = w + st * (e.r - kTermRows);
     sm.ux[o] = rx;
     sm.uz[o] = rz;
 }
 
-// The SAT terms of the left and right boundary columns of a tile (we_op.cpp:776-822,
-// 1754-1800), one cell per thread.
+// The impedance terms of absorbing left and right boundary columns of a tile (we_op.cpp:776-822,
+// 1754-1800; the SAT's other terms are in the columns' D2 weights and D1 coefficients, as along
+// z), one cell per thread.
 template <bool VTI, class S>
 __device__ __forceinline__ void x_sat_pass(const StepArgs& a, const StepSmem& sm, const TileInfo& t, int tid,
                                            bool left, bool right, const float* prev, long long nxz)
@@ -654,28 +643,12 @@ __device__ __forceinline__ void x_sat_pass(const StepArgs& a, const StepSmem& sm
         if (!(rt ? right : left) || gz >= t.ez) continue;
         const int gx = rt ? a.nx - 1 : 0, sn = rt ? -S::WZ : S::WZ;
         const int w = (gx - t.wsx) * S::WZ + (gz - t.wsz), g = gx * a.ldz + gz;
-        const float *ux = &sm.ux[w], *uz = &sm.uz[w];
-        const float mu0 = sm.mu[w], lam0 = a.lam[g], rho0 = a.rho[g], f1 = VTI ? a.c13[g] : lam0;
+        const float mu0 = sm.mu[w], lam0 = a.lam[g], rho0 = a.rho[g];
         const float epsf = VTI ? 1.f + 2.f * a.eps[g] : 1.f;
-        const int bc = rt ? a.bc_right : a.bc_left;
-        float rx = 0.f, rz = 0.f;
-        if (bc != 0) {
-            const float out = rt ? a.rdz : -a.rdz;
-            float dzx, dzz;
-            d1_pair(ux, uz, 1, gz, a.nz, sm.tb, dzx, dzz);
-            float tx = f1 * (out * dzz) + (epsf * (2.f * mu0)) * bnd_deriv(ux, sn) * a.rdx;
-            float tz = mu0 * (out * dzx) + mu0 * bnd_deriv(uz, sn) * a.rdx;
-            if (bc == 2) {
-                float prx, prz;
-                prev_at(a, prev, nxz, gx, gz, prx, prz);
-                tx -= (0.5f * sqrtf(epsf * (lam0 + 2.f * mu0) * rho0)) * prx / a.dt;
-                tz -= (0.5f * sqrtf(mu0 * rho0)) * prz / a.dt;
-            }
-            rx = (a.sat_x * a.rdx) * (epsf * lam0) * d1_row0(ux, sn) - a.sat_x * tx;
-            rz = -a.sat_x * tz;
-        }
-        sm.ux[w - sn] = rx;
-        sm.uz[w - sn] = rz;
+        float prx, prz;
+        prev_at(a, prev, nxz, gx, gz, prx, prz);
+        sm.ux[w - sn] = a.sat_x * ((0.5f * sqrtf(epsf * (lam0 + 2.f * mu0) * rho0)) * prx / a.dt);
+        sm.uz[w - sn] = a.sat_x * ((0.5f * sqrtf(mu0 * rho0)) * prz / a.dt);
     }
 }
 
@@ -746,7 +719,8 @@ __device__ __forceinline__ void rhs_quad(const StepArgs& a, const StepSmem& sm, 
 #pragma unroll 2
         for (int j = 0; j < 8; j++) {
             const int o = e.o + j * e.st;
-            const float c = sm.tb.c[sm.tb.rs * e.r + j];
+            float c = sm.tb.c[sm.tb.rs * e.r + j];
+            if (j == 0 && e.r == 0 && (gx ? a.bc_right : a.bc_left) != 0) c = -c;  // with the SAT's share
             float wj[4], xj[4], U[4], Z[4];
             unpack(ld4(W + (size_t)j * a.ldz), wj);
             if (VTI) unpack(ld4(WX + (size_t)j * a.ldz), xj);
@@ -847,7 +821,7 @@ __device__ __forceinline__ void frame_terms(const StepArgs& a, const StepSmem& s
         rx[k] += zx[k];
         rz[k] += zz[k];
     }
-    if (gx == 0 || gx == nx - 1) {
+    if ((gx == 0 && a.bc_left == 2) || (gx == nx - 1 && a.bc_right == 2)) {
         const int o = gx == 0 ? w - S::WZ : w + S::WZ;
         unpack(ld4(&sm.ux[o]), tx);
         unpack(ld4(&sm.uz[o]), tz);
@@ -1158,7 +1132,7 @@ __device__ __forceinline__ void step_tile(const StepArgs& a, const StepSmem& sm,
     product_range(t.sz, t.ez, nz, t.plz, t.phz);
     // closure rows in the tile
     const bool top = EDGE && t.sz == 0, bot = EDGE && tiz == a.ntz - 1;
-    const bool left = EDGE && t.sx == 0, right = EDGE && tix == a.ntx - 1;
+    const bool left = EDGE && t.sx == 0 && a.bc_left == 2, right = EDGE && tix == a.ntx - 1 && a.bc_right == 2;
     const long long nxz = (long long)nx * ldz;
     const int tid = threadIdx.x;
 
@@ -1293,7 +1267,7 @@ __device__ __forceinline__ void step_tile(const StepArgs& a, const StepSmem& sm,
         bool has_p = false, has_z = false;
         if (EDGE && (top || bot)) {
             has_p = p_cell<VTI, S>(a, t, kThreads - 1 - tid, top, bot, pc);
-            has_z = z_cell<VTI, S>(a, t, ztid, top, bot, pux, nxz, zc);
+            has_z = z_cell<S>(a, t, ztid, top, bot, pux, nxz, zc);
         }
         __syncthreads();  // the previous shot is done with the LDS state and products
         if (EDGE && VTI && shot == s0 && tid < 48)
@@ -1360,7 +1334,7 @@ __device__ __forceinline__ void step_tile(const StepArgs& a, const StepSmem& sm,
         if constexpr (EDGE) {
             if (top || bot) {
                 if (has_z) z_cell_run<VTI, S>(a, sm, t, zc);
-                if (12 * S::TX > kThreads && z_cell<VTI, S>(a, t, kThreads + ztid, top, bot, pux, nxz, zc))
+                if (12 * S::TX > kThreads && z_cell<S>(a, t, kThreads + ztid, top, bot, pux, nxz, zc))
                     z_cell_run<VTI, S>(a, sm, t, zc);
             }
             if (left || right) x_sat_pass<VTI, S>(a, sm, t, tid, left, right, pux, nxz);
@@ -2397,7 +2371,8 @@ void launch_reduce_f64(const double* partial, int n, double* out, hipStream_t s)
 // ---------------------------------------------------------------------------
 static_assert(kAcTX * (kAcTZ / 4) == kThreads, "one quad per thread");
 
-// bnd_deriv of 4 values with the order of its roundings written out
+// one-sided outward boundary derivative sum_k SC[k] u_k (times h), the order of its roundings
+// written out
 __device__ __forceinline__ float ac_bnd(float u0, float u1, float u2, float u3)
 {
     return __builtin_fmaf(cSC[3], u3, __builtin_fmaf(cSC[2], u2, __builtin_fmaf(cSC[0], u0, cSC[1] * u1)));
@@ -2424,11 +2399,11 @@ __device__ __forceinline__ W5 ac_weights(float m2, float m1, float f0, float p1,
     };
     W5 w;
     const float s = m1 + p1;
-    w.c = fma(cD2I[2], m2 + p2, sf ? fma(cD2I[0], f0, cD2I[1] * s) : fma(cD2I[1], s, cD2I[0] * f0));
-    w.m1 = fma(cD2I[6], p1, fma(cD2I[5], f0, two(MN, cD2I[3], m2, cD2I[4], m1)));
-    w.p1 = fma(cD2I[6], m1, fma(cD2I[5], f0, two(PN, cD2I[3], p2, cD2I[4], p1)));
-    w.m2 = fma(cD2I[9], f0, two(MN, cD2I[7], m2, cD2I[8], m1));
-    w.p2 = fma(cD2I[9], f0, two(PN, cD2I[7], p2, cD2I[8], p1));
+    w.c = fma(cD2A[2], m2 + p2, sf ? fma(cD2A[0], f0, cD2A[1] * s) : fma(cD2A[1], s, cD2A[0] * f0));
+    w.m1 = fma(cD2A[6], p1, fma(cD2A[5], f0, two(MN, cD2A[3], m2, cD2A[4], m1)));
+    w.p1 = fma(cD2A[6], m1, fma(cD2A[5], f0, two(PN, cD2A[3], p2, cD2A[4], p1)));
+    w.m2 = fma(cD2A[9], f0, two(MN, cD2A[7], m2, cD2A[8], m1));
+    w.p2 = fma(cD2A[9], f0, two(PN, cD2A[7], p2, cD2A[8], p1));
     return w;
 }
 
@@ -2630,7 +2605,7 @@ __device__ __forceinline__ void ac_d1x(const AcousticArgs& a, const float* u, co
 #pragma unroll
             for (int c = 0; c < 4; c++) unpack(ld4(&f[w + (c < 2 ? c - 2 : c - 1) * AcShape<EDGE>::WZ]), X[c]);
 #pragma unroll
-            for (int k = 0; k < 4; k++) d[k] = cD1I[0] * (X[2][k] - X[1][k]) + cD1I[1] * (X[3][k] - X[0][k]);
+            for (int k = 0; k < 4; k++) d[k] = cD1A[0] * (X[2][k] - X[1][k]) + cD1A[1] * (X[3][k] - X[0][k]);
         };
         d1x(u, du);
         d1x(v, dv);
@@ -2857,8 +2832,8 @@ __device__ __forceinline__ void astep_tile(const AcousticArgs& a, int tix, int t
             ac_d1x<EDGE>(a, U, F, w, gx, tb, ax, fx);
 #pragma unroll
             for (int k = 0; k < 4; k++) {
-                az[k] = (cD1I[0] * (Uc[5 + k] - Uc[3 + k]) + cD1I[1] * (Uc[6 + k] - Uc[2 + k])) * a.rdz;
-                fz[k] = (cD1I[0] * (Fc[5 + k] - Fc[3 + k]) + cD1I[1] * (Fc[6 + k] - Fc[2 + k])) * a.rdz;
+                az[k] = (cD1A[0] * (Uc[5 + k] - Uc[3 + k]) + cD1A[1] * (Uc[6 + k] - Uc[2 + k])) * a.rdz;
+                fz[k] = (cD1A[0] * (Fc[5 + k] - Fc[3 + k]) + cD1A[1] * (Fc[6 + k] - Fc[2 + k])) * a.rdz;
             }
             if (EDGE && ntop + nbot > 0) {
                 float c[4], d[4];
@@ -3034,8 +3009,8 @@ __global__ void __launch_bounds__(kThreads, 5) k_agrad(const AcousticArgs a)
             const float f = Fc[4 + k];
             const float d2 = a.mode == 0 ? fp[k] - 2.f * f + fm[k] : (a.mode == 1 ? fp[k] - f : -f + fm[k]);
             gk[k] -= kw[k] * Ac[4 + k] * d2;
-            az[k] = (cD1I[0] * (Ac[5 + k] - Ac[3 + k]) + cD1I[1] * (Ac[6 + k] - Ac[2 + k])) * a.rdz;
-            fz[k] = (cD1I[0] * (Fc[5 + k] - Fc[3 + k]) + cD1I[1] * (Fc[6 + k] - Fc[2 + k])) * a.rdz;
+            az[k] = (cD1A[0] * (Ac[5 + k] - Ac[3 + k]) + cD1A[1] * (Ac[6 + k] - Ac[2 + k])) * a.rdz;
+            fz[k] = (cD1A[0] * (Fc[5 + k] - Fc[3 + k]) + cD1A[1] * (Fc[6 + k] - Fc[2 + k])) * a.rdz;
         }
         ac_d1x<true>(a, A, F, w, gx, tb, ax, fx);
         if (ntop + nbot > 0) {
