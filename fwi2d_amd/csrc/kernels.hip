@@ -1006,7 +1006,8 @@ __device__ __forceinline__ void image_accumulate(const StepArgs& a, long long g,
 // recomputed inside the shot loop instead of being hoisted out and kept live in
 // registers across it (which multiplies the register footprint of the loop body).
 __device__ __forceinline__ void opaque(int& v) { __asm__ volatile("" : "+s"(v)); }
-__device__ __forceinline__ void opaque_v(int& v) { __asm__ volatile("" : "+v"(v)); }
+template <class I>
+__device__ __forceinline__ void opaque_v(I& v) { __asm__ volatile("" : "+v"(v)); }
 __device__ __forceinline__ void opaque(TileInfo& t)
 {
     opaque(t.sx);
@@ -2444,33 +2445,35 @@ __device__ __forceinline__ float sel4(const float (&v)[4], int k)
     return k == 0 ? v[0] : (k == 1 ? v[1] : (k == 2 ? v[2] : v[3]));
 }
 
-// 4 floats at a uniform address plus a 32-bit offset in floats (an address in scalar registers
-// and one vector register)
-__device__ __forceinline__ const float* at(const float* base, unsigned i)
+// Cell i of a level at a uniform address.  I = int: a level below 4 GiB, whose byte offsets fit 32
+// bits (an address in scalar registers and one vector register); I = long long: any level.
+__device__ __forceinline__ const float* at(const float* base, int i)
 {
-    return reinterpret_cast<const float*>(reinterpret_cast<const char*>(base) + 4 * i);
+    return reinterpret_cast<const float*>(reinterpret_cast<const char*>(base) + 4 * (unsigned)i);
 }
-__device__ __forceinline__ float* at(float* base, unsigned i)
+__device__ __forceinline__ float* at(float* base, int i)
 {
-    return reinterpret_cast<float*>(reinterpret_cast<char*>(base) + 4 * i);
+    return reinterpret_cast<float*>(reinterpret_cast<char*>(base) + 4 * (unsigned)i);
 }
+__device__ __forceinline__ const float* at(const float* base, long long i) { return base + i; }
+__device__ __forceinline__ float* at(float* base, long long i) { return base + i; }
 
 // The thread's quads of a window: window quad i goes to float 4 i of the LDS window and comes
 // from float off of the level (kOutside: outside the grid, zeros).  Interior tiles' windows lie
 // inside the grid: such a tile starts at a multiple of 32 rows, ends before row nz - 6, and
 // before column nx - 6.
 constexpr int kOutside = -1;
-template <bool EDGE>
+template <bool EDGE, class I>
 struct AcQuads {
     using S = AcShape<EDGE>;
-    int off[S::NQ];
+    I off[S::NQ];
     __device__ __forceinline__ AcQuads(const AcousticArgs& a, const AcTile& t)
     {
 #pragma unroll
         for (int m = 0; m < S::NQ; m++) {
             const int i = threadIdx.x + m * kThreads, lx = i / S::WQ;
             const int gx = t.wsx + lx, gz = t.wsz + 4 * (i - lx * S::WQ);
-            off[m] = !EDGE || (gx >= 0 && gx < a.nx && gz >= 0 && gz < a.ldz) ? gx * a.ldz + gz : kOutside;
+            off[m] = !EDGE || (gx >= 0 && gx < a.nx && gz >= 0 && gz < a.ldz) ? (I)gx * a.ldz + gz : kOutside;
         }
     }
     __device__ __forceinline__ void load(const float* u, float* w) const
@@ -2491,6 +2494,7 @@ struct AcCell {
     float w[8], K, p;
 };
 // cell c of the tile's pass: rows 0-5 of the top (where the tile holds it), then of the bottom
+template <class I>
 __device__ __forceinline__ bool ac_cell(const AcousticArgs& a, const AcTile& t, int c, int ntop, int nbot,
                                         const float* prev, AcCell& e)
 {
@@ -2500,11 +2504,11 @@ __device__ __forceinline__ bool ac_cell(const AcousticArgs& a, const AcTile& t, 
     e.bot = row >= ntop;
     const int gz = e.bot ? max(a.nz - 6, t.sz) + (row - ntop) : row;
     e.r = e.bot ? a.nz - 1 - gz : gz;
-    const float* W = a.wz + (((e.bot ? a.nx : 0) + e.gx) * 6 + e.r) * 8;
+    const float* W = a.wz + ((I)((e.bot ? a.nx : 0) + e.gx) * 6 + e.r) * 8;
     unpack(ld4(W), e.w);
     unpack(ld4(W + 4), e.w + 4);
     if (e.r == 0) {
-        const int g = e.gx * a.ldz + gz;
+        const I g = (I)e.gx * a.ldz + gz;
         e.K = a.K[g];
         e.p = prev[g];
         if (a.taper_prev) e.p = (e.p * a.taper_z[gz]) * a.taper_x[e.gx];
@@ -2552,8 +2556,9 @@ __device__ __forceinline__ void ac_cell_run(const AcousticArgs& a, const AcTile&
 // x part of the Laplacian (times h^2) of a closure column's quad (columns 0-5 from a side), and
 // its SAT terms into sat;
 // w: the quad's window index, g its model index, p the tapered previous level
+template <class I>
 __device__ __forceinline__ void ac_closure_column(const AcousticArgs& a, const float* U, const float* R, int w, int gx,
-                                                  int z0, int g, const float* p, float* rhs, float* sat)
+                                                  int z0, I g, const float* p, float* rhs, float* sat)
 {
     const EdgeRow e = edge_row(gx, a.nx, 1);
     const float* W = a.wx + ((size_t)((e.sg < 0 ? 6 : 0) + e.r) * 8) * a.ldz + z0;
@@ -2623,7 +2628,7 @@ __device__ __forceinline__ void ac_d1x(const AcousticArgs& a, const float* u, co
 // level's cells c0, c0 + 256, ... before c1 get dt^2 K f over the divisor, tapered; sums in
 // injector order.  IMG: the increment's share of the K gradient by parts, which the imaging did
 // not see, goes to the group's slab.
-template <bool IMG>
+template <bool IMG, class I>
 __device__ __forceinline__ void ac_inject(const AcousticArgs& a, int c0, int c1, float* G)
 {
     const PointTable& pt = *a.points;
@@ -2631,7 +2636,7 @@ __device__ __forceinline__ void ac_inject(const AcousticArgs& a, int c0, int c1,
         const InjCell cell = pt.cells[c];
         float f = 0.f;
         for (int k = pt.ptr[c]; k < pt.ptr[c + 1]; k++) f += pt.w[k] * a.inj_trace[pt.ctx[k] + a.it];
-        const int g = cell.gx * a.ldz + cell.gz;
+        const I g = (I)cell.gx * a.ldz + cell.gz;
         const float inc = ((a.kdt2[g] * f / a.div[g]) * a.taper_z[cell.gz]) * a.taper_x[cell.gx];
         a.next[cell.shot * a.shot_stride + g] += inc;
         if (IMG) G[g] -= (a.wk + a.dwn) * inc * a.f0[cell.shot * a.fshot_stride + g] / (a.K[g] * a.K[g]);
@@ -2647,7 +2652,7 @@ __device__ __forceinline__ void ac_inject(const AcousticArgs& a, int c0, int c1,
 // dwn next + dwp prev (prev as stored; the point sources' share of next is ac_inject's), so a
 // step reads one snapshot, and its 1/rho term meets the step's own level (img_deriv): 16 B per
 // shot-cell instead of the 12 B of a step and 16 B of a separate k_agrad.
-template <bool EDGE, bool IMG>
+template <bool EDGE, bool IMG, class I>
 __device__ __forceinline__ void astep_tile(const AcousticArgs& a, int tix, int tiz, int grp, float* sR, float* sU,
                                            float* sF, EdgeTable tb)
 {
@@ -2656,14 +2661,15 @@ __device__ __forceinline__ void astep_tile(const AcousticArgs& a, int tix, int t
     const int nx = a.nx, nz = a.nz, ldz = a.ldz, tid = threadIdx.x;
     const int s0 = grp * a.spb, s1 = min(s0 + a.spb, a.nshots);
     const int* const tile_ptr = a.points->tile_ptr + (tix * a.ntz + tiz) * a.nshots;
-    AcQuads<EDGE> q(a, t);
+    AcQuads<EDGE, I> q(a, t);
     q.load(a.ri, sR);
     q.load(a.curr + s0 * a.shot_stride, sU);
     if (IMG) q.load(a.f0 + s0 * a.fshot_stride, sF);
     // threads past the last column compute the tile's first one and store nothing
     const bool active = t.sx + tid / (kAcTZ / 4) < t.ex;
     int gx = active ? t.sx + tid / (kAcTZ / 4) : t.sx, z0 = t.sz + 4 * (tid % (kAcTZ / 4));
-    int g = gx * ldz + z0, w = (gx - t.wsx) * WZ + (z0 - t.wsz);
+    I g = (I)gx * ldz + z0;
+    int w = (gx - t.wsx) * WZ + (z0 - t.wsz);
     float kd[4], tz[4], pn[4];  // pn: the previous level of the next shot, in flight with its windows
     unpack(ld4(at(a.prev + s0 * a.shot_stride, g), a.stream), pn);
     unpack(ld4(a.kdt2 + g), kd);
@@ -2772,12 +2778,12 @@ __device__ __forceinline__ void astep_tile(const AcousticArgs& a, int tix, int t
         if (EDGE && ntop + nbot > 0) {
 #pragma unroll
             for (int k = 0; k < 4; k++) __asm__ volatile("" : "+v"(zt[k]));
-            bool has = ac_cell(a, t, cell, ntop, nbot, prev, e);
+            bool has = ac_cell<I>(a, t, cell, ntop, nbot, prev, e);
 #pragma unroll 1
             while (has) {
                 ac_cell_run<IMG>(a, t, e, U, sR, F, tb);
                 cell += kThreads;
-                has = ac_cell(a, t, cell, ntop, nbot, prev, e);
+                has = ac_cell<I>(a, t, cell, ntop, nbot, prev, e);
             }
             __syncthreads();  // the closure rows' terms are in the windows
             float c[4];
@@ -2857,7 +2863,7 @@ __device__ __forceinline__ void astep_tile(const AcousticArgs& a, int tix, int t
         }
         __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();  // the next shot's windows are in, this one's are read, the new level is stored
-        if (inj1 > inj0) ac_inject<IMG>(a, inj0 + tid, inj1, G);
+        if (inj1 > inj0) ac_inject<IMG, I>(a, inj0 + tid, inj1, G);
     }
     if (IMG) __syncthreads();  // the point sources' shares are in the slab
     if (IMG && active) {
@@ -2885,7 +2891,7 @@ __device__ __forceinline__ void astep_tile(const AcousticArgs& a, int tix, int t
 // the windows in flight, so the bounds are the tightest ones that do not spill there (5 and 4
 // instead: 246 and 650 us); what the frame spills costs 1%.  Streamed levels (stream): 151
 // instead of 168 us above the memory-side cache's size, 2 to 12% slower below it.
-template <bool IMG>
+template <bool IMG, class I>
 __global__ void __launch_bounds__(kThreads, IMG ? 3 : 4) k_astep(const AcousticArgs a)
 {
     __shared__ __attribute__((aligned(16))) float sR[kAcWin];
@@ -2916,11 +2922,11 @@ __global__ void __launch_bounds__(kThreads, IMG ? 3 : 4) k_astep(const AcousticA
             tiz = a.itz0 + r / w;
             tix = c < a.itx0 ? c : a.itx1 + (c - a.itx0);
         }
-        astep_tile<true, IMG>(a, tix, tiz, grp, sR, sU, sF, tb);
+        astep_tile<true, IMG, I>(a, tix, tiz, grp, sR, sU, sF, tb);
     } else if (b < ne8 + nin * groups) {
         const int lin = xcd_remap(b - ne8, nin * groups);
         const int grp = lin / nin, tile = lin - grp * nin;
-        astep_tile<false, IMG>(a, a.itx0 + tile / nin_z, a.itz0 + tile % nin_z, grp, sR, sU, sF, tb);
+        astep_tile<false, IMG, I>(a, a.itx0 + tile / nin_z, a.itz0 + tile % nin_z, grp, sR, sU, sF, tb);
     } else {
         const int r = (b - ne8 - nin * groups) * kThreads + threadIdx.x;
         if (r < a.nrec) {
@@ -2941,6 +2947,7 @@ __global__ void __launch_bounds__(kThreads, IMG ? 3 : 4) k_astep(const AcousticA
 // shots (the step kernel's groups and windows, adjoint level and snapshot windows one shot
 // ahead), sums their terms in shot order in registers and adds the sum to the group's
 // gradient slab once.
+template <class I>
 __global__ void __launch_bounds__(kThreads, 5) k_agrad(const AcousticArgs a)
 {
     __shared__ __attribute__((aligned(16))) float sA[2 * kAcWin];
@@ -2956,13 +2963,14 @@ __global__ void __launch_bounds__(kThreads, 5) k_agrad(const AcousticArgs a)
     const AcTile t = ac_tile<true>(a, tix, tiz);
     const int nz = a.nz, ldz = a.ldz;
     const int s0 = grp * a.spb, s1 = min(s0 + a.spb, a.nshots);
-    const AcQuads<true> q(a, t);
+    const AcQuads<true, I> q(a, t);
     q.load(a.curr + s0 * a.shot_stride, sA);
     q.load(a.f0 + s0 * a.fshot_stride, sF);
     // threads past the last column compute the tile's first one and store nothing
     const bool active = t.sx + tid / (kAcTZ / 4) < t.ex;
     const int gx = active ? t.sx + tid / (kAcTZ / 4) : t.sx, z0 = t.sz + 4 * (tid % (kAcTZ / 4));
-    const int g = gx * ldz + z0, w = (gx - t.wsx) * WZ + (z0 - t.wsz);
+    const I g = (I)gx * ldz + z0;
+    const int w = (gx - t.wsx) * WZ + (z0 - t.wsz);
     const int zr = min(t.ez, nz);
     const int ntop = t.sz == 0 ? min(4, zr) : 0, nbot = max(0, zr - max(nz - 4, t.sz));
     float K[4], kw[4], gk[4], gr[4];  // kw: the K term's weight w / (dtg K^2)
@@ -3068,20 +3076,28 @@ __global__ void k_aextract(const float* u, long long shot_stride, int ldz, const
     trace[e.trace + it] = v;
 }
 
+// Whether 32-bit offsets reach every cell of a level (in bytes, see at) and every closure weight
+// (2 nx 48 of wz).  64-bit ones everywhere, also in the closure and point cells alone, cost 3 to 5%.
+static bool small_level(const AcousticArgs& a) { return (long long)a.nx * std::max(a.ldz, 48) < (1LL << 30); }
+
 void launch_astep(const AcousticArgs& a, hipStream_t s)
 {
     const int groups = (a.nshots + a.spb - 1) / a.spb;
     const int nin = (a.itx1 - a.itx0) * (a.itz1 - a.itz0), ne = (a.ntx * a.ntz - nin) * groups;
     const int nrec = a.rec_trace ? (a.nrec + kThreads - 1) / kThreads : 0;
     const dim3 grid(((ne + 7) & ~7) + nin * groups + nrec);
-    if (a.img) hipLaunchKernelGGL(k_astep<true>, grid, dim3(kThreads), 0, s, a);
-    else hipLaunchKernelGGL(k_astep<false>, grid, dim3(kThreads), 0, s, a);
+    if (a.img && small_level(a)) hipLaunchKernelGGL((k_astep<true, int>), grid, dim3(kThreads), 0, s, a);
+    else if (a.img) hipLaunchKernelGGL((k_astep<true, long long>), grid, dim3(kThreads), 0, s, a);
+    else if (small_level(a)) hipLaunchKernelGGL((k_astep<false, int>), grid, dim3(kThreads), 0, s, a);
+    else hipLaunchKernelGGL((k_astep<false, long long>), grid, dim3(kThreads), 0, s, a);
 }
 
 void launch_agrad(const AcousticArgs& a, hipStream_t s)
 {
     const int groups = (a.nshots + a.spb - 1) / a.spb;
-    hipLaunchKernelGGL(k_agrad, dim3(a.ntx * a.ntz * groups), dim3(kThreads), 0, s, a);
+    const dim3 grid(a.ntx * a.ntz * groups);
+    if (small_level(a)) hipLaunchKernelGGL(k_agrad<int>, grid, dim3(kThreads), 0, s, a);
+    else hipLaunchKernelGGL(k_agrad<long long>, grid, dim3(kThreads), 0, s, a);
 }
 
 void launch_ainit(const InjCell* cells, int ncell, const int* ptr, const long long* off, const float* w,
