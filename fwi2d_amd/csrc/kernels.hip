@@ -583,7 +583,7 @@ __device__ __forceinline__ bool z_cell(const StepArgs& a, const TileInfo& t, int
     e.gx = t.sx + i % S::TX;
     if (e.gx >= t.ex) return false;
     // weights [side][nx][6 rows][8 points], divided by dz^2
-    const float* W = a.wz + (((e.bot ? a.nx : 0) + e.gx) * 6 + e.r) * 8;
+    const float* W = a.wz + ((size_t)((e.bot ? a.nx : 0) + e.gx) * 6 + e.r) * 8;
     unpack(ld4(W), e.w);
     unpack(ld4(W + 4), e.w + 4);
     if (e.r == 0 && (e.bot ? a.bc_bottom : a.bc_top) == 2) {

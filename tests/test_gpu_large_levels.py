@@ -1,6 +1,6 @@
 """Grids whose level or closure weights lie past 32-bit offsets: an acoustic level of 1.6e9 cells
-(6 GiB: byte offsets past 2^32) and 22.4 million columns (2 nx 48 closure weights: indices past 2^31).
-Ten steps next to the far side equal those of a small grid with the same
+(6 GiB: byte offsets past 2^32) and 22.4 million columns (2 nx 48 closure weights: indices past 2^31),
+on both engines.  Ten steps next to the far side equal those of a small grid with the same
 cells there; 22.4 million and 96 columns are whole tiles, so the same cells fall into the same kinds
 of tiles and the values are the same bit for bit.  (All positions are binary fractions, so that the
 points' weights are the same too.)"""
@@ -60,3 +60,18 @@ def test_acoustic_level_past_4_gib(lib):
     assert np.abs(out[0][0]).max() > 0 and np.abs(out[0][1]).max() > 0
     assert np.array_equal(out[0][0], out[1][0])
     assert np.array_equal(out[0][1], out[1][1])
+
+
+def test_elastic_closure_weights_past_2_31(lib):
+    nz = 12
+    src = np.random.default_rng(2).standard_normal((2, 2, NT)).astype(np.float32)
+    out = []
+    for nx in (SMALL, NX):
+        e = lib.Engine(grid(lib, nx, nz, 0, (1, 1, 2)))
+        e.set_model(fields((2.5, 1.7, 2.0), nz, nx))
+        e.set_shots(*points(nx, nz, 2))
+        out.append(e.forward(src))
+        print("nx %d: done" % nx, flush=True)
+        e.close()
+    assert np.abs(out[0]).max() > 0
+    assert np.array_equal(out[0], out[1])
