@@ -1546,8 +1546,8 @@ long long fwi2d_engine_get_stat(fwi2d_engine* e, const char* key)
     if (k == "segment") return x->seg_K;
     if (k == "nseg") return x->nseg;
     if (k == "tile_x") return x->tile_x;
-    if (k == "shots_per_block") return x->spb();
-    if (k == "shots_per_block_edge") return x->spb_edge();
+    if (k == "shots_per_block") return x->opt_spb > 0 ? x->opt_spb : x->spb();
+    if (k == "shots_per_block_edge") return x->opt_spb_edge > 0 ? x->opt_spb_edge : x->spb_edge();
     if (k == "shots_per_block_edge_img") return x->opt_spb_edge_img;
     if (k == "band_rows") return x->opt_band_rows;
     if (k == "shots_per_block_img") return x->opt_spb_img;

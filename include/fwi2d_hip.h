@@ -119,9 +119,10 @@ int fwi2d_dot_f64_noalloc(int device, const float* a, const float* b, const floa
 /* Tuning and test options (no reference counterpart): "tile_x" (16 | 32 cells per tile
    along x), "shots_per_block" (1..64 shots advanced in turn by one step workgroup of an
    interior tile; by default up to 8, fewer where the launch would otherwise have less than
-   2048 workgroups; the stat reads the number in effect), "shots_per_block_edge" (the same
-   for tiles at the grid edge), "shots_per_block_edge_img" (the same for edge tiles of
-   adjoint steps with the imaging fused in; 0, the default: "shots_per_block_edge"),
+   2048 workgroups; the stat reads what was set, or while nothing was the number in
+   effect), "shots_per_block_edge" (the same for tiles at the grid edge),
+   "shots_per_block_edge_img" (the same for edge tiles of adjoint steps with the imaging
+   fused in; 0, the default: "shots_per_block_edge"),
    "edge_stream" (0, 1 or 2) and "band_rows" (8, 12 or 16) (accepted without effect: a step
    is one launch over all tiles),
    "shots_per_block_img" (shots per imaging workgroup; 0: up to 4, or "shots_per_block"
