@@ -60,7 +60,7 @@ def parse():
                          "0: in a separate imaging kernel after each adjoint step; -1: the engine's default "
                          "(1 on isotropic grids, 0 on VTI grids)")
     ap.add_argument("--engine-preset", action="append", default=[], metavar="KEY=VALUE",
-                    help="an engine option set before the autotuner runs, e.g. band_rows=16; repeatable")
+                    help="an engine option set before the autotuner runs, e.g. lag=0; repeatable")
     ap.add_argument("--engine-option", action="append", default=[], metavar="KEY=VALUE",
                     help="an engine option (fwi2d_engine_set_option) set after the autotuner ran, e.g. "
                          "shots_per_block_img=8; repeatable")
@@ -96,10 +96,8 @@ def parse():
     ap.add_argument("--acoustic", type=int, metavar="SUB", default=None,
                     help="the acoustic operator (nl_we_op_a) on the C2 geometry: batched gradients with snapshots "
                          "every SUB steps, kept whole")
-    ap.add_argument("--step-only", type=int, metavar="EDGE_STREAM", default=None,
-                    help="only autotune and time the forward time step of the workload with this edge_stream "
-                         "setting (0: every launch of a step on one stream, for per-launch kernel traces), "
-                         "print the step time and exit")
+    ap.add_argument("--step-only", action="store_true",
+                    help="only autotune and time the forward time step of the workload, print the step time and exit")
     return ap.parse_args()
 
 
@@ -110,7 +108,7 @@ ACOUSTIC_TRAFFIC_FILE = os.path.join(ROOT, "profiles", "k_astep_acoustic_64shots
 def measured_traffic(spb=None, path=TRAFFIC_FILE):
     """HBM bytes per forward step from the committed counter summary (FETCH_SIZE and
     WRITE_SIZE per dispatch, calibrated against a copy kernel of known size) for the
-    core launch's shots per workgroup spb (the autotuner's choice), or None."""
+    step's shots per workgroup spb (the autotuner's choice), or None."""
     try:
         lines = open(path).read().splitlines()
     except OSError:
@@ -337,8 +335,8 @@ def cpu_baseline(nt_sample=400, kind="c2"):
 
 
 def step_only(args):
-    """The forward time step alone: autotuned as in the bench, then 40 eager steps with the
-    given edge_stream setting, timed with HIP events on the engine stream."""
+    """The forward time step alone: autotuned as in the bench, then 40 eager steps timed with HIP
+    events on the engine stream."""
     import torch
     import fwi2d_amd
     fwi2d_amd.load()
@@ -347,12 +345,11 @@ def step_only(args):
     prob, m_true, m0, sxz, rxz, src, dt = workload(args.workload, ns, nt)
     B = Batch(fwi2d_amd, torch, prob, m_true, m0, sxz, rxz, src, nt, dt, args.tile_x, presets=args.engine_preset)
     B.eng.set_option("graph", 0)
-    B.eng.set_option("edge_stream", args.step_only)
     B.eng.set_option("timing", 1)
     for _ in range(2):
         B.eng.forward_device(B.src.data_ptr(), B.rcv.data_ptr(), keep_checkpoints=False)
     us = B.eng.stat("fwd_loop_ns") / 1e3 / B.eng.stat("fwd_loop_steps")
-    print(json.dumps({"workload": args.workload, "edge_stream": args.step_only, "step_us": round(us, 2),
+    print(json.dumps({"workload": args.workload, "step_us": round(us, 2),
                       "presets": args.engine_preset,
                       "tile_x": B.eng.stat("tile_x"), "shots_per_block": B.eng.stat("shots_per_block"),
                       "shots_per_block_edge": B.eng.stat("shots_per_block_edge")}))
@@ -542,7 +539,7 @@ def acoustic_run(args):
             "misfit_f64": res.get("misfit"),
             "grad_rel_err_vs_fp64": err,
             "grad_err_sample": "1 shot, 160x100 grid, nt=600, sub=2, raw K and 1/rho gradients vs FP64 oracle",
-            "roofline": {"bound": "hbm", "kernel": "k_astep + k_ainject per step (eager forward, no snapshots)",
+            "roofline": {"bound": "hbm", "kernel": "k_astep (time step of all shots with point sources and receivers; eager forward, no snapshots)",
                          "achieved": round(fwd_bytes / step_s / 1e9, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                          "frac": round(fwd_bytes / step_s / 1e9 / HBM_PEAK_GBS, 4),
                          "traffic": measured_traffic(path=ACOUSTIC_TRAFFIC_FILE) if ns == 64 else None,
@@ -662,7 +659,7 @@ def main():
     if args.calibrate_copy:
         calibrate_copy()
         return
-    if args.step_only is not None:
+    if args.step_only:
         step_only(args)
         return
     if args.operator:  # with --acoustic SUB: the acoustic operator at the operator level
@@ -717,10 +714,10 @@ def main():
     traffic = measured_traffic(B.eng.stat("shots_per_block")) if (args.workload, ns) == ("c2", 64) else None
 
     # ---- dominant kernel: fused step, timed with HIP events on its stream ----
-    # (eager launches: one step = the core-box launch plus the edge-band launches beside it)
+    # (eager launches: one step = k_step over all tiles and k_points)
     image_fused = B.eng.stat("image_fused")
     tune = {"tile_x": B.eng.stat("tile_x"), "shots_per_block": B.eng.stat("shots_per_block"),
-            "shots_per_block_edge": B.eng.stat("shots_per_block_edge"), "edge_stream": B.eng.stat("edge_stream"),
+            "shots_per_block_edge": B.eng.stat("shots_per_block_edge"),
             "report": B.eng.tune_report()}
     graph_replays = B.eng.stat("graph_replays")
     recompute = B.eng.stat("recompute_steps")
@@ -806,7 +803,7 @@ def main():
         "misfit_f64": misfit,
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
-                     "kernel": "k_step (fused time step of all shots: core-box launch + edge-band launches)",
+                     "kernel": "k_step + k_points (fused time step of all shots, point sources and receivers)",
                      "avg_launch_us": round(step_s * 1e6, 2),
                      "bytes_per_cell_update": bytes_per_cell, "cells_per_launch": cells_per_launch,
                      # the whole gradient (forward + checkpointed adjoint with imaging) against the

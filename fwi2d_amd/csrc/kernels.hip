@@ -225,16 +225,18 @@ __device__ __forceinline__ float d2_apply(const W5& w, const float* pu, int s)
 //     table.
 //   * Along z a closure row is part of a quad.  Every quad forms the interior rows, and the
 //     closure rows are dealt one cell per thread in passes of their own: the products of
-//     rows 0-3 from either side, then the z terms (with the top and bottom SAT terms) of
-//     rows 0-5, and the left and right SAT terms, which go to the quads' owners through the
-//     out-of-grid cells of the state windows.
+//     rows 0-3 from either side, then the z terms of rows 0-5, and the impedance terms of
+//     absorbing left and right sides, which go to the quads' owners through the out-of-grid
+//     cells of the state windows.
+//   * The SAT terms of a side are part of its boundary row: its D2 weights and its first D1
+//     coefficient (see z_cell).
 // The instance-per-row form this replaced (34-60 KB of code per kernel, edge bands beside a
 // core launch) was bound by instruction fetch: one band workgroup took 30 us alone, and a
-// step of one shot on 201 x 601 cells 117 us (the core launch 6.4 us of it); it takes 14 us
-// in this form (one launch), a 64-shot step on 500 x 1700 392 us instead of 401.  A frame
-// tile costs about 1.7 times an interior one, in VALU work (1209 against 527 vector
-// instructions per wavefront and shot at first, most of the surplus addresses), so it loads
-// per shot what its passes need and keeps no D2 weights: spills cost it more than both.
+// step of one shot on 201 x 601 cells 105 us; it takes 11 us in this form (one launch), and
+// 64 shots of 500 x 1700 394 us instead of 407.  A frame tile costs more than an interior one
+// in VALU work (at first 1209 against 527 vector instructions per wavefront and shot, most of
+// the surplus addresses), so it loads per shot what its passes need and keeps no D2 weights:
+// spills cost it more than both.
 // ---------------------------------------------------------------------------
 template <int TX_>
 struct StepShape {
@@ -267,7 +269,7 @@ __device__ __forceinline__ void out_quad(const TileInfo& t, int i, int& gx, int&
 
 // D1 rows 0-5 on points 0-7 in LDS (rows 4 and 5 are interior rows), row stride rs
 struct EdgeTable {
-    const float* c;
+    float* c;
     int rs;
 };
 
@@ -333,10 +335,6 @@ constexpr EdgeD1 edge_d1_table()
 }
 __constant__ EdgeD1 cEdgeD1 = edge_d1_table();
 
-// One launch for all tiles: the frame's workgroups first (their extra passes make them the
-// slowest), then the interior rectangle's, each class spread over all XCDs (the frame's
-// block count rounded up to a multiple of 8, the extra blocks idle) and remapped within its
-// class so that an XCD runs neighbouring tiles.
 // ---- table-driven closure rows -------------------------------------------------------
 // A closure row of point g of n: the edge point's offset o from g and the inward step st
 // along a line of stride s, the row r from the edge, and the sign of D1 there.
@@ -913,6 +911,7 @@ __device__ __forceinline__ void d1z_pass(const StepArgs& a, float* u, float* v, 
 // snapshot idx (x_x, z_z, z_x, x_z), f0/fm/fp the snapshots idx, idx-1, idx+1 at the
 // cells, o the adjoint level of the density term.  Adds to the accumulators of the
 // lambda, mu, rho gradients (VTI stiffness mode: c11, c13, c33, c55, rho).
+//
 // Density term of the imaging condition of one quad: o is the adjoint level after the
 // step, f0/fm/fp the snapshots idx, idx-1, idx+1 at the cells (second time difference;
 // one-sided at the first and last snapshot, mode 1 and 2).  It goes to gr, or to g4 in
@@ -1272,7 +1271,7 @@ __device__ __forceinline__ void step_tile(const StepArgs& a, const StepSmem& sm,
         }
         __syncthreads();  // the previous shot is done with the LDS state and products
         if (EDGE && VTI && shot == s0 && tid < 48)
-            const_cast<float*>(sm.tb.c)[sm.tb.rs * (tid >> 3) + (tid & 7)] = cEdgeD1.c[tid];
+            sm.tb.c[sm.tb.rs * (tid >> 3) + (tid & 7)] = cEdgeD1.c[tid];
         const float* cux = a.curr + shot * a.shot_stride;
 #pragma unroll
         for (int m = 0; m < S::NQ1; m++) {
@@ -1535,7 +1534,11 @@ __device__ __forceinline__ void step_tile(const StepArgs& a, const StepSmem& sm,
 // wavefronts per SIMD the registers must leave room for: the LDS's share
 constexpr int step_waves(bool vti, int tx, bool img) { return tx == 32 ? 2 : (vti || img ? (vti && img ? 2 : 3) : 4); }
 
-// PTS: the launch also takes the point sources and receivers (see step_launch).
+// One launch for all tiles: the frame's workgroups first (their extra passes make them the
+// slowest), then the interior rectangle's, each class spread over all XCDs (the frame's
+// block count rounded up to a multiple of 8, the extra blocks idle) and remapped within its
+// class so that an XCD runs neighbouring tiles.  PTS: the launch also takes the point sources
+// and receivers (see step_launch).
 template <bool VTI, int TX, bool IMG, bool PTS>
 __global__ void __launch_bounds__(kThreads, step_waves(VTI, TX, IMG)) k_step(const StepArgs a)
 {
@@ -2192,10 +2195,10 @@ static void step_launch(const StepArgs& a, bool image, int ncell, hipStream_t s)
     const int nstep = ((ne + 7) & ~7) + nin * a.ngroups;
     const int nrec = a.rec_trace ? (2 * a.nrec + kThreads - 1) / kThreads : 0;
     // Point sources and receivers: in the step's launch while its workgroups fit the chip about
-    // once (4 per CU): one shot on 201 x 601 takes 12.4 us a step instead of 14.6 and 8.5 in
-    // launches of their own.  In larger launches the step kernel without their code keeps its
-    // registers: 64 shots of 500 x 1700 took 455 us a step with them in the launch, 392 us and
-    // 8 us for k_points without.
+    // once (4 per CU): one shot on 201 x 601 takes 11.2 us a step, and 14.5 us with a launch of
+    // their own.  In larger launches the step kernel without their code keeps its registers:
+    // 64 shots of 500 x 1700 take 394 us a step, k_points included, and 445 us with them in the
+    // launch.
     if constexpr (TX == 16) {
         if (nstep <= 1024) {
             const dim3 grid(nstep + nrec);
@@ -2378,12 +2381,15 @@ __device__ __forceinline__ float ac_bnd(float u0, float u1, float u2, float u3)
 {
     return __builtin_fmaf(cSC[3], u3, __builtin_fmaf(cSC[2], u2, __builtin_fmaf(cSC[0], u0, cSC[1] * u1)));
 }
-// d2_apply and d2_weights with the order of their roundings written out, so
-// that the results do not depend on how the compiler contracts the expressions around them (the
-// 1/rho gradient on a free surface is a sum of large cancelling terms: a change of the rounding
-// alone moves single values by up to 1e-3 of the gradient's rms).  CF: the centre's product is
-// rounded, not the lower neighbour's; MN, PN: on the lower and the upper side the nearer
-// coefficient's product is; sf: the nearest pair's product is, not the centre's.
+// d2_apply and d2_weights with the order of their roundings written out, so that the results do
+// not depend on how the compiler contracts the expressions around them.  The orders, and where each
+// holds, are those of the first kernel of this operator, kept so that its results stay the same bit
+// for bit; no order is more accurate than another.  On a free surface the 1/rho gradient is a sum
+// of large cancelling terms: with one order for all cells, or with the elastic step's consistent
+// rows, single values move by 5 to 9e-4 of the gradient's rms, and stay 1.4 to 2.4e-3 of it off
+// FP64 (1.6 to 2.8e-3 as it is), which is the rounding of the stored levels.
+// CF: the centre's product is rounded, not the lower neighbour's; MN, PN: on the lower and the upper
+// side the nearer coefficient's product is; sf: the nearest pair's product is, not the centre's.
 template <bool CF>
 __device__ __forceinline__ float ac_d2(const W5& w, float m2, float m1, float u0, float p1, float p2)
 {
