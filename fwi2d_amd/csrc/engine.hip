@@ -99,6 +99,9 @@ struct Engine {
     // state and checkpoints
     DevMem d_fwd, d_adj, d_ckpt, d_seg, d_gshot, d_gout, d_src, d_rcv, d_adjsrc, d_partial, d_scalar;
     DevMem d_ckpt16, d_ckpt_scale, d_amax;  // 16-bit checkpoint levels, their per-shot scales
+    // the carry of the rows below a free surface (StepArgs::carry): of the forward run and its
+    // recomputation and of the adjoint run, and with the checkpoint of every segment after the first
+    DevMem d_carry, d_ckpt_carry;
     DevMem d_tm_ptr, d_tm_col, d_tm_w, d_tdata;  // operator-level trace matrix and data traces
     int opt_bf16 = 0;                       // checkpoint levels: 0 FP32, 1 BF16, 2 FP16 (max-abs scaled)
     int opt_stiff = 0;                      // VTI raw gradients w.r.t. c11, c13, c33, c55, rho
@@ -637,11 +640,19 @@ struct Engine {
         return L;
     }
 
+    long long carry_stride() const { return g.bc_top == 1 ? (long long)ns * 2 * g.nx * kCarryRows : 0; }
+    float* carry(bool adjoint) const { return carry_stride() ? d_carry.as<float>() + (adjoint ? carry_stride() : 0) : nullptr; }
+    float* ckpt_carry(int j) const { return d_ckpt_carry.as<float>() + (j - 1) * carry_stride(); }
+
     // zero state, then prev = 1/2 dt^2/rho * inject(trace sample 0)
     void init_levels(Levels& L, bool adjoint, const float* traces)
     {
         const long long ss = state_stride();
         launch_fill(L.b[0], L.n * ss, 0.f, st);
+        if (carry_stride() > 0) {
+            d_carry.reserve((size_t)2 * carry_stride() * sizeof(float));
+            launch_fill(carry(adjoint), carry_stride(), 0.f, st);
+        }
         L.prev = 0;
         L.curr = 1;
         L.next = 2;
@@ -695,6 +706,7 @@ struct Engine {
         a.inj_trace = traces;
         a.rec_trace = rcv;
         a.nrec = nr;
+        a.carry = carry(adjoint);
         launch_step(a, vti, tile_x, fuse_img, (int)(adjoint ? inj_rcv : inj_src).cells.size(), st);
         if (img_idx >= 0 && !fuse_img) {
             ia.aprev = L.P();
@@ -833,7 +845,7 @@ struct Engine {
                 P(inj_src.d_tile_ptr.p), P(inj_rcv.d_tile_ptr.p),
                 P(inj_rcv.d_cw.p), (long long)inj_src.cells.size(), (long long)inj_rcv.cells.size(),
                 P(d_rcv_ext_ents.p), P(d_tx.p), P(d_tz.p),
-                P(d_div_tb.p), P(d_div_lr.p)};
+                P(d_div_tb.p), P(d_div_lr.p), P(d_carry.p), P(d_ckpt_carry.p)};
     }
 
     // Runs body (which only enqueues device work on st) directly, or, with the
@@ -965,6 +977,7 @@ struct Engine {
                 d_ckpt.reserve(nslot * state_stride() * sizeof(float));
             }
             d_seg.reserve((size_t)(seg_K + 2) * state_stride() * sizeof(float));
+            if (carry_stride() > 0) d_ckpt_carry.reserve((size_t)std::max(nseg - 1, 1) * carry_stride() * sizeof(float));
             jlast = nseg - 1;
         }
         const int nt = g.nt;
@@ -1016,6 +1029,7 @@ struct Engine {
             if (level == (j * seg_K - 1) * g.sub && level < g.nt - 1) {
                 ckpt_store(2 * (j - 1), L.C());
                 ckpt_store(2 * (j - 1) + 1, L.P());
+                if (carry_stride() > 0) launch_copy(ckpt_carry(j), carry(false), carry_stride(), st);
             }
         if (level % g.sub == 0) {
             int idx = level / g.sub;
@@ -1095,6 +1109,7 @@ struct Engine {
         img_join();  // the recompute overwrites snapshot slots the imaging reads
         const long long ss = state_stride();
         Levels F = levels_in(d_fwd);
+        if (j > 0 && carry_stride() > 0) launch_copy(carry(false), ckpt_carry(j), carry_stride(), st);
         if (g.sub == 1) {
             // every level is a snapshot: step straight from slot to slot of the segment
             // buffer (the level before the first slot lives in a scratch level)

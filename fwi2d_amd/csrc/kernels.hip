@@ -230,6 +230,13 @@ __device__ __forceinline__ float d2_apply(const W5& w, const float* pu, int s)
 //     cells of the state windows.
 //   * The SAT terms of a side are part of its boundary row: its D2 weights and its first D1
 //     coefficient (see z_cell).
+//   * In the rows below a free surface at the top the leapfrog carries, per cell, what the
+//     rounding of the new level leaves of its increment to the next step (StepArgs::carry).  Every
+//     rounding of a level is a kick that the scheme integrates twice; surface waves meet them all
+//     the way and do not spread, and they were nearly the whole error: 14 rows in FP64 bring a
+//     one-shot gradient of 1500 steps from 4.8e-6 to 2.3e-7 off FP64.  With the carry such
+//     gradients are 1.0 to 1.3e-6 off, 3.0 to 7.0e-6 without.  16 rows are 3% of 500: a step of
+//     64 shots takes 397 instead of 394 us, of one on 201 x 601 11.4 instead of 11.1 us.
 // The instance-per-row form this replaced (34-60 KB of code per kernel, edge bands beside a
 // core launch) was bound by instruction fetch: one band workgroup took 30 us alone, and a
 // step of one shot on 201 x 601 cells 105 us; it takes 11 us in this form (one launch), and
@@ -1078,8 +1085,14 @@ __device__ __forceinline__ void inject_cells(const StepArgs& a, int c0, int c1, 
         const float f = a.irho[g] * a.taper_z[gz] * a.taper_x[gx];
         const float ix = f * fx / dx, iz = f * fz / dz;
         float* u = a.next + cell.shot * a.shot_stride + g;
-        u[0] += ix;
-        u[nxz] += iz;
+        const float ux = u[0], uz = u[nxz], nx1 = ux + ix, nz1 = uz + iz;
+        u[0] = nx1;
+        u[nxz] = nz1;
+        if (a.carry && gz < kCarryRows) {
+            float* e = a.carry + ((cell.shot * 2LL) * nx + gx) * kCarryRows + gz;
+            e[0] += ix - (nx1 - ux);
+            e[(long long)nx * kCarryRows] += iz - (nz1 - uz);
+        }
         if (img) {
             const long long fo = cell.shot * a.fshot_stride + g;
             a.grad[cell.shot * a.gslab_stride + (a.stiff ? 4 : 2) * nxz + g] +=
@@ -1238,8 +1251,8 @@ __device__ __forceinline__ void step_tile(const StepArgs& a, const StepSmem& sm,
         int tid = tid0;
         opaque(t);
         opaque_v(tid);
-        // previous level of this shot's new-level quads
-        float4 qprx[S::NQ3], qprz[S::NQ3];
+        // previous level of this shot's new-level quads; frame tiles: what their last step carries over
+        float4 qprx[S::NQ3], qprz[S::NQ3], qex[EDGE ? S::NQ3 : 1], qez[EDGE ? S::NQ3 : 1];
         const float* pux = a.prev + shot * a.shot_stride;
         const int inj0 = PTS ? tile_ptr[shot] : 0, inj1 = PTS ? tile_ptr[shot + 1] : 0;  // the sources' cells
         auto load_prev = [&] {
@@ -1253,6 +1266,12 @@ __device__ __forceinline__ void step_tile(const StepArgs& a, const StepSmem& sm,
             const float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
             qprx[m] = ok ? ld4(pux + g) : z4;
             qprz[m] = ok ? ld4(pux + nxz + g) : z4;
+            if constexpr (EDGE) {
+                const bool c = ok && a.carry && gz < kCarryRows;
+                const float* e = a.carry + ((shot * 2LL) * nx + gx) * kCarryRows + gz;
+                qex[m] = c ? ld4(e) : z4;
+                qez[m] = c ? ld4(e + (long long)nx * kCarryRows) : z4;
+            }
         }
         };
         if (!EDGE) load_prev();
@@ -1389,11 +1408,31 @@ __device__ __forceinline__ void step_tile(const StepArgs& a, const StepSmem& sm,
             float cx[4], cz[4], vx[4], vz[4];
             unpack(ld4(&sm.ux[wq]), cx);
             unpack(ld4(&sm.uz[wq]), cz);
+            // leapfrog (we_op.cpp:824-830) with ir = dt^2 / rho
+            if constexpr (EDGE) {
+                float ex[4], ez[4];
+                unpack(qex[m], ex);
+                unpack(qez[m], ez);
 #pragma unroll
-            for (int k = 0; k < 4; k++) {
-                // leapfrog (we_op.cpp:824-830) with ir = dt^2 / rho
-                vx[k] = ir[k] * rx[k] + (2.f * cx[k] - prx[k]);
-                vz[k] = ir[k] * rz[k] + (2.f * cz[k] - prz[k]);
+                for (int k = 0; k < 4; k++) {
+                    const float wx = (ir[k] * rx[k] + (cx[k] - prx[k])) + ex[k];
+                    const float wz = (ir[k] * rz[k] + (cz[k] - prz[k])) + ez[k];
+                    vx[k] = cx[k] + wx;
+                    vz[k] = cz[k] + wz;
+                    ex[k] = wx - (vx[k] - cx[k]);
+                    ez[k] = wz - (vz[k] - cz[k]);
+                }
+                if (a.carry && z0 < kCarryRows) {
+                    float* e = a.carry + ((shot * 2LL) * nx + gx) * kCarryRows + z0;
+                    st4(e, make_float4(ex[0], ex[1], ex[2], ex[3]));
+                    st4(e + (long long)nx * kCarryRows, make_float4(ez[0], ez[1], ez[2], ez[3]));
+                }
+            } else {
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    vx[k] = ir[k] * rx[k] + (2.f * cx[k] - prx[k]);
+                    vz[k] = ir[k] * rz[k] + (2.f * cz[k] - prz[k]);
+                }
             }
             if constexpr (EDGE) {
                 // implicit part of the absorbing SAT on the perimeter (spatial_operators.cpp:307-521)

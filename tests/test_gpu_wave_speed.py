@@ -28,8 +28,8 @@ def delay(out, ref):
     return float((d * du).sum() / (du * du).sum()), float(np.linalg.norm(d) / np.linalg.norm(ref))
 
 
-@pytest.mark.parametrize("physics", ["iso", "vti", "acoustic"])
-def test_no_delay(orc64, physics):
+def traces(orc64, physics):
+    """the engine's traces and the oracle's"""
     import fwi2d_amd as lib
 
     x, z = np.arange(NX)[:, None] * H, np.arange(NZ)[None, :] * H
@@ -61,6 +61,24 @@ def test_no_delay(orc64, physics):
         src = np.stack([0.3 * wav[None], wav[None]])
         ref = el.oracle_forward(orc64, prob, model, sxz, rxz, src, NT, DT)
         _, out = el.run_engine(lib, prob, model, sxz, rxz, src, NT, DT)
-    a, err = delay(out, ref)
+    return out, ref
+
+
+@pytest.mark.parametrize("physics", ["iso", "vti", "acoustic"])
+def test_no_delay(orc64, physics):
+    a, err = delay(*traces(orc64, physics))
     print("%s: delay %.2e steps, relative error %.2e" % (physics, a, err))
     assert abs(a) <= 1e-4
+
+
+@pytest.mark.parametrize("physics", ["iso", "vti"])
+def test_surface_waves_below_the_rounding_of_the_levels(orc64, physics):
+    """The traces of a free surface are nearer to FP64 than levels rounded to FP32 at every step leave
+    them, since the rows below it carry their rounding over.  Tolerance 2.5e-6, two thirds of the
+    3.7e-6 that exact arithmetic on rounded levels leaves here (rounding errors of rms 0.3 ulp,
+    integrated twice over 1500 steps): the right-hand side's own rounding, of terms a tenth of
+    the levels' size, and the waves' share below the 16 rows remain."""
+    out, ref = traces(orc64, physics)
+    err = delay(out, ref)[1]
+    print("%s: relative error %.2e" % (physics, err))
+    assert err <= 2.5e-6
