@@ -34,11 +34,13 @@ BYTES_PER_CELL_UPDATE_FWD = 36.0   # iso forward step: read curr 2 + prev 2 + mo
 BYTES_PER_GRADIENT_CELL_STEP = {False: 36.0 + 68.0, True: 44.0 + 76.0}
 # acoustic operator (nl_we_op_a), per shot-cell: a step reads prev and curr and writes next
 # (12 B; its per-cell factors dt^2 K, 1/rho and the boundary divisor are read once per cell
-# for all shots); imaging every sub steps reads the adjoint level and snapshots j-1, j, j+1
-# and read-modify-writes the K and 1/rho slabs (32 B); the forward run writes snapshot j
+# for all shots).  Imaging at sub = 1 is part of the adjoint step and reads one snapshot more;
+# otherwise a snapshot's launch reads the adjoint level and snapshots j-1, j, j+1.  Either
+# reads and writes the K and 1/rho slabs once per cell and group of 8 shots.  Snapshots are
+# written in the new level's place.
 ACOUSTIC_BYTES_FWD = 12.0
 ACOUSTIC_BYTES_MODEL = 12.0
-ACOUSTIC_BYTES_IMAGING = 32.0
+ACOUSTIC_BYTES_SLABS = 16.0
 
 
 def parse():
@@ -101,8 +103,8 @@ def parse():
     return ap.parse_args()
 
 
-TRAFFIC_FILE = os.path.join(ROOT, "profiles", "k_step_iso_64shots_500x1700_traffic.md")
-ACOUSTIC_TRAFFIC_FILE = os.path.join(ROOT, "profiles", "k_astep_acoustic_64shots_500x1700.md")
+TRAFFIC_FILE = os.path.join(ROOT, "profiles", "elastic_64shots_500x1700.md")
+ACOUSTIC_TRAFFIC_FILE = os.path.join(ROOT, "profiles", "acoustic_64shots_500x1700.md")
 
 
 def measured_traffic(spb=None, path=TRAFFIC_FILE):
@@ -526,7 +528,8 @@ def acoustic_run(args):
     step_s = fwd_s / (nt - 1)
     cells = ns * nx * nz
     fwd_bytes = ACOUSTIC_BYTES_FWD * cells + ACOUSTIC_BYTES_MODEL * nx * nz
-    grad_bytes = (2 * fwd_bytes * (nt - 1) + (4.0 + ACOUSTIC_BYTES_IMAGING) * cells * (nt // sub + 1))
+    img_bytes = (4.0 if sub == 1 else 16.0) * cells + ACOUSTIC_BYTES_SLABS * nx * nz * ((ns + 7) // 8)
+    grad_bytes = 2 * fwd_bytes * (nt - 1) + img_bytes * (nt - 1 if sub == 1 else nt // sub + 1)
     err = None if args.no_check else acoustic_grad_error_small()
     cpu = None if args.no_cpu else acoustic_cpu_baseline(800, sub)
     line = {"metric": "acoustic FWI gradient shots/s (nl_we_op_a, batched)", "value": round(shots_per_s, 4),
