@@ -26,7 +26,6 @@
 namespace fwi2d {
 
 extern thread_local std::string g_last_error;
-void upload_constants(hipStream_t s);
 
 namespace {
 
@@ -70,7 +69,6 @@ struct Acoustic {
         alpha = kFreeSurfaceA / std::max(stiffness, 1.0);
         HIPCHECK(hipSetDevice(device));
         HIPCHECK(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
-        upload_constants(st);
         ldz = (g.nz + 31) / 32 * 32;  // columns start on 128-byte lines
         nxz = (long long)g.nx * ldz;
         ntx = (g.nx + kAcTX - 1) / kAcTX;

@@ -131,7 +131,6 @@ struct Engine {
         HIPCHECK(hipStreamCreateWithFlags(&st_img, hipStreamNonBlocking));
         HIPCHECK(hipEventCreateWithFlags(&ev_img_in, hipEventDisableTiming));
         for (auto& e : ev_img_done) HIPCHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-        upload_constants(st);
         set_tile(opt_tile_x);
         build_tapers();
     }

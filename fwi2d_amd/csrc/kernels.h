@@ -119,8 +119,6 @@ struct ImageArgs {
     int lag;                 // 1: derivatives of adj_prev (reference), 0: of adj
 };
 
-void upload_constants(hipStream_t s);
-
 int tiles_x(int nx, int tile_x);
 int tiles_z(int ldz);
 void tile_range_x(int k, int ntile, int T, int n, int& s, int& e);

@@ -17,26 +17,23 @@
 
 namespace fwi2d {
 
-__constant__ float cD1I[2];   // elastic interior rows (see kD2Interior24)
-__constant__ float cD2I[10];
-__constant__ float cD1A[2];   // acoustic: the rows rounded one by one
-__constant__ float cD2A[10];
-__constant__ float cSC[4];
-
-void upload_constants(hipStream_t s)
+// Interior rows and the SAT's boundary derivative, as literals in the kernels (the frame tiles are
+// short of scalar registers).  Elastic rows: see kD2Interior24; the acoustic ones are rounded one
+// by one.
+template <int N>
+struct Row {
+    float c[N];
+};
+template <int N>
+constexpr Row<N> rounded(const double (&v)[N])
 {
-    float d1a[2], sc[4], d2a[10];
-    for (int i = 0; i < 2; i++) d1a[i] = (float)kD1Interior[i];
-    for (int i = 0; i < 4; i++) sc[i] = (float)kBoundaryDeriv[i];
-    for (int i = 0; i < 10; i++) d2a[i] = (float)kD2Interior[i];
-    (void)hipMemcpyToSymbolAsync(HIP_SYMBOL(cD1I), kD1InteriorF, sizeof(kD1InteriorF), 0, hipMemcpyHostToDevice, s);
-    (void)hipMemcpyToSymbolAsync(HIP_SYMBOL(cD2I), kD2Interior24, sizeof(kD2Interior24), 0, hipMemcpyHostToDevice, s);
-    (void)hipMemcpyToSymbolAsync(HIP_SYMBOL(cD1A), d1a, sizeof(d1a), 0, hipMemcpyHostToDevice, s);
-    (void)hipMemcpyToSymbolAsync(HIP_SYMBOL(cD2A), d2a, sizeof(d2a), 0, hipMemcpyHostToDevice, s);
-    (void)hipMemcpyToSymbolAsync(HIP_SYMBOL(cSC), sc, sizeof(sc), 0, hipMemcpyHostToDevice, s);
-    (void)hipStreamSynchronize(s);
+    Row<N> r{};
+    for (int i = 0; i < N; i++) r.c[i] = (float)v[i];
+    return r;
 }
-
+constexpr Row<2> kD1A = rounded(kD1Interior);
+constexpr Row<10> kD2A = rounded(kD2Interior);
+constexpr Row<4> kSC = rounded(kBoundaryDeriv);
 
 // ---------------------------------------------------------------------------
 // Tile geometry.  x: tiles of TX columns; z: tiles of 64 cells aligned on quads.  The
@@ -128,7 +125,7 @@ __device__ __forceinline__ void unpack(float4 v, float* d)
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ float d1_int(const float* p, int s)
 {
-    return cD1I[0] * (p[s] - p[-s]) + cD1I[1] * (p[2 * s] - p[-2 * s]);
+    return kD1InteriorF[0] * (p[s] - p[-s]) + kD1InteriorF[1] * (p[2 * s] - p[-2 * s]);
 }
 
 // Closure row R of D1 from the edge point q along stride st, with the coefficients as
@@ -178,11 +175,11 @@ __device__ __forceinline__ W5 d2_weights(const float* pc, int s)
 {
     const float fm2 = pc[-2 * s], fm1 = pc[-s], f0 = pc[0], fp1 = pc[s], fp2 = pc[2 * s];
     W5 w;
-    w.c = cD2I[0] * f0 + cD2I[1] * (fm1 + fp1) + cD2I[2] * (fm2 + fp2);
-    w.m1 = cD2I[3] * fm2 + cD2I[4] * fm1 + cD2I[5] * f0 + cD2I[6] * fp1;
-    w.p1 = cD2I[3] * fp2 + cD2I[4] * fp1 + cD2I[5] * f0 + cD2I[6] * fm1;
-    w.m2 = cD2I[7] * fm2 + cD2I[8] * fm1 + cD2I[9] * f0;
-    w.p2 = cD2I[7] * fp2 + cD2I[8] * fp1 + cD2I[9] * f0;
+    w.c = kD2Interior24[0] * f0 + kD2Interior24[1] * (fm1 + fp1) + kD2Interior24[2] * (fm2 + fp2);
+    w.m1 = kD2Interior24[3] * fm2 + kD2Interior24[4] * fm1 + kD2Interior24[5] * f0 + kD2Interior24[6] * fp1;
+    w.p1 = kD2Interior24[3] * fp2 + kD2Interior24[4] * fp1 + kD2Interior24[5] * f0 + kD2Interior24[6] * fm1;
+    w.m2 = kD2Interior24[7] * fm2 + kD2Interior24[8] * fm1 + kD2Interior24[9] * f0;
+    w.p2 = kD2Interior24[7] * fp2 + kD2Interior24[8] * fp1 + kD2Interior24[9] * f0;
     return w;
 }
 
@@ -2421,7 +2418,7 @@ static_assert(kAcTX * (kAcTZ / 4) == kThreads, "one quad per thread");
 // written out
 __device__ __forceinline__ float ac_bnd(float u0, float u1, float u2, float u3)
 {
-    return __builtin_fmaf(cSC[3], u3, __builtin_fmaf(cSC[2], u2, __builtin_fmaf(cSC[0], u0, cSC[1] * u1)));
+    return __builtin_fmaf(kSC.c[3], u3, __builtin_fmaf(kSC.c[2], u2, __builtin_fmaf(kSC.c[0], u0, kSC.c[1] * u1)));
 }
 // d2_apply and d2_weights with the order of their roundings written out, so that the results do
 // not depend on how the compiler contracts the expressions around them.  The orders, and where each
@@ -2448,11 +2445,11 @@ __device__ __forceinline__ W5 ac_weights(float m2, float m1, float f0, float p1,
     };
     W5 w;
     const float s = m1 + p1;
-    w.c = fma(cD2A[2], m2 + p2, sf ? fma(cD2A[0], f0, cD2A[1] * s) : fma(cD2A[1], s, cD2A[0] * f0));
-    w.m1 = fma(cD2A[6], p1, fma(cD2A[5], f0, two(MN, cD2A[3], m2, cD2A[4], m1)));
-    w.p1 = fma(cD2A[6], m1, fma(cD2A[5], f0, two(PN, cD2A[3], p2, cD2A[4], p1)));
-    w.m2 = fma(cD2A[9], f0, two(MN, cD2A[7], m2, cD2A[8], m1));
-    w.p2 = fma(cD2A[9], f0, two(PN, cD2A[7], p2, cD2A[8], p1));
+    w.c = fma(kD2A.c[2], m2 + p2, sf ? fma(kD2A.c[0], f0, kD2A.c[1] * s) : fma(kD2A.c[1], s, kD2A.c[0] * f0));
+    w.m1 = fma(kD2A.c[6], p1, fma(kD2A.c[5], f0, two(MN, kD2A.c[3], m2, kD2A.c[4], m1)));
+    w.p1 = fma(kD2A.c[6], m1, fma(kD2A.c[5], f0, two(PN, kD2A.c[3], p2, kD2A.c[4], p1)));
+    w.m2 = fma(kD2A.c[9], f0, two(MN, kD2A.c[7], m2, kD2A.c[8], m1));
+    w.p2 = fma(kD2A.c[9], f0, two(PN, kD2A.c[7], p2, kD2A.c[8], p1));
     return w;
 }
 
@@ -2658,7 +2655,7 @@ __device__ __forceinline__ void ac_d1x(const AcousticArgs& a, const float* u, co
 #pragma unroll
             for (int c = 0; c < 4; c++) unpack(ld4(&f[w + (c < 2 ? c - 2 : c - 1) * AcShape<EDGE>::WZ]), X[c]);
 #pragma unroll
-            for (int k = 0; k < 4; k++) d[k] = cD1A[0] * (X[2][k] - X[1][k]) + cD1A[1] * (X[3][k] - X[0][k]);
+            for (int k = 0; k < 4; k++) d[k] = kD1A.c[0] * (X[2][k] - X[1][k]) + kD1A.c[1] * (X[3][k] - X[0][k]);
         };
         d1x(u, du);
         d1x(v, dv);
@@ -2886,8 +2883,8 @@ __device__ __forceinline__ void astep_tile(const AcousticArgs& a, int tix, int t
             ac_d1x<EDGE>(a, U, F, w, gx, tb, ax, fx);
 #pragma unroll
             for (int k = 0; k < 4; k++) {
-                az[k] = (cD1A[0] * (Uc[5 + k] - Uc[3 + k]) + cD1A[1] * (Uc[6 + k] - Uc[2 + k])) * a.rdz;
-                fz[k] = (cD1A[0] * (Fc[5 + k] - Fc[3 + k]) + cD1A[1] * (Fc[6 + k] - Fc[2 + k])) * a.rdz;
+                az[k] = (kD1A.c[0] * (Uc[5 + k] - Uc[3 + k]) + kD1A.c[1] * (Uc[6 + k] - Uc[2 + k])) * a.rdz;
+                fz[k] = (kD1A.c[0] * (Fc[5 + k] - Fc[3 + k]) + kD1A.c[1] * (Fc[6 + k] - Fc[2 + k])) * a.rdz;
             }
             if (EDGE && ntop + nbot > 0) {
                 float c[4], d[4];
@@ -3065,8 +3062,8 @@ __global__ void __launch_bounds__(kThreads, 5) k_agrad(const AcousticArgs a)
             const float f = Fc[4 + k];
             const float d2 = a.mode == 0 ? fp[k] - 2.f * f + fm[k] : (a.mode == 1 ? fp[k] - f : -f + fm[k]);
             gk[k] -= kw[k] * Ac[4 + k] * d2;
-            az[k] = (cD1A[0] * (Ac[5 + k] - Ac[3 + k]) + cD1A[1] * (Ac[6 + k] - Ac[2 + k])) * a.rdz;
-            fz[k] = (cD1A[0] * (Fc[5 + k] - Fc[3 + k]) + cD1A[1] * (Fc[6 + k] - Fc[2 + k])) * a.rdz;
+            az[k] = (kD1A.c[0] * (Ac[5 + k] - Ac[3 + k]) + kD1A.c[1] * (Ac[6 + k] - Ac[2 + k])) * a.rdz;
+            fz[k] = (kD1A.c[0] * (Fc[5 + k] - Fc[3 + k]) + kD1A.c[1] * (Fc[6 + k] - Fc[2 + k])) * a.rdz;
         }
         ac_d1x<true>(a, A, F, w, gx, tb, ax, fx);
         if (ntop + nbot > 0) {
