@@ -347,10 +347,10 @@ struct Engine {
 
     // D2 closure rows of the model (layout in StepArgs: wx[, wxx], wz): the weight of field
     // point j in row r is the sum over the table's entries (r, j, k) of coefficient times
-    // model value at point k, formed in double, times 1 / h^2.  Row 0 of a side with a boundary
-    // condition takes the SAT's boundary derivative, -1 / (H0 h) c S u, with it: the two cancel to
-    // a tenth of either, and rounded apart they left the free surface with an error of its own at
-    // every step.
+    // model value at point k, formed in double, times 1 / h^2.  Row 0 takes the SAT's boundary
+    // derivative, -1 / (H0 h) c S u, with it (every side has a free surface or absorbs): the two
+    // cancel to a tenth of either, and rounded apart they left the free surface with an error of
+    // its own at every step.
     void build_closures(const float* m)
     {
         const int nx = g.nx, nz = g.nz;
@@ -359,7 +359,6 @@ struct Engine {
         const long long nc = (long long)nx * nz;
         const double rdx2 = 1.0 / (g.dx * g.dx), rdz2 = 1.0 / (g.dz * g.dz);
         std::vector<double> acc(nz);
-        const int bcx[2] = {g.bc_left, g.bc_right}, bcz[2] = {g.bc_top, g.bc_bottom};
         double sat[8] = {};
         for (int j = 0; j < 4; j++) sat[j] = -kBoundaryDeriv[j] / kH0;
         for (int f = 0; f < (vti ? 2 : 1); f++) {
@@ -377,7 +376,7 @@ struct Engine {
                         for (const D2Entry& e : kD2ClosureNZ)
                             if (e.row == r && e.point == j)
                                 add(e.num / e.den, (long long)(side ? nx - 1 - e.coef : e.coef) * nz);
-                        if (r == 0 && bcx[side] != 0) add(sat[j], (long long)(side ? nx - 1 : 0) * nz);
+                        if (r == 0) add(sat[j], (long long)(side ? nx - 1 : 0) * nz);
                         float* o = w.data() + f * nwx + ((size_t)(side * 6 + r) * 8 + j) * ldz;
                         for (int iz = 0; iz < nz; iz++) o[iz] = (float)(acc[iz] * rdx2);
                     }
@@ -390,8 +389,7 @@ struct Engine {
                 const float* p = mu + (long long)ix * nz + (side ? nz - 1 : 0);
                 for (const D2Entry& e : kD2ClosureNZ)
                     v[e.point][e.row] += e.num / e.den * p[side ? -(int)e.coef : e.coef];
-                if (bcz[side] != 0)
-                    for (int j = 0; j < 8; j++) v[j][0] += sat[j] * p[0];
+                for (int j = 0; j < 8; j++) v[j][0] += sat[j] * p[0];
                 for (int j = 0; j < 8; j++)
                     for (int r = 0; r < 6; r++) wz[(((size_t)side * nx + ix) * 6 + r) * 8 + j] = (float)(v[j][r] * rdz2);
             }

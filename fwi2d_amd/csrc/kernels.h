@@ -66,8 +66,8 @@ struct StepArgs {
     const float *mux, *lamx;  // VTI: (1 + 2 eps) mu, (1 + 2 eps) lambda
     // D2 closure rows of the model, times 1 / h^2: x columns 0-5 from the left and right
     // [2 sides][6 columns][8 points][ldz] for mu (wx) and, VTI, (1 + 2 eps) mu (wxx); z rows
-    // 0-5 from the top and bottom [2 sides][nx][6 rows][8 points] for mu.  Row 0 of a side with a
-    // boundary condition includes its SAT's boundary derivative
+    // 0-5 from the top and bottom [2 sides][nx][6 rows][8 points] for mu.  Row 0 includes the
+    // SAT's boundary derivative
     const float *wx, *wxx, *wz;
     const float *div_tb;   // [2 sides][2 comps][nx] absorbing divisors, top then bottom
     const float *div_lr;   // [2 sides][2 comps][ldz]

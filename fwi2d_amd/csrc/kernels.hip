@@ -271,7 +271,9 @@ __device__ __forceinline__ void out_quad(const TileInfo& t, int i, int& gx, int&
     z0 = t.sz + 4 * (i % S::QC);
 }
 
-// D1 rows 0-5 on points 0-7 in LDS (rows 4 and 5 are interior rows), row stride rs
+// D1 rows 0-5 on points 0-7 in LDS (rows 4 and 5 are interior rows), row stride rs; the step's
+// table holds as row kSatRow the row 0 of the products, with the SAT terms' share (see z_cell)
+constexpr int kSatRow = 6;
 struct EdgeTable {
     float* c;
     int rs;
@@ -320,9 +322,10 @@ __device__ __forceinline__ void load_col12(const float* base, int i, float* c)
 }
 
 // D1 rows 0-5 from a side on the 8 points next to it: four closure rows and the first two
-// interior ones
+// interior ones; then the products' row 0, whose first coefficient -24/17 the SAT terms turn into
+// 24/17 (+ 1 / H0)
 struct EdgeD1 {
-    float c[48];
+    float c[56];
 };
 constexpr EdgeD1 edge_d1_table()
 {
@@ -335,6 +338,7 @@ constexpr EdgeD1 edge_d1_table()
         t.c[8 * r + r + 1] = kD1InteriorF[0];
         t.c[8 * r + r + 2] = kD1InteriorF[1];
     }
+    for (int j = 0; j < 8; j++) t.c[8 * kSatRow + j] = j ? t.c[j] : -t.c[0];
     return t;
 }
 __constant__ EdgeD1 cEdgeD1 = edge_d1_table();
@@ -603,9 +607,7 @@ __device__ __forceinline__ void z_cell_run(const StepArgs& a, const StepSmem& sm
     const int w = (e.gx - t.wsx) * S::WZ + (edge - t.wsz);  // the boundary cell
     const int q = (e.gx - t.plx) * S::PZ + (edge - t.pz0);
     float c[8], ux[8], uz[8], v[8];
-    edge_coefficients(sm.tb, e.r, c);
-    const int bc = e.bot ? a.bc_bottom : a.bc_top;
-    if (e.r == 0 && bc != 0) c[0] = -c[0];
+    edge_coefficients(sm.tb, e.r ? e.r : kSatRow, c);
     edge_cells<8>(&sm.ux[w], e.bot, ux);
     edge_cells<8>(&sm.uz[w], e.bot, uz);
     float d2x = 0.f, d2z = 0.f, dp = 0.f, dq = 0.f;
@@ -622,7 +624,7 @@ __device__ __forceinline__ void z_cell_run(const StepArgs& a, const StepSmem& sm
     for (int j = 0; j < 8; j++) dq += c[j] * v[j];
     const float sg = e.bot ? -a.rdz : a.rdz;
     float rx = d2x + sg * dq, rz = 2.f * d2z + sg * dp;
-    if (e.r == 0 && bc == 2) {
+    if (e.r == 0 && (e.bot ? a.bc_bottom : a.bc_top) == 2) {
         const float mu0 = sm.mu[w];
         rx += a.sat_z * ((0.5f * sqrtf(mu0 * e.rho)) * e.prx / a.dt);
         rz += a.sat_z * ((0.5f * sqrtf((e.lam + 2.f * mu0) * e.rho)) * e.prz / a.dt);
@@ -715,14 +717,14 @@ __device__ __forceinline__ void rhs_quad(const StepArgs& a, const StepSmem& sm, 
         const EdgeRow e = edge_row(gx, nx, 1);
         const size_t wo = (size_t)((gx >= 6 ? 6 : 0) + e.r) * 8 * a.ldz + z0;
         const float *W = a.wx + wo, *WX = VTI ? a.wxx + wo : W;
+        const float* crow = sm.tb.c + sm.tb.rs * (e.r ? e.r : kSatRow);
         float d2u[4], d2z[4], dp[4], dq[4];
 #pragma unroll
         for (int k = 0; k < 4; k++) d2u[k] = d2z[k] = dp[k] = dq[k] = 0.f;
 #pragma unroll 2
         for (int j = 0; j < 8; j++) {
             const int o = e.o + j * e.st;
-            float c = sm.tb.c[sm.tb.rs * e.r + j];
-            if (j == 0 && e.r == 0 && (gx ? a.bc_right : a.bc_left) != 0) c = -c;  // with the SAT's share
+            const float c = crow[j];
             float wj[4], xj[4], U[4], Z[4];
             unpack(ld4(W + (size_t)j * a.ldz), wj);
             if (VTI) unpack(ld4(WX + (size_t)j * a.ldz), xj);
@@ -1286,7 +1288,7 @@ __device__ __forceinline__ void step_tile(const StepArgs& a, const StepSmem& sm,
             has_z = z_cell<S>(a, t, ztid, top, bot, pux, nxz, zc);
         }
         __syncthreads();  // the previous shot is done with the LDS state and products
-        if (EDGE && VTI && shot == s0 && tid < 48)
+        if (EDGE && VTI && shot == s0 && tid < 56)
             sm.tb.c[sm.tb.rs * (tid >> 3) + (tid & 7)] = cEdgeD1.c[tid];
         const float* cux = a.curr + shot * a.shot_stride;
 #pragma unroll
@@ -1589,7 +1591,7 @@ __global__ void __launch_bounds__(kThreads, step_waves(VTI, TX, IMG)) k_step(con
     __shared__ __attribute__((aligned(16))) float sQz[S::IX * S::PZ];
     // frame tiles' D1 table; VTI: in the (1 + 2 eps) mu window, for the 42 LDS granules that
     // leave 3 workgroups per CU
-    __shared__ __attribute__((aligned(16))) float sT[VTI ? 4 : 48];
+    __shared__ __attribute__((aligned(16))) float sT[VTI ? 4 : 56];
     StepSmem sm{sUx, sUz, sMu, sMuX, sPx, sPz, sQx, sQz, {sT, 8}};
 
     const int nin_x = a.itx1 - a.itx0, nin_z = a.itz1 - a.itz0;
@@ -1598,7 +1600,7 @@ __global__ void __launch_bounds__(kThreads, step_waves(VTI, TX, IMG)) k_step(con
     const int b = blockIdx.x;
     if (b < ne8) {
         if (b >= ne) return;  // padding: the whole workgroup leaves before any barrier
-        if (!VTI && threadIdx.x < 48) sT[threadIdx.x] = cEdgeD1.c[threadIdx.x];  // read after the first barrier
+        if (!VTI && threadIdx.x < 56) sT[threadIdx.x] = cEdgeD1.c[threadIdx.x];  // read after the first barrier
         // frame: the rows of tiles above and below the rectangle, then its side columns
         const int lin = xcd_remap(b, ne);
         const int tile = lin / a.ngroups_e, grp = lin - tile * a.ngroups_e;
