@@ -2232,16 +2232,18 @@ static void step_launch(const StepArgs& a, bool image, int ncell, hipStream_t s)
     const int nin = (a.itx1 - a.itx0) * (a.itz1 - a.itz0), ne = (a.ntx * a.ntz - nin) * a.ngroups_e;
     const int nstep = ((ne + 7) & ~7) + nin * a.ngroups;
     const int nrec = a.rec_trace ? (2 * a.nrec + kThreads - 1) / kThreads : 0;
-    // Point sources and receivers: in the step's launch below 4096 tiles x shots (where the automatic
-    // groups hold one shot), which saves a launch of 3 us: us a step with them in the launch and
-    // in one of their own,
+    // Point sources and receivers: in the step's launch below 6144 tiles x shots (24 a CU), which saves
+    // a launch of 3 us: us a step with them in the launch and in one of their own,
     //   201 x 601, 1 shot (152 tiles x shots)   11.4  14.8     500 x 1700, 2 (1712)    20.3  22.6
     //   200 x 800, 10 shots (2000)              24.2  27.4     the same, VTI (2000)    32.4  35.2
-    //   200 x 800, 20 shots (4000)              42.2  45.0     the same, VTI (4000)    57.0  59.2
-    // Far above, the step kernel without their code gains more from its registers: 64 shots of
-    // 500 x 1700 (54784) 445 and 397 us.
+    //   100 x 1200, 30 (4500)                   56.8  65.7     the same, VTI (4500)    68.0  77.3
+    //   500 x 1700, 6 (5136)                    42.1  42.3     the same, VTI (5136)    55.5  57.6
+    // Above, the step kernel without their code gains more from its registers, most where tiles
+    // are interior ones: 500 x 1700, 12 shots (10272) 89.4 and 79.2 us, VTI 113.6 and 112.6; a
+    // gradient of 200 steps on 200 x 800, 48 shots (9600), 71.6 and 69.6 ms, of 100 x 1200, 60
+    // (9000), 94.1 and 93.0 ms.
     if constexpr (TX == 16) {
-        if ((long long)a.ntx * a.ntz * a.nshots < 4096) {
+        if ((long long)a.ntx * a.ntz * a.nshots < 6144) {
             const dim3 grid(nstep + nrec);
             if (image) hipLaunchKernelGGL((k_step<VTI, TX, true, true>), grid, dim3(kThreads), 0, s, a);
             else hipLaunchKernelGGL((k_step<VTI, TX, false, true>), grid, dim3(kThreads), 0, s, a);

@@ -1,6 +1,6 @@
 """Batches past the sizes at which the step changes its form: acoustic levels streamed past the caches
-(three levels above 256 MiB), elastic steps of 4096 tiles x shots and more, whose point sources and
-receivers run in a launch of their own.  Three shots of the batch against the FP64 oracle (the other
+(three levels above 256 MiB), elastic steps of several shots per workgroup, and of 6144 tiles x
+shots and more, whose point sources and receivers run in a launch of their own.  Three shots of the batch against the FP64 oracle (the other
 shots' adjoint sources are zero, so the gradient is the three shots'), with the engines'
 tolerances: traces within twice the FP32 gap of the oracle itself (at least 1e-5), gradients within
 1e-4.  The same three shots alone, which take the other form, agree too: the acoustic traces bit for
@@ -61,13 +61,14 @@ def test_acoustic_streamed_levels(lib, orc64, orc32):
     assert rel(ga, g.astype(np.float64)) <= 1e-6  # the same terms, the shots summed in other groups
 
 
+# 9 x 3 tiles: 4131 and 6183 tiles x shots, groups of 2 and 3 shots, the last of 1
 @pytest.mark.parametrize("vti", [False, True])
-def test_elastic_points_in_their_own_launch(lib, orc64, orc32, vti):
-    ns = 153  # 9 x 3 tiles: 4131 tiles x shots, groups of 2 shots, the last of 1
+@pytest.mark.parametrize("ns, group", [(153, 2), (229, 3)])
+def test_elastic_points_in_their_own_launch(lib, orc64, orc32, vti, ns, group):
     prob, model, sxz, rxz, src, nt, dt = el.engine_case(nx=130, nz=150, nt=240, ns=ns, vti=vti)
     rxz = [r[:12 + s % 5] for s, r in enumerate(rxz)]
     src = np.stack([np.stack([W.ricker(nt, dt, 20.0 + s % 7) * a for s in range(ns)]) for a in (0.3, 1.0)])
-    pick = [0, 77, 152]
+    pick = [0, 77, ns - 1]
     tr = pick_traces(rxz, pick)
     few = (prob, model, sxz[pick], [rxz[s] for s in pick], src[:, pick], nt, dt)
     adj = np.zeros((2, sum(len(r) for r in rxz), nt), np.float32)
@@ -80,7 +81,7 @@ def test_elastic_points_in_their_own_launch(lib, orc64, orc32, vti):
     for fused in (0, 1):
         e, out = el.run_engine(lib, prob, model, sxz, rxz, src, nt, dt, sub=1, keep=True,
                                options=(("image_fused", fused),))
-        assert e.stat("ntiles") * ns >= 4096 and e.stat("shots_per_block") == 2
+        assert e.stat("ntiles") * ns  == 27 * ns and e.stat("shots_per_block") == group
         assert e.stat("image_fused") == fused
         g = e.adjoint(adj)
         e.close()
