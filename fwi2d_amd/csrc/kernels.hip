@@ -233,11 +233,11 @@ __device__ __forceinline__ float d2_apply(const W5& w, const float* pu, int s)
 //     the way and do not spread, and they were nearly the whole error: 14 rows in FP64 bring a
 //     one-shot gradient of 1500 steps from 4.8e-6 to 2.3e-7 off FP64.  With the carry such
 //     gradients are 1.0 to 1.3e-6 off, 3.0 to 7.0e-6 without.  16 rows are 3% of 500: a step of
-//     64 shots takes 397 instead of 394 us, of one on 201 x 601 11.4 instead of 11.1 us.
+//     64 shots takes 391.5 instead of 389.6 us, of one on 201 x 601 11.1 us with or without.
 // The instance-per-row form this replaced (34-60 KB of code per kernel, edge bands beside a
 // core launch) was bound by instruction fetch: one band workgroup took 30 us alone, and a
 // step of one shot on 201 x 601 cells 105 us; it takes 11 us in this form (one launch), and
-// 64 shots of 500 x 1700 394 us instead of 407.  A frame tile costs more than an interior one
+// 64 shots of 500 x 1700 392 us instead of 407.  A frame tile costs more than an interior one
 // in VALU work (at first 1209 against 527 vector instructions per wavefront and shot, most of
 // the surplus addresses), so it loads per shot what its passes need and keeps no D2 weights:
 // spills cost it more than both.
@@ -2234,14 +2234,14 @@ static void step_launch(const StepArgs& a, bool image, int ncell, hipStream_t s)
     const int nrec = a.rec_trace ? (2 * a.nrec + kThreads - 1) / kThreads : 0;
     // Point sources and receivers: in the step's launch below 6144 tiles x shots (24 a CU), which saves
     // a launch of 3 us: us a step with them in the launch and in one of their own,
-    //   201 x 601, 1 shot (152 tiles x shots)   11.4  14.8     500 x 1700, 2 (1712)    20.3  22.6
-    //   200 x 800, 10 shots (2000)              24.2  27.4     the same, VTI (2000)    32.4  35.2
-    //   100 x 1200, 30 (4500)                   56.8  65.7     the same, VTI (4500)    68.0  77.3
-    //   500 x 1700, 6 (5136)                    42.1  42.3     the same, VTI (5136)    55.5  57.6
+    //   201 x 601, 1 shot (152 tiles x shots)   11.1  14.8     500 x 1700, 2 (1712)    20.1  22.3
+    //   200 x 800, 10 shots (2000)              23.6  26.6     the same, VTI (2000)    31.6  34.8
+    //   100 x 1200, 30 (4500)                   56.5  66.1     the same, VTI (4500)    68.5  78.1
+    //   500 x 1700, 6 (5136)                    42.2  42.7     the same, VTI (5136)    55.7  58.1
     // Above, the step kernel without their code gains more from its registers, most where tiles
-    // are interior ones: 500 x 1700, 12 shots (10272) 89.4 and 79.2 us, VTI 113.6 and 112.6; a
-    // gradient of 200 steps on 200 x 800, 48 shots (9600), 71.6 and 69.6 ms, of 100 x 1200, 60
-    // (9000), 94.1 and 93.0 ms.
+    // are interior ones: 500 x 1700, 12 shots (10272) 89.7 and 78.3 us, VTI 113.7 and 113.2, 64
+    // shots 446 and 391 us; a gradient of 200 steps on 200 x 800, 48 shots (9600), 71.6 and
+    // 69.6 ms, of 100 x 1200, 60 (9000), 94.1 and 93.0 ms.
     if constexpr (TX == 16) {
         if ((long long)a.ntx * a.ntz * a.nshots < 6144) {
             const dim3 grid(nstep + nrec);
@@ -2932,11 +2932,11 @@ __device__ __forceinline__ void astep_tile(const AcousticArgs& a, int tix, int t
 // frame's block count rounded up to a multiple of 8, the extra blocks idle) and remapped
 // within its class so that an XCD runs neighbouring tiles; then the receivers of the current
 // level.
-// Bound by memory latency: 12 B per shot-cell (16 imaged) at 4.1 (3.3) TB/s for 64 shots of
-// 500 x 1700, 159 us a step and 266 us an imaged one.  The form before (loads through
-// registers, the frame's cells dealt one per thread with one code instance per closure row, a
-// launch of its own for the imaging, the points and each kept level) took 208 us a step, 299 us
-// an imaging launch and 78 us a copy.  Waves per SIMD: scratch reloads in the shot loop wait for
+// Bound by HBM: 64 shots of 500 x 1700 move 0.89 GB in 158 us a step (5.6 TB/s; 0.66 GB without
+// the windows' halos) and 1.30 GB in 269 us an imaged one (4.8 TB/s); a large copy reaches 4.9 TB/s.
+// The form before (loads through registers, the frame's cells dealt one per thread with one code
+// instance per closure row, a launch of its own for the imaging, the points and each kept level)
+// took 208 us a step, 299 us an imaging launch and 78 us a copy.  Waves per SIMD: scratch reloads in the shot loop wait for
 // the windows in flight, so the bounds are the tightest ones that do not spill there (5 and 4
 // instead: 246 and 650 us); what the frame spills costs 1%.  Streamed levels (stream): 151
 // instead of 168 us above the memory-side cache's size, 2 to 12% slower below it.
