@@ -725,16 +725,17 @@ struct Engine {
         int K = opt_segment > 0 ? opt_segment : (int)std::ceil(std::sqrt(2.0 * nsnap));
         K = std::max(1, std::min(K, nsnap));
         if (opt_segment == 0 && opt_ckpt_budget_mb > 0) {
-            // the longest segments whose checkpoints (2 levels per segment after the first)
-            // and snapshot slots (K + 2 levels) fit the budget: the last segment is kept
+            // the longest segments whose checkpoints (2 levels and the carry of the rows below a
+            // free surface per segment after the first) and snapshot slots (K + 2 levels) fit the budget: the last segment is kept
             // whole by the forward run, so every snapshot beyond the first nsnap - K is
             // never recomputed
             const double level = (double)state_stride() * sizeof(float);
             const double ck_level = (double)state_stride() * (opt_bf16 ? 2 : 4);
+            const double ck_carry = (double)carry_stride() * sizeof(float);
             const double budget = (double)opt_ckpt_budget_mb * 1048576.0;
             for (int k = nsnap; k > K; k--) {
                 const int nseg_k = (nsnap + k - 1) / k;
-                if (2.0 * (nseg_k - 1) * ck_level + (k + 2.0) * level <= budget) {
+                if ((nseg_k - 1) * (2.0 * ck_level + ck_carry) + (k + 2.0) * level <= budget) {
                     // the same number of segments of balanced length, so that the last one
                     // (kept whole) is not a short remainder
                     K = (nsnap + nseg_k - 1) / nseg_k;
@@ -890,7 +891,7 @@ struct Engine {
     }
 
     // Step-shape autotuner: times a few forward steps of the current shots for every
-    // (tile_x, shots per core workgroup, shots per edge workgroup) and keeps the fastest.
+    // (tile_x, shots per interior workgroup, shots per frame workgroup) and keeps the fastest.
     // Forward results do not depend on the choice (bit for bit); gradients only through
     // the order in which a workgroup sums its shots.
     void autotune(const float* dsrc)
